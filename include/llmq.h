@@ -124,6 +124,20 @@ int llmq_wq_gemv_batched_fused(const void* x, int64_t x_row_stride, const void* 
 int llmq_moe_combine(const void* rows_out, const int64_t* order, const void* weights, void* final_out,
                      int n_rows, int top_k, int n_tokens, int width, int dtype, llmq_stream_t stream);
 
+/* A whole gated experts block over many tokens (KernelQuantExperts.forward, kernel.py:216-289, which walks the experts
+ * one at a time beyond a few tokens): out[t] = sum over t's experts e of weight * down_e(silu(gate_e(x_t)) * up_e(x_t)),
+ * rounded to `dtype` (fp16 / bf16) after each projection, activation, product, weighted row and addition (added in the
+ * order of the experts). Groups of 128, one scale per weight row; gate_up: [experts, 2 I, H/128, ..], gate rows first;
+ * down: [experts, H, I/128, ..]; x, out: [tokens, H]; top_k_index, top_k_weights: [tokens, top_k]. An expert id outside
+ * the stack counts as the nearest valid one. `supported`: hidden and intermediate whole groups, up to 1024 experts,
+ * 256 experts a token, activations and one expert's weight below 4 GiB. */
+int llmq_wq_experts_supported(int n_tokens, int top_k, int n_experts, int hidden, int intermediate);
+size_t llmq_wq_experts_workspace_bytes(int n_tokens, int top_k, int n_experts, int hidden, int intermediate);
+int llmq_wq_experts(const void* x, const int64_t* top_k_index, const void* top_k_weights, const void* gate_up,
+                    const float* gate_up_scale, const void* down, const float* down_scale, void* out,
+                    void* workspace, size_t workspace_bytes, int n_tokens, int top_k, int n_experts, int hidden,
+                    int intermediate, int wformat, int dtype, llmq_stream_t stream);
+
 /* The decode-step form of llmq_wq_gemv (M = 1, group size 128): the same product with the
  * elementwise operations that surround a Linear in a Llama decoder layer folded in, so that a
  * layer is five launches instead of ~40. There is no counterpart in the reference, which leaves

@@ -465,6 +465,52 @@ at::Tensor moe_combine(const at::Tensor& rows_out, const at::Tensor& order, cons
   return out;
 }
 
+// A whole gated experts block over many tokens (see llmq_wq_experts): x [tokens, hidden], top_k_index and
+// top_k_weights [tokens, top_k], the stacked weights as KernelQuantExperts stores them. Returns [tokens, hidden].
+at::Tensor wq_experts(const at::Tensor& x, const at::Tensor& top_k_index, const at::Tensor& top_k_weights,
+                      const at::Tensor& gate_up, const at::Tensor& gate_up_scale, const at::Tensor& down,
+                      const at::Tensor& down_scale) {
+  TORCH_CHECK(x.is_cuda() && top_k_index.is_cuda() && top_k_weights.is_cuda() && gate_up.is_cuda() &&
+                  gate_up_scale.is_cuda() && down.is_cuda() && down_scale.is_cuda(), "all tensors must be CUDA");
+  TORCH_CHECK(x.dim() == 2 && x.is_contiguous(), "x must be contiguous [tokens, hidden]");
+  TORCH_CHECK(gate_up.dim() == 4 && gate_up.is_contiguous() && down.dim() == 4 && down.is_contiguous() &&
+                  gate_up.scalar_type() == down.scalar_type() && gate_up.size(0) == down.size(0),
+              "the weights must be contiguous [experts, N, groups, group_size] of one format");
+  const bool packed = gate_up.scalar_type() == at::kByte;
+  TORCH_CHECK(packed || gate_up.scalar_type() == at::kChar, "weights must be int8, or uint8 for nibble-packed int4");
+  const int64_t E = gate_up.size(0), H = down.size(1), I = gate_up.size(1) / 2, per_byte = packed ? 2 : 1;
+  TORCH_CHECK(gate_up.size(3) * per_byte == 128 && down.size(3) * per_byte == 128, "the experts' GEMM needs group_size 128");
+  TORCH_CHECK(x.size(1) == H && gate_up.size(1) == 2 * I && gate_up.size(2) * 128 == H && down.size(2) * 128 == I,
+              "gate_up must be [experts, 2 I, H / 128, ...], down [experts, H, I / 128, ...] and x [tokens, H]");
+  auto scales = [&](const at::Tensor& s, const at::Tensor& w) {
+    return s.scalar_type() == at::kFloat && s.is_contiguous() && s.dim() == 3 && s.size(0) == w.size(0) &&
+           s.size(1) == w.size(1) && s.size(2) == w.size(2);
+  };
+  TORCH_CHECK(scales(gate_up_scale, gate_up) && scales(down_scale, down),
+              "scales must be contiguous float32 [experts, N, groups]");
+  const int64_t T = x.size(0), top_k = top_k_index.size(-1);
+  TORCH_CHECK(top_k_index.dim() == 2 && top_k_index.size(0) == T && at::isIntegralType(top_k_index.scalar_type(), false),
+              "top_k_index must hold integers, [tokens, top_k]");
+  TORCH_CHECK(top_k_weights.sizes() == top_k_index.sizes() && top_k_weights.scalar_type() == x.scalar_type(),
+              "top_k_weights must be [tokens, top_k] of x's dtype");
+  const int dtype = dtype_code(x, "x");
+  auto out = at::empty_like(x);
+  if (out.numel() == 0) return out;
+  const at::Tensor index = top_k_index.to(at::kLong).contiguous(), weights = top_k_weights.contiguous();
+  const int t = static_cast<int>(T), k = static_cast<int>(top_k), e = static_cast<int>(E), h = static_cast<int>(H),
+            i = static_cast<int>(I);
+  const c10::OptionalDeviceGuard guard(at::device_of(x));
+  const int64_t bytes = static_cast<int64_t>(llmq_wq_experts_workspace_bytes(t, k, e, h, i));
+  auto workspace = at::empty({bytes}, x.options().dtype(at::kByte));
+  check_rc(llmq_wq_experts(x.const_data_ptr(), index.const_data_ptr<int64_t>(), weights.const_data_ptr(),
+                           gate_up.const_data_ptr(), gate_up_scale.const_data_ptr<float>(), down.const_data_ptr(),
+                           down_scale.const_data_ptr<float>(), out.mutable_data_ptr(), workspace.mutable_data_ptr(),
+                           static_cast<size_t>(bytes), t, k, e, h, i, packed ? LLMQ_W_INT4_PACKED : LLMQ_W_INT8, dtype,
+                           current_stream(x)),
+           "wq_experts");
+  return out;
+}
+
 // One-row gate|up Linear of a gated MLP with act(gate) * up folded into the store (see
 // llmq_wq_gemv_gate_up_silu). qweight: [2I, groups, group_size], gate rows first; returns [1, I].
 at::Tensor wq_gemv_gate_up_silu(const at::Tensor& x, const at::Tensor& qweight, const at::Tensor& wscale,
@@ -1391,6 +1437,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("block_expert"), py::arg("block_row0"), py::arg("block_rows"), py::arg("act_pair"));
   m.def("moe_combine", &moe_combine, "Routing-weighted sum of the experts' rows per token",
         py::arg("rows_out"), py::arg("order"), py::arg("weights"), py::arg("n_tokens"));
+  m.def("wq_experts", &wq_experts, "A gated experts block over many tokens: plan, two grouped GEMMs, combination",
+        py::arg("x"), py::arg("top_k_index"), py::arg("top_k_weights"), py::arg("gate_up"), py::arg("gate_up_scale"),
+        py::arg("down"), py::arg("down_scale"));
+  m.def("wq_experts_supported", [](int64_t tokens, int64_t top_k, int64_t experts, int64_t hidden, int64_t intermediate) {
+    constexpr int64_t kMost = INT32_MAX;
+    return tokens <= kMost && top_k <= kMost && experts <= kMost && hidden <= kMost && intermediate <= kMost &&
+           llmq_wq_experts_supported(static_cast<int>(tokens), static_cast<int>(top_k), static_cast<int>(experts),
+                                     static_cast<int>(hidden), static_cast<int>(intermediate)) != 0;
+  }, py::arg("tokens"), py::arg("top_k"), py::arg("experts"), py::arg("hidden"), py::arg("intermediate"));
   m.def("route_plan", &route_plan, "Routing plan of the batched GEMV in one launch",
         py::arg("top_k_index"), py::arg("num_experts"), py::arg("limit"));
   m.def("route_plan_supported", [](int64_t rows, int64_t experts) {

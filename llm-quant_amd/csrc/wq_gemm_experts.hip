@@ -1,0 +1,294 @@
+// A Mixture-of-Experts block over a prompt (or a batch of sequences), gfx950: every token through the experts it is
+// routed to, five launches whatever the number of experts, nothing read back to the host.
+//
+// KernelQuantExperts.forward walks the experts one at a time for more than a few tokens
+// (llmquant/quantizers/kernel.py:216-289): per expert a nonzero / where on the routing mask (which the host waits
+// for), a gather of its rows, two projections, an index_add. For 300 tokens through 64 experts of 2048 x 1024 that is
+// 1180 launches and 7.7 ms around 0.2 GB of int4 codes.
+// Here:
+//   plan + prepare  one launch: a workgroup counts the rows of every expert and lists the row tiles (runs of up to BM
+//                   rows of one expert); the other workgroups put the tokens' rows in the tiled GEMM's prepared form
+//   gate|up         wq_gemm_a16_tile_kernel, GROUPED: a tile's rows are gathered by the transfers into LDS
+//                   (row -> token), its weight is its expert's; stores silu(gate) * up as the next GEMM's prepared rows
+//   down            the same kernel on those rows (now contiguous per expert)
+//   combine         per token, its rows times their routing weights, in the order of the experts
+// with the rounding points of the per-expert form: gate and up, silu(gate), silu(gate) * up, the down projection, each
+// weighted row and each partial sum are rounded to the activation dtype.
+//
+// Bound: the experts' codes (64 x 2048 x 1024 int4: 201 MB) for up to about 40 rows an expert, the tiled GEMM's rate
+// beyond. Measured, 64 experts, 8 a token, 2048 x 1024, bf16, us a pass, per-expert loop -> here: 300 tokens int4
+// 6970 -> 104; by kernel trace (with the profiler's overhead) at 12 / 60 / 300 / 600 tokens int4 the gate|up GEMM takes
+// 33.5 / 39 / 67 / 90 us (4.0 TB/s of codes at 12 tokens), down 18 / 21 / 36 / 48, the plan 5-11, the combination 6-8.
+#include "wq_gemm_a16_tile.h"
+
+namespace {
+
+constexpr int kPlanThreads = 512;
+constexpr int kMaxExperts = 1024;
+constexpr int kMaxTopK = 256;
+
+// The shapes: 256 columns (128 gate + 128 up rows of the weight make a whole group of the next reduction axis), rows by
+// what an expert gets. Two workgroups a CU where their stages fit (int4), so that one's first transfers and store run
+// under the other's multiplications: a tile is only 8 to 16 groups long here.
+using Rows32 = Shape<32, 8, 1, 2>;
+using Rows64 = Shape<64, 8, 1, 2>;
+using Rows32Whole = Shape<32, 8, 1, 1>;
+using Rows64Whole = Shape<64, 8, 1, 1>;
+
+struct PlanArgs {
+  const int64_t* expert_of_row;   // [n_rows] (token-major: row i is of token i / top_k)
+  int n_rows, n_experts, top_k, tile_rows;
+  int4* tiles;
+  int* n_tiles;
+  int* row_source;                // [n_rows]: sorted row -> token
+  int* sorted_of_row;             // [n_rows]: row -> sorted row
+};
+
+__device__ __forceinline__ int expert_id(int64_t raw, int n_experts) {
+  // an id outside the layer's experts is counted with the nearest valid one
+  return raw < 0 ? 0 : (raw >= n_experts ? n_experts - 1 : static_cast<int>(raw));
+}
+
+// Block 0: the plan. Where a row lands inside its expert's run depends on the order of the atomics; nothing downstream
+// does: a row's result does not depend on its neighbours, and the combination goes by expert and slot.
+// Other blocks: x -> prepared form, a lane per 16-byte chunk (act_prep_kernel's work).
+template <typename T>
+__global__ __launch_bounds__(kPlanThreads) void experts_plan_kernel(const PlanArgs p, const u32x4* __restrict__ x,
+                                                                    u32x4* __restrict__ xp, u32x4* __restrict__ rec,
+                                                                    const int64_t n_chunks) {
+  const int tid = threadIdx.x;
+  if (blockIdx.x > 0) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x - 1) * kPlanThreads + tid;
+    const bool active = i < n_chunks;  // n_chunks is a multiple of 16: a row of 16 lanes is active or idle as one
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (active) v = x[i];
+    emit_prepared<T>(v, active, (tid & 15) == 0, xp + (active ? i : 0), rec + (active ? i >> 4 : 0));
+    return;
+  }
+  __shared__ int s_count[kMaxExperts], s_first[kMaxExperts], s_tile[kMaxExperts];
+  for (int e = tid; e < p.n_experts; e += kPlanThreads) s_count[e] = 0;
+  __syncthreads();
+  for (int i = tid; i < p.n_rows; i += kPlanThreads) atomicAdd(&s_count[expert_id(p.expert_of_row[i], p.n_experts)], 1);
+  __syncthreads();
+  if (tid < kWave) {
+    // exclusive prefix sums of rows and of row tiles: a lane takes `per` experts in a row, then a scan over the lanes
+    const int per = (p.n_experts + kWave - 1) / kWave;
+    int rows = 0, tiles = 0;
+    for (int k = 0; k < per; ++k) {
+      const int e = tid * per + k;
+      if (e < p.n_experts) rows += s_count[e], tiles += (s_count[e] + p.tile_rows - 1) / p.tile_rows;
+    }
+    int row_end = rows, tile_end = tiles;
+#pragma unroll
+    for (int step = 1; step < kWave; step <<= 1) {
+      const int r = __shfl_up(row_end, step), t = __shfl_up(tile_end, step);
+      if (tid >= step) row_end += r, tile_end += t;
+    }
+    int row = row_end - rows, tile = tile_end - tiles;
+    for (int k = 0; k < per; ++k) {
+      const int e = tid * per + k;
+      if (e < p.n_experts) {
+        s_first[e] = row, s_tile[e] = tile;
+        row += s_count[e], tile += (s_count[e] + p.tile_rows - 1) / p.tile_rows;
+      }
+    }
+    if (tid == kWave - 1) *p.n_tiles = tile_end;
+  }
+  __syncthreads();
+  for (int e = tid; e < p.n_experts; e += kPlanThreads) {
+    const int count = s_count[e], first = s_first[e], tile = s_tile[e];
+    for (int done = 0, t = tile; done < count; done += p.tile_rows, ++t) {
+      p.tiles[t] = int4{e, first + done, min(p.tile_rows, count - done), 0};
+    }
+    s_count[e] = first;   // from here on: where the expert's next row goes
+  }
+  __syncthreads();
+  for (int i = tid; i < p.n_rows; i += kPlanThreads) {
+    const int at = atomicAdd(&s_count[expert_id(p.expert_of_row[i], p.n_experts)], 1);
+    p.row_source[at] = i / p.top_k;
+    p.sorted_of_row[i] = at;
+  }
+}
+
+// final[t] = the rows of token t, each times its routing weight, added up in the order of the experts (of the slots
+// where two are the same), every product and sum rounded to T. One workgroup per token, eight columns a thread and turn.
+template <typename T>
+__global__ __launch_bounds__(256) void experts_combine_kernel(const T* __restrict__ rows_out,
+                                                              const int64_t* __restrict__ expert_of_row,
+                                                              const int* __restrict__ sorted_of_row,
+                                                              const T* __restrict__ weights, T* __restrict__ final_out,
+                                                              const int top_k, const int n_experts, const int width) {
+  __shared__ int s_expert[kMaxTopK], s_row[kMaxTopK];
+  __shared__ float s_weight[kMaxTopK];
+  const int t = blockIdx.x, tid = threadIdx.x;
+  const int64_t first = static_cast<int64_t>(t) * top_k;
+  for (int k = tid; k < top_k; k += 256) s_expert[k] = expert_id(expert_of_row[first + k], n_experts);
+  __syncthreads();
+  for (int k = tid; k < top_k; k += 256) {
+    const int e = s_expert[k];
+    int rank = 0;
+    for (int j = 0; j < top_k; ++j) rank += s_expert[j] < e || (s_expert[j] == e && j < k);
+    s_row[rank] = sorted_of_row[first + k];
+    s_weight[rank] = llmq::to_float(weights[first + k]);
+  }
+  __syncthreads();
+  for (int c = tid * 8; c < width; c += 256 * 8) {
+    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int k = 0; k < top_k; ++k) {
+      float v[8];
+      Pack<T>::unpack(load16(rows_out + static_cast<int64_t>(s_row[k]) * width + c), v);
+      const float w = s_weight[k];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = round_through<T>(acc[e] + round_through<T>(v[e] * w));
+    }
+    store16(final_out + static_cast<int64_t>(t) * width + c, Pack<T>::pack(acc));
+  }
+}
+
+size_t aligned(size_t bytes) { return (bytes + 255) / 256 * 256; }
+
+struct Layout {
+  size_t xp, rec, act_xp, act_rec, rows_out, tiles, n_tiles, row_source, sorted, total;
+};
+
+Layout layout_for(int T, int top_k, int E, int H, int I) {
+  const size_t rows = static_cast<size_t>(T) * top_k;
+  const size_t max_tiles = rows / 32 + (rows < static_cast<size_t>(E) ? rows : E) + 1;   // (of the smallest tile)
+  Layout l{};
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t here = at;
+    at += aligned(bytes);
+    return here;
+  };
+  l.xp = take(static_cast<size_t>(T) * H * 2);
+  l.rec = take(static_cast<size_t>(T) * (H / kGroup) * 16);
+  l.act_xp = take(rows * I * 2);
+  l.act_rec = take(rows * (I / kGroup) * 16);
+  l.rows_out = take(rows * H * 2);
+  l.tiles = take(max_tiles * sizeof(int4));
+  l.n_tiles = take(sizeof(int));
+  l.row_source = take(rows * sizeof(int));
+  l.sorted = take(rows * sizeof(int));
+  l.total = at;
+  return l;
+}
+
+template <typename T, int BITS, int EPI, typename S>
+int launch_grouped(const TileArgs& a, int max_row_tiles, hipStream_t stream) {
+  auto kernel = wq_gemm_a16_tile_kernel<T, BITS, EPI, S, true>;
+  constexpr int kLds = S::template kLdsBytes<BITS>;
+  static bool raised = false;  // per instantiation; worst case two threads both set it
+  if (!raised) {
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (err != hipSuccess) {
+      llmq_host::set_error("raising the LDS limit failed: %s", hipGetErrorString(err));
+      return static_cast<int>(err);
+    }
+    raised = true;
+  }
+  const int work = max_row_tiles * a.n_tiles;
+  hipLaunchKernelGGL(kernel, dim3((work + 7) / 8 * 8), dim3(S::kThreads), kLds, stream, a);
+  return llmq_host::check_launch("wq_gemm_a16_tile_kernel (grouped)");
+}
+
+template <typename T, int BITS, typename S>
+int run_shape(const TileArgs& gate_up, const TileArgs& down, int max_row_tiles, hipStream_t stream) {
+  if (int rc = launch_grouped<T, BITS, kEpiGateUpSilu, S>(gate_up, max_row_tiles, stream)) return rc;
+  return launch_grouped<T, BITS, kEpiStore, S>(down, max_row_tiles, stream);
+}
+
+template <typename T, int BITS>
+int run(const void* x, const int64_t* index, const void* weights, const void* q1, const float* s1, const void* q2,
+        const float* s2, void* out, uint8_t* ws, int n_tokens, int top_k, int E, int H, int I, hipStream_t stream) {
+  const Layout l = layout_for(n_tokens, top_k, E, H, I);
+  const int rows = n_tokens * top_k;
+  // 64-row tiles from 40 rows an expert on: below, most 64-row tiles would be half empty
+  const int tile_rows = rows > 40 * E ? 64 : 32;
+  const PlanArgs p{index, rows, E, top_k, tile_rows, reinterpret_cast<int4*>(ws + l.tiles),
+                   reinterpret_cast<int*>(ws + l.n_tiles), reinterpret_cast<int*>(ws + l.row_source),
+                   reinterpret_cast<int*>(ws + l.sorted)};
+  const int64_t n_chunks = static_cast<int64_t>(n_tokens) * (H / 8);
+  const dim3 plan_grid(1 + static_cast<unsigned>((n_chunks + kPlanThreads - 1) / kPlanThreads));
+  hipLaunchKernelGGL(experts_plan_kernel<T>, plan_grid, dim3(kPlanThreads), 0, stream, p, static_cast<const u32x4*>(x),
+                     reinterpret_cast<u32x4*>(ws + l.xp), reinterpret_cast<u32x4*>(ws + l.rec), n_chunks);
+  if (int rc = llmq_host::check_launch("experts_plan_kernel")) return rc;
+
+  const int g1 = H / kGroup, g2 = I / kGroup;
+  TileArgs up{};
+  up.xp = ws + l.xp, up.rec = ws + l.rec, up.qw = static_cast<const uint8_t*>(q1), up.sw = s1;
+  up.M = rows, up.N = 2 * I, up.G = g1, up.n_tiles = I / 128, up.splits = 1, up.groups_per_split = g1;
+  up.next_xp = ws + l.act_xp, up.next_rec = ws + l.act_rec, up.next_G = g2;
+  up.tiles = p.tiles, up.n_row_tiles = p.n_tiles, up.row_source = p.row_source;
+  up.expert_codes = static_cast<int64_t>(2) * I * H * BITS / 8, up.expert_scales = static_cast<int64_t>(2) * I * g1;
+  TileArgs down{};
+  down.xp = ws + l.act_xp, down.rec = ws + l.act_rec, down.qw = static_cast<const uint8_t*>(q2), down.sw = s2;
+  down.out = ws + l.rows_out;
+  down.M = rows, down.N = H, down.G = g2, down.n_tiles = (H + 255) / 256, down.splits = 1, down.groups_per_split = g2;
+  down.tiles = p.tiles, down.n_row_tiles = p.n_tiles;
+  down.expert_codes = static_cast<int64_t>(H) * I * BITS / 8, down.expert_scales = static_cast<int64_t>(H) * g2;
+  const int max_row_tiles = rows / tile_rows + (rows < E ? rows : E);
+  int rc;
+  if constexpr (BITS == 4) {
+    rc = tile_rows == 32 ? run_shape<T, BITS, Rows32>(up, down, max_row_tiles, stream)
+                         : run_shape<T, BITS, Rows64>(up, down, max_row_tiles, stream);
+  } else {
+    rc = tile_rows == 32 ? run_shape<T, BITS, Rows32Whole>(up, down, max_row_tiles, stream)
+                         : run_shape<T, BITS, Rows64Whole>(up, down, max_row_tiles, stream);
+  }
+  if (rc) return rc;
+  hipLaunchKernelGGL(experts_combine_kernel<T>, dim3(n_tokens), dim3(256), 0, stream,
+                     reinterpret_cast<const T*>(ws + l.rows_out), index, p.sorted_of_row, static_cast<const T*>(weights),
+                     static_cast<T*>(out), top_k, E, H);
+  return llmq_host::check_launch("experts_combine_kernel");
+}
+
+}  // namespace
+
+extern "C" int llmq_wq_experts_supported(int n_tokens, int top_k, int n_experts, int hidden, int intermediate) {
+  if (n_tokens < 1 || top_k < 1 || top_k > kMaxTopK || n_experts < 1 || n_experts > kMaxExperts) return 0;
+  if (hidden < kGroup || intermediate < kGroup || hidden % kGroup || intermediate % kGroup) return 0;
+  // the GEMMs' 32-bit offsets: an activation, and one expert's weight
+  const uint64_t rows = static_cast<uint64_t>(n_tokens) * top_k, limit = 1ull << 32;
+  const uint64_t wide = hidden > intermediate ? hidden : intermediate;
+  if (rows * wide * 2 >= limit || rows > (1u << 24) || 2ull * hidden * intermediate >= limit) return 0;
+  return 1;
+}
+
+extern "C" size_t llmq_wq_experts_workspace_bytes(int n_tokens, int top_k, int n_experts, int hidden, int intermediate) {
+  if (!llmq_wq_experts_supported(n_tokens, top_k, n_experts, hidden, intermediate)) return 0;
+  return layout_for(n_tokens, top_k, n_experts, hidden, intermediate).total;
+}
+
+extern "C" int llmq_wq_experts(const void* x, const int64_t* top_k_index, const void* top_k_weights,
+                               const void* gate_up, const float* gate_up_scale, const void* down,
+                               const float* down_scale, void* out, void* workspace, size_t workspace_bytes,
+                               int n_tokens, int top_k, int n_experts, int hidden, int intermediate, int wformat,
+                               int dtype, llmq_stream_t stream) {
+  if (n_tokens == 0) return 0;
+  if (!llmq_wq_experts_supported(n_tokens, top_k, n_experts, hidden, intermediate))
+    return llmq_host::fail_invalid("the experts' GEMM does not take tokens=%d top_k=%d experts=%d hidden=%d intermediate=%d",
+                                   n_tokens, top_k, n_experts, hidden, intermediate);
+  if (wformat != LLMQ_W_INT8 && wformat != LLMQ_W_INT4_PACKED)
+    return llmq_host::fail_invalid("unsupported weight format %d, expected 8 or 4", wformat);
+  if (dtype != LLMQ_BF16 && dtype != LLMQ_F16)
+    return llmq_host::fail_invalid("the experts' GEMM takes bfloat16 or float16 activations, got dtype code %d", dtype);
+  if (!x || !top_k_index || !top_k_weights || !gate_up || !gate_up_scale || !down || !down_scale || !out || !workspace)
+    return llmq_host::fail_invalid("null tensor pointer");
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(gate_up) | reinterpret_cast<uintptr_t>(down) |
+       reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(workspace)) & 15u)
+    return llmq_host::fail_invalid("activation, weight, output and workspace pointers must be 16-byte aligned");
+  const size_t need = layout_for(n_tokens, top_k, n_experts, hidden, intermediate).total;
+  if (workspace_bytes < need)
+    return llmq_host::fail_invalid("workspace of %zu bytes is too small, need %zu", workspace_bytes, need);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  uint8_t* ws = static_cast<uint8_t*>(workspace);
+  const bool int4 = wformat == LLMQ_W_INT4_PACKED;
+#define LLMQ_EXPERTS(T, BITS)                                                                                      \
+  run<T, BITS>(x, top_k_index, top_k_weights, gate_up, gate_up_scale, down, down_scale, out, ws, n_tokens, top_k, \
+               n_experts, hidden, intermediate, s)
+  if (dtype == LLMQ_BF16) return int4 ? LLMQ_EXPERTS(bf16_t, 4) : LLMQ_EXPERTS(bf16_t, 8);
+  return int4 ? LLMQ_EXPERTS(f16_t, 4) : LLMQ_EXPERTS(f16_t, 8);
+#undef LLMQ_EXPERTS
+}

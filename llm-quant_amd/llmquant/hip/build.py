@@ -89,6 +89,12 @@ def load_capi() -> ctypes.CDLL:
     lib.llmq_wq_gemv_batched_fused.restype = c_int
     lib.llmq_moe_combine.argtypes = [c_p] * 4 + [c_int] * 5 + [c_p]
     lib.llmq_moe_combine.restype = c_int
+    lib.llmq_wq_experts_supported.argtypes = [c_int] * 5
+    lib.llmq_wq_experts_supported.restype = c_int
+    lib.llmq_wq_experts_workspace_bytes.argtypes = [c_int] * 5
+    lib.llmq_wq_experts_workspace_bytes.restype = ctypes.c_size_t
+    lib.llmq_wq_experts.argtypes = [c_p] * 9 + [ctypes.c_size_t] + [c_int] * 7 + [c_p]
+    lib.llmq_wq_experts.restype = c_int
     lib.llmq_route_plan_blocks_per_expert.argtypes = [c_int, c_int]
     lib.llmq_route_plan_blocks_per_expert.restype = c_int
     lib.llmq_route_plan_supported.argtypes = [c_int, c_int]

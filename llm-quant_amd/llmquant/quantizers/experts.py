@@ -264,6 +264,19 @@ class KernelQuantExperts(_QuantExperts):
                 and top_k_weights.dtype == hidden_states.dtype and top_k_weights.shape == top_k_index.shape
                 and self._ext.route_plan_supported(top_k_index.numel(), self.num_experts))
 
+    def _takes_gemm(self, hidden_states, top_k_index, top_k_weights) -> bool:
+        """Whether a prompt's tokens go through the grouped GEMMs (five launches whatever the number of experts): SiLU
+        experts of unpadded groups of 128, one scale per weight row, 16-bit activations and routing weights."""
+        return (self._act_is_silu and self._weight_args.group_size == 128
+                and self._gate_up_padded == self.hidden_dim and self._down_padded == self.intermediate_dim
+                and self.sgate_up.shape[1] == self.gate_up_data.shape[1] and self.sdown.shape[1] == self.down_data.shape[1]
+                and hidden_states.dtype in (torch.bfloat16, torch.float16)
+                and hidden_states.dim() == 2 and hidden_states.is_contiguous()
+                and top_k_weights.dtype == hidden_states.dtype and top_k_weights.shape == top_k_index.shape
+                and top_k_index.dim() == 2 and top_k_index.shape[0] == hidden_states.shape[0]
+                and self._ext.wq_experts_supported(hidden_states.shape[0], top_k_index.shape[1], self.num_experts,
+                                                   self.hidden_dim, self.intermediate_dim))
+
     def _forward_fused(self, hidden_states, top_k_index, top_k_weights):
         """Plan, gate|up (storing act(gate) * up), down, weighted sum per token: four launches. With one
         token every row reads that token's activation, so `hidden_states[tokens_per_row]` is not formed."""
@@ -282,6 +295,9 @@ class KernelQuantExperts(_QuantExperts):
         # An expert cannot be picked twice by one token, so no expert sees more rows than there
         # are tokens: the shape alone says whether the batched kernel's run length suffices.
         if hidden_states.shape[0] > self._batched_max_rows:
+            if self._takes_gemm(hidden_states, top_k_index, top_k_weights):
+                return self._ext.wq_experts(hidden_states, top_k_index, top_k_weights, self.gate_up_data, self.sgate_up,
+                                            self.down_data, self.sdown)
             return self._each_hit_expert(hidden_states, top_k_index, top_k_weights)
         if self._fusable(hidden_states, top_k_index, top_k_weights):
             return self._forward_fused(hidden_states, top_k_index, top_k_weights)
