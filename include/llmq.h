@@ -51,6 +51,13 @@ const char* llmq_last_error(void);
 int llmq_fake_quant_group(const void* x, void* out, float* scale_or_null, int64_t n_groups,
                           int group_size, int num_bits, int dtype, llmq_stream_t stream);
 
+/* The same over rows of `width` elements that need not be a whole number of groups: every row's last group is what is
+ * left of it (the zeros that the reference pads with, llmquant/cuda/ops.py, never raise an abs-max). x, out:
+ * [rows, width], read and written in place of a padded copy; scale: [rows, ceil(width / group_size)] or null. Groups of
+ * 1, 2, 4, .. 64 packets of 16 bytes, rows of at least one. */
+int llmq_fake_quant_rows(const void* x, void* out, float* scale_or_null, int64_t rows, int width, int group_size,
+                         int num_bits, int dtype, llmq_stream_t stream);
+
 /* Same arithmetic, but emits the integer codes instead of the dequantized values:
  * codes int8 [n_groups*group_size] (pack4 == 0) or nibble-packed uint8
  * [n_groups*group_size/2] (pack4 != 0, num_bits <= 4), scale fp32 [n_groups].

@@ -68,6 +68,32 @@ std::tuple<at::Tensor, at::Tensor> fake_quant_group(const at::Tensor& x, int64_t
   return std::make_tuple(out.reshape(x.sizes()), scale);
 }
 
+// fake_quant_group for a last axis that is not a whole number of groups: a row's last group is what is left of it.
+std::tuple<at::Tensor, at::Tensor> fake_quant_rows(const at::Tensor& x, int64_t num_bits, int64_t group_size,
+                                                   bool return_scale) {
+  TORCH_CHECK(x.is_cuda(), "x must be a CUDA tensor");
+  TORCH_CHECK(x.dim() >= 1, "x must have at least one dimension");
+  TORCH_CHECK(num_bits >= 2 && num_bits <= 8, "num_bits must be in [2, 8], got ", num_bits);
+  TORCH_CHECK(group_size > 0 && group_size <= INT32_MAX && x.size(-1) <= INT32_MAX, "group_size must be positive, got ",
+              group_size);
+  const int dtype = dtype_code(x, "x");
+  const auto xc = x.contiguous();
+  const int64_t width = xc.size(-1);
+  auto out = at::empty_like(xc);
+  auto scale_sizes = xc.sizes().vec();
+  scale_sizes.back() = (width + group_size - 1) / group_size;
+  const auto scale_opts = xc.options().dtype(at::kFloat);
+  if (xc.numel() == 0) return std::make_tuple(out, at::empty({0}, scale_opts));
+  auto scale = return_scale ? at::empty(scale_sizes, scale_opts) : at::empty({0}, scale_opts);
+  const c10::OptionalDeviceGuard guard(at::device_of(xc));
+  check_rc(llmq_fake_quant_rows(xc.const_data_ptr(), out.mutable_data_ptr(),
+                                return_scale ? scale.mutable_data_ptr<float>() : nullptr, xc.numel() / width,
+                                static_cast<int>(width), static_cast<int>(group_size), static_cast<int>(num_bits), dtype,
+                                current_stream(xc)),
+           "fake_quant_rows");
+  return std::make_tuple(out, scale);
+}
+
 std::tuple<at::Tensor, at::Tensor> quant_group_codes(const at::Tensor& x, int64_t num_bits,
                                                      int64_t group_size, bool pack4) {
   TORCH_CHECK(x.is_cuda(), "x must be a CUDA tensor");
@@ -1419,6 +1445,8 @@ at::Tensor argmax_advance(const at::Tensor& x, at::Tensor& token, at::Tensor& st
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fake_quant_group", &fake_quant_group,
         "Fused symmetric RTN quant-dequant, grouped along the last axis (HIP, gfx950)",
+        py::arg("x"), py::arg("num_bits"), py::arg("group_size"), py::arg("return_scale") = false);
+  m.def("fake_quant_rows", &fake_quant_rows, "fake_quant_group over rows that are not a whole number of groups",
         py::arg("x"), py::arg("num_bits"), py::arg("group_size"), py::arg("return_scale") = false);
   m.def("quant_group_codes", &quant_group_codes,
         "Symmetric RTN quantize to integer codes + fp32 scales, grouped along the last axis",

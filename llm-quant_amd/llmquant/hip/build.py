@@ -74,6 +74,8 @@ def load_capi() -> ctypes.CDLL:
     lib.llmq_abi_version.restype = c_int
     lib.llmq_last_error.restype = ctypes.c_char_p
     lib.llmq_fake_quant_group.argtypes = [c_p, c_p, c_p, c_i64, c_int, c_int, c_int, c_p]
+    lib.llmq_fake_quant_rows.argtypes = [c_p, c_p, c_p, c_i64] + [c_int] * 4 + [c_p]
+    lib.llmq_fake_quant_rows.restype = c_int
     lib.llmq_quant_group_codes.argtypes = [c_p, c_p, c_p, c_i64, c_int, c_int, c_int, c_int, c_p]
     lib.llmq_wq_gemv.argtypes = [c_p, c_p, c_p, c_p] + [c_int] * 7 + [c_p]
     lib.llmq_kv_append.argtypes = [c_p, c_p, c_i64, c_i64, c_p, c_p, c_p, c_p, c_p, c_p, c_p] + [c_int] * 6 + [c_p]

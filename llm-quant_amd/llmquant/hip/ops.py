@@ -20,11 +20,17 @@ def _group_size_for(x: torch.Tensor, args: QuantizationArgs) -> int:
 def fake_quantize_hip(x: torch.Tensor, args: QuantizationArgs, return_scale: bool = False):
     """Quant-dequant on the GPU, bit-exact with llmquant.core.quant_ops.fake_quantize.
 
-    Groups run along the last axis. A last axis that is not a whole number of groups gets
-    the same zero padding the PyTorch form applies, and the padding is trimmed again.
+    Groups run along the last axis. A last axis that is not a whole number of groups gives
+    what the PyTorch form's zero padding and trimming give: for groups of a power of two 16-byte
+    packets the kernel reads and writes the rows as they lie, others are padded and trimmed.
     """
     group_size = _group_size_for(x, args)
     width = x.shape[-1]
+    if width % group_size and x.is_cuda and x.element_size() <= 4:
+        packets, rest = divmod(group_size * x.element_size(), 16)
+        if rest == 0 and packets <= 64 and packets & (packets - 1) == 0 and width >= 8 and x.numel() < 1 << 30:
+            out, scale = load_extension().fake_quant_rows(x, args.num_bits, group_size, return_scale)
+            return (out, scale) if return_scale else out
     padded = pad_to_group(x, group_size)
     out, scale = load_extension().fake_quant_group(padded, args.num_bits, group_size, return_scale)
     if padded.shape[-1] != width:

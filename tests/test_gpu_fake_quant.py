@@ -173,3 +173,26 @@ def test_bare_c_abi_call():
     assert same_bits(out, oracle.fake_quantize(to_np(x), 8, "bf16", "group", GROUP))
     rc = lib.llmq_fake_quant_group(x.data_ptr(), out.data_ptr(), None, 4, GROUP, 9, 2, None)
     assert rc == 1 and b"num_bits" in lib.llmq_last_error()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [8, 9, 127, 129, 135, 250, 1003, 5000])
+def test_rows_that_are_no_whole_number_of_groups(hip_fake_quantize, dtype, width):
+    """One packet, a tail of one element, a last group shorter than a packet, odd widths (rows at every alignment)."""
+    torch.manual_seed(width)
+    x = (torch.randn(7, width) * 2).to(dtype)
+    got, scale = hip_fake_quantize(x.cuda(), args(4), return_scale=True)
+    assert got.shape == x.shape
+    assert same_bits(got, oracle.fake_quantize(to_np(x), 4, tag_of(dtype), "group", GROUP))
+    assert np.array_equal(to_np(scale), oracle.compute_scale(to_np(x), 4, "group", GROUP)[..., 0])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [5, 8, 100, 513, 2047, 2049, 8191, 16392, 20001])
+def test_groups_of_any_width(hip_fake_quantize, dtype, width):
+    """One group a row: below a packet, one wave and four, the last packet overlapping, beyond what registers hold."""
+    torch.manual_seed(width)
+    x = (torch.randn(5, width) * 2).to(dtype)
+    got, scale = hip_fake_quantize(x.cuda(), args(8, strategy="channel"), return_scale=True)
+    assert same_bits(got, oracle.fake_quantize(to_np(x), 8, tag_of(dtype), "channel"))
+    assert np.array_equal(to_np(scale).reshape(-1), oracle.compute_scale(to_np(x), 8, "channel").reshape(-1))
