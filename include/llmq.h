@@ -131,6 +131,18 @@ int llmq_wq_gemv_batched_fused(const void* x, int64_t x_row_stride, const void* 
 int llmq_moe_combine(const void* rows_out, const int64_t* order, const void* weights, void* final_out,
                      int n_rows, int top_k, int n_tokens, int width, int dtype, llmq_stream_t stream);
 
+/* The same block for a token or two, in two launches: a (token, slot) row reads its expert's id itself, and the down
+ * launch adds up a token's experts in their order. Rounding points and bits of llmq_route_plan +
+ * llmq_wq_gemv_batched_fused + llmq_moe_combine; every row reads its expert's weight (nothing is shared between tokens).
+ * act: [tokens * top_k, intermediate] of the activation dtype, 16-byte aligned. Weights, scales and index as for
+ * llmq_wq_experts below, any float dtype. `supported`: hidden and intermediate multiples of 512, intermediate up to
+ * 8192, top_k up to 16, a token's rows within the LDS. */
+int llmq_wq_experts_direct_supported(int n_tokens, int top_k, int n_experts, int hidden, int intermediate, int wformat);
+int llmq_wq_experts_direct(const void* x, const int64_t* top_k_index, const void* top_k_weights, const void* gate_up,
+                           const float* gate_up_scale, const void* down, const float* down_scale, void* out, void* act,
+                           int n_tokens, int top_k, int n_experts, int hidden, int intermediate, int wformat, int dtype,
+                           llmq_stream_t stream);
+
 /* A whole gated experts block over many tokens (KernelQuantExperts.forward, kernel.py:216-289, which walks the experts
  * one at a time beyond a few tokens): out[t] = sum over t's experts e of weight * down_e(silu(gate_e(x_t)) * up_e(x_t)),
  * rounded to `dtype` (fp16 / bf16) after each projection, activation, product, weighted row and addition (added in the

@@ -337,6 +337,12 @@ int gemv_mfma_launch_fused(const void* x, const void* qw, const float* ws, void*
                            int attn_splits = 0, int attn_head_dim = 0, int pair_half = 0);
 // Batched form (a plan of expert / row runs read on the device): see llmq_wq_gemv_batched.
 bool gemv_batched_mfma_supported(const void* x, const void* qw, const float* ws, int G, int gs, int wformat);
+// The routed experts of a few tokens, no plan (csrc/wq_gemv_mfma.hip); act: [tokens * top_k, intermediate] scratch.
+bool experts_direct_supported(int tokens, int top_k, int n_experts, int hidden, int intermediate, bool int4);
+int experts_direct_launch(const void* x, const int64_t* index, const void* weights, const void* gate_up,
+                          const float* gate_up_scale, const void* down, const float* down_scale, void* out, void* act,
+                          int tokens, int top_k, int n_experts, int hidden, int intermediate, int wformat, int dtype,
+                          hipStream_t stream);
 int gemv_batched_mfma_launch(const void* x, const void* qw, const float* ws, void* out, const int32_t* block_expert,
                              const int32_t* block_row0, const int32_t* block_rows, int n_blocks, int n_rows,
                              int n_experts, int N, int G, int out_group, int wformat, int dtype,

@@ -141,3 +141,31 @@ extern "C" int llmq_route_plan(const int64_t* expert_of_row, int n_rows, int n_e
                      block_expert, block_row0, block_rows);
   return llmq_host::check_launch("route_plan_kernel");
 }
+
+extern "C" int llmq_wq_experts_direct_supported(int n_tokens, int top_k, int n_experts, int hidden, int intermediate,
+                                                int wformat) {
+  return llmq_host::experts_direct_supported(n_tokens, top_k, n_experts, hidden, intermediate,
+                                             wformat == LLMQ_W_INT4_PACKED) ? 1 : 0;
+}
+
+extern "C" int llmq_wq_experts_direct(const void* x, const int64_t* top_k_index, const void* top_k_weights,
+                                      const void* gate_up, const float* gate_up_scale, const void* down,
+                                      const float* down_scale, void* out, void* act, int n_tokens, int top_k,
+                                      int n_experts, int hidden, int intermediate, int wformat, int dtype,
+                                      llmq_stream_t stream) {
+  if (n_tokens == 0) return 0;
+  if (wformat != LLMQ_W_INT8 && wformat != LLMQ_W_INT4_PACKED)
+    return llmq_host::fail_invalid("unsupported weight format %d, expected 8 or 4", wformat);
+  if (!llmq_host::experts_direct_supported(n_tokens, top_k, n_experts, hidden, intermediate, wformat == LLMQ_W_INT4_PACKED))
+    return llmq_host::fail_invalid("the direct experts launches do not take tokens=%d top_k=%d experts=%d hidden=%d "
+                                   "intermediate=%d", n_tokens, top_k, n_experts, hidden, intermediate);
+  if (!x || !top_k_index || !top_k_weights || !gate_up || !gate_up_scale || !down || !down_scale || !out || !act)
+    return llmq_host::fail_invalid("null tensor pointer");
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(gate_up) | reinterpret_cast<uintptr_t>(down) |
+       reinterpret_cast<uintptr_t>(gate_up_scale) | reinterpret_cast<uintptr_t>(down_scale) |
+       reinterpret_cast<uintptr_t>(act)) & 15u)
+    return llmq_host::fail_invalid("activation, weight, scale and scratch pointers must be 16-byte aligned");
+  return llmq_host::experts_direct_launch(x, top_k_index, top_k_weights, gate_up, gate_up_scale, down, down_scale, out,
+                                          act, n_tokens, top_k, n_experts, hidden, intermediate, wformat, dtype,
+                                          static_cast<hipStream_t>(stream));
+}

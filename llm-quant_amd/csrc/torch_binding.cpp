@@ -491,11 +491,14 @@ at::Tensor moe_combine(const at::Tensor& rows_out, const at::Tensor& order, cons
   return out;
 }
 
-// A whole gated experts block over many tokens (see llmq_wq_experts): x [tokens, hidden], top_k_index and
-// top_k_weights [tokens, top_k], the stacked weights as KernelQuantExperts stores them. Returns [tokens, hidden].
-at::Tensor wq_experts(const at::Tensor& x, const at::Tensor& top_k_index, const at::Tensor& top_k_weights,
-                      const at::Tensor& gate_up, const at::Tensor& gate_up_scale, const at::Tensor& down,
-                      const at::Tensor& down_scale) {
+// What the two forms of a gated experts block take: x [tokens, hidden], top_k_index and top_k_weights [tokens, top_k],
+// the stacked weights as KernelQuantExperts stores them.
+struct ExpertsProblem {
+  int tokens, top_k, experts, hidden, intermediate, wformat, dtype;
+};
+ExpertsProblem check_experts(const at::Tensor& x, const at::Tensor& top_k_index, const at::Tensor& top_k_weights,
+                             const at::Tensor& gate_up, const at::Tensor& gate_up_scale, const at::Tensor& down,
+                             const at::Tensor& down_scale) {
   TORCH_CHECK(x.is_cuda() && top_k_index.is_cuda() && top_k_weights.is_cuda() && gate_up.is_cuda() &&
                   gate_up_scale.is_cuda() && down.is_cuda() && down_scale.is_cuda(), "all tensors must be CUDA");
   TORCH_CHECK(x.dim() == 2 && x.is_contiguous(), "x must be contiguous [tokens, hidden]");
@@ -505,7 +508,7 @@ at::Tensor wq_experts(const at::Tensor& x, const at::Tensor& top_k_index, const 
   const bool packed = gate_up.scalar_type() == at::kByte;
   TORCH_CHECK(packed || gate_up.scalar_type() == at::kChar, "weights must be int8, or uint8 for nibble-packed int4");
   const int64_t E = gate_up.size(0), H = down.size(1), I = gate_up.size(1) / 2, per_byte = packed ? 2 : 1;
-  TORCH_CHECK(gate_up.size(3) * per_byte == 128 && down.size(3) * per_byte == 128, "the experts' GEMM needs group_size 128");
+  TORCH_CHECK(gate_up.size(3) * per_byte == 128 && down.size(3) * per_byte == 128, "the experts need group_size 128");
   TORCH_CHECK(x.size(1) == H && gate_up.size(1) == 2 * I && gate_up.size(2) * 128 == H && down.size(2) * 128 == I,
               "gate_up must be [experts, 2 I, H / 128, ...], down [experts, H, I / 128, ...] and x [tokens, H]");
   auto scales = [&](const at::Tensor& s, const at::Tensor& w) {
@@ -514,26 +517,52 @@ at::Tensor wq_experts(const at::Tensor& x, const at::Tensor& top_k_index, const 
   };
   TORCH_CHECK(scales(gate_up_scale, gate_up) && scales(down_scale, down),
               "scales must be contiguous float32 [experts, N, groups]");
-  const int64_t T = x.size(0), top_k = top_k_index.size(-1);
-  TORCH_CHECK(top_k_index.dim() == 2 && top_k_index.size(0) == T && at::isIntegralType(top_k_index.scalar_type(), false),
+  TORCH_CHECK(top_k_index.dim() == 2 && top_k_index.size(0) == x.size(0) &&
+                  at::isIntegralType(top_k_index.scalar_type(), false),
               "top_k_index must hold integers, [tokens, top_k]");
   TORCH_CHECK(top_k_weights.sizes() == top_k_index.sizes() && top_k_weights.scalar_type() == x.scalar_type(),
               "top_k_weights must be [tokens, top_k] of x's dtype");
-  const int dtype = dtype_code(x, "x");
+  return {static_cast<int>(x.size(0)), static_cast<int>(top_k_index.size(1)), static_cast<int>(E), static_cast<int>(H),
+          static_cast<int>(I), packed ? LLMQ_W_INT4_PACKED : LLMQ_W_INT8, dtype_code(x, "x")};
+}
+
+// A whole gated experts block over many tokens (see llmq_wq_experts). Returns [tokens, hidden].
+at::Tensor wq_experts(const at::Tensor& x, const at::Tensor& top_k_index, const at::Tensor& top_k_weights,
+                      const at::Tensor& gate_up, const at::Tensor& gate_up_scale, const at::Tensor& down,
+                      const at::Tensor& down_scale) {
+  const auto p = check_experts(x, top_k_index, top_k_weights, gate_up, gate_up_scale, down, down_scale);
   auto out = at::empty_like(x);
   if (out.numel() == 0) return out;
   const at::Tensor index = top_k_index.to(at::kLong).contiguous(), weights = top_k_weights.contiguous();
-  const int t = static_cast<int>(T), k = static_cast<int>(top_k), e = static_cast<int>(E), h = static_cast<int>(H),
-            i = static_cast<int>(I);
   const c10::OptionalDeviceGuard guard(at::device_of(x));
-  const int64_t bytes = static_cast<int64_t>(llmq_wq_experts_workspace_bytes(t, k, e, h, i));
+  const int64_t bytes = static_cast<int64_t>(
+      llmq_wq_experts_workspace_bytes(p.tokens, p.top_k, p.experts, p.hidden, p.intermediate));
   auto workspace = at::empty({bytes}, x.options().dtype(at::kByte));
   check_rc(llmq_wq_experts(x.const_data_ptr(), index.const_data_ptr<int64_t>(), weights.const_data_ptr(),
                            gate_up.const_data_ptr(), gate_up_scale.const_data_ptr<float>(), down.const_data_ptr(),
                            down_scale.const_data_ptr<float>(), out.mutable_data_ptr(), workspace.mutable_data_ptr(),
-                           static_cast<size_t>(bytes), t, k, e, h, i, packed ? LLMQ_W_INT4_PACKED : LLMQ_W_INT8, dtype,
-                           current_stream(x)),
+                           static_cast<size_t>(bytes), p.tokens, p.top_k, p.experts, p.hidden, p.intermediate, p.wformat,
+                           p.dtype, current_stream(x)),
            "wq_experts");
+  return out;
+}
+
+// The same block for a token or two, two launches (see llmq_wq_experts_direct).
+at::Tensor wq_experts_direct(const at::Tensor& x, const at::Tensor& top_k_index, const at::Tensor& top_k_weights,
+                             const at::Tensor& gate_up, const at::Tensor& gate_up_scale, const at::Tensor& down,
+                             const at::Tensor& down_scale) {
+  const auto p = check_experts(x, top_k_index, top_k_weights, gate_up, gate_up_scale, down, down_scale);
+  auto out = at::empty_like(x);
+  if (out.numel() == 0) return out;
+  const at::Tensor index = top_k_index.to(at::kLong).contiguous(), weights = top_k_weights.contiguous();
+  const c10::OptionalDeviceGuard guard(at::device_of(x));
+  auto act = at::empty({static_cast<int64_t>(p.tokens) * p.top_k, p.intermediate}, x.options());
+  check_rc(llmq_wq_experts_direct(x.const_data_ptr(), index.const_data_ptr<int64_t>(), weights.const_data_ptr(),
+                                  gate_up.const_data_ptr(), gate_up_scale.const_data_ptr<float>(), down.const_data_ptr(),
+                                  down_scale.const_data_ptr<float>(), out.mutable_data_ptr(), act.mutable_data_ptr(),
+                                  p.tokens, p.top_k, p.experts, p.hidden, p.intermediate, p.wformat, p.dtype,
+                                  current_stream(x)),
+           "wq_experts_direct");
   return out;
 }
 
@@ -1468,6 +1497,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("wq_experts", &wq_experts, "A gated experts block over many tokens: plan, two grouped GEMMs, combination",
         py::arg("x"), py::arg("top_k_index"), py::arg("top_k_weights"), py::arg("gate_up"), py::arg("gate_up_scale"),
         py::arg("down"), py::arg("down_scale"));
+  m.def("wq_experts_direct", &wq_experts_direct, "A gated experts block for a token or two in two launches",
+        py::arg("x"), py::arg("top_k_index"), py::arg("top_k_weights"), py::arg("gate_up"), py::arg("gate_up_scale"),
+        py::arg("down"), py::arg("down_scale"));
+  m.def("wq_experts_direct_supported", [](int64_t tokens, int64_t top_k, int64_t experts, int64_t hidden,
+                                          int64_t intermediate, int64_t weight_bits) {
+    constexpr int64_t kMost = INT32_MAX;
+    return tokens <= kMost && top_k <= kMost && experts <= kMost && hidden <= kMost && intermediate <= kMost &&
+           llmq_wq_experts_direct_supported(static_cast<int>(tokens), static_cast<int>(top_k), static_cast<int>(experts),
+                                            static_cast<int>(hidden), static_cast<int>(intermediate),
+                                            weight_bits == 4 ? LLMQ_W_INT4_PACKED : LLMQ_W_INT8) != 0;
+  }, py::arg("tokens"), py::arg("top_k"), py::arg("experts"), py::arg("hidden"), py::arg("intermediate"),
+     py::arg("weight_bits"));
   m.def("wq_experts_supported", [](int64_t tokens, int64_t top_k, int64_t experts, int64_t hidden, int64_t intermediate) {
     constexpr int64_t kMost = INT32_MAX;
     return tokens <= kMost && top_k <= kMost && experts <= kMost && hidden <= kMost && intermediate <= kMost &&

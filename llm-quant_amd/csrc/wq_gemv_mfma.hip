@@ -620,6 +620,137 @@ __global__ __launch_bounds__(MAXT) void wq_gemv_mfma_batched_kernel(MfmaArgs a, 
   }
 }
 
+// The routed experts of a token or two in two launches, with no plan: a (token, slot) row names its expert itself.
+//
+// gate|up: grid (row tiles, rows); the single-row body on the expert's weight, act(gate) * up in its store.
+struct RoutedArgs {
+  const int64_t* expert_of_row;  // [tokens * top_k]
+  int n_experts, top_k;
+  int64_t weight_stride;         // bytes between experts' weights
+  int64_t scale_stride;          // floats between experts' scales
+  // an id outside the layer's experts is counted with the nearest valid one
+  __device__ __forceinline__ int expert(int row) const {
+    const int64_t raw = expert_of_row[row];
+    return raw < 0 ? 0 : (raw >= n_experts ? n_experts - 1 : static_cast<int>(raw));
+  }
+};
+
+template <typename T, int BITS, int MAXT, bool MULTI>
+__global__ __launch_bounds__(MAXT) void wq_gemv_mfma_routed_kernel(MfmaArgs a, const RoutedArgs route) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int row = blockIdx.y, e = route.expert(row);
+  a.qw += e * route.weight_stride;
+  a.ws += e * route.scale_stride;
+  a.x = static_cast<const T*>(a.x) + static_cast<int64_t>(row / route.top_k) * a.G * kGroup;
+  a.out = static_cast<T*>(a.out) + static_cast<int64_t>(row) * a.pair_half;
+  ksplit_body<T, BITS, 1, MULTI>(a, smem, blockIdx.x, gridDim.x, 1);
+}
+
+// down and the weighted sum over a token's experts: grid (row tiles, tokens). A workgroup owns a tile of the token's
+// output columns for all of its experts, so that the sum needs no launch of its own. The token's activation rows lie
+// one after the other and are staged as one long row; a wave takes (slot, chunk of four groups) units of it, each
+// against its expert's weight. What meets in LDS is added up as the single-row body does (a row's bits are
+// llmq_wq_gemv's), rounded, weighted, rounded, and the slots are added in the order of their experts (equal experts:
+// of the slots), rounding after each: the arithmetic of moe_combine_kernel over the sorted rows.
+// Bound: the chain of dependent steps (ids -> weights from memory -> multiply -> two meetings in LDS). With both
+// launches a token of 64 experts of 2048 x 1024 int4, eight routed (27 MB of codes), takes the time stated at
+// experts_direct_pays in quantizers/experts.py.
+constexpr int kRoutedMaxTopK = 16;
+constexpr int kRoutedMaxChunks = 16;   // of one row: longer ones are added up per wave by the single-row body
+template <typename T, int BITS>
+__global__ __launch_bounds__(1024) void wq_gemv_mfma_routed_down_kernel(const MfmaArgs a, const RoutedArgs route,
+                                                                        const T* __restrict__ weights) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ float s_product[kRoutedMaxTopK][kTileRows];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), waves = blockDim.x / kWave;
+  const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int top_k = route.top_k, row0 = blockIdx.y * top_k, tile = blockIdx.x;
+  const int G = top_k * a.G, n_chunks = a.G / kGW, units = G / kGW;
+  const LdsLayout L(1, G, 0, BITS == 4);
+  int8_t* dig = reinterpret_cast<int8_t*>(smem + L.dig_off);
+  float* cxs = reinterpret_cast<float*>(smem + L.cx_off);
+  float* red = reinterpret_cast<float*>(smem + L.red_off);
+  int* csum = reinterpret_cast<int*>(smem + L.csum_off);
+  float* part = reinterpret_cast<float*>(smem + L.part_off);   // [unit][digit][row of the tile]
+  const int j = lane & 15, blk = lane >> 4;
+
+  constexpr int kB = BITS == 8 ? 2 : 1;
+  v4i b[kB * kGW];
+  float sc[kGW];
+  auto issue_loads = [&](int unit) {
+    const int slot = unit / n_chunks, g0 = (unit - slot * n_chunks) * kGW;
+    const int e = route.expert(row0 + slot), n = tile_row(a, tile, j);
+    const uint8_t* row = a.qw + e * route.weight_stride + static_cast<int64_t>(n) * a.row_bytes;
+#pragma unroll
+    for (int gi = 0; gi < kGW; ++gi) {
+      const uint8_t* p = row + (g0 + gi) * (kGroup * BITS / 8) + blk * 16;
+      b[kB * gi] = *reinterpret_cast<const v4i*>(p);
+      if constexpr (BITS == 8) b[kB * gi + 1] = *reinterpret_cast<const v4i*>(p + 64);
+    }
+    const u32x4 s4 = load16(a.ws + e * route.scale_stride + static_cast<int64_t>(n) * a.G + g0);
+    sc[0] = __builtin_bit_cast(float, s4.x); sc[1] = __builtin_bit_cast(float, s4.y);
+    sc[2] = __builtin_bit_cast(float, s4.z); sc[3] = __builtin_bit_cast(float, s4.w);
+  };
+  // (A row 4 * digit + m: every lane reads a valid plane; see wq_gemv_mfma_fullk_kernel)
+  const int8_t* a_base = dig + min(j >> 2, kDigits - 1) * L.plane + blk * 16;
+  const float digit_weight = blk == 0 ? 1.0f : (blk == 1 ? 256.0f : (blk == 2 ? 65536.0f : 0.0f));
+  const int* csum_row = csum + (blk < kDigits ? blk : 0) * G;
+
+  const T* x = static_cast<const T*>(a.x) + static_cast<int64_t>(row0) * a.G * kGroup;
+  const Prologue pro{LLMQ_PRO_NONE, nullptr, 0.0f, 0};
+  const StageFirst first = stage_first<T, 1>(x, G, pro);
+  stage_activation<T, BITS, 1>(x, G, L, dig, cxs, csum, pro, red, first, 1, [&] { issue_loads(wv); });
+  __syncthreads();
+
+  for (int unit = wv; unit < units; unit += waves) {
+    v4i d[kGW];
+    float s_now[kGW];
+#pragma unroll
+    for (int gi = 0; gi < kGW; ++gi) {
+      const int g = unit * kGW + gi;
+      const v4i a0 = *reinterpret_cast<const v4i*>(a_base + g * kGroup);
+      const v4i a1 = *reinterpret_cast<const v4i*>(a_base + g * kGroup + 64);
+      s_now[gi] = sc[gi] * (cxs[g] * digit_weight);
+      d[gi] = v4i{BITS == 4 ? -8 * csum_row[g] : 0, 0, 0, 0};
+      if constexpr (BITS == 8) {
+        d[gi] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b[kB * gi], d[gi], 0, 0, 0);
+        d[gi] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b[kB * gi + 1], d[gi], 0, 0, 0);
+      } else {
+        d[gi] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b[gi] & 0x0f0f0f0f, d[gi], 0, 0, 0);
+        d[gi] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, (b[gi] >> 4) & 0x0f0f0f0f, d[gi], 0, 0, 0);
+      }
+    }
+    if (unit + waves < units) issue_loads(unit + waves);
+    float acc = 0.0f;
+#pragma unroll
+    for (int gi = 0; gi < kGW; ++gi) acc = fmaf(static_cast<float>(d[gi][0]), s_now[gi], acc);
+    if (blk < kDigits) part[(unit * kDigits + blk) * kTileRows + j] = acc;
+  }
+  __syncthreads();
+  // a wave per slot: the row's sum in the order of the single-row body, its weighted value into the slot's place in
+  // the order of the experts
+  for (int slot = wv; slot < top_k; slot += waves) {
+    float total = 0.0f;
+    for (int c = blk; c < n_chunks; c += 4) {
+#pragma unroll
+      for (int q = kDigits - 1; q >= 0; --q) total += part[((slot * n_chunks + c) * kDigits + q) * kTileRows + j];
+    }
+    total += __shfl_xor(total, 16, kWave);
+    total += __shfl_xor(total, 32, kWave);
+    const int e = route.expert(row0 + slot);
+    const int theirs = lane < top_k ? route.expert(row0 + lane) : 0;
+    const int place = __popcll(__ballot(lane < top_k && (theirs < e || (theirs == e && lane < slot))));
+    if (lane < kTileRows) s_product[place][j] = round_through<T>(round_through<T>(total) * to_float(weights[row0 + slot]));
+  }
+  __syncthreads();
+  const int n = tile * a.tile_rows + tid;
+  if (tid < a.tile_rows && n < a.N) {
+    float acc = 0.0f;
+    for (int k = 0; k < top_k; ++k) acc = round_through<T>(acc + s_product[k][tid]);
+    static_cast<T*>(a.out)[static_cast<int64_t>(blockIdx.y) * a.N + n] = from_float<T>(acc);
+  }
+}
+
 // Large N: a wave owns whole rows. With every group of the row in one wave there is nothing
 // to exchange between waves, so after the activation is staged the main loop has no barrier:
 // per chunk of four groups a wave issues its weight loads together with the LDS reads of the
@@ -1154,6 +1285,98 @@ int gemv_batched_mfma_launch(const void* x, const void* qw, const float* ws, voi
     case LLMQ_F32: return LLMQ_DISPATCH(float);
     case LLMQ_F16: return LLMQ_DISPATCH(f16_t);
     case LLMQ_BF16: return LLMQ_DISPATCH(bf16_t);
+  }
+#undef LLMQ_DISPATCH
+  return fail_invalid("x must be float32, float16 or bfloat16, got dtype code %d", dtype);
+}
+
+namespace {
+// LDS of the down launch: the staged rows of a token, and a partial tile per unit.
+int routed_down_lds(int top_k, int G, bool int4) {
+  return LdsLayout(1, top_k * G, 0, int4).part_off + top_k * (G / kGW) * kDigits * kTileRows * static_cast<int>(sizeof(float));
+}
+
+template <typename T, int BITS>
+int launch_routed(const T* x, const int64_t* index, const T* weights, const uint8_t* q1, const float* s1,
+                  const uint8_t* q2, const float* s2, T* out, T* act, int tokens, int top_k, int E, int H, int I,
+                  hipStream_t stream) {
+  MfmaArgs up{};
+  up.x = x; up.qw = q1; up.ws = s1; up.out = act;
+  up.N = 2 * I; up.G = H / kGroup; up.x_row_stride = -1; up.pair_half = I; up.tile_rows = kTileRows;
+  up.n_tiles = 2 * I / kTileRows;
+  up.row_bytes = H * BITS / 8;
+  const int rows = tokens * top_k;
+  RoutedArgs route{index, E, top_k, static_cast<int64_t>(up.N) * up.row_bytes, static_cast<int64_t>(up.N) * up.G};
+  const int wk = waves_for(up.G / kGW);
+  const bool multi = wk * kGW < up.G;
+  const LdsLayout L(1, up.G, wk, BITS == 4);
+  // sixteen waves a CU, and every workgroup the same number of row tiles
+  int resident = 256 * (16 / wk) / rows;
+  if (resident < 1) resident = 1;
+  const int turns = (up.n_tiles + resident - 1) / resident;
+  const dim3 grid((up.n_tiles + turns - 1) / turns, rows), block(wk * kWave);
+#define LLMQ_ROUTED(KERNEL, GRID, BLOCK, LDS, ...)                                                  \
+  do {                                                                                              \
+    auto kernel = KERNEL;                                                                           \
+    static bool raised = false; /* per instantiation; worst case two threads both set it */        \
+    if ((LDS) > kLdsDefault && !raised) {                                                           \
+      const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),             \
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax - 1024); \
+      if (err != hipSuccess) {                                                                      \
+        set_error("raising the LDS limit failed: %s", hipGetErrorString(err));                      \
+        return static_cast<int>(err);                                                               \
+      }                                                                                             \
+      raised = true;                                                                                \
+    }                                                                                               \
+    hipLaunchKernelGGL(kernel, GRID, BLOCK, LDS, stream, __VA_ARGS__);                              \
+    if (int rc = check_launch("wq_gemv_mfma_routed_kernel")) return rc;                             \
+  } while (0)
+  if (multi) LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 512, true>), grid, block, L.total, up, route);
+  else if (wk <= 4) LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 256, false>), grid, block, L.total, up, route);
+  else if (wk <= 8) LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 512, false>), grid, block, L.total, up, route);
+  else LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 1024, false>), grid, block, L.total, up, route);
+
+  MfmaArgs down{};
+  down.x = act; down.qw = q2; down.ws = s2; down.out = out;
+  down.N = H; down.G = I / kGroup; down.x_row_stride = -1;
+  down.row_bytes = I * BITS / 8;
+  // tiles of eight rows (the other lanes repeat them) where sixteen would leave CUs without a workgroup
+  down.tile_rows = static_cast<int64_t>(H) * tokens <= 128 * kTileRows ? 8 : kTileRows;
+  down.n_tiles = (H + down.tile_rows - 1) / down.tile_rows;
+  route.weight_stride = static_cast<int64_t>(H) * down.row_bytes;
+  route.scale_stride = static_cast<int64_t>(H) * down.G;
+  const int units = top_k * (down.G / kGW), waves = units < 16 ? units : 16;
+  const int lds = routed_down_lds(top_k, down.G, BITS == 4);
+  LLMQ_ROUTED((wq_gemv_mfma_routed_down_kernel<T, BITS>), dim3(down.n_tiles, tokens), dim3(waves * kWave), lds, down, route,
+              weights);
+#undef LLMQ_ROUTED
+  return 0;
+}
+}  // namespace
+
+bool experts_direct_supported(int tokens, int top_k, int n_experts, int hidden, int intermediate, bool int4) {
+  if (tokens < 1 || tokens > 2048 || top_k < 1 || top_k > kRoutedMaxTopK || n_experts < 1) return false;
+  if (hidden < kGroup * kGW || intermediate < kGroup * kGW || hidden % (kGroup * kGW) || intermediate % (kGroup * kGW))
+    return false;
+  if (hidden > (1 << 20) || intermediate / (kGroup * kGW) > kRoutedMaxChunks) return false;
+  return LdsLayout(1, hidden / kGroup, waves_for(hidden / kGroup / kGW), int4).total <= kLdsMax - 1024 &&
+         routed_down_lds(top_k, intermediate / kGroup, int4) <= kLdsMax - 2048;
+}
+
+int experts_direct_launch(const void* x, const int64_t* index, const void* weights, const void* gate_up,
+                          const float* gate_up_scale, const void* down, const float* down_scale, void* out, void* act,
+                          int tokens, int top_k, int n_experts, int hidden, int intermediate, int wformat, int dtype,
+                          hipStream_t stream) {
+#define LLMQ_DISPATCH(T, BITS)                                                                                      \
+  launch_routed<T, BITS>(static_cast<const T*>(x), index, static_cast<const T*>(weights),                         \
+                         static_cast<const uint8_t*>(gate_up), gate_up_scale, static_cast<const uint8_t*>(down),  \
+                         down_scale, static_cast<T*>(out), static_cast<T*>(act), tokens, top_k, n_experts, hidden, \
+                         intermediate, stream)
+  const bool int4 = wformat == LLMQ_W_INT4_PACKED;
+  switch (dtype) {
+    case LLMQ_F32: return int4 ? LLMQ_DISPATCH(float, 4) : LLMQ_DISPATCH(float, 8);
+    case LLMQ_F16: return int4 ? LLMQ_DISPATCH(f16_t, 4) : LLMQ_DISPATCH(f16_t, 8);
+    case LLMQ_BF16: return int4 ? LLMQ_DISPATCH(bf16_t, 4) : LLMQ_DISPATCH(bf16_t, 8);
   }
 #undef LLMQ_DISPATCH
   return fail_invalid("x must be float32, float16 or bfloat16, got dtype code %d", dtype);

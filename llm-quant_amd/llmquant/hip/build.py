@@ -91,6 +91,10 @@ def load_capi() -> ctypes.CDLL:
     lib.llmq_wq_gemv_batched_fused.restype = c_int
     lib.llmq_moe_combine.argtypes = [c_p] * 4 + [c_int] * 5 + [c_p]
     lib.llmq_moe_combine.restype = c_int
+    lib.llmq_wq_experts_direct_supported.argtypes = [c_int] * 6
+    lib.llmq_wq_experts_direct_supported.restype = c_int
+    lib.llmq_wq_experts_direct.argtypes = [c_p] * 9 + [c_int] * 7 + [c_p]
+    lib.llmq_wq_experts_direct.restype = c_int
     lib.llmq_wq_experts_supported.argtypes = [c_int] * 5
     lib.llmq_wq_experts_supported.restype = c_int
     lib.llmq_wq_experts_workspace_bytes.argtypes = [c_int] * 5

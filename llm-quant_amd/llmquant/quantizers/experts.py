@@ -130,7 +130,7 @@ class RealQuantExperts(_QuantExperts):
 
 
 class KernelQuantExperts(_QuantExperts):
-    """Every routed expert of a projection in one launch of the batched GEMV.
+    """Every routed expert of a projection in one launch: by row for up to eight tokens, by grouped GEMM beyond.
 
     4-bit stacks live in HBM nibble-packed ([E, N, groups, gs/2] uint8, the bytes of the packed
     file); `qgate_up` / `qdown` hand back the canonical int8 view on demand."""
@@ -277,8 +277,26 @@ class KernelQuantExperts(_QuantExperts):
                 and self._ext.wq_experts_supported(hidden_states.shape[0], top_k_index.shape[1], self.num_experts,
                                                    self.hidden_dim, self.intermediate_dim))
 
+    def _takes_direct(self, hidden_states, top_k_index, top_k_weights) -> bool:
+        """Whether a few tokens go through the two-launch form, where every (token, slot) row reads its expert's id
+        itself and its expert's weight for itself: the four-launch form's conditions, and rows that fit the LDS of the
+        launch that adds a token's experts up. It is the faster one at every count of tokens up to the batched GEMV's
+        reach, although it shares no weight between tokens. Measured, graph replay, us, four launches / two / the
+        grouped GEMMs: 64 experts, 8 a token, 2048 x 1024 int4, 1 token 21.4 / 12.8 / 33.4, 2: 38.8 / 15.2 / 34.9,
+        4: 57.1 / 23.2 / 36.5, 8: 85.8 / 39.3 / 49.5, int8 1: 24.3 / 16.1 / 41.4, 8: 99.5 / 62.8 / 75.9; 8 experts, 2 a
+        token, 2048 x 4096 int4 1: 17.3 / 12.7 / 47.9, 8: 87.7 / 38.8 / 50.6, int8 8: 97.9 / 62.2 / 65.7."""
+        return (self._act_is_silu and self._weight_args.group_size == 128
+                and self._gate_up_padded == self.hidden_dim and self._down_padded == self.intermediate_dim
+                and self.sgate_up.shape[1] == self.gate_up_data.shape[1] and self.sdown.shape[1] == self.down_data.shape[1]
+                and hidden_states.dim() == 2 and hidden_states.is_contiguous()
+                and top_k_weights.dtype == hidden_states.dtype and top_k_weights.shape == top_k_index.shape
+                and top_k_index.dim() == 2 and top_k_index.shape[0] == hidden_states.shape[0]
+                and self._ext.wq_experts_direct_supported(hidden_states.shape[0], top_k_index.shape[1], self.num_experts,
+                                                          self.hidden_dim, self.intermediate_dim, 4 if self._packed else 8))
+
     def _forward_fused(self, hidden_states, top_k_index, top_k_weights):
-        """Plan, gate|up (storing act(gate) * up), down, weighted sum per token: four launches. With one
+        """Plan, gate|up (storing act(gate) * up), down, weighted sum per token: four launches (a token's rows too many
+        or too long for the two-launch form's LDS). With one
         token every row reads that token's activation, so `hidden_states[tokens_per_row]` is not formed."""
         ext = self._ext
         tokens, top_k = hidden_states.shape[0], top_k_index.shape[-1]
@@ -299,6 +317,9 @@ class KernelQuantExperts(_QuantExperts):
                 return self._ext.wq_experts(hidden_states, top_k_index, top_k_weights, self.gate_up_data, self.sgate_up,
                                             self.down_data, self.sdown)
             return self._each_hit_expert(hidden_states, top_k_index, top_k_weights)
+        if self._takes_direct(hidden_states, top_k_index, top_k_weights):
+            return self._ext.wq_experts_direct(hidden_states, top_k_index, top_k_weights, self.gate_up_data, self.sgate_up,
+                                               self.down_data, self.sdown)
         if self._fusable(hidden_states, top_k_index, top_k_weights):
             return self._forward_fused(hidden_states, top_k_index, top_k_weights)
         return self._forward_unfused(hidden_states, top_k_index, top_k_weights)

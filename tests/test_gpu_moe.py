@@ -286,6 +286,41 @@ def test_experts_that_are_not_silu_keep_the_unfused_forward(ext):
 
 
 @pytest.mark.parametrize("bits,dtype", [("int4", torch.bfloat16), ("int8", torch.bfloat16), ("int4", torch.float16),
+                                        ("int8", torch.float32)])
+@pytest.mark.parametrize("tokens,hidden,inter,experts,top_k", [
+    (1, 512, 512, 4, 1),       # one unit: a workgroup of one wave; sixteen-row tiles that fill half the chip
+    (3, 512, 512, 4, 2),
+    (1, 2048, 1024, 64, 8),    # a unit a wave, tiles of eight rows
+    (8, 2048, 1024, 64, 8),
+    (2, 512, 1536, 20, 16),    # 48 units on 16 waves, the largest top_k
+    (1, 8704, 8192, 3, 2),     # gate|up rows of more chunks than waves, down rows of sixteen chunks
+])
+def test_direct_launches_equal_the_planned_ones(ext, bits, dtype, tokens, hidden, inter, experts, top_k):
+    """Every row's own expert id instead of a plan: the same arithmetic, so the same bits, also for ids that one token
+    holds twice and ids outside the layer (counted with the nearest valid one by both)."""
+    from llmquant.quantizers import KernelQuantExperts
+
+    gen = torch.Generator(device="cuda").manual_seed(hidden + inter)
+    source = torch.nn.Module()
+    source.act_fn = torch.nn.SiLU()
+    for name, shape in (("gate_up_proj", (experts, 2 * inter, hidden)), ("down_proj", (experts, hidden, inter))):
+        weight = torch.randn(shape, device="cuda", generator=gen) * 0.05
+        setattr(source, name, torch.nn.Parameter(weight.to(dtype), requires_grad=False))
+    quant = KernelQuantExperts.from_experts(source, QuantConfig(mlp_weight=bits).scheme("mlp_weight"))
+    x = torch.randn(tokens, hidden, device="cuda", generator=gen).to(dtype)
+    weights, index = torch.randn(tokens, experts, device="cuda", generator=gen).softmax(-1).topk(top_k, dim=-1)
+    weights = weights.to(dtype)
+    odd = index.clone()
+    odd[0, 0], odd[-1, -1] = -3, experts + 5
+    if top_k > 1:
+        odd[0, 1] = odd[-1, 0]
+    assert quant._takes_direct(x, index, weights)
+    with torch.no_grad():
+        for ids in (index, odd, index.int()):
+            assert torch.equal(quant(x, ids, weights), quant._forward_fused(x, ids, weights))
+
+
+@pytest.mark.parametrize("bits,dtype", [("int4", torch.bfloat16), ("int8", torch.bfloat16), ("int4", torch.float16),
                                         ("int8", torch.float16)])
 @pytest.mark.parametrize("tokens,hidden,inter,experts,top_k,skew", [
     (9, 128, 128, 4, 2, False),      # one group a row, one column tile, runs of a few rows
