@@ -507,6 +507,16 @@ int llmq_argmax_advance_embed(const void* x, int n, int64_t* out_index, int64_t*
                               void* hidden_out_or_null, int hidden_dim, void* workspace, int dtype,
                               llmq_stream_t stream);
 
+/* What a decode step that does not continue from the one before reads, in one launch (the reference sets its step's
+ * inputs with a copy and a fill each, llmquant/runtime/graph_decode.py:131-140): *token = *token_src, *step64 and
+ * *position = position_value, *length = length_value, hidden_out[0 .. row_bytes) = embed[*token_src * row_bytes ..] (a
+ * token outside [0, vocab): a row of NaN). Every pointer may be null but for: a token or a row needs token_src, and
+ * embed and hidden_out (16-byte aligned, row_bytes a multiple of 16) go together. token may be token_src. */
+int llmq_seed_step(const int64_t* token_src_or_null, int64_t* token_or_null, int64_t* step64_or_null,
+                   int32_t* position_or_null, int32_t* length_or_null, int64_t position_value, int length_value,
+                   const void* embed_or_null, void* hidden_out_or_null, int row_bytes, int64_t vocab,
+                   llmq_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1453,6 +1453,46 @@ at::Tensor argmax_advance_embed(const at::Tensor& x, at::Tensor& token, at::Tens
   return out;
 }
 
+// position / length (int32 [1]) <- the values, and where given: token (int64 [1]) <- token_src (int64 [1]), step64 (int64
+// [1]) <- position, hidden_out <- embed[token_src].
+void seed_step(const c10::optional<at::Tensor>& token_src, const c10::optional<at::Tensor>& token,
+               const c10::optional<at::Tensor>& step64, at::Tensor& position, at::Tensor& length, int64_t position_value,
+               int64_t length_value, const c10::optional<at::Tensor>& embed, const c10::optional<at::Tensor>& hidden_out) {
+  auto one = [&](const at::Tensor& t, at::ScalarType type, const char* name) {
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == type && t.numel() == 1 && t.device() == position.device(), name,
+                " must be one ", type, " on the cache's GPU");
+  };
+  one(position, at::kInt, "position");
+  one(length, at::kInt, "length");
+  TORCH_CHECK(position_value >= INT32_MIN && position_value <= INT32_MAX && length_value >= INT32_MIN &&
+                  length_value <= INT32_MAX, "position and length must fit 32 bits, got ", position_value, " and ", length_value);
+  auto given = [](const c10::optional<at::Tensor>& t) { return t.has_value() && t->defined(); };
+  if (given(token_src)) one(*token_src, at::kLong, "token_src");
+  if (given(token)) one(*token, at::kLong, "token");
+  if (given(step64)) one(*step64, at::kLong, "step64");
+  TORCH_CHECK(given(embed) == given(hidden_out), "embed and hidden_out go together");
+  int64_t row_bytes = 0, vocab = 0;
+  if (given(embed)) {
+    TORCH_CHECK(embed->device() == position.device() && embed->is_contiguous() && embed->dim() == 2,
+                "embed must be a contiguous [vocab, hidden] tensor on the cache's GPU");
+    TORCH_CHECK(hidden_out->device() == position.device() && hidden_out->is_contiguous() &&
+                    hidden_out->numel() == embed->size(1) && hidden_out->scalar_type() == embed->scalar_type(),
+                "hidden_out must be a contiguous tensor of ", embed->size(1), " elements of embed's dtype");
+    row_bytes = embed->size(1) * static_cast<int64_t>(embed->element_size());
+    TORCH_CHECK(row_bytes <= INT32_MAX, "embedding rows of ", row_bytes, " bytes");
+    vocab = embed->size(0);
+  }
+  const c10::OptionalDeviceGuard guard(at::device_of(position));
+  check_rc(llmq_seed_step(given(token_src) ? token_src->const_data_ptr<int64_t>() : nullptr,
+                          given(token) ? token->mutable_data_ptr<int64_t>() : nullptr,
+                          given(step64) ? step64->mutable_data_ptr<int64_t>() : nullptr, position.mutable_data_ptr<int32_t>(),
+                          length.mutable_data_ptr<int32_t>(), position_value, static_cast<int>(length_value),
+                          given(embed) ? embed->const_data_ptr() : nullptr,
+                          given(hidden_out) ? hidden_out->mutable_data_ptr() : nullptr, static_cast<int>(row_bytes), vocab,
+                          current_stream(position)),
+           "seed_step");
+}
+
 // argmax_row plus: token <- index, step64 += 1, step32 += 1 (one-element int64 / int64 / int32 device tensors).
 at::Tensor argmax_advance(const at::Tensor& x, at::Tensor& token, at::Tensor& step64, at::Tensor& step32) {
   TORCH_CHECK(x.is_cuda() && x.is_contiguous() && x.numel() > 0, "x must be a non-empty contiguous CUDA tensor");
@@ -1630,6 +1670,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "argmax_advance over 32 workgroups; with embed / hidden_out also hidden_out <- embed[index]", py::arg("x"),
         py::arg("token"), py::arg("step64"), py::arg("step32"), py::arg("embed") = py::none(),
         py::arg("hidden_out") = py::none(), py::arg("workspace"));
+  m.def("seed_step", &seed_step, "Token, positions, cache length and embedding row of a decode step in one launch",
+        py::arg("token_src"), py::arg("token"), py::arg("step64"), py::arg("position"), py::arg("length"),
+        py::arg("position_value"), py::arg("length_value"), py::arg("embed"), py::arg("hidden_out"));
   m.def("argmax_workspace_ints", []() { return static_cast<int64_t>((llmq_argmax_workspace_bytes() + 3) / 4); },
         "elements of the int32 zeros tensor argmax_advance_embed takes as workspace");
   m.def("argmax_advance", &argmax_advance, "argmax_row, then token <- index, step64 += 1, step32 += 1",

@@ -129,6 +129,8 @@ def load_capi() -> ctypes.CDLL:
     lib.llmq_prefill_attention.restype = c_int
     lib.llmq_argmax_advance_embed.argtypes = [c_p, c_int, c_p, c_p, c_p, c_p, c_p, c_p, c_int, c_p, c_int, c_p]
     lib.llmq_argmax_advance_embed.restype = c_int
+    lib.llmq_seed_step.argtypes = [c_p] * 5 + [c_i64, c_int, c_p, c_p, c_int, c_i64, c_p]
+    lib.llmq_seed_step.restype = c_int
     lib.llmq_argmax_workspace_bytes.argtypes = []
     lib.llmq_argmax_workspace_bytes.restype = ctypes.c_size_t
     lib.llmq_wq_gemm_a8.argtypes = [c_p] * 6 + [c_int] * 7 + [c_p]

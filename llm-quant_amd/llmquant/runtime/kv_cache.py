@@ -58,9 +58,16 @@ class KernelQuantCache:
 
     def set_position(self, position: int) -> None:
         """Next write position (host call; inside a graph the tensors are advanced instead)."""
+        self.set_counters(position, position)
+
+    def set_counters(self, position: int, length: int) -> None:
+        """Write position and valid length, one launch on the GPU."""
         self._host_length = position
-        self.position.fill_(position)
-        self.length.fill_(position)
+        if self.position.is_cuda:
+            self._ext.seed_step(None, None, None, self.position, self.length, position, length, None, None)
+        else:
+            self.position.fill_(position)
+            self.length.fill_(length)
 
     def advance(self, tokens: int = 1) -> None:
         """Move the write position forward on the device (capturable)."""

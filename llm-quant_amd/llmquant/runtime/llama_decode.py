@@ -206,8 +206,7 @@ class LlamaKernelRuntime:
         tokens = ids.shape[0]
         if tokens + 1 > self.max_len:
             raise ValueError(f"prompt of {tokens} tokens does not fit a cache of {self.max_len}")
-        self.cache.set_position(0)
-        self.cache.length.fill_(tokens)
+        self.cache.set_counters(0, tokens)
         logits = self._forward(ids, self.cos_table[:tokens], self.sin_table[:tokens], decode=False)
         self.cache.set_position(tokens)
         # (one row of logits: the kernel that the decode step uses, first maximum like torch.argmax)
@@ -228,9 +227,18 @@ class LlamaKernelRuntime:
         return logits, nxt
 
     def _set_step_inputs(self, token, position: int):
-        self.token.copy_(token.reshape(1))
-        self.pos_index.fill_(position)
-        self.cache.set_position(position)
+        self._seed(token, position, None, None)
+
+    def _seed(self, token, position: int, embed, hidden_out):
+        """Token and position of the next step onto the device, and with `embed` the token's row of it into
+        `hidden_out`: one launch (a token that is not an int64 on this GPU is copied and cast by PyTorch first)."""
+        if token.numel() != 1 or token.dtype != torch.long or token.device != self.token.device:
+            self.token.copy_(token.reshape(1))
+            token = self.token
+        cache = self.cache
+        cache._host_length = position
+        self._ext.seed_step(token, self.token, self.pos_index, cache.position, cache.length, position, position, embed,
+                            hidden_out)
 
     @torch.no_grad()
     def capture(self, token, position: int):

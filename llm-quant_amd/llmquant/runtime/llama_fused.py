@@ -332,10 +332,17 @@ class LlamaFusedRuntime(LlamaKernelRuntime):
         return splits
 
     def _set_step_inputs(self, token, position: int):
-        super()._set_step_inputs(token, position)
         self._splits_now = self._splits_for(position)
+        table = self.model.model.embed_tokens
+        # (the table that the captured step looks its next rows up in, and nothing that watches the module's calls)
+        if (self._embed_table is not None and type(table) is torch.nn.Embedding
+                and table.weight.data_ptr() == self._embed_table.data_ptr()
+                and not (table._forward_hooks or table._forward_pre_hooks)):
+            self._seed(token, position, self._embed_table, self._hidden0)
+            return
+        super()._set_step_inputs(token, position)
         if self._embed_table is not None:
-            self._hidden0.copy_(self.model.model.embed_tokens(self.token))
+            self._hidden0.copy_(table(self.token))
 
     def _use_graph_of(self, splits: int) -> bool:
         kept = self._graphs.get(splits)

@@ -374,6 +374,31 @@ def test_argmax_advance_embed_picks_the_same_token_and_hands_over_its_row(ext, d
         ext.argmax_advance_embed(x, token, step64, step32, None, None, ws[:8])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hidden", [8, 64, 2056, 8192])   # one packet; within, just past and four times a workgroup's reach
+def test_seed_step_sets_what_a_step_reads(ext, dtype, hidden):
+    table = torch.randn(50, hidden, generator=torch.Generator().manual_seed(hidden)).to(dtype).cuda()
+    row = torch.zeros(1, hidden, dtype=dtype, device="cuda")
+    token, step64 = (torch.zeros(1, dtype=torch.long, device="cuda") for _ in range(2))
+    position, length = (torch.zeros(1, dtype=torch.int32, device="cuda") for _ in range(2))
+    for value in (0, 49):
+        given = torch.tensor([value], device="cuda")
+        ext.seed_step(given, token, step64, position, length, 7 + value, 9, table, row)
+        assert (token.item(), step64.item(), position.item(), length.item()) == (value, 7 + value, 7 + value, 9)
+        assert torch.equal(row[0], table[value])
+    ext.seed_step(token, token, step64, position, length, 3, 3, table, row)   # the token where it already lies
+    assert token.item() == 49 and position.item() == 3 and torch.equal(row[0], table[49])
+    for outside in (-1, 50):
+        ext.seed_step(torch.tensor([outside], device="cuda"), token, step64, position, length, 3, 3, table, row)
+        assert torch.isnan(row).all()
+    ext.seed_step(None, None, None, position, length, 5, 6, None, None)       # only the cache's counters
+    assert (token.item(), step64.item(), position.item(), length.item()) == (50, 3, 5, 6)
+    with pytest.raises(RuntimeError, match="go together"):
+        ext.seed_step(token, token, step64, position, length, 0, 0, table, None)
+    with pytest.raises(RuntimeError, match="needs a token"):
+        ext.seed_step(None, None, None, position, length, 0, 0, table, row)
+
+
 def test_fused_runtime_equals_the_unfused_one():
     """Whole decode steps on a small model: fused and operation-by-operation runtimes give the
     same logits to the bit (hidden 512: the variance reduction happens to agree), the same
