@@ -642,6 +642,28 @@ def test_dense_linear_takes_a_shape_the_library_has_no_plan_for():
     assert torch.equal(ext.dense_linear(x, w), first)
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("n,groups,out_group,keep", [
+    (70, 3, 0, 40), (70, 3, 7, 40),        # five packets to a group: no shift; rows that share scales, a last tile of them
+    (1, 1, 0, 8), (1025, 1, 64, 0),        # one packet; just past a workgroup's four packets a thread
+    (16640, 32, 0, 0), (16640, 32, 128, 0),  # more packets than the grid covers at once: a second stripe, partly filled
+])
+def test_dequant_weight_indexing(bits, n, groups, out_group, keep):
+    """Codes and scales are found by shift or division, per row or shared, in one stripe or more: bit for bit."""
+    from llmquant.hip import load_extension
+
+    gen = torch.Generator(device="cuda").manual_seed(n + groups)
+    codes = torch.randint(-8 if bits == 4 else -127, 8 if bits == 4 else 128, (n, groups, GROUP), device="cuda", generator=gen,
+                          dtype=torch.int8)
+    biased = (codes + 8).to(torch.uint8)
+    stored = codes if bits == 8 else biased[..., 0::2] | (biased[..., 1::2] << 4)
+    scales = torch.rand(-(-n // out_group) if out_group else n, groups, device="cuda", generator=gen) + 0.01
+    rows = scales.repeat_interleave(out_group, 0)[:n] if out_group else scales
+    want = (codes[..., :keep or GROUP].float() * rows[..., None]).to(torch.bfloat16).reshape(n, -1)
+    got = load_extension().dequant_weight(stored.contiguous(), scales, out_group, keep, torch.bfloat16)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("bits", [8, 4])
 def test_wq_dense_linear_is_dequantize_then_matmul(bits):
     """One call for the dense branch: the dequantized matrix (bit-exact, tested above) times x, whole
