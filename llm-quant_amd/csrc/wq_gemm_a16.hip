@@ -27,6 +27,8 @@
 // and issues 4 MFMAs per activation tile. The next group's transfer and codes are requested once this group's
 // operands are in registers. Rows past M or N are clamped for the loads and dropped at the store, so the load
 // sequence is the same for every lane.
+#include <type_traits>
+
 #include "llmq_device.h"
 
 namespace {
@@ -74,9 +76,10 @@ __device__ __forceinline__ typename Mfma16<T>::Vec codes_to_operand(const uint32
   using E = typename Mfma16<T>::Elem;
   typename Mfma16<T>::Vec v;
   if constexpr (BITS == 4) {
-    const uint32_t w = raw[step];  // nibble i: even i is the low nibble of byte i/2, +8 biased
+    // nibble i (even i is the low nibble of byte i/2) is code + 8: with its top bit flipped, the code in two's complement
+    const uint32_t w = raw[step] ^ 0x88888888u;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = static_cast<E>(static_cast<float>(static_cast<int>((w >> (4 * i)) & 0xfu) - 8));
+    for (int i = 0; i < 8; ++i) v[i] = static_cast<E>(static_cast<float>(static_cast<int>(w << (28 - 4 * i)) >> 28));
   } else {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -86,11 +89,11 @@ __device__ __forceinline__ typename Mfma16<T>::Vec codes_to_operand(const uint32
   return v;
 }
 
-template <typename T, int BITS, int MT, int NT>
+template <typename T, int BITS, int MT, int NT, bool BIASED>
 __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A16Args a) {
   using Vec = typename Mfma16<T>::Vec;
   constexpr int kRaw = BITS == 4 ? 4 : 8;  // dwords of codes per lane per group and row tile
-  constexpr bool kBiased = BITS == 4 && MT <= 2;   // codes as biased operands (see multiply)
+  constexpr bool kBiased = BIASED;
   constexpr int kRows = NT * kTileN;       // weight rows of the workgroup
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   float* part = reinterpret_cast<float*>(smem);  // [waves][MT * 16][NT * 16]
@@ -105,33 +108,34 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   const int64_t K = static_cast<int64_t>(G) * kGroup;
 
   const int n0 = blockIdx.x * kRows;
-  const uint8_t* wrow[NT];
-  const float* srow[NT];
+  // (four row tiles: offsets of 32 bits from a scalar base instead of addresses; their registers are needed)
+  using Offset = typename std::conditional<NT == 4, uint32_t, int64_t>::type;
+  Offset wrow[NT], srow[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int n = min(n0 + nt * kTileN + j, a.N - 1);
-    wrow[nt] = a.qw + static_cast<int64_t>(n) * a.row_bytes + blk * (BITS == 4 ? 16 : 32);
-    srow[nt] = a.ws + static_cast<int64_t>(a.out_group > 0 ? n / a.out_group : n) * G;
+    wrow[nt] = static_cast<Offset>(n) * static_cast<Offset>(a.row_bytes) + blk * (BITS == 4 ? 16 : 32);
+    srow[nt] = static_cast<Offset>(a.out_group > 0 ? n / a.out_group : n) * G * 4;
   }
   // ---- x of one group: [16 MT rows][16 slots of 16 bytes], slot p of row r holds chunk p ^ (r & 15) ------------
   // transfer i of the wave covers rows 4 i .. 4 i + 3; lane = (row 4 i + lane / 16, slot lane % 16)
   constexpr int kXInstr = MT * 4;
   constexpr int kXTileBytes = MT * kTileM * kGroup * 2;
   unsigned char* xtile = smem + wv * kXTileBytes;
-  const unsigned char* xsrc[kXInstr];
+  Offset xsrc[kXInstr];
 #pragma unroll
   for (int i = 0; i < kXInstr; ++i) {
     const int row = 4 * i + (lane >> 4), chunk = (lane & 15) ^ (row & 15);
-    xsrc[i] = reinterpret_cast<const unsigned char*>(static_cast<const T*>(a.x) + static_cast<int64_t>(min(row, a.M - 1)) * K +
-                                                     chunk * 8);
+    xsrc[i] = static_cast<Offset>(min(row, a.M - 1)) * static_cast<Offset>(K * 2) + chunk * 16;
   }
   auto request_rows = [&](int g) {
+    const unsigned char* xg = static_cast<const unsigned char*>(a.x) + static_cast<int64_t>(g) * (kGroup * 2);
 #pragma unroll
     for (int i = 0; i < kXInstr; ++i) {
       // (four rows past the activation's end are not fetched: what the tile holds there feeds only result rows
       // that are dropped at the store)
       if (4 * i < a.M) {
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(xsrc[i] + static_cast<int64_t>(g) * (kGroup * 2)),
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(xg + xsrc[i]),
                                          reinterpret_cast<u32x4*>(xtile + 1024 * i), 16, 0, 0);
       }
     }
@@ -151,13 +155,13 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   auto load_weights = [&](int g, Weights& W) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      const uint8_t* p = wrow[nt] + static_cast<int64_t>(g) * (kGroup * BITS / 8);
+      const uint8_t* p = a.qw + static_cast<int64_t>(g) * (kGroup * BITS / 8) + wrow[nt];
 #pragma unroll
       for (int q = 0; q < kRaw / 4; ++q) {
         const u32x4 r = load16(p + 16 * q);
         W.raw[nt][4 * q] = r.x; W.raw[nt][4 * q + 1] = r.y; W.raw[nt][4 * q + 2] = r.z; W.raw[nt][4 * q + 3] = r.w;
       }
-      W.scale[nt] = srow[nt][g];
+      W.scale[nt] = *reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.ws + g) + srow[nt]);
     }
   };
   auto read_rows = [&](Rows& X) {
@@ -177,13 +181,13 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
-  // int4 codes, up to 32 activation rows: the codes become operands without a conversion per element (BiasedCodes:
-  // a nibble placed in the mantissa of 16.0 is the value 16 + n; converting the signed code takes five vector
-  // instructions per code, 160 per row tile and group). The matrix core then sums x (code + bias); bias * sum_k x
-  // comes out per group through four more MFMAs per activation tile against a vector of ones, shared by the
-  // workgroup's row tiles. Measured, 14336 x 4096 int4, M = 8 / 16 / 32: 16.0 / 16.4 / 21.9 -> 13.9 / 14.8 /
-  // 20.9 us; with three or four activation tiles the extra MFMAs take back what the conversion saves, and int8
-  // codes (a v_cvt_f32_ubyte each for bf16) gain nothing: those keep the signed conversion.
+  // BIASED (int4): the codes become operands without a conversion per element (BiasedCodes: a nibble placed in the
+  // mantissa of 16.0 is the value 16 + n: 0.9 vector instructions a code; the signed code takes 2.5). The matrix core then
+  // sums x (code + bias); bias * sum_k x comes out per group through four more MFMAs per activation tile against a vector
+  // of ones, and the activation's halves are interleaved, both shared by the workgroup's row tiles. It pays where they
+  // are: four row tiles, or two with up to two activation tiles. Measured, signed / biased us: 14336 x 4096 int4, four
+  // tiles, M = 16: 14.1 / 12.4, 32: 15.9 / 14.7, 48: 18.1 / 17.8; two, 16: 13.8 / 13.0, 48: 21.2 / 22.1; one,
+  // 4096 x 14336, 16: 12.4 / 12.8. int8 codes gain nothing: a v_cvt either way.
   using Codes = BiasedCodes<T, BITS>;
   uint32_t magic = Codes::kMagic;
   asm volatile("" : "+v"(magic));   // (in a vector register: see and_or)
@@ -269,19 +273,19 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   }
 }
 
-template <typename T, int BITS, int MT, int NT>
+template <typename T, int BITS, int MT, int NT, bool BIASED>
 int launch_tile(const A16Args& a, int wk, hipStream_t stream) {
   const int grid = (a.N + NT * kTileN - 1) / (NT * kTileN);
   // the waves' activation tiles, then (the same memory) their partial sums
   const int part = wk * MT * kTileM * NT * kTileN * static_cast<int>(sizeof(float));
   const int tiles = wk * MT * kTileM * kGroup * 2;
   const int lds = part > tiles ? part : tiles;
-  auto kernel = wq_gemm_a16_kernel<T, BITS, MT, NT>;
+  auto kernel = wq_gemm_a16_kernel<T, BITS, MT, NT, BIASED>;
   if (lds > 64 * 1024) {
     static bool raised = false;  // per instantiation; worst case two threads both set it
     if (!raised) {
       const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, kMaxWaves * MT * kTileM * kGroup * 2);
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
       if (err != hipSuccess) {
         llmq_host::set_error("raising the LDS limit failed: %s", hipGetErrorString(err));
         return static_cast<int>(err);
@@ -300,11 +304,17 @@ int launch_typed(const void* x, const void* qw, const float* ws, void* out, int 
   int wk = G < kMaxWaves ? G : kMaxWaves;
   // rows of few groups: two groups per wave at least
   if (G >= 4 && wk * 2 > G) wk = G / 2;
-  // Two row tiles per workgroup share the activation rows a wave loads (the activation comes from L2
-  // once per workgroup: 16 rows per workgroup make that traffic four times the codes' at M = 16),
-  // as long as a workgroup per CU and more is left. Measured, M = 8 / 64, 14336 x 4096 int4:
-  // 21 / 86 us with one tile, 17 / 48 us with two; 4096 x 4096: 7 / 23 against 9 / 24.
+  // Row tiles of a workgroup share the activation rows a wave loads: those come from L2 once per workgroup, and 16
+  // weight rows a workgroup make that traffic four times the codes' at M = 16. Two tiles as long as a workgroup per CU
+  // and more is left, four where that leaves most CUs one. Measured, us with 1 / 2 / 4 tiles: 14336 x 4096 int4 bf16
+  // M = 16: 14.6 / 13.0 / 12.4, 32: 19.6 / 17.8 / 14.7, 48: 29.4 / 21.2 / 17.8; int8 M = 32: 29.5 / 24.8 / 20.1;
+  // 28672 x 4096 int4 32: 41 / 39 / 31; 128256 x 2048 int4 M = 16: 62 / 49 / 56, 32: 90 / 93 / 70, 48: 160 / 108 / 87;
+  // 8192 x 2048 M = 32: 7.4 / 6.7 / 9.1; 4096 x 4096 M = 64: 10.2 / 13.7 / -. Four tiles against 64 rows, and int8 codes
+  // against 48, are more registers than a wave has (spills: 41 us against 26).
   const bool wide = N >= 2 * kTileN * 256;
+  const int quads = (N + 4 * kTileN - 1) / (4 * kTileN);
+  const int64_t limit = int64_t{1} << 32;   // the four-tile form's offsets from its scalar bases
+  const bool offsets32 = N * (K * BITS / 8) < limit && static_cast<int64_t>(N) * G * 4 < limit && kSlabRows * K * 2 < limit;
   // (Sixteen waves for few row tiles of long rows, down_proj, measured no faster than eight.)
   for (int m0 = 0; m0 < M; m0 += kSlabRows) {
     A16Args a{};
@@ -316,20 +326,30 @@ int launch_typed(const void* x, const void* qw, const float* ws, void* out, int 
     a.N = N; a.G = G; a.out_group = out_group;
     a.row_bytes = K * BITS / 8;
     const int mt = (a.M + kTileM - 1) / kTileM;
+    // Four row tiles (see above): outputs that still give three quarters of the CUs a workgroup; for one activation tile,
+    // where there are few rows to share, only where those workgroups are one round and rows long enough to fill it.
+    const bool four = quads >= 192 && offsets32 &&
+                      (mt == 1 ? quads <= 256 && G >= 32 : mt == 2 || (mt == 3 && BITS == 4));
     int rc;
-    if (wide) {
+    if (four) {
+      constexpr bool kBi = BITS == 4;
+      if (mt == 1) rc = launch_tile<T, BITS, 1, 4, kBi>(a, wk, stream);
+      else if (mt == 2) rc = launch_tile<T, BITS, 2, 4, kBi>(a, wk, stream);
+      else if constexpr (BITS == 4) rc = launch_tile<T, BITS, 3, 4, kBi>(a, wk, stream);
+      else rc = llmq_host::fail_invalid("internal: no such tile");
+    } else if (wide) {
       switch (mt) {
-        case 1: rc = launch_tile<T, BITS, 1, 2>(a, wk, stream); break;
-        case 2: rc = launch_tile<T, BITS, 2, 2>(a, wk, stream); break;
-        case 3: rc = launch_tile<T, BITS, 3, 2>(a, wk, stream); break;
-        default: rc = launch_tile<T, BITS, 4, 2>(a, wk, stream); break;
+        case 1: rc = launch_tile<T, BITS, 1, 2, BITS == 4>(a, wk, stream); break;
+        case 2: rc = launch_tile<T, BITS, 2, 2, BITS == 4>(a, wk, stream); break;
+        case 3: rc = launch_tile<T, BITS, 3, 2, false>(a, wk, stream); break;
+        default: rc = launch_tile<T, BITS, 4, 2, false>(a, wk, stream); break;
       }
     } else {
       switch (mt) {
-        case 1: rc = launch_tile<T, BITS, 1, 1>(a, wk, stream); break;
-        case 2: rc = launch_tile<T, BITS, 2, 1>(a, wk, stream); break;
-        case 3: rc = launch_tile<T, BITS, 3, 1>(a, wk, stream); break;
-        default: rc = launch_tile<T, BITS, 4, 1>(a, wk, stream); break;
+        case 1: rc = launch_tile<T, BITS, 1, 1, false>(a, wk, stream); break;
+        case 2: rc = launch_tile<T, BITS, 2, 1, false>(a, wk, stream); break;
+        case 3: rc = launch_tile<T, BITS, 3, 1, false>(a, wk, stream); break;
+        default: rc = launch_tile<T, BITS, 4, 1, false>(a, wk, stream); break;
       }
     }
     if (rc) return rc;

@@ -103,6 +103,21 @@ def test_llama_shapes_on_sampled_entries(ext, n, k, m, split):
     assert rel_l2(got[:, cols], exact) <= 2e-3
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k,out_group", [
+    (5, 12225, 4096, 0),                                              # four row tiles, one activation tile; ragged in rows
+    (17, 12289, 640, 0), (32, 12352, 512, 64), (33, 12289, 384, 0), (48, 12300, 256, 0),   # two and three activation tiles
+    (64, 12289, 256, 0), (16, 16448, 256, 0), (33, 8201, 384, 0),     # two row tiles: past 48 rows, short rows, fewer rows
+])
+def test_wide_outputs_take_more_row_tiles_a_workgroup(ext, bits, dtype, m, n, k, out_group):
+    x, q, s, canonical, scales = make_case(m, n, k, bits, dtype, out_group=out_group, seed=5)
+    got = to_np(ext.wq_gemm_a16(x.cuda(), q, s, out_group, False))
+    cols = np.r_[0:70, n // 2 // 64 * 64:n // 2 // 64 * 64 + 64, n - 70:n]
+    rows = scales[cols // out_group] if out_group else scales[cols]
+    assert rel_l2(got[:, cols], oracle.gemv_float64(to_np(x), canonical[cols], rows)) <= 2e-3
+
+
 def test_argument_checks(ext):
     x, q, s, _, _ = make_case(8, 64, 256, 4, torch.bfloat16)
     with pytest.raises(RuntimeError, match="float16 or bfloat16"):
