@@ -165,6 +165,37 @@ at::Tensor wq_gemv(const at::Tensor& x, const at::Tensor& qweight, const at::Ten
   return out;
 }
 
+at::Tensor wq_gemv_fused(const at::Tensor& x, const at::Tensor& qweight, const at::Tensor& wscale,
+                         int64_t out_group, int64_t prologue, const c10::optional<at::Tensor>& norm_weight,
+                         double eps, int64_t in_head_dim, const c10::optional<at::Tensor>& residual);
+
+// A Linear's whole forward for a row or two: x [..., K] -> [..., N], no other launch and no view in front of or behind it.
+// in_head_dim > 0: x holds heads of that many values, one to a group of 128 (M == 1; the GEMV pads them while it stages
+// the row). The module's own buffers: their shapes are checked by the entry points below it.
+at::Tensor wq_linear_rows(const at::Tensor& x, const at::Tensor& qweight, const at::Tensor& wscale, int64_t out_group,
+                          int64_t in_head_dim) {
+  at::Tensor out;
+  if (in_head_dim > 0) {
+    const auto xc = x.contiguous();
+    const auto wc = qweight.contiguous(), sc = wscale.contiguous();
+    const auto misaligned = (reinterpret_cast<uintptr_t>(xc.const_data_ptr()) | reinterpret_cast<uintptr_t>(wc.const_data_ptr()) |
+                             reinterpret_cast<uintptr_t>(sc.const_data_ptr())) & 15u;
+    if (misaligned || xc.numel() == 0) {
+      // (operands that the matrix-core GEMV does not take: padded here, for the other one)
+      out = wq_gemv(at::constant_pad_nd(xc.view({-1, in_head_dim}), {0, 128 - in_head_dim}).view({-1, wc.size(1) * 128}), wc,
+                    sc, out_group);
+    } else {
+      out = wq_gemv_fused(xc, wc, sc, out_group, LLMQ_PRO_NONE, {}, 0.0, in_head_dim, {});
+    }
+  } else {
+    out = wq_gemv(x, qweight, wscale, out_group);
+  }
+  if (x.dim() == 2) return out;
+  auto sizes = x.sizes().vec();
+  sizes.back() = out.size(1);
+  return out.view(sizes);
+}
+
 // x [R, G*gs]; qweight [E, N, G, gs] int8 or [E, N, G, gs/2] packed; wscale [E, scale_rows, G]; the plan is
 // three int32 device tensors of equal length. Returns [R, N]; rows no plan entry covers are zero.
 at::Tensor wq_gemv_batched(const at::Tensor& x, const at::Tensor& qweight, const at::Tensor& wscale,
@@ -1670,6 +1701,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "argmax_advance over 32 workgroups; with embed / hidden_out also hidden_out <- embed[index]", py::arg("x"),
         py::arg("token"), py::arg("step64"), py::arg("step32"), py::arg("embed") = py::none(),
         py::arg("hidden_out") = py::none(), py::arg("workspace"));
+  m.def("wq_linear_rows", &wq_linear_rows, "wq_gemv of a row or two with x's leading axes kept; heads padded in the launch",
+        py::arg("x"), py::arg("qweight"), py::arg("wscale"), py::arg("out_group"), py::arg("in_head_dim"));
   m.def("seed_step", &seed_step, "Token, positions, cache length and embedding row of a decode step in one launch",
         py::arg("token_src"), py::arg("token"), py::arg("step64"), py::arg("position"), py::arg("length"),
         py::arg("position_value"), py::arg("length_value"), py::arg("embed"), py::arg("hidden_out"));

@@ -130,6 +130,8 @@ class KernelQuantLinear(nn.Module):
     """Linear over a canonical quantized weight: [N, groups, group_size] codes with padding
     and head splits already applied, plus fp32 scales [scale_rows, groups]."""
 
+    _few_elements, _head_rows = -1, 0   # (of a module pickled without them)
+
     def __init__(self, qweight, wscale, bias, scheme: QuantizationScheme, in_features: int):
         super().__init__()
         bits = scheme.weights.num_bits
@@ -174,6 +176,17 @@ class KernelQuantLinear(nn.Module):
         # looked up once: a decode step runs ~113 of these modules
         self._ext = load_extension()
         self._gemv = self._ext.wq_gemv
+        # One or two rows go to the GEMV whatever their type, and the launch takes a few microseconds: the host's way to it
+        # (shapes, the routing questions below, views) took twice that (2048 x 2048 int8, calls back to back: 9.9 us a
+        # call, 5.4 through forward's first branch). Elements of x up to which that branch applies; -1: never. One row of
+        # 64- or 32-wide heads is padded inside the launch where the matrix-core GEMV takes it.
+        self._few_elements = -1
+        self._head_rows = 0
+        if not self._int8_act:
+            if not self._needs_padding:
+                self._few_elements = (FUSED_GEMM_MIN_ROWS - 1) * self.in_features
+            elif self._head_keep and group_size == 128 and stored.shape[1] % 4 == 0 and self._head_keep % 8 == 0:
+                self._few_elements, self._head_rows = self.in_features, self._head_keep
 
     # the loaded extension is a module object, which copy and pickle refuse: a copy (copy.deepcopy(model),
     # torch.save of the module) carries everything else and looks the extension up again
@@ -255,19 +268,24 @@ class KernelQuantLinear(nn.Module):
         return rows @ self._dequantized_weight(rows.dtype, real_width).T
 
     def forward(self, x):
+        # (the buffers through their dict: nn.Module.__getattr__ costs a third of a microsecond a look)
+        held, bias = self._buffers, self.bias
+        qdata, wscale = held["qdata"], held["wscale"]
+        if bias is None and x.numel() <= self._few_elements and x.shape[-1] == self.in_features:
+            return self._ext.wq_linear_rows(x, qdata, wscale, self.out_group, self._head_rows)
         rows = x.reshape(-1, x.shape[-1])
+        count, groups = rows.shape[0], qdata.shape[1]
+        sixteen = rows.dtype in (torch.bfloat16, torch.float16) and self._fused_max_rows > 0 and not self._int8_act
         # (heads padded to groups: above 64 rows the dense branch on the real width reads half the codes)
-        fused = (self._fused_max_rows > 0 and fused_gemm_takes(rows.shape[0], self.out_features, self.qdata.shape[1])
-                 and (rows.shape[0] <= self._fused_max_rows or not self._head_keep)
-                 and rows.dtype in (torch.bfloat16, torch.float16) and not self._int8_act)
-        tiled = (self._fused_max_rows > 0 and rows.dtype in (torch.bfloat16, torch.float16) and not self._int8_act
-                 and tiled_gemm_pays(rows.shape[0], self.out_features, self.qdata.shape[1],
-                                     4 if self.qdata.dtype == torch.uint8 else 8))
-        if rows.shape[0] > KERNEL_MAX_ROWS and not self._int8_act and self._head_keep and not fused and not tiled:
+        fused = (sixteen and fused_gemm_takes(count, self.out_features, groups)
+                 and (count <= self._fused_max_rows or not self._head_keep))
+        tiled = (sixteen and count > FUSED_GEMM_MAX_ROWS
+                 and tiled_gemm_pays(count, self.out_features, groups, 4 if self._packed else 8))
+        if count > KERNEL_MAX_ROWS and not self._int8_act and self._head_keep and not fused and not tiled:
             # dense branch on the real width: neither the activation nor the weight is padded
             out = self._dense(rows, real_width=True)
-            if self.bias is not None:
-                out = out + self.bias.to(out.dtype)
+            if bias is not None:
+                out = out + bias.to(out.dtype)
             return out.reshape(*x.shape[:-1], self.out_features).to(x.dtype)
         if self._needs_padding:
             rows = pad_activation(rows, self._weight_args)
@@ -286,16 +304,17 @@ class KernelQuantLinear(nn.Module):
                                        x.dtype, self.a8_exact)
             return out.reshape(*x.shape[:-1], self.out_features)
         if fused:
-            out = self._ext.wq_gemm_a16(rows, self.qdata, self.wscale, self.out_group,
-                                        fused_gemm_splits(rows.shape[0], self.qdata.shape[1]))
-        elif rows.shape[0] <= KERNEL_MAX_ROWS:
-            out = self._gemv(rows, self.qdata, self.wscale, self.out_group)
+            out = self._ext.wq_gemm_a16(rows, qdata, wscale, self.out_group, fused_gemm_splits(count, groups))
+        elif count <= KERNEL_MAX_ROWS:
+            out = self._gemv(rows, qdata, wscale, self.out_group)
         elif tiled:
-            out = self._ext.wq_gemm_a16_tile(rows, self.qdata, self.wscale, self.out_group)
+            out = self._ext.wq_gemm_a16_tile(rows, qdata, wscale, self.out_group)
         else:
             out = self._dense(rows)
-        if self.bias is not None:
-            out = out + self.bias.to(out.dtype)
+        if bias is not None:
+            out = out + bias.to(out.dtype)
+        if x.dim() == 2 and out.dtype == x.dtype:
+            return out
         return out.reshape(*x.shape[:-1], self.out_features).to(x.dtype)
 
     def extra_repr(self):

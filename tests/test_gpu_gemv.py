@@ -664,6 +664,33 @@ def test_dequant_weight_indexing(bits, n, groups, out_group, keep):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("spec,width", [(dict(), 640), (dict(), 600), (dict(head_dim=64), 8 * 64), (dict(head_dim=32), 4 * 32),
+                                        (dict(head_dim=64), 6 * 64), (dict(out_group=64), 512)])
+def test_the_short_way_of_a_row_or_two_is_the_general_one(bits, spec, width):
+    """KernelQuantLinear.forward on few rows (its first branch) against the same module without that branch, to the bit:
+    rows, leading axes, types, strides and alignments; padded widths, heads and a bias keep their own ways."""
+    from llmquant.quantizers import KernelQuantLinear
+
+    gen = torch.Generator().manual_seed(width + bits)
+    for bias in (False, True):
+        linear = nn.Linear(width, 192, bias=bias).to(torch.bfloat16)
+        with torch.no_grad():
+            linear.weight.normal_(0, 0.05, generator=gen)
+        short = KernelQuantLinear.from_linear(linear.cuda(), weight_only(bits, **spec))
+        general = KernelQuantLinear.from_linear(linear.cuda(), weight_only(bits, **spec))
+        general._few_elements = -1
+        for dtype in (torch.bfloat16, torch.float16, torch.float32):
+            base = torch.randn(6, width + 8, generator=gen).to(dtype).cuda()
+            for x in (base[0, :width], base[:1, :width], base[:2, :width], base[:3, :width], base[None, 1:2, :width],
+                      base[0, 1:width + 1], base[:1, 1:width + 1], base[::2, :width][:2], base[:0, :width],
+                      base[:0, :width].reshape(2, 0, width), base[:2, :width][:, None].expand(2, 1, width)):
+                got, want = short(x), general(x)
+                assert got.shape == want.shape and got.dtype == want.dtype and torch.equal(got, want)
+        with pytest.raises(RuntimeError):
+            short(torch.zeros(1, width + 128, dtype=torch.bfloat16, device="cuda"))
+
+
 @pytest.mark.parametrize("bits", [8, 4])
 def test_wq_dense_linear_is_dequantize_then_matmul(bits):
     """One call for the dense branch: the dequantized matrix (bit-exact, tested above) times x, whole
