@@ -27,7 +27,7 @@
 // group's activation sum, cut into three bf16 pieces, against the constant -B. The fp32 group sum is then
 // folded into the fp32 total with one multiply-add by the group's weight scale.
 //
-// The activation is prepared once per call by act_prep_kernel: rows padded to whole tiles, within every
+// A bfloat16 activation is prepared once per call by act_prep_kernel: rows padded to whole tiles, within every
 // 16-byte chunk the eight values reordered to (0, 4, 1, 5, 2, 6, 3, 7), the order in which the AND-OR above
 // leaves the codes (a sum does not care about the order of its terms, as long as both operands agree), and
 // the per-group sums written as records of bf16 pieces.
@@ -50,8 +50,8 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
 // bfloat16: the matrix core sums x * (code + B) and B * sum x is taken out again (below). float16 has the mantissa
 // to hold B + code as well, but the pieces of a group's activation sum do not fit its exponent range (128 values of
-// up to 65504, and pieces of a small sum fall below its smallest step), so there the bias is subtracted from the
-// operand itself, exactly, with one packed add per two codes, and there is no correction step.
+// up to 65504, and pieces of a small sum fall below its smallest step), so there the bias is taken off the
+// operand itself, exactly, with one packed instruction per two codes, and there is no correction step (operand_words).
 template <typename T> constexpr bool kBiased = std::is_same<T, bf16_t>::value;
 typedef float v16f __attribute__((ext_vector_type(16)));
 
@@ -105,9 +105,10 @@ template <typename T>
 __device__ __forceinline__ void emit_prepared(const u32x4 v, const bool active, const bool first_of_row,
                                               u32x4* __restrict__ chunk_out, u32x4* __restrict__ record_out) {
   if constexpr (!kBiased<T>) {
-    // (no correction step: the records stay part of the layout and are zeros)
+    // (the operands are in the chunk's own order, and without a correction step the records, which stay part of the
+    // layout, are read by nobody: a float16 activation in rows of its own needs no preparation)
     if (!active) return;
-    *chunk_out = interleave_halves(v);
+    *chunk_out = v;
     if (first_of_row) *record_out = u32x4{0u, 0u, 0u, 0u};
     return;
   }
@@ -237,19 +238,34 @@ template <int BITS> __device__ __forceinline__ int code_slot(int row, int c) {
 
 
 // The four operand words of a k-step of the wave (`raw`: its k-steps' codes one after the other, one 32-bit word
-// of int4 or two of int8 a step); operand word i pairs codes i and i + 4.
+// of int4 or two of int8 a step). bfloat16: word i pairs the biased codes i and i + 4. float16: word i pairs codes 2 i and
+// 2 i + 1, the order of the activation as it lies in memory, so that there nothing prepares it (333 x 14336 values: a
+// launch of 5.8 us; 333 x 4096 x 14336 int4 60.7 -> 55.2 us, 200 x 4096 x 4096 23.1 -> 19.9): a byte of two nibbles goes to both halves, the even code stays where it is (1024 + n) and the odd
+// one sixteen times as high (1024 + 16 n), and the multiply-add that takes the bias out brings it down, all exact.
+template <typename T, int BITS>
+constexpr uint32_t kOperandMagic = std::is_same<T, f16_t>::value && BITS == 4 ? 0x64006400u : BiasedCodes<T, BITS>::kMagic;
 template <typename T, int BITS>
 __device__ __forceinline__ u32x4 operand_words(const uint32_t* raw, int step, uint32_t magic) {
-  u32x4 w = BiasedCodes<T, BITS>::operand(raw, step, magic);
-  if constexpr (!kBiased<T>) {
-    const _Float16 b = static_cast<_Float16>(BiasedCodes<T, BITS>::kBias);
-    const h2 bias = {b, b};
-    w.x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, w.x) - bias);
-    w.y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, w.y) - bias);
-    w.z = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, w.z) - bias);
-    w.w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, w.w) - bias);
+  if constexpr (kBiased<T>) return BiasedCodes<T, BITS>::operand(raw, step, magic);
+  uint32_t out[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (BITS == 4) {
+      const uint32_t both = __builtin_amdgcn_perm(0u, raw[step], 0x0c000c00u | (i << 16) | i);
+      const h2 v = __builtin_bit_cast(h2, and_or(both, 0x00f0000fu, magic));
+      const h2 down = {static_cast<_Float16>(1.0f), static_cast<_Float16>(0.0625f)};
+      const h2 bias = {static_cast<_Float16>(-1032.0f), static_cast<_Float16>(-72.0f)};
+      out[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, down, bias));
+    } else {
+      // bytes 2 i and 2 i + 1 into the two halves, in the mantissa of 256.0
+      const uint32_t w = raw[2 * step + i / 2] ^ 0x80808080u;
+      const uint32_t pick = i % 2 ? 0x0c030c02u : 0x0c010c00u;
+      const h2 v = __builtin_bit_cast(h2, (__builtin_amdgcn_perm(0u, w, pick) << 2) | magic);
+      const h2 bias = {static_cast<_Float16>(-384.0f), static_cast<_Float16>(-384.0f)};
+      out[i] = __builtin_bit_cast(uint32_t, v + bias);
+    }
   }
-  return w;
+  return u32x4{out[0], out[1], out[2], out[3]};
 }
 
 template <typename T> __device__ __forceinline__ v16f mfma(const u32x4& a, const u32x4& b, const v16f& c) {
@@ -268,7 +284,8 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   static_assert(EPI == kEpiStore || (S::kBN == 256 && S::kKH == 1), "the gate|up epilogue is laid out for 128 + 128 columns");
   constexpr int kBM = S::kBM, kBN = S::kBN, kWaveM = S::kWaveM, kWaveN = S::kWaveN, kWaves = S::kWaves;
   constexpr int kThreads = S::kThreads, kTileBytes = S::kTileBytes, kMT = S::kMT, kNT = S::kNT;
-  constexpr int kRecTileBytes = S::kRecTileBytes, kRecWaves = S::kRecWaves, kScaleWaves = S::kScaleWaves;
+  // (float16: the records are not read)
+  constexpr int kRecTileBytes = S::kRecTileBytes, kRecWaves = kBiased<T> ? S::kRecWaves : 0, kScaleWaves = S::kScaleWaves;
   constexpr int kCodeTileB = S::template kCodeTileBytes<BITS>, kStageB = S::template kStageBytes<BITS>;
   constexpr int kStagesN = S::template kStages<BITS>;
   constexpr int kKH = S::kKH, kSteps = 8 / kKH;   // k-steps of a group that one wave multiplies
@@ -310,13 +327,14 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   // One instruction moves 64 x 16 bytes into 1 KB of consecutive LDS; which global chunk a lane fetches
   // for its place there carries the swizzle. The activation and its records are the kernel's own
   // buffers, padded to whole tiles of rows, so their rows need no clamping.
+  // (float16: an activation may be the caller's, whose last tile of rows repeats the last row.)
   // activation: instruction i of a wave = rows wv*16 + 4 i .. + 3, lane = (row, slot); slot p of row r
   // holds chunk p ^ (r & 15), and r & 15 = 4 i + lane / 16
   constexpr int kXInstr = kBM / 4 / kWaves;  // 4
   const uint32_t x_row_bytes = static_cast<uint32_t>(a.G) * kRowBytes;
   // row `row` of the tile in the prepared activation (GROUPED: rows past the run's end repeat its last one)
   auto source_row = [&](int row) {
-    if constexpr (!GROUPED) return static_cast<uint32_t>(m0 + row);
+    if constexpr (!GROUPED) return static_cast<uint32_t>(kBiased<T> ? m0 + row : min(m0 + row, m_end - 1));
     const int r = min(m0 + row, m_end - 1);
     return static_cast<uint32_t>(a.row_source != nullptr ? a.row_source[r] : r);
   };
@@ -344,7 +362,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   // scales (kScaleWaves waves, 64 columns each).
   constexpr int kExtraWaves = kLeftCodes + kRecWaves + kScaleWaves;
   static_assert(kExtraWaves <= kWaves, "at most one transfer instruction per wave beyond the even share");
-  const int rec_wave = (wv + kWaves - kLeftCodes) % kWaves % kRecWaves;
+  const int rec_wave = (wv + kWaves - kLeftCodes) % kWaves % (kRecWaves ? kRecWaves : 1);
   const int scale_wave = (wv + kWaves - kLeftCodes - kRecWaves) % kWaves % kScaleWaves;
   const uint32_t r_off = source_row(rec_wave * 64 + lane) * a.G * 16;
   const float* sw_lane;
@@ -421,7 +439,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
     for (int ni = 0; ni < kNT; ++ni)
 #pragma unroll
       for (int r = 0; r < 16; ++r) total[mi][ni][r] = 0.0f;
-  uint32_t sixteen = BiasedCodes<T, BITS>::kMagic;  // 16.0 (int8 in float16: 256.0) twice; kept in a vector register (see and_or)
+  uint32_t sixteen = kOperandMagic<T, BITS>;  // 16.0 (float16: 1024.0, int8 256.0) twice; kept in a vector register (see and_or)
   asm volatile("" : "+v"(sixteen));
   const uint32_t nb = bf16_bits_rne(-BiasedCodes<T, BITS>::kBias);  // exact (read where kBiased<T> only)
   const uint32_t nb2 = (lh || kh) ? 0u : (nb | (nb << 16));   // (the correction step belongs to the group's first k-steps)

@@ -153,16 +153,10 @@ int check_common(const void* x, bool prepared, const void* qweight, const float*
   return 0;
 }
 
-int prepare(const void* x, uint8_t* xp, uint8_t* rec, int M, int G, int dtype, hipStream_t s) {
+int prepare(const void* x, uint8_t* xp, uint8_t* rec, int M, int G, hipStream_t s) {
   const int64_t n_chunks = static_cast<int64_t>(M) * G * 16;
-  const dim3 grid(static_cast<unsigned>((n_chunks + 255) / 256));
-  if (dtype == LLMQ_BF16) {
-    hipLaunchKernelGGL(act_prep_kernel<bf16_t>, grid, dim3(256), 0, s, static_cast<const u32x4*>(x),
-                       reinterpret_cast<u32x4*>(xp), reinterpret_cast<u32x4*>(rec), n_chunks);
-  } else {
-    hipLaunchKernelGGL(act_prep_kernel<f16_t>, grid, dim3(256), 0, s, static_cast<const u32x4*>(x),
-                       reinterpret_cast<u32x4*>(xp), reinterpret_cast<u32x4*>(rec), n_chunks);
-  }
+  hipLaunchKernelGGL(act_prep_kernel<bf16_t>, dim3(static_cast<unsigned>((n_chunks + 255) / 256)), dim3(256), 0, s,
+                     static_cast<const u32x4*>(x), reinterpret_cast<u32x4*>(xp), reinterpret_cast<u32x4*>(rec), n_chunks);
   return llmq_host::check_launch("act_prep_kernel");
 }
 
@@ -187,11 +181,13 @@ int run_store(const void* x, const void* qweight, const float* wscale, void* out
     return llmq_host::fail_invalid("workspace of %zu bytes is too small, need %zu", workspace_bytes,
                                    p.xp_bytes + p.rec_bytes + p.partial_bytes);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
-  uint8_t* xp = ws;
+  const uint8_t* xp = ws;
   uint8_t* rec = ws + p.xp_bytes;
   float* partial = reinterpret_cast<float*>(ws + p.xp_bytes + p.rec_bytes);
-  if (x != nullptr) {
-    if (int rc = prepare(x, xp, rec, M, G, dtype, s)) return rc;
+  if (x != nullptr && dtype == LLMQ_F16) {
+    xp = static_cast<const uint8_t*>(x);   // (read as it lies)
+  } else if (x != nullptr) {
+    if (int rc = prepare(x, ws, rec, M, G, s)) return rc;
   }
   TileArgs a{xp, rec, static_cast<const uint8_t*>(qweight), wscale, out, partial, M, N, G, out_group,
              p.m_tiles, p.n_tiles, p.splits, p.groups_per_split, nullptr, nullptr, 0};
@@ -260,10 +256,12 @@ int run_gate_up_silu(const void* x, const void* qweight, const float* wscale, vo
     return llmq_host::fail_invalid("activation of %d x %d values is beyond the next GEMM's 32-bit offsets", M, I);
   hipStream_t s = static_cast<hipStream_t>(stream);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
-  uint8_t* xp = ws;
+  const uint8_t* xp = ws;
   uint8_t* rec = ws + p.xp_bytes;
-  if (x != nullptr) {
-    if (int rc = prepare(x, xp, rec, M, G, dtype, s)) return rc;
+  if (x != nullptr && dtype == LLMQ_F16) {
+    xp = static_cast<const uint8_t*>(x);   // (read as it lies)
+  } else if (x != nullptr) {
+    if (int rc = prepare(x, ws, rec, M, G, s)) return rc;
   }
   uint8_t* nws = static_cast<uint8_t*>(next_workspace);
   // whole reduction axis per workgroup: a tile's epilogue needs its finished totals

@@ -62,7 +62,8 @@ def tiled_gemm_cost(rows: int, out_features: int, groups: int, bits: int = 8, pr
     """Estimated microseconds of llmq_wq_gemm_a16_tile (within a tenth of the measured launches, 128-2048 rows on
     weights of 2048-28672 rows): rounds of 256 workgroups, each a fixed part plus a time per group, the partial sums'
     way through memory where the reduction axis is cut, and 3.5 us for the activation's preparation unless the rows
-    arrive prepared (llmq_add_rmsnorm_prepared, the gate|up epilogue)."""
+    arrive prepared (llmq_add_rmsnorm_prepared, the gate|up epilogue). (float16 rows are read as they lie; the estimate
+    does not tell the types apart, which leaves them that much in hand.)"""
     launch = min(_tile_plan_cost(rows, out_features, groups, narrow, bits == 4) for narrow in (False, True))
     return launch + (0.0 if prepared else 3.5)
 
