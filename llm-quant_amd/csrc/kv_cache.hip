@@ -1227,6 +1227,46 @@ __global__ __launch_bounds__(256) void kv_attend_merge_kernel(const float* __res
   for (int e = 0; e < 8; ++e) out[i + e] = from_float<T>(f[e]);
 }
 
+// The same with a workgroup per head, whose records it brings into LDS at once, a thread per element behind that (the
+// arithmetic per element, and so the bits, are merge_partials8's). What bounds it is one trip to memory; a thread that
+// merges 32 records on its own takes four, eight records at a time.
+constexpr int kMergeThreads = 256;
+constexpr int kMergeLdsFloats = 12 * 1024;
+template <typename T>
+__global__ __launch_bounds__(kMergeThreads) void kv_attend_merge_head_kernel(const float* __restrict__ partials,
+                                                                             T* __restrict__ out, const int head_dim,
+                                                                             const int n_splits) {
+  extern __shared__ __attribute__((aligned(16))) float recs[];
+  const int stride = head_dim + kAttnRecordHeader, floats = n_splits * stride;   // (multiples of four)
+  const float* src = partials + static_cast<int64_t>(blockIdx.x) * floats;
+  for (int i = threadIdx.x * 4; i < floats; i += kMergeThreads * 4)
+    *reinterpret_cast<u32x4*>(recs + i) = load16(src + i);
+  __syncthreads();
+  for (int d = threadIdx.x; d < head_dim; d += kMergeThreads) {
+    float mm = -INFINITY, ll = 0.0f, f = 0.0f;
+    for (int s0 = 0; s0 < n_splits; s0 += 8) {
+      float m_s[8], m_new = mm;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        m_s[j] = recs[min(s0 + j, n_splits - 1) * stride];
+        if (s0 + j < n_splits) m_new = fmaxf(m_new, m_s[j]);
+      }
+      const float corr = mm == -INFINITY ? 0.0f : exp2f(mm - m_new);
+      ll *= corr;
+      f *= corr;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float* rec = recs + min(s0 + j, n_splits - 1) * stride;
+        const float a = (s0 + j < n_splits && m_s[j] != -INFINITY) ? exp2f(m_s[j] - m_new) : 0.0f;
+        ll += rec[1] * a;
+        f += rec[kAttnRecordHeader + d] * a;
+      }
+      mm = m_new;
+    }
+    out[static_cast<int64_t>(blockIdx.x) * head_dim + d] = from_float<T>(f * (ll > 0.0f ? 1.0f / ll : 0.0f));
+  }
+}
+
 // ---- argmax of one row (the greedy sampler of the decode loop) ------------------------------------------
 // First index of the maximum, like torch.argmax on a row without ties broken otherwise.
 template <typename T>
@@ -1348,7 +1388,7 @@ __global__ __launch_bounds__(256) void argmax_split_kernel(const T* __restrict__
     for (int w = 1; w < static_cast<int>(blockDim.x) / kWave; ++w) take(s_val[w], s_idx[w]);
     __hip_atomic_store(part_val + blockIdx.x, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(part_idx + blockIdx.x, best_i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __threadfence();   // the slice's result is visible to the other XCDs before the ticket is
+    // (the slice's result is visible to the other XCDs before the ticket is: the increment releases it)
     const unsigned ticket = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
     s_winner = ticket == gridDim.x - 1 ? 0 : -1;
   }
@@ -1918,6 +1958,22 @@ extern "C" int llmq_kv_attend_merge(const float* partials, void* out, int q_head
   if (total == 0) return 0;
   if (!partials || !out) return llmq_host::fail_invalid("null tensor pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // records of a head that fit LDS (the default limit), 16-byte aligned: a workgroup a head
+  const int64_t floats = static_cast<int64_t>(n_splits) * (head_dim + kAttnRecordHeader);
+  if (floats <= kMergeLdsFloats && (reinterpret_cast<uintptr_t>(partials) & 15u) == 0) {
+    const size_t lds = static_cast<size_t>(floats) * sizeof(float);
+#define LLMQ_MERGE(T)                                                                                              \
+  hipLaunchKernelGGL((kv_attend_merge_head_kernel<T>), dim3(q_heads), dim3(kMergeThreads), lds, s, partials,      \
+                     static_cast<T*>(out), head_dim, n_splits)
+    switch (dtype) {
+      case LLMQ_F32: LLMQ_MERGE(float); break;
+      case LLMQ_F16: LLMQ_MERGE(f16_t); break;
+      case LLMQ_BF16: LLMQ_MERGE(bf16_t); break;
+      default: return llmq_host::fail_invalid("unsupported dtype code %d", dtype);
+    }
+#undef LLMQ_MERGE
+    return llmq_host::check_launch("kv_attend_merge_head_kernel");
+  }
   const dim3 grid((total / 8 + 255) / 256), block(256);
   switch (dtype) {
     case LLMQ_F32:

@@ -51,6 +51,11 @@ def _fusable(*mods) -> bool:
 # (the vector-ALU form, which caches below 2048 rows keep, with 8 splits: 546-551 / 555 / 578 / 595 at 600 / 1000 / 2000 /
 # 3500, 673 at 7000)
 MID_CONTEXT_FROM = 5120
+# Splits from which the records are merged by a launch of their own in front of o_proj instead of inside it, where every
+# workgroup of the GEMV merges all of them, eight records at a time. A step of four 1B layers / two 8B layers and lm_head,
+# merged inside / by a launch, us: 8 splits 175 / 177 and 219 / 217, 16 splits (8000 cached) 190.7 / 189.5 and
+# 228.7 / 225.0, 32 splits (24000, 20000) 209.1 / 205.8 and 243 / 235.
+MERGE_LAUNCH_FROM = 16
 LONG_CONTEXT_FROM = 16384
 
 
@@ -299,9 +304,14 @@ class LlamaFusedRuntime(LlamaKernelRuntime):
                                                 cache.v_codes[index], cache.k_scale[index], cache.v_scale[index],
                                                 self._partials, cache.position, self.scaling, self.q_heads,
                                                 splits)
-                hidden = ext.wq_gemv_attn_merge(self._partials, splits, self.head_dim, f["o"].qdata,
-                                                f["o"].wscale, f["o"].out_group, f["o_head_dim"], hidden,
-                                                hidden.dtype)
+                if splits >= MERGE_LAUNCH_FROM:
+                    ctx = ext.kv_attend_merge(self._partials, self.q_heads, self.head_dim, splits, hidden.dtype)
+                    hidden = ext.wq_gemv_fused(ctx, f["o"].qdata, f["o"].wscale, f["o"].out_group, PRO_NONE, None, 0.0,
+                                               f["o_head_dim"], hidden)
+                else:
+                    hidden = ext.wq_gemv_attn_merge(self._partials, splits, self.head_dim, f["o"].qdata,
+                                                    f["o"].wscale, f["o"].out_group, f["o_head_dim"], hidden,
+                                                    hidden.dtype)
             else:
                 ctx = ext.kv_rope_append_attend(qkv, self.cos_table, self.sin_table, cache.k_codes[index],
                                                 cache.v_codes[index], cache.k_scale[index], cache.v_scale[index],

@@ -401,3 +401,28 @@ def test_heads_of_128_take_the_matrix_core_form_on_short_caches_too(ext, bits, c
     assert rel_l2(got, want) <= 1e-2
     per_head = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
     assert per_head.max() <= 2e-2, per_head.argmax()
+
+
+@pytest.mark.parametrize("head_dim", [8, 64, 128, 264])
+@pytest.mark.parametrize("splits", [1, 8, 9, 32, 46, 256])   # one batch of eight, one over, a long walk, past LDS at 264
+def test_merge_of_records_against_the_closed_form(ext, head_dim, splits):
+    """softmax merge of (max, sum, weighted output) records, base 2, in float64: records of empty splits (max -inf) weigh
+    nothing whatever they hold, a head of empty records is zero, large maxima do not overflow. The fp32 sum of `splits`
+    terms of one sign differs by at most splits * 2^-23 of the sum of their magnitudes (twice, numerator and denominator)."""
+    heads = 5
+    gen = torch.Generator().manual_seed(head_dim * 1000 + splits)
+    rec = torch.randn(heads, splits, head_dim + 4, generator=gen)
+    rec[..., 0] *= 30
+    rec[1, ..., 0] += 1e4
+    rec[..., 1] = rec[..., 1].abs() + 0.1
+    rec[2, 1:, 0] = -float("inf")
+    rec[3, :, 0] = -float("inf")
+    got = ext.kv_attend_merge(rec.cuda().flatten(), heads, head_dim, splits, torch.float32).cpu().double().view(heads, head_dim)
+    r = rec.double()
+    top = r[..., 0].max(-1, keepdim=True).values
+    weight = torch.where(r[..., 0] == -float("inf"), 0.0, torch.exp2(r[..., 0] - torch.where(top.isinf(), 0.0, top)))
+    total = (weight * r[..., 1]).sum(-1)
+    live = total > 0
+    want = torch.where(live[:, None], (weight[..., None] * r[..., 4:]).sum(1) / total.clamp(min=1e-300)[:, None], 0.0)
+    size = (weight[..., None] * r[..., 4:].abs()).sum(1) / total.clamp(min=1e-300)[:, None]
+    assert ((got - want).abs() <= (2 * splits + 16) * 2.0 ** -23 * size + 1e-30).all()
