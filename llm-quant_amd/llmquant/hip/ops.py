@@ -17,6 +17,17 @@ def _group_size_for(x: torch.Tensor, args: QuantizationArgs) -> int:
     raise ValueError(f"unsupported strategy {args.strategy!r}")
 
 
+def _rows_in_place(numel: int, width: int, element_size: int, group_size: int) -> bool:
+    """Whether ragged rows go to the kernel that takes them as they lie: groups of a power of two 16-byte packets that
+    one wave holds, rows of a packet or more, and fewer than 2^31 packets counting each row's zeros up to whole groups
+    (narrow rows under wide groups are mostly zeros)."""
+    if numel == 0 or width < 8 or width % group_size == 0 or element_size > 4:
+        return False
+    packets, rest = divmod(group_size * element_size, 16)
+    padded_packets = numel // width * -(-width // group_size) * packets
+    return rest == 0 and packets <= 64 and packets & (packets - 1) == 0 and padded_packets < 1 << 31
+
+
 def fake_quantize_hip(x: torch.Tensor, args: QuantizationArgs, return_scale: bool = False):
     """Quant-dequant on the GPU, bit-exact with llmquant.core.quant_ops.fake_quantize.
 
@@ -26,11 +37,9 @@ def fake_quantize_hip(x: torch.Tensor, args: QuantizationArgs, return_scale: boo
     """
     group_size = _group_size_for(x, args)
     width = x.shape[-1]
-    if width % group_size and x.is_cuda and x.element_size() <= 4:
-        packets, rest = divmod(group_size * x.element_size(), 16)
-        if rest == 0 and packets <= 64 and packets & (packets - 1) == 0 and width >= 8 and x.numel() < 1 << 30:
-            out, scale = load_extension().fake_quant_rows(x, args.num_bits, group_size, return_scale)
-            return (out, scale) if return_scale else out
+    if x.is_cuda and _rows_in_place(x.numel(), width, x.element_size(), group_size):
+        out, scale = load_extension().fake_quant_rows(x, args.num_bits, group_size, return_scale)
+        return (out, scale) if return_scale else out
     padded = pad_to_group(x, group_size)
     out, scale = load_extension().fake_quant_group(padded, args.num_bits, group_size, return_scale)
     if padded.shape[-1] != width:

@@ -437,3 +437,19 @@ def test_deployed_cost_of_a_bf16_model_and_the_row_columns():
     shared = deployed_cost(tied, None)
     per_layer = 64 * 64 * 2 + 2 * 32 * 64 + 3 * 64 * 128
     assert shared["deployed_bytes"] == 2 * (per_layer + 3 * 64 + 100 * 64)   # the shared table once
+
+
+@pytest.mark.parametrize("numel,width,element_size,group_size,taken", [
+    (4096 * 5000, 5000, 2, 128, True),
+    (4096 * 5120, 5120, 2, 128, False),        # whole groups
+    (100, 4, 2, 128, False),                   # less than a packet
+    (0, 40, 2, 128, False),
+    (40 * 96, 40, 2, 96, False),               # twelve packets a group
+    (40 * 96, 40, 4, 512, False),              # more packets than a wave has lanes
+    (8 * ((1 << 26) - 1), 8, 2, 256, True),    # 32 packets a row once padded: just below 2^31 of them
+    (8 * (1 << 26), 8, 2, 256, False),         # 2^31: what the launch refuses is padded and trimmed
+])
+def test_which_ragged_rows_the_quantizer_takes_in_place(numel, width, element_size, group_size, taken):
+    from llmquant.hip.ops import _rows_in_place
+
+    assert _rows_in_place(numel, width, element_size, group_size) is taken
