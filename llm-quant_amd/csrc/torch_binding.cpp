@@ -557,13 +557,20 @@ ExpertsProblem check_experts(const at::Tensor& x, const at::Tensor& top_k_index,
           static_cast<int>(I), packed ? LLMQ_W_INT4_PACKED : LLMQ_W_INT8, dtype_code(x, "x")};
 }
 
+// The kernels read 16-byte packets: a view that starts elsewhere is copied (allocations start at one).
+at::Tensor on_a_packet(const at::Tensor& t) {
+  return (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) ? t.clone() : t;
+}
+
 // A whole gated experts block over many tokens (see llmq_wq_experts). Returns [tokens, hidden].
-at::Tensor wq_experts(const at::Tensor& x, const at::Tensor& top_k_index, const at::Tensor& top_k_weights,
-                      const at::Tensor& gate_up, const at::Tensor& gate_up_scale, const at::Tensor& down,
-                      const at::Tensor& down_scale) {
-  const auto p = check_experts(x, top_k_index, top_k_weights, gate_up, gate_up_scale, down, down_scale);
-  auto out = at::empty_like(x);
+at::Tensor wq_experts(const at::Tensor& x_in, const at::Tensor& top_k_index, const at::Tensor& top_k_weights,
+                      const at::Tensor& gate_up_in, const at::Tensor& gate_up_scale_in, const at::Tensor& down_in,
+                      const at::Tensor& down_scale_in) {
+  const auto p = check_experts(x_in, top_k_index, top_k_weights, gate_up_in, gate_up_scale_in, down_in, down_scale_in);
+  auto out = at::empty_like(x_in);
   if (out.numel() == 0) return out;
+  const at::Tensor x = on_a_packet(x_in), gate_up = on_a_packet(gate_up_in), down = on_a_packet(down_in),
+                   gate_up_scale = on_a_packet(gate_up_scale_in), down_scale = on_a_packet(down_scale_in);
   const at::Tensor index = top_k_index.to(at::kLong).contiguous(), weights = top_k_weights.contiguous();
   const c10::OptionalDeviceGuard guard(at::device_of(x));
   const int64_t bytes = static_cast<int64_t>(
@@ -578,13 +585,15 @@ at::Tensor wq_experts(const at::Tensor& x, const at::Tensor& top_k_index, const 
   return out;
 }
 
-// The same block for a token or two, two launches (see llmq_wq_experts_direct).
-at::Tensor wq_experts_direct(const at::Tensor& x, const at::Tensor& top_k_index, const at::Tensor& top_k_weights,
-                             const at::Tensor& gate_up, const at::Tensor& gate_up_scale, const at::Tensor& down,
-                             const at::Tensor& down_scale) {
-  const auto p = check_experts(x, top_k_index, top_k_weights, gate_up, gate_up_scale, down, down_scale);
-  auto out = at::empty_like(x);
+// The same block for a few tokens, two launches (see llmq_wq_experts_direct).
+at::Tensor wq_experts_direct(const at::Tensor& x_in, const at::Tensor& top_k_index, const at::Tensor& top_k_weights,
+                             const at::Tensor& gate_up_in, const at::Tensor& gate_up_scale_in, const at::Tensor& down_in,
+                             const at::Tensor& down_scale_in) {
+  const auto p = check_experts(x_in, top_k_index, top_k_weights, gate_up_in, gate_up_scale_in, down_in, down_scale_in);
+  auto out = at::empty_like(x_in);
   if (out.numel() == 0) return out;
+  const at::Tensor x = on_a_packet(x_in), gate_up = on_a_packet(gate_up_in), down = on_a_packet(down_in),
+                   gate_up_scale = on_a_packet(gate_up_scale_in), down_scale = on_a_packet(down_scale_in);
   const at::Tensor index = top_k_index.to(at::kLong).contiguous(), weights = top_k_weights.contiguous();
   const c10::OptionalDeviceGuard guard(at::device_of(x));
   auto act = at::empty({static_cast<int64_t>(p.tokens) * p.top_k, p.intermediate}, x.options());
@@ -1568,7 +1577,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("wq_experts", &wq_experts, "A gated experts block over many tokens: plan, two grouped GEMMs, combination",
         py::arg("x"), py::arg("top_k_index"), py::arg("top_k_weights"), py::arg("gate_up"), py::arg("gate_up_scale"),
         py::arg("down"), py::arg("down_scale"));
-  m.def("wq_experts_direct", &wq_experts_direct, "A gated experts block for a token or two in two launches",
+  m.def("wq_experts_direct", &wq_experts_direct, "A gated experts block for a few tokens in two launches",
         py::arg("x"), py::arg("top_k_index"), py::arg("top_k_weights"), py::arg("gate_up"), py::arg("gate_up_scale"),
         py::arg("down"), py::arg("down_scale"));
   m.def("wq_experts_direct_supported", [](int64_t tokens, int64_t top_k, int64_t experts, int64_t hidden,

@@ -354,3 +354,24 @@ def test_grouped_gemms_against_real_mode(ext, bits, dtype, tokens, hidden, inter
         got, want = quant(x, index, weights), real(x.float(), index, weights.float())
         assert torch.equal(got, quant(x, index, weights))   # whatever order the rows were placed in
     assert rel_l2(to_np(got), to_np(want)) <= (1e-2 if dtype == torch.bfloat16 else 1.5e-3)
+
+
+@pytest.mark.parametrize("tokens", [2, 12])
+def test_an_activation_that_starts_inside_a_packet(ext, tokens):
+    """A contiguous view at an odd storage offset, through the two-launch form and the grouped GEMMs: the bits of the
+    same values in a tensor of their own."""
+    from llmquant.quantizers import KernelQuantExperts
+
+    gen = torch.Generator(device="cuda").manual_seed(tokens)
+    source = torch.nn.Module()
+    source.act_fn = torch.nn.SiLU()
+    for name, shape in (("gate_up_proj", (4, 1024, 512)), ("down_proj", (4, 512, 512))):
+        weight = torch.randn(shape, device="cuda", generator=gen) * 0.05
+        setattr(source, name, torch.nn.Parameter(weight.to(torch.bfloat16), requires_grad=False))
+    quant = KernelQuantExperts.from_experts(source, QuantConfig(mlp_weight="int4").scheme("mlp_weight"))
+    x = torch.randn(tokens * 512 + 1, device="cuda", generator=gen).to(torch.bfloat16)[1:].view(tokens, 512)
+    assert x.data_ptr() % 16 and x.is_contiguous()
+    weights, index = torch.randn(tokens, 4, device="cuda", generator=gen).softmax(-1).topk(2, dim=-1)
+    weights = weights.to(torch.bfloat16)
+    with torch.no_grad():
+        assert torch.equal(quant(x, index, weights), quant(x.clone(), index, weights))
