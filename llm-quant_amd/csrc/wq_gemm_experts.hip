@@ -1,5 +1,5 @@
 // A Mixture-of-Experts block over a prompt (or a batch of sequences), gfx950: every token through the experts it is
-// routed to, five launches whatever the number of experts, nothing read back to the host.
+// routed to, four launches whatever the number of experts, nothing read back to the host.
 //
 // KernelQuantExperts.forward walks the experts one at a time for more than a few tokens
 // (llmquant/quantizers/kernel.py:216-289): per expert a nonzero / where on the routing mask (which the host waits
@@ -204,7 +204,11 @@ int run(const void* x, const int64_t* index, const void* weights, const void* q1
         const float* s2, void* out, uint8_t* ws, int n_tokens, int top_k, int E, int H, int I, hipStream_t stream) {
   const Layout l = layout_for(n_tokens, top_k, E, H, I);
   const int rows = n_tokens * top_k;
-  // 64-row tiles from 40 rows an expert on: below, most 64-row tiles would be half empty
+  // 64-row tiles from 40 rows an expert on. Measured, us a pass, 32-row tiles / 64-row: 64 experts of 2048 x 1024 int4 at
+  // 10 rows an expert 58.9 / 68.5, 25: 74.4 / 90.2, 37.5: 89.8 / 92.6, 45: 93.0 / 96.8, 52: 108.5 / 98.5, 75: 128.8 / 122.3;
+  // int8 25: 120.0 / 142.6, 37.5: 147.1 / 146.4, 41: 150.1 / 144.5, 52: 174.1 / 151.2. Eight experts of 2048 x 4096 int4 at
+  // 30: 61.4 / 74.7, 50: 74.6 / 77.8, 75: 77.3 / 79.7, 125: 120.0 / 98.9 (between 40 and 48 rows int4 would keep the lower
+  // tile, int8 would not).
   const int tile_rows = rows > 40 * E ? 64 : 32;
   const PlanArgs p{index, rows, E, top_k, tile_rows, reinterpret_cast<int4*>(ws + l.tiles),
                    reinterpret_cast<int*>(ws + l.n_tiles), reinterpret_cast<int*>(ws + l.row_source),

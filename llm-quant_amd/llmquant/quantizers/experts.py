@@ -265,7 +265,7 @@ class KernelQuantExperts(_QuantExperts):
                 and self._ext.route_plan_supported(top_k_index.numel(), self.num_experts))
 
     def _takes_gemm(self, hidden_states, top_k_index, top_k_weights) -> bool:
-        """Whether a prompt's tokens go through the grouped GEMMs (five launches whatever the number of experts): SiLU
+        """Whether a prompt's tokens go through the grouped GEMMs (four launches whatever the number of experts): SiLU
         experts of unpadded groups of 128, one scale per weight row, 16-bit activations and routing weights."""
         return (self._act_is_silu and self._weight_args.group_size == 128
                 and self._gate_up_padded == self.hidden_dim and self._down_padded == self.intermediate_dim
