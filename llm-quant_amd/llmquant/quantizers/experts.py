@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.autograd.forward_ad import unpack_dual
 
 from llmquant.core.observers import group_view
 from llmquant.core.scheme import QuantizationScheme
@@ -264,9 +265,18 @@ class KernelQuantExperts(_QuantExperts):
                 and top_k_weights.dtype == hidden_states.dtype and top_k_weights.shape == top_k_index.shape
                 and self._ext.route_plan_supported(top_k_index.numel(), self.num_experts))
 
+    @staticmethod
+    def _differentiated(*tensors) -> bool:
+        """Whether a derivative is asked for with respect to one of the inputs (reverse or forward mode). The loop over
+        the experts carries the routing weights' (and, beyond the fused GEMM's rows, the activation's); a kernel that
+        does the whole block carries none."""
+        reverse = torch.is_grad_enabled()
+        return any((reverse and t.requires_grad) or unpack_dual(t).tangent is not None for t in tensors)
+
     def _takes_gemm(self, hidden_states, top_k_index, top_k_weights) -> bool:
         """Whether a prompt's tokens go through the grouped GEMMs (four launches whatever the number of experts): SiLU
-        experts of unpadded groups of 128, one scale per weight row, 16-bit activations and routing weights."""
+        experts of unpadded groups of 128, one scale per weight row, 16-bit activations and routing weights, no
+        derivative to carry."""
         return (self._act_is_silu and self._weight_args.group_size == 128
                 and self._gate_up_padded == self.hidden_dim and self._down_padded == self.intermediate_dim
                 and self.sgate_up.shape[1] == self.gate_up_data.shape[1] and self.sdown.shape[1] == self.down_data.shape[1]
@@ -274,6 +284,7 @@ class KernelQuantExperts(_QuantExperts):
                 and hidden_states.dim() == 2 and hidden_states.is_contiguous()
                 and top_k_weights.dtype == hidden_states.dtype and top_k_weights.shape == top_k_index.shape
                 and top_k_index.dim() == 2 and top_k_index.shape[0] == hidden_states.shape[0]
+                and not self._differentiated(hidden_states, top_k_weights)
                 and self._ext.wq_experts_supported(hidden_states.shape[0], top_k_index.shape[1], self.num_experts,
                                                    self.hidden_dim, self.intermediate_dim))
 
@@ -292,7 +303,10 @@ class KernelQuantExperts(_QuantExperts):
                 and top_k_weights.dtype == hidden_states.dtype and top_k_weights.shape == top_k_index.shape
                 and top_k_index.dim() == 2 and top_k_index.shape[0] == hidden_states.shape[0]
                 and self._ext.wq_experts_direct_supported(hidden_states.shape[0], top_k_index.shape[1], self.num_experts,
-                                                          self.hidden_dim, self.intermediate_dim, 4 if self._packed else 8))
+                                                          self.hidden_dim, self.intermediate_dim, 4 if self._packed else 8)
+                # (the four-launch form carries no derivative either; the one behind it, for more experts, does)
+                and (self._ext.route_plan_supported(top_k_index.numel(), self.num_experts)
+                     or not self._differentiated(hidden_states, top_k_weights)))
 
     def _forward_fused(self, hidden_states, top_k_index, top_k_weights):
         """Plan, gate|up (storing act(gate) * up), down, weighted sum per token: four launches (a token's rows too many

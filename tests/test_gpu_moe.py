@@ -375,3 +375,28 @@ def test_an_activation_that_starts_inside_a_packet(ext, tokens):
     weights = weights.to(torch.bfloat16)
     with torch.no_grad():
         assert torch.equal(quant(x, index, weights), quant(x.clone(), index, weights))
+
+
+def test_a_prompt_carries_the_derivative_of_its_routing_weights(ext):
+    """Beyond eight tokens, reverse and forward mode: d out / d weight is the expert's row. In float32 from the real-mode
+    block; here its rows are rounded to bfloat16 a few times (each 2^-9), as in the forward pass."""
+    from torch.autograd import forward_ad
+
+    _, quant, real, cfg = kernel_block("int8", experts=4, top_k=2)
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    hidden = torch.randn(20, cfg.hidden_size, device="cuda", generator=gen).to(torch.bfloat16)
+    weights, index = torch.randn(20, 4, device="cuda", generator=gen).softmax(-1).topk(2, dim=-1)
+    weights = weights.to(torch.bfloat16)
+    cotangent = torch.randn(20, cfg.hidden_size, device="cuda", generator=gen)
+    with torch.no_grad():
+        assert quant._takes_gemm(hidden, index, weights)
+    mine, theirs = weights.clone().requires_grad_(), weights.float().requires_grad_()
+    out = quant(hidden, index, mine)
+    assert out.requires_grad and not quant(hidden, index, weights).requires_grad
+    out.backward(cotangent.to(torch.bfloat16))
+    real(hidden.float(), index, theirs).backward(cotangent)
+    assert rel_l2(to_np(mine.grad), to_np(theirs.grad)) <= 2e-2
+    with torch.no_grad(), forward_ad.dual_level():
+        tangent = torch.randn(20, 2, device="cuda", generator=gen).to(torch.bfloat16)
+        along = forward_ad.unpack_dual(quant(hidden, index, forward_ad.make_dual(weights, tangent))).tangent
+        assert rel_l2(to_np(along), to_np(real(hidden.float(), index, tangent.float()))) <= 1e-2
