@@ -135,8 +135,8 @@ int llmq_moe_combine(const void* rows_out, const int64_t* order, const void* wei
  * launch adds up a token's experts in their order. Rounding points and bits of llmq_route_plan +
  * llmq_wq_gemv_batched_fused + llmq_moe_combine; every row reads its expert's weight (nothing is shared between tokens).
  * act: [tokens * top_k, intermediate] of the activation dtype, 16-byte aligned. Weights, scales and index as for
- * llmq_wq_experts below, any float dtype. `supported`: hidden and intermediate multiples of 512, intermediate up to
- * 8192, top_k up to 16, a token's rows within the LDS. */
+ * llmq_wq_experts below, any float dtype; an expert id outside the stack counts as the nearest valid one. `supported`:
+ * hidden and intermediate multiples of 512, intermediate up to 8192, top_k up to 16, a token's rows within the LDS. */
 int llmq_wq_experts_direct_supported(int n_tokens, int top_k, int n_experts, int hidden, int intermediate, int wformat);
 int llmq_wq_experts_direct(const void* x, const int64_t* top_k_index, const void* top_k_weights, const void* gate_up,
                            const float* gate_up_scale, const void* down, const float* down_scale, void* out, void* act,
@@ -147,9 +147,9 @@ int llmq_wq_experts_direct(const void* x, const int64_t* top_k_index, const void
  * one at a time beyond a few tokens): out[t] = sum over t's experts e of weight * down_e(silu(gate_e(x_t)) * up_e(x_t)),
  * rounded to `dtype` (fp16 / bf16) after each projection, activation, product, weighted row and addition (added in the
  * order of the experts). Groups of 128, one scale per weight row; gate_up: [experts, 2 I, H/128, ..], gate rows first;
- * down: [experts, H, I/128, ..]; x, out: [tokens, H]; top_k_index, top_k_weights: [tokens, top_k]. An expert id outside
- * the stack counts as the nearest valid one. `supported`: hidden and intermediate whole groups, up to 1024 experts,
- * 256 experts a token, activations and one expert's weight below 4 GiB. */
+ * down: [experts, H, I/128, ..]; x, out: [tokens, H]; top_k_index, top_k_weights: [tokens, top_k]. A token
+ * with an expert id outside the stack gets a row of NaN. `supported`: hidden and intermediate whole groups, up to 1024
+ * experts, 256 experts a token, activations and one expert's weight below 4 GiB. */
 int llmq_wq_experts_supported(int n_tokens, int top_k, int n_experts, int hidden, int intermediate);
 size_t llmq_wq_experts_workspace_bytes(int n_tokens, int top_k, int n_experts, int hidden, int intermediate);
 int llmq_wq_experts(const void* x, const int64_t* top_k_index, const void* top_k_weights, const void* gate_up,

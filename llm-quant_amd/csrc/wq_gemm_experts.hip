@@ -45,7 +45,7 @@ struct PlanArgs {
 };
 
 __device__ __forceinline__ int expert_id(int64_t raw, int n_experts) {
-  // an id outside the layer's experts is counted with the nearest valid one
+  // an id outside the layer's experts is planned with the nearest valid one; the combination makes its token's row NaN
   return raw < 0 ? 0 : (raw >= n_experts ? n_experts - 1 : static_cast<int>(raw));
 }
 
@@ -112,6 +112,7 @@ __global__ __launch_bounds__(kPlanThreads) void experts_plan_kernel(const PlanAr
 
 // final[t] = the rows of token t, each times its routing weight, added up in the order of the experts (of the slots
 // where two are the same), every product and sum rounded to T. One workgroup per token, eight columns a thread and turn.
+// A token with an id outside the layer's experts: a row of NaN.
 template <typename T>
 __global__ __launch_bounds__(256) void experts_combine_kernel(const T* __restrict__ rows_out,
                                                               const int64_t* __restrict__ expert_of_row,
@@ -129,7 +130,8 @@ __global__ __launch_bounds__(256) void experts_combine_kernel(const T* __restric
     int rank = 0;
     for (int j = 0; j < top_k; ++j) rank += s_expert[j] < e || (s_expert[j] == e && j < k);
     s_row[rank] = sorted_of_row[first + k];
-    s_weight[rank] = llmq::to_float(weights[first + k]);
+    const bool known = expert_of_row[first + k] == e;
+    s_weight[rank] = known ? llmq::to_float(weights[first + k]) : __builtin_nanf("");
   }
   __syncthreads();
   for (int c = tid * 8; c < width; c += 256 * 8) {

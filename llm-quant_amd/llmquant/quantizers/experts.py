@@ -134,7 +134,11 @@ class KernelQuantExperts(_QuantExperts):
     """Every routed expert of a projection in one launch: by row for up to eight tokens, by grouped GEMM beyond.
 
     4-bit stacks live in HBM nibble-packed ([E, N, groups, gs/2] uint8, the bytes of the packed
-    file); `qgate_up` / `qdown` hand back the canonical int8 view on demand."""
+    file); `qgate_up` / `qdown` hand back the canonical int8 view on demand.
+
+    Expert ids outside the layer: up to eight tokens they count as the nearest valid one; beyond, the grouped GEMMs give
+    a token that holds one a row of NaN (the host would have to wait for the ids to raise), and the loop over the
+    experts refuses them."""
 
     _what = "kernel"
 
@@ -275,8 +279,8 @@ class KernelQuantExperts(_QuantExperts):
 
     def _takes_gemm(self, hidden_states, top_k_index, top_k_weights) -> bool:
         """Whether a prompt's tokens go through the grouped GEMMs (four launches whatever the number of experts): SiLU
-        experts of unpadded groups of 128, one scale per weight row, 16-bit activations and routing weights, no
-        derivative to carry."""
+        experts of unpadded groups of 128, one scale per weight row, 16-bit activations and routing weights, int64 expert
+        ids (the loop refuses others), no derivative to carry."""
         return (self._act_is_silu and self._weight_args.group_size == 128
                 and self._gate_up_padded == self.hidden_dim and self._down_padded == self.intermediate_dim
                 and self.sgate_up.shape[1] == self.gate_up_data.shape[1] and self.sdown.shape[1] == self.down_data.shape[1]
@@ -284,6 +288,7 @@ class KernelQuantExperts(_QuantExperts):
                 and hidden_states.dim() == 2 and hidden_states.is_contiguous()
                 and top_k_weights.dtype == hidden_states.dtype and top_k_weights.shape == top_k_index.shape
                 and top_k_index.dim() == 2 and top_k_index.shape[0] == hidden_states.shape[0]
+                and top_k_index.dtype == torch.int64
                 and not self._differentiated(hidden_states, top_k_weights)
                 and self._ext.wq_experts_supported(hidden_states.shape[0], top_k_index.shape[1], self.num_experts,
                                                    self.hidden_dim, self.intermediate_dim))

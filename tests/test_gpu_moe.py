@@ -400,3 +400,31 @@ def test_a_prompt_carries_the_derivative_of_its_routing_weights(ext):
         tangent = torch.randn(20, 2, device="cuda", generator=gen).to(torch.bfloat16)
         along = forward_ad.unpack_dual(quant(hidden, index, forward_ad.make_dual(weights, tangent))).tangent
         assert rel_l2(to_np(along), to_np(real(hidden.float(), index, tangent.float()))) <= 1e-2
+
+
+@pytest.mark.parametrize("bits,dtype", [("int4", torch.bfloat16), ("int8", torch.float16)])
+def test_a_prompt_with_ids_outside_the_layer(ext, bits, dtype):
+    """Beyond eight tokens: tokens that hold such an id get a row of NaN, the others the bits they have without them; ids
+    that are not int64 are refused."""
+    from llmquant.quantizers import KernelQuantExperts
+
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    source = torch.nn.Module()
+    source.act_fn = torch.nn.SiLU()
+    for name, shape in (("gate_up_proj", (3, 512, 128)), ("down_proj", (3, 128, 256))):
+        weight = torch.randn(shape, device="cuda", generator=gen) * 0.05
+        setattr(source, name, torch.nn.Parameter(weight.to(dtype), requires_grad=False))
+    quant = KernelQuantExperts.from_experts(source, QuantConfig(mlp_weight=bits).scheme("mlp_weight"))
+    x = torch.randn(40, 128, device="cuda", generator=gen).to(dtype)
+    weights, index = torch.randn(40, 3, device="cuda", generator=gen).softmax(-1).topk(2, dim=-1)
+    weights = weights.to(dtype)
+    odd, bad = index.clone(), [0, 7, 39]
+    odd[0, 0], odd[7, 1], odd[39, 0] = 3, -1, 2 ** 40
+    with torch.no_grad():
+        assert quant._takes_gemm(x, odd, weights)
+        want, got = quant(x, index, weights), quant(x, odd, weights)
+        assert got[bad].isnan().all()
+        rest = [t for t in range(40) if t not in bad]
+        assert torch.equal(got[rest], want[rest]) and want.isfinite().all()
+        with pytest.raises(RuntimeError, match="LongTensor"):
+            quant(x, index.int(), weights)
