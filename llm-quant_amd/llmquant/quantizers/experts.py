@@ -277,10 +277,26 @@ class KernelQuantExperts(_QuantExperts):
         reverse = torch.is_grad_enabled()
         return any((reverse and t.requires_grad) or unpack_dual(t).tangent is not None for t in tensors)
 
+    def _grouped_pays(self, rows: int) -> bool:
+        """Whether the grouped GEMMs are the faster form for this many (token, slot) rows. They run at 820 (int4) or 550
+        (int8) TFLOP/s on many rows: a tile is at most 64 rows, and every tile converts its expert's codes again. The loop
+        waits for the host 150 us an expert, dequantizes its weight once (4 TB/s) and multiplies at the BLAS library's
+        1.2 PFLOP/s, with element-wise passes beside it. Measured, us, grouped / loop: 8 experts, 2 a token, 2048 x 4096,
+        int4 at 512 / 4096 / 16384 rows an expert 294 / 1406, 1973 / 3121, 7864 / 8163, int8 at 4096 / 6144 / 16384
+        2911 / 3113, 4377 / 3826, 11993 / 8248; 4 experts, 2 a token, 4096 x 14336, int4 at 1024 / 2048 / 4096 1850 / 2195,
+        3561 / 3433, 6979 / 6462, int8 at 512 / 1024 / 4096 1456 / 1741, 2866 / 2274, 10622 / 6561."""
+        weights = 3.0 * self.hidden_dim * self.intermediate_dim
+        multiply = 2.0 * rows * weights
+        grouped = multiply / (820e6 if self._packed else 550e6)
+        loop = (min(rows, self.num_experts) * (150.0 + weights * ((0.5 if self._packed else 1.0) + 2.0) / 4e6)
+                + rows * (self.hidden_dim + self.intermediate_dim) * 1.6e-6 + multiply / 1200e6)
+        return grouped <= loop
+
     def _takes_gemm(self, hidden_states, top_k_index, top_k_weights) -> bool:
         """Whether a prompt's tokens go through the grouped GEMMs (four launches whatever the number of experts): SiLU
         experts of unpadded groups of 128, one scale per weight row, 16-bit activations and routing weights, int64 expert
-        ids (the loop refuses others), no derivative to carry."""
+        ids (the loop refuses others), no derivative to carry, and not so many rows that the loop is faster (a stream
+        capture, which the loop cannot be part of, takes them all)."""
         return (self._act_is_silu and self._weight_args.group_size == 128
                 and self._gate_up_padded == self.hidden_dim and self._down_padded == self.intermediate_dim
                 and self.sgate_up.shape[1] == self.gate_up_data.shape[1] and self.sdown.shape[1] == self.down_data.shape[1]
@@ -290,6 +306,7 @@ class KernelQuantExperts(_QuantExperts):
                 and top_k_index.dim() == 2 and top_k_index.shape[0] == hidden_states.shape[0]
                 and top_k_index.dtype == torch.int64
                 and not self._differentiated(hidden_states, top_k_weights)
+                and (self._grouped_pays(top_k_index.numel()) or torch.cuda.is_current_stream_capturing())
                 and self._ext.wq_experts_supported(hidden_states.shape[0], top_k_index.shape[1], self.num_experts,
                                                    self.hidden_dim, self.intermediate_dim))
 

@@ -428,3 +428,24 @@ def test_a_prompt_with_ids_outside_the_layer(ext, bits, dtype):
         assert torch.equal(got[rest], want[rest]) and want.isfinite().all()
         with pytest.raises(RuntimeError, match="LongTensor"):
             quant(x, index.int(), weights)
+
+
+def test_a_prompt_too_long_for_the_grouped_gemms_goes_through_the_loop_unless_captured(ext):
+    _, quant, _, cfg = kernel_block("int4", experts=4, top_k=2)
+    hidden = torch.randn(20, cfg.hidden_size, device="cuda", dtype=torch.bfloat16)
+    index, weights = routing(20, 4, 2, seed=1)
+    index, weights = index.cuda(), weights.cuda()
+    with torch.no_grad():
+        grouped = quant(hidden, index, weights)
+        quant._grouped_pays = lambda rows: False
+        assert not quant._takes_gemm(hidden, index, weights)
+        assert rel_l2(to_np(quant(hidden, index, weights)), to_np(grouped)) <= 1e-2
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            captured = quant(hidden, index, weights)
+        for _ in range(3):
+            captured.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(captured, grouped)

@@ -138,3 +138,24 @@ def test_experts_lookup_and_structure_checks():
         stacked_expert_blocks(odd)
     with pytest.raises(ValueError, match="needs a weight scheme"):
         RealQuantExperts.from_experts(expert_block()[0], QuantizationScheme(weights=None, input_activations=None))
+
+
+@pytest.mark.parametrize("experts,hidden,inter,packed,rows,grouped", [
+    (64, 2048, 1024, True, 8 * 600, True),
+    (64, 2048, 1024, False, 8 * 16384, True),
+    (8, 2048, 4096, True, 2 * 16384, True),
+    (8, 2048, 4096, False, 2 * 16384, True),       # 2911 us grouped, 3113 looped
+    (8, 2048, 4096, False, 2 * 24576, False),      # 4377, 3826
+    (4, 4096, 14336, True, 2 * 2048, True),        # 1850, 2195
+    (4, 4096, 14336, True, 2 * 8192, False),       # 6979, 6462
+    (4, 4096, 14336, False, 2 * 1024, True),       # 1456, 1741
+    (4, 4096, 14336, False, 2 * 2048, False),      # 2866, 2274
+    (64, 2048, 1024, True, 9, True),
+])
+def test_which_prompts_the_grouped_gemms_take(experts, hidden, inter, packed, rows, grouped):
+    from types import SimpleNamespace
+
+    from llmquant.quantizers import KernelQuantExperts
+
+    module = SimpleNamespace(num_experts=experts, hidden_dim=hidden, intermediate_dim=inter, _packed=packed)
+    assert KernelQuantExperts._grouped_pays(module, rows) is grouped
