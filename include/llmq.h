@@ -174,6 +174,9 @@ int llmq_wq_gemv_fused(const void* x, const void* qweight, const float* wscale, 
                        int G, int out_group, int wformat, int dtype, int prologue,
                        const void* norm_weight, float eps, int in_head_dim,
                        const void* residual_or_null, llmq_stream_t stream);
+/* Whether llmq_wq_gemv sends such a row to the kernel behind llmq_wq_gemv_fused (which takes no other): a multiple of
+ * four groups of 128, operands aligned to 16 bytes, a staged row that fits the LDS (up to about 390 groups). */
+int llmq_wq_gemv_fused_supported(const void* x, const void* qweight, const float* wscale, int G, int wformat);
 
 /* llmq_wq_gemv_fused for the gate|up weight of a gated MLP with the activation folded into the
  * store: qweight is [2 * intermediate, G, gs] (gate rows, then up rows: transformers' fused

@@ -178,14 +178,14 @@ at::Tensor wq_linear_rows(const at::Tensor& x, const at::Tensor& qweight, const 
   if (in_head_dim > 0) {
     const auto xc = x.contiguous();
     const auto wc = qweight.contiguous(), sc = wscale.contiguous();
-    const auto misaligned = (reinterpret_cast<uintptr_t>(xc.const_data_ptr()) | reinterpret_cast<uintptr_t>(wc.const_data_ptr()) |
-                             reinterpret_cast<uintptr_t>(sc.const_data_ptr())) & 15u;
-    if (misaligned || xc.numel() == 0) {
-      // (operands that the matrix-core GEMV does not take: padded here, for the other one)
+    const int format = wc.scalar_type() == at::kByte ? LLMQ_W_INT4_PACKED : LLMQ_W_INT8;
+    if (xc.numel() > 0 && llmq_wq_gemv_fused_supported(xc.const_data_ptr(), wc.const_data_ptr(), sc.const_data_ptr<float>(),
+                                                       static_cast<int>(wc.size(1)), format)) {
+      out = wq_gemv_fused(xc, wc, sc, out_group, LLMQ_PRO_NONE, {}, 0.0, in_head_dim, {});
+    } else {
+      // (what the matrix-core GEMV does not take, misaligned operands or a row of some 400 groups: padded here)
       out = wq_gemv(at::constant_pad_nd(xc.view({-1, in_head_dim}), {0, 128 - in_head_dim}).view({-1, wc.size(1) * 128}), wc,
                     sc, out_group);
-    } else {
-      out = wq_gemv_fused(xc, wc, sc, out_group, LLMQ_PRO_NONE, {}, 0.0, in_head_dim, {});
     }
   } else {
     out = wq_gemv(x, qweight, wscale, out_group);

@@ -408,6 +408,10 @@ extern "C" int llmq_wq_gemv(const void* x, const void* qweight, const float* wsc
              : launch_bits<4>(x, qweight, wscale, out, M, N, G, gs, out_group, dtype, s);
 }
 
+extern "C" int llmq_wq_gemv_fused_supported(const void* x, const void* qweight, const float* wscale, int G, int wformat) {
+  return llmq_host::gemv_mfma_supported(x, qweight, wscale, 1, G, 128, wformat) && !llmq_host::gemv_force_alu() ? 1 : 0;
+}
+
 extern "C" int llmq_wq_gemv_fused(const void* x, const void* qweight, const float* wscale, void* out,
                                   int N, int G, int out_group, int wformat, int dtype, int prologue,
                                   const void* norm_weight, float eps, int in_head_dim,
@@ -426,8 +430,8 @@ extern "C" int llmq_wq_gemv_fused(const void* x, const void* qweight, const floa
   if (N == 0) return 0;
   if (!x || !qweight || !wscale || !out) return llmq_host::fail_invalid("null tensor pointer");
   if (!llmq_host::gemv_mfma_supported(x, qweight, wscale, 1, G, 128, wformat))
-    return llmq_host::fail_invalid("the fused GEMV needs group size 128, a multiple of 4 groups "
-                                   "and 16-byte aligned operands");
+    return llmq_host::fail_invalid("the fused GEMV needs group size 128, a multiple of 4 groups, 16-byte aligned "
+                                   "operands and a row that fits the LDS, got %d groups", G);
   return llmq_host::gemv_mfma_launch_fused(x, qweight, wscale, out, 1, N, G, out_group, wformat, dtype, prologue,
                                            norm_weight, eps, in_head_dim, residual_or_null,
                                            static_cast<hipStream_t>(stream));

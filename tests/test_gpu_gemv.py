@@ -666,7 +666,8 @@ def test_dequant_weight_indexing(bits, n, groups, out_group, keep):
 
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("spec,width", [(dict(), 640), (dict(), 600), (dict(head_dim=64), 8 * 64), (dict(head_dim=32), 4 * 32),
-                                        (dict(head_dim=64), 6 * 64), (dict(out_group=64), 512)])
+                                        (dict(head_dim=64), 6 * 64), (dict(out_group=64), 512),
+                                        (dict(head_dim=32), 512 * 32)])   # (more groups than the LDS holds staged)
 def test_the_short_way_of_a_row_or_two_is_the_general_one(bits, spec, width):
     """KernelQuantLinear.forward on few rows (its first branch) against the same module without that branch, to the bit:
     rows, leading axes, types, strides and alignments; padded widths, heads and a bias keep their own ways."""
