@@ -1315,13 +1315,14 @@ int launch_routed(const T* x, const int64_t* index, const T* weights, const uint
   if (resident < 1) resident = 1;
   const int turns = (up.n_tiles + resident - 1) / resident;
   const dim3 grid((up.n_tiles + turns - 1) / turns, rows), block(wk * kWave);
-#define LLMQ_ROUTED(KERNEL, GRID, BLOCK, LDS, ...)                                                  \
+// (STATIC: LDS that the kernel declares beside the dynamic part; the limit is on both)
+#define LLMQ_ROUTED(KERNEL, GRID, BLOCK, LDS, STATIC, ...)                                          \
   do {                                                                                              \
     auto kernel = KERNEL;                                                                           \
     static bool raised = false; /* per instantiation; worst case two threads both set it */        \
-    if ((LDS) > kLdsDefault && !raised) {                                                           \
+    if ((LDS) + (STATIC) > kLdsDefault && !raised) {                                                \
       const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),             \
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax - 1024); \
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax - (STATIC)); \
       if (err != hipSuccess) {                                                                      \
         set_error("raising the LDS limit failed: %s", hipGetErrorString(err));                      \
         return static_cast<int>(err);                                                               \
@@ -1331,10 +1332,10 @@ int launch_routed(const T* x, const int64_t* index, const T* weights, const uint
     hipLaunchKernelGGL(kernel, GRID, BLOCK, LDS, stream, __VA_ARGS__);                              \
     if (int rc = check_launch("wq_gemv_mfma_routed_kernel")) return rc;                             \
   } while (0)
-  if (multi) LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 512, true>), grid, block, L.total, up, route);
-  else if (wk <= 4) LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 256, false>), grid, block, L.total, up, route);
-  else if (wk <= 8) LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 512, false>), grid, block, L.total, up, route);
-  else LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 1024, false>), grid, block, L.total, up, route);
+  if (multi) LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 512, true>), grid, block, L.total, 0, up, route);
+  else if (wk <= 4) LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 256, false>), grid, block, L.total, 0, up, route);
+  else if (wk <= 8) LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 512, false>), grid, block, L.total, 0, up, route);
+  else LLMQ_ROUTED((wq_gemv_mfma_routed_kernel<T, BITS, 1024, false>), grid, block, L.total, 0, up, route);
 
   MfmaArgs down{};
   down.x = act; down.qw = q2; down.ws = s2; down.out = out;
@@ -1347,8 +1348,8 @@ int launch_routed(const T* x, const int64_t* index, const T* weights, const uint
   route.scale_stride = static_cast<int64_t>(H) * down.G;
   const int units = top_k * (down.G / kGW), waves = units < 16 ? units : 16;
   const int lds = routed_down_lds(top_k, down.G, BITS == 4);
-  LLMQ_ROUTED((wq_gemv_mfma_routed_down_kernel<T, BITS>), dim3(down.n_tiles, tokens), dim3(waves * kWave), lds, down, route,
-              weights);
+  LLMQ_ROUTED((wq_gemv_mfma_routed_down_kernel<T, BITS>), dim3(down.n_tiles, tokens), dim3(waves * kWave), lds,
+              kRoutedMaxTopK * kTileRows * static_cast<int>(sizeof(float)), down, route, weights);
 #undef LLMQ_ROUTED
   return 0;
 }

@@ -293,6 +293,7 @@ def test_experts_that_are_not_silu_keep_the_unfused_forward(ext):
     (1, 2048, 1024, 64, 8),    # a unit a wave, tiles of eight rows
     (8, 2048, 1024, 64, 8),
     (2, 512, 1536, 20, 16),    # 48 units on 16 waves, the largest top_k
+    (2, 512, 3072, 8, 6),      # int4: the down launch's LDS passes 64 KB only with the products it holds beside the rows
     (1, 8704, 8192, 3, 2),     # gate|up rows of more chunks than waves, down rows of sixteen chunks
 ])
 def test_direct_launches_equal_the_planned_ones(ext, bits, dtype, tokens, hidden, inter, experts, top_k):
