@@ -22,6 +22,7 @@ q/k/v sharing bit width and out_group, gate/up sharing bit width.
 from __future__ import annotations
 
 import torch
+from torch.nn.modules import module as nn_module
 
 from llmquant.hip.build import load_extension
 from llmquant.quantizers.kernel import KernelQuantLinear
@@ -344,10 +345,11 @@ class LlamaFusedRuntime(LlamaKernelRuntime):
     def _set_step_inputs(self, token, position: int):
         self._splits_now = self._splits_for(position)
         table = self.model.model.embed_tokens
-        # (the table that the captured step looks its next rows up in, and nothing that watches the module's calls)
-        if (self._embed_table is not None and type(table) is torch.nn.Embedding
+        # (the table that the captured step looks its next rows up in, and nothing that watches or replaces the module's call)
+        if (self._embed_table is not None and type(table) is torch.nn.Embedding and "forward" not in table.__dict__
                 and table.weight.data_ptr() == self._embed_table.data_ptr()
-                and not (table._forward_hooks or table._forward_pre_hooks)):
+                and not (table._forward_hooks or table._forward_pre_hooks or nn_module._global_forward_hooks
+                         or nn_module._global_forward_pre_hooks)):
             self._seed(token, position, self._embed_table, self._hidden0)
             return
         super()._set_step_inputs(token, position)

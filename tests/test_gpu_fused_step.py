@@ -399,6 +399,37 @@ def test_seed_step_sets_what_a_step_reads(ext, dtype, hidden):
         ext.seed_step(None, None, None, position, length, 0, 0, table, row)
 
 
+@pytest.mark.parametrize("how", ["forward", "hook", "pre_hook", "global_hook", "global_pre_hook"])
+def test_a_given_token_goes_through_an_embedding_whose_call_is_watched_or_replaced(how):
+    """The row a step from a given token starts from is what the module's call returns, as for any other module."""
+    from test_gpu_decode import build_model, quantized_pair
+
+    from llmquant.runtime import LlamaFusedRuntime
+
+    _, kernel = quantized_pair(build_model(512, 1024, 1, 8, 2, 4096))
+    runtime, table, token = LlamaFusedRuntime(kernel, 80, 8), kernel.model.embed_tokens, torch.tensor([7], device="cuda")
+    runtime._set_step_inputs(token, 5)
+    row = table.weight[7:8].detach()
+    assert torch.equal(runtime._hidden0, row)
+    module = torch.nn.modules.module
+    other, twice = (lambda ids: table.weight.detach()[ids + 1]), (lambda mod, args, out: out * 2 if mod is table else None)
+    shifted = lambda mod, args: (args[0] + 1,) if mod is table else None  # noqa: E731
+    if how == "forward":
+        table.forward = other
+    else:
+        handle = {"hook": lambda: table.register_forward_hook(twice), "pre_hook": lambda: table.register_forward_pre_hook(shifted),
+                  "global_hook": lambda: module.register_module_forward_hook(twice),
+                  "global_pre_hook": lambda: module.register_module_forward_pre_hook(shifted)}[how]()
+    try:
+        with torch.no_grad():
+            runtime._set_step_inputs(token, 5)
+    finally:
+        if how != "forward":
+            handle.remove()
+    want = row * 2 if "pre" not in how and how != "forward" else table.weight[8:9].detach()
+    assert torch.equal(runtime._hidden0, want)
+
+
 def test_fused_runtime_equals_the_unfused_one():
     """Whole decode steps on a small model: fused and operation-by-operation runtimes give the
     same logits to the bit (hidden 512: the variance reduction happens to agree), the same
