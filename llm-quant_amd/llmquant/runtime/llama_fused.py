@@ -52,12 +52,25 @@ def _fusable(*mods) -> bool:
 # (the vector-ALU form, which caches below 2048 rows keep, with 8 splits: 546-551 / 555 / 578 / 595 at 600 / 1000 / 2000 /
 # 3500, 673 at 7000)
 MID_CONTEXT_FROM = 5120
-# Splits from which the records are merged by a launch of their own in front of o_proj instead of inside it, where every
-# workgroup of the GEMV merges all of them, eight records at a time. A step of four 1B layers / two 8B layers and lm_head,
-# merged inside / by a launch, us: 8 splits 175 / 177 and 219 / 217, 16 splits (8000 cached) 190.7 / 189.5 and
-# 228.7 / 225.0, 32 splits (24000, 20000) 209.1 / 205.8 and 243 / 235.
+# From this many splits on, and for attention outputs of at least this many values (heads x head size), the records are
+# merged by a launch of their own in front of o_proj instead of inside it, where every workgroup of the GEMV merges all of
+# them, eight records at a time. A step of four 1B layers / two 8B layers and lm_head, merged inside / by a launch, us:
+# 8 splits 175 / 177 and 219 / 217, 16 splits (8000 cached) 190.7 / 189.5 and 228.7 / 225.0, 32 splits (24000, 20000)
+# 209.1 / 205.8 and 243 / 235. A narrow o_proj is a launch of few workgroups that merge side by side, and there the launch
+# costs more than it saves. Four layers of hidden size heads x head size, MLP four times that, vocabulary 4096, at 100 / 8000
+# / 24000 cached: 8 x 128 (32 splits) 124.0 / 126.3, 128.8 / 131.3, 140.4 / 142.1; 16 x 64 (16 splits, 32 at 24000)
+# 112.1 / 112.9, 119.8 / 122.1, 133.0 / 132.5; 12 x 64 (21) 115.7 / 116.2, 127.3 / 127.5, 149.7 / 150.4; 20 x 64 (16)
+# at 8000 146.3 / 147.2; 8 x 64 (32) is the exception, 105.4 / 104.2, 118.9 / 116.0, 134.0 / 133.9. Wider: 16 x 128 (16)
+# 136.0 / 135.3, 147.0 / 144.0, 167.1 / 164.3; 32 x 64 (16) at 8000 138.6 / 138.2; 24 x 128 (16) 275.9 / 271.2, 366 / 360;
+# 28 x 128 (16) 300 / 292.6, 389 / 383; 40 x 128 (16) 546 / 482, 680 / 617.
 MERGE_LAUNCH_FROM = 16
+MERGE_LAUNCH_MIN_WIDTH = 2048
 LONG_CONTEXT_FROM = 16384
+
+
+def merge_launch_pays(splits: int, width: int) -> bool:
+    """Whether a step merges its attention records by a launch of their own: `splits` a head, `width` = heads x head size."""
+    return splits >= MERGE_LAUNCH_FROM and width >= MERGE_LAUNCH_MIN_WIDTH
 
 
 def _code_bits(qdata) -> int:
@@ -305,7 +318,7 @@ class LlamaFusedRuntime(LlamaKernelRuntime):
                                                 cache.v_codes[index], cache.k_scale[index], cache.v_scale[index],
                                                 self._partials, cache.position, self.scaling, self.q_heads,
                                                 splits)
-                if splits >= MERGE_LAUNCH_FROM:
+                if merge_launch_pays(splits, self.q_heads * self.head_dim):
                     ctx = ext.kv_attend_merge(self._partials, self.q_heads, self.head_dim, splits, hidden.dtype)
                     hidden = ext.wq_gemv_fused(ctx, f["o"].qdata, f["o"].wscale, f["o"].out_group, PRO_NONE, None, 0.0,
                                                f["o_head_dim"], hidden)

@@ -453,3 +453,14 @@ def test_which_ragged_rows_the_quantizer_takes_in_place(numel, width, element_si
     from llmquant.hip.ops import _rows_in_place
 
     assert _rows_in_place(numel, width, element_size, group_size) is taken
+
+
+@pytest.mark.parametrize("splits,width,launch", [
+    (8, 32 * 128, False), (16, 32 * 64, True), (15, 32 * 64, False), (32, 32 * 64, True),
+    (64, 4 * 128, False), (32, 8 * 128, False), (16, 16 * 64, False), (21, 12 * 64, False),   # narrow: slower by a launch
+    (16, 16 * 128, True),
+])
+def test_which_decode_steps_merge_their_records_by_a_launch(splits, width, launch):
+    from llmquant.runtime.llama_fused import merge_launch_pays
+
+    assert merge_launch_pays(splits, width) is launch
