@@ -306,11 +306,21 @@ int launch_typed(const void* x, const void* qw, const float* ws, void* out, int 
   if (G >= 4 && wk * 2 > G) wk = G / 2;
   // Row tiles of a workgroup share the activation rows a wave loads: those come from L2 once per workgroup, and 16
   // weight rows a workgroup make that traffic four times the codes' at M = 16. Two tiles as long as a workgroup per CU
-  // and more is left, four where that leaves most CUs one. Measured, us with 1 / 2 / 4 tiles: 14336 x 4096 int4 bf16
-  // M = 16: 14.6 / 13.0 / 12.4, 32: 19.6 / 17.8 / 14.7, 48: 29.4 / 21.2 / 17.8; int8 M = 32: 29.5 / 24.8 / 20.1;
-  // 28672 x 4096 int4 32: 41 / 39 / 31; 128256 x 2048 int4 M = 16: 62 / 49 / 56, 32: 90 / 93 / 70, 48: 160 / 108 / 87;
-  // 8192 x 2048 M = 32: 7.4 / 6.7 / 9.1; 4096 x 4096 M = 64: 10.2 / 13.7 / -. Four tiles against 64 rows, and int8 codes
-  // against 48, are more registers than a wave has (spills: 41 us against 26).
+  // and more is left (14336 x 4096 int4 bf16, one / two tiles, us: M = 16 14.6 / 13.0, 32 19.6 / 17.8, 48 29.4 / 21.2; 4096
+  // x 4096, M = 64: 10.2 / 13.7).
+  // Four tiles (one workgroup a CU) by how full their last round of 256 workgroups is. Measured, two / four tiles, us,
+  // weights rotated through 600 MB, bf16; fp16 is within 3 % of it, also where its 33 to 48 rows against int4 spill two
+  // registers (14336 x 4096, M = 48: 24.7 / 19.9):
+  //  17 rows and more, K = 4096: 192 workgroups int4 M = 17 / 32 / 48: 17.3 / 14.8, 20.7 / 16.4, 24.3 / 19.1, int8 32: 24.3 /
+  //  19.8; 256: 18.0 / 15.2, 21.3 / 17.0, 25.2 / 19.8, int8 26.4 / 21.2; but 260 to 384, a second round at most half full:
+  //  288 24.9 / 26.8, 29.8 / 30.0, 34.9 / 35.1, int8 17 29.8 / 33.3; 384 26.9 / 27.9, 30.8 / 30.5, int8 17 33.9 / 34.4; 416
+  //  32.9 / 27.7, 39.1 / 30.8, int8 39.5 / 35.1; 528, where the third is nearly empty, int4 M = 32 8 % faster, int8 4 %.
+  //  Below 192: 8192 x 2048 M = 32 6.7 / 9.1.
+  //  Up to 16 rows there is less to share: one round only (288: M = 3 16.7 / 22.1, 16 20.3 / 24.7; 448: 21.9 / 23.2, 26.3 /
+  //  25.9), rows of 32 groups (256 workgroups, M = 3 / 16: K = 2048 7.9 / 8.5, 9.3 / 9.2; K = 4096 14.1 / 13.9, 15.5 / 14.2;
+  //  K = 8192 25.1 / 24.7, 28.1 / 25.7), and for int8 codes nine rows (256: M = 4 17.4 / 18.1, 8 17.8 / 18.1, 12 18.7 / 18.7,
+  //  16 19.7 / 18.9).
+  // Four tiles against 64 rows, and int8 codes against 48, are more registers than a wave has (spills: 41 us against 26).
   const bool wide = N >= 2 * kTileN * 256;
   const int quads = (N + 4 * kTileN - 1) / (4 * kTileN);
   const int64_t limit = int64_t{1} << 32;   // the four-tile form's offsets from its scalar bases
@@ -326,17 +336,18 @@ int launch_typed(const void* x, const void* qw, const float* ws, void* out, int 
     a.N = N; a.G = G; a.out_group = out_group;
     a.row_bytes = K * BITS / 8;
     const int mt = (a.M + kTileM - 1) / kTileM;
-    // Four row tiles (see above): outputs that still give three quarters of the CUs a workgroup; for one activation tile,
-    // where there are few rows to share, only where those workgroups are one round and rows long enough to fill it.
-    const bool four = quads >= 192 && offsets32 &&
-                      (mt == 1 ? quads <= 256 && G >= 32 : mt == 2 || (mt == 3 && BITS == 4));
+    const bool few_rows = mt == 1 && quads <= 256 && G >= 32 && (BITS == 4 || a.M > 8);
+    const bool more_rows = (mt == 2 || (mt == 3 && BITS == 4)) && (quads <= 256 || quads > 384);
     int rc;
-    if (four) {
+    if (quads >= 192 && offsets32 && (few_rows || more_rows)) {
       constexpr bool kBi = BITS == 4;
-      if (mt == 1) rc = launch_tile<T, BITS, 1, 4, kBi>(a, wk, stream);
-      else if (mt == 2) rc = launch_tile<T, BITS, 2, 4, kBi>(a, wk, stream);
-      else if constexpr (BITS == 4) rc = launch_tile<T, BITS, 3, 4, kBi>(a, wk, stream);
-      else rc = llmq_host::fail_invalid("internal: no such tile");
+      if (mt == 1) {
+        rc = launch_tile<T, BITS, 1, 4, kBi>(a, wk, stream);
+      } else if constexpr (BITS == 4) {
+        rc = mt == 2 ? launch_tile<T, BITS, 2, 4, kBi>(a, wk, stream) : launch_tile<T, BITS, 3, 4, kBi>(a, wk, stream);
+      } else {
+        rc = launch_tile<T, BITS, 2, 4, kBi>(a, wk, stream);
+      }
     } else if (wide) {
       switch (mt) {
         case 1: rc = launch_tile<T, BITS, 1, 2, BITS == 4>(a, wk, stream); break;

@@ -109,6 +109,7 @@ def test_llama_shapes_on_sampled_entries(ext, n, k, m, split):
     (5, 12225, 4096, 0),                                              # four row tiles, one activation tile; ragged in rows
     (17, 12289, 640, 0), (32, 12352, 512, 64), (33, 12289, 384, 0), (48, 12300, 256, 0),   # two and three activation tiles
     (64, 12289, 256, 0), (16, 16448, 256, 0), (33, 8201, 384, 0),     # two row tiles: past 48 rows, short rows, fewer rows
+    (9, 12225, 4096, 0), (17, 16385, 256, 0), (48, 24577, 256, 0),    # int8's first row count; a full round + 1, 1.5 + 1
 ])
 def test_wide_outputs_take_more_row_tiles_a_workgroup(ext, bits, dtype, m, n, k, out_group):
     x, q, s, canonical, scales = make_case(m, n, k, bits, dtype, out_group=out_group, seed=5)
