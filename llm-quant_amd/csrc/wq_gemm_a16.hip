@@ -108,34 +108,42 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   const int64_t K = static_cast<int64_t>(G) * kGroup;
 
   const int n0 = blockIdx.x * kRows;
-  // (four row tiles: offsets of 32 bits from a scalar base instead of addresses; their registers are needed)
-  using Offset = typename std::conditional<NT == 4, uint32_t, int64_t>::type;
-  Offset wrow[NT], srow[NT];
+  // (four row tiles: offsets of 32 bits from a scalar base instead of addresses, their registers are needed; the others
+  // keep addresses: 8192 x 2048 int4, M = 16: 5.85 us, 5.98 from offsets)
+  using Place = typename std::conditional<NT == 4, uint32_t, const uint8_t*>::type;
+  auto place = [](const auto* base, int64_t count) {
+    if constexpr (NT == 4) return static_cast<uint32_t>(count * sizeof(*base));
+    else return reinterpret_cast<const uint8_t*>(base + count);
+  };
+  auto address = [](const void* base, Place at, int64_t step) {
+    if constexpr (NT == 4) return static_cast<const uint8_t*>(base) + step + at;
+    else return at + step;
+  };
+  Place wrow[NT], srow[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int n = min(n0 + nt * kTileN + j, a.N - 1);
-    wrow[nt] = static_cast<Offset>(n) * static_cast<Offset>(a.row_bytes) + blk * (BITS == 4 ? 16 : 32);
-    srow[nt] = static_cast<Offset>(a.out_group > 0 ? n / a.out_group : n) * G * 4;
+    wrow[nt] = place(a.qw, static_cast<int64_t>(n) * a.row_bytes + blk * (BITS == 4 ? 16 : 32));
+    srow[nt] = place(a.ws, static_cast<int64_t>(a.out_group > 0 ? n / a.out_group : n) * G);
   }
   // ---- x of one group: [16 MT rows][16 slots of 16 bytes], slot p of row r holds chunk p ^ (r & 15) ------------
   // transfer i of the wave covers rows 4 i .. 4 i + 3; lane = (row 4 i + lane / 16, slot lane % 16)
   constexpr int kXInstr = MT * 4;
   constexpr int kXTileBytes = MT * kTileM * kGroup * 2;
   unsigned char* xtile = smem + wv * kXTileBytes;
-  Offset xsrc[kXInstr];
+  Place xsrc[kXInstr];
 #pragma unroll
   for (int i = 0; i < kXInstr; ++i) {
     const int row = 4 * i + (lane >> 4), chunk = (lane & 15) ^ (row & 15);
-    xsrc[i] = static_cast<Offset>(min(row, a.M - 1)) * static_cast<Offset>(K * 2) + chunk * 16;
+    xsrc[i] = place(static_cast<const T*>(a.x), min(row, a.M - 1) * K + chunk * 8);
   }
   auto request_rows = [&](int g) {
-    const unsigned char* xg = static_cast<const unsigned char*>(a.x) + static_cast<int64_t>(g) * (kGroup * 2);
 #pragma unroll
     for (int i = 0; i < kXInstr; ++i) {
       // (four rows past the activation's end are not fetched: what the tile holds there feeds only result rows
       // that are dropped at the store)
       if (4 * i < a.M) {
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(xg + xsrc[i]),
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(address(a.x, xsrc[i], static_cast<int64_t>(g) * (kGroup * 2))),
                                          reinterpret_cast<u32x4*>(xtile + 1024 * i), 16, 0, 0);
       }
     }
@@ -155,13 +163,13 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   auto load_weights = [&](int g, Weights& W) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      const uint8_t* p = a.qw + static_cast<int64_t>(g) * (kGroup * BITS / 8) + wrow[nt];
+      const uint8_t* p = address(a.qw, wrow[nt], static_cast<int64_t>(g) * (kGroup * BITS / 8));
 #pragma unroll
       for (int q = 0; q < kRaw / 4; ++q) {
         const u32x4 r = load16(p + 16 * q);
         W.raw[nt][4 * q] = r.x; W.raw[nt][4 * q + 1] = r.y; W.raw[nt][4 * q + 2] = r.z; W.raw[nt][4 * q + 3] = r.w;
       }
-      W.scale[nt] = *reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.ws + g) + srow[nt]);
+      W.scale[nt] = *reinterpret_cast<const float*>(address(a.ws, srow[nt], static_cast<int64_t>(g) * 4));
     }
   };
   auto read_rows = [&](Rows& X) {
