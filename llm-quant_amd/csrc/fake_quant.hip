@@ -106,26 +106,26 @@ template <typename T> __device__ __forceinline__ u32x4 load_packet(const T* p) {
   return v;
 }
 template <typename T, int V = Pack<T>::N> __device__ __forceinline__ void load_elements(const T* p, int n, float* f) {
-  if constexpr (V == 1) {
-    f[0] = n > 0 ? to_float(p[0]) : 0.0f;
-  } else if (n >= V) {
-    Pack<T>::unpack(load_packet(p), f);
-  } else {
-#pragma unroll
-    for (int i = 0; i < V; ++i) f[i] = i < n ? to_float(p[i]) : 0.0f;
+  if constexpr (V == Pack<T>::N) {
+    if (n >= V) {
+      Pack<T>::unpack(load_packet(p), f);
+      return;
+    }
   }
+#pragma unroll
+  for (int i = 0; i < V; ++i) f[i] = i < n ? to_float(p[i]) : 0.0f;
 }
 template <typename T, int V = Pack<T>::N> __device__ __forceinline__ void store_elements(T* p, int n, const float* q) {
-  if constexpr (V == 1) {
-    if (n > 0) p[0] = from_float<T>(q[0]);
-  } else if (n >= V) {
-    const u32x4 v = Pack<T>::pack(q);
-    __builtin_memcpy(p, &v, sizeof v);
-  } else {
-#pragma unroll
-    for (int i = 0; i < V; ++i) {
-      if (i < n) p[i] = from_float<T>(q[i]);
+  if constexpr (V == Pack<T>::N) {
+    if (n >= V) {
+      const u32x4 v = Pack<T>::pack(q);
+      __builtin_memcpy(p, &v, sizeof v);
+      return;
     }
+  }
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    if (i < n) p[i] = from_float<T>(q[i]);
   }
 }
 
@@ -175,8 +175,11 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(
 
 // Any group size, any alignment: WAVES waves per group (one: four groups a workgroup), every thread HELD packets of it
 // in registers between the reduction and the quantize step; what goes beyond is read again. Packets are V elements: 16
-// bytes of 16-bit types at any address (4096 x 14336 bf16, a group a row: 102 us element by element, 48.5 here), one
-// element of fp32 (a wave's 256 bytes are whole cache lines either way; 3000 x 3000: 12.2 us, 13.1 in packets).
+// bytes at any address (a group a row, one element at a time / here, us: 4096 x 14336 bf16 73 / 37, fp32 137 / 107, int8
+// codes of fp32 81 / 60; 3000 x 3000 fp32 12.1 / 11.9, its int8 codes 9.5 / 9.9; 1024 x 4096 bf16 7.0 / 5.3). Groups below
+// a packet, and fp32 groups that a wave's lanes hold in four elements each, go element by element (codes of two: nibble
+// pairs): one division a lane instead of a chain of eight (64 groups of 4 bf16 2.3 us, 3.0 in a packet; 100000 groups of 20
+// fp32 13.3 us, 19.9 in packets).
 constexpr int kBlockThreads = 256;
 
 template <typename T, int MODE, int WAVES, int HELD, int V>
@@ -186,22 +189,26 @@ __global__ __launch_bounds__(kBlockThreads) void quant_group_kernel(
   constexpr int kThreads = WAVES * kWave;   // threads of a group
   __shared__ float s_part[kBlockThreads / kWave];
   const int tid = threadIdx.x % kThreads;
-  const int64_t group = static_cast<int64_t>(blockIdx.x) * (kBlockThreads / kThreads) + threadIdx.x / kThreads;
-  if (group >= n_groups) return;   // (whole waves; with four waves a group every workgroup has one)
+  const int64_t group = WAVES * kWave == kBlockThreads ? blockIdx.x
+                                                       : static_cast<int64_t>(blockIdx.x) * (kBlockThreads / kThreads) + threadIdx.x / kThreads;
+  if (kThreads < kBlockThreads && group >= n_groups) return;   // (whole waves)
   const int64_t base = group * group_size;
 
   // A packet that would run past the group's end starts earlier: what it repeats changes no maximum, and is written
-  // twice with the same values. (Groups below a packet: element by element.)
+  // twice with the same values. (Groups below a packet come with a smaller V, element by element.)
+  constexpr bool kPackets = V == Pack<T>::N;
   const int last = group_size - V;
   float held[HELD][V];
   float amax = 0.0f;
-  if constexpr (V == 1) {
-#pragma unroll
-    for (int j = 0; j < HELD; ++j) held[j][0] = to_float(x[base + min(tid + j * kThreads, last)]);
-  } else if (last >= 0) {
+  if constexpr (kPackets) {
+    // (four waves: threads past the group's end load nothing, clamped loads that nobody needs cost up to a seventh there;
+    // one wave: they repeat the last packet, 514 elements 5.25 us a launch of 4096 groups against 5.5)
     u32x4 raw[HELD];
 #pragma unroll
-    for (int j = 0; j < HELD; ++j) raw[j] = load_packet(x + base + min((tid + j * kThreads) * V, last));
+    for (int j = 0; j < HELD; ++j) {
+      const int i = (tid + j * kThreads) * V;
+      raw[j] = WAVES == 1 || i < group_size ? load_packet(x + base + min(i, last)) : u32x4{0u, 0u, 0u, 0u};
+    }
 #pragma unroll
     for (int j = 0; j < HELD; ++j) Pack<T>::unpack(raw[j], held[j]);
   } else {
@@ -233,8 +240,7 @@ __global__ __launch_bounds__(kBlockThreads) void quant_group_kernel(
   const float scale = scale_from_amax(amax, qmax);
   if (scale_out != nullptr && tid == 0) scale_out[group] = scale;
 
-  auto emit = [&](int i, const float* f) {
-    const int n = group_size - i;
+  auto emit = [&](int i, int n, const float* f) {   // (n: elements from there to the group's end, V if more do not matter)
     float q[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) q[e] = quant_code(f[e], scale, qmin, qmax);
@@ -277,12 +283,12 @@ __global__ __launch_bounds__(kBlockThreads) void quant_group_kernel(
 #pragma unroll
   for (int j = 0; j < HELD; ++j) {
     const int i = (tid + j * kThreads) * V;
-    if (i < group_size) emit(last >= 0 ? min(i, last) : i, held[j]);
+    if (i < group_size) emit(kPackets ? min(i, last) : i, kPackets ? V : group_size - i, held[j]);
   }
   for (int i = (tid + HELD * kThreads) * V; i < group_size; i += kThreads * V) {
     float f[V];
     load_elements<T, V>(x + base + i, group_size - i, f);
-    emit(i, f);
+    emit(i, group_size - i, f);
   }
 }
 
@@ -361,14 +367,11 @@ int launch_typed(const void* x, void* out, float* scale, int64_t n_groups, int g
 #define LLMQ_GROUP(WAVES, HELD, V)                                                                                   \
   hipLaunchKernelGGL((quant_group_kernel<T, MODE, WAVES, HELD, V>), grid, block, 0, stream,                          \
                      static_cast<const T*>(x), out, scale, n_groups, group_size, qmin, qmax)
-  if constexpr (MODE != kCodes4 && V == 4) {
-    if (group_size <= kWave * 4) LLMQ_GROUP(1, 4, 1);
-    else if (one_wave) LLMQ_GROUP(1, 16, 1);
-    else LLMQ_GROUP(4, 16, 1);
-    return llmq_host::check_launch("quant_group_kernel");
-  }
-  if (group_size <= kWave * V) LLMQ_GROUP(1, 1, V);
+  if (MODE != kCodes4 && V == 4 && group_size <= kWave * 4) LLMQ_GROUP(1, 4, 1);
+  else if (group_size < V) LLMQ_GROUP(1, 1, MODE == kCodes4 ? 2 : 1);
+  else if (group_size <= kWave * V) LLMQ_GROUP(1, 1, V);
   else if (one_wave) LLMQ_GROUP(1, 4, V);
+  else if (group_size <= 4 * kWave * V * 2) LLMQ_GROUP(4, 2, V);   // (2048 groups of 2050 bf16: 6.3 us, 6.9 with four turns)
   else if (group_size <= 4 * kWave * V * 4) LLMQ_GROUP(4, 4, V);
   else LLMQ_GROUP(4, 8, V);
 #undef LLMQ_GROUP

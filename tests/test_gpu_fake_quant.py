@@ -156,6 +156,29 @@ def test_codes_variant(bits, pack4, dtype):
     assert np.array_equal(to_np(scale), want_scale)
 
 
+@pytest.mark.parametrize("bits,pack4", [(8, False), (4, True)])
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("group_size", [2, 4, 6, 7, 100, 254, 258, 514, 1026, 2046, 2050, 2051, 4098, 8190, 8194, 16392, 20002])
+def test_codes_of_groups_of_any_width(bits, pack4, dtype, group_size):
+    """Integer codes where the lanes of a wave do not hold the group: below a packet, one wave and four at every number of
+    packets a thread, the last packet overlapping, beyond what registers hold, odd widths; and whole packets on a tensor
+    that starts inside one."""
+    from llmquant.hip import load_extension
+
+    if pack4 and group_size % 2:
+        pytest.skip("nibble pairs need an even group")
+    torch.manual_seed(group_size)
+    offset = 1 if group_size % 2 == 0 else 0   # (the other widths bring every alignment themselves)
+    shape = (5, 3 * group_size)
+    x = (torch.randn(5 * 3 * group_size + offset) * 4).to(dtype)
+    on_device = x.cuda()[offset:].view(shape)
+    assert (on_device.data_ptr() % 16 != 0) == bool(offset)
+    codes, scale = load_extension().quant_group_codes(on_device, bits, group_size, pack4)
+    want_codes, want_scale = oracle.quant_group_codes(to_np(x[offset:].view(shape)), bits, group_size)
+    assert np.array_equal(codes.cpu().numpy(), oracle.pack_int4(want_codes) if pack4 else want_codes)
+    assert np.array_equal(to_np(scale), want_scale)
+
+
 def test_bare_c_abi_call():
     """The same kernel through ctypes: plain pointers, sizes and a stream, no torch types."""
     from llmquant.hip import load_capi
@@ -188,7 +211,7 @@ def test_rows_that_are_no_whole_number_of_groups(hip_fake_quantize, dtype, width
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("width", [5, 8, 100, 513, 2047, 2049, 8191, 16392, 20001])
+@pytest.mark.parametrize("width", [5, 8, 100, 513, 2047, 2049, 4097, 8191, 16392, 20001])
 def test_groups_of_any_width(hip_fake_quantize, dtype, width):
     """One group a row: below a packet, one wave and four, the last packet overlapping, beyond what registers hold."""
     torch.manual_seed(width)
