@@ -223,9 +223,10 @@ __global__ __launch_bounds__(kBlockThreads) void quant_group_kernel(
 #pragma unroll
     for (int e = 0; e < V; ++e) amax = fmaxf(amax, fabsf(held[j][e]));
   }
-  for (int i = (tid + HELD * kThreads) * V; i < group_size; i += kThreads * V) {
+  // (unsigned: the last step of a group of close to 2^31 elements passes that)
+  for (uint32_t i = (tid + HELD * kThreads) * V; i < static_cast<uint32_t>(group_size); i += kThreads * V) {
     float f[V];
-    load_elements<T, V>(x + base + i, group_size - i, f);
+    load_elements<T, V>(x + base + i, static_cast<int>(group_size - i), f);
 #pragma unroll
     for (int e = 0; e < V; ++e) amax = fmaxf(amax, fabsf(f[e]));
   }
@@ -285,9 +286,9 @@ __global__ __launch_bounds__(kBlockThreads) void quant_group_kernel(
     const int i = (tid + j * kThreads) * V;
     if (i < group_size) emit(kPackets ? min(i, last) : i, kPackets ? V : group_size - i, held[j]);
   }
-  for (int i = (tid + HELD * kThreads) * V; i < group_size; i += kThreads * V) {
+  for (uint32_t i = (tid + HELD * kThreads) * V; i < static_cast<uint32_t>(group_size); i += kThreads * V) {
     float f[V];
-    load_elements<T, V>(x + base + i, group_size - i, f);
+    load_elements<T, V>(x + base + i, static_cast<int>(group_size - i), f);
     emit(i, group_size - i, f);
   }
 }

@@ -219,3 +219,17 @@ def test_groups_of_any_width(hip_fake_quantize, dtype, width):
     got, scale = hip_fake_quantize(x.cuda(), args(8, strategy="channel"), return_scale=True)
     assert same_bits(got, oracle.fake_quantize(to_np(x), 8, tag_of(dtype), "channel"))
     assert np.array_equal(to_np(scale).reshape(-1), oracle.compute_scale(to_np(x), 8, "channel").reshape(-1))
+
+
+def test_a_group_of_close_to_two_to_the_31_values(hip_fake_quantize):
+    """One row, one group, whose last step of 2048 values passes 2^31: a repeated pattern comes out as the pattern does."""
+    width, period = 2 ** 31 - 1000, 1 << 12
+    pattern = torch.randn(period, generator=torch.Generator().manual_seed(0)).to(torch.bfloat16).cuda()
+    x = torch.empty(1, width, dtype=torch.bfloat16, device="cuda")
+    whole = width // period * period
+    x[0, :whole].view(-1, period).copy_(pattern.expand(whole // period, period))
+    x[0, whole:] = pattern[: width - whole]
+    got = hip_fake_quantize(x, args(8, strategy="channel"))[0]
+    want = hip_fake_quantize(pattern[None], args(8, strategy="channel"))[0]
+    assert all(bool((part == want).all()) for part in got[:whole].view(-1, period).split(1 << 16))
+    assert torch.equal(got[whole:], want[: width - whole])
