@@ -19,6 +19,7 @@ from torch.autograd.forward_ad import unpack_dual
 
 from llmquant.core.observers import group_view
 from llmquant.core.scheme import QuantizationScheme
+from llmquant.hip.build import load_extension
 from llmquant.packing.packing import pack_int4, unpack_int4
 from llmquant.quantizers.real import exact_fp32_matmul, quantize_weight
 
@@ -143,8 +144,6 @@ class KernelQuantExperts(_QuantExperts):
     _what = "kernel"
 
     def _store(self, qgate_up, sgate_up, qdown, sdown):
-        from llmquant.hip.build import load_extension
-
         bits = self.scheme.weights.num_bits
         pack = (lambda t: t.contiguous() if t.dtype == torch.uint8 else pack_int4(t)) if bits == 4 else (
             lambda t: t.contiguous())

@@ -450,3 +450,20 @@ def test_a_prompt_too_long_for_the_grouped_gemms_goes_through_the_loop_unless_ca
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(captured, grouped)
+
+
+def test_a_copied_and_a_pickled_block_give_the_same_rows(ext):
+    import copy
+    import io
+
+    _, quant, _, cfg = kernel_block("int4")
+    hidden = torch.randn(3, cfg.hidden_size, device="cuda", dtype=torch.bfloat16)
+    index, weights = routing(3, cfg.num_local_experts, cfg.num_experts_per_tok, seed=2)
+    index, weights = index.cuda(), weights.cuda()
+    file = io.BytesIO()
+    torch.save(quant, file)
+    file.seek(0)
+    with torch.no_grad():
+        want = quant(hidden, index, weights)
+        for other in (copy.deepcopy(quant), torch.load(file, weights_only=False)):
+            assert torch.equal(other(hidden, index, weights), want)
