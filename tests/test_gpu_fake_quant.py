@@ -66,7 +66,7 @@ def test_other_group_sizes(hip_fake_quantize, group_size):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("group_size", [8, 16, 64, 512, 1024, 4096, 100, 36])
 def test_every_kernel_variant(hip_fake_quantize, dtype, group_size):
-    """Lane-group widths 1..64 and the block kernel (wide, non power-of-two groups)."""
+    """Lane-group widths 1..64, and groups that the lanes of a wave do not hold (wide, non power-of-two)."""
     torch.manual_seed(1)
     x = (torch.randn(24, group_size * 3) * 2).to(dtype)
     got, scale = hip_fake_quantize(x.cuda(), args(8, group_size=group_size), return_scale=True)

@@ -136,8 +136,15 @@ def test_wide_batches_take_the_per_expert_path():
     index, weights = routing(tokens, cfg.num_local_experts, cfg.num_experts_per_tok)
     with torch.no_grad():
         out = quant(hidden, index.cuda(), weights.cuda())
+        looped = quant._forward_looped(hidden, index.cuda(), weights.cuda())   # (where the grouped GEMMs do not apply)
         want = real(hidden, index.cuda(), weights.cuda())
-    assert out.shape == hidden.shape and rel_l2(to_np(out), to_np(want)) <= 2e-2
+    for got in (out, looped):
+        assert got.shape == hidden.shape and rel_l2(to_np(got), to_np(want)) <= 2e-2
+    quant.act_fn = torch.nn.GELU()
+    quant._act_is_silu = quant._probe_silu()
+    with torch.no_grad():
+        assert not quant._takes_gemm(hidden, index.cuda(), weights.cuda())
+        assert torch.isfinite(quant(hidden, index.cuda(), weights.cuda())).all()
 
 
 def test_the_expert_block_replays_from_a_graph():
