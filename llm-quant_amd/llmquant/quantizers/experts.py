@@ -142,6 +142,7 @@ class KernelQuantExperts(_QuantExperts):
     experts refuses them."""
 
     _what = "kernel"
+    _plan_in_one_launch = False   # (of a module pickled without it)
 
     def _store(self, qgate_up, sgate_up, qdown, sdown):
         bits = self.scheme.weights.num_bits
@@ -163,6 +164,7 @@ class KernelQuantExperts(_QuantExperts):
         self._gemv = self._ext.wq_gemv
         self._gemv_batched = self._ext.wq_gemv_batched
         self._batched_max_rows = self._ext.wq_gemv_batched_max_rows()
+        self._plan_in_one_launch = self._ext.route_plan_supported(1, self.num_experts)   # (the rows of a few tokens always fit)
 
     # (the loaded extension is a module object, which copy and pickle refuse: a copy looks it up again)
     def __getstate__(self):
@@ -326,8 +328,7 @@ class KernelQuantExperts(_QuantExperts):
                 and self._ext.wq_experts_direct_supported(hidden_states.shape[0], top_k_index.shape[1], self.num_experts,
                                                           self.hidden_dim, self.intermediate_dim, 4 if self._packed else 8)
                 # (the four-launch form carries no derivative either; the one behind it, for more experts, does)
-                and (self._ext.route_plan_supported(top_k_index.numel(), self.num_experts)
-                     or not self._differentiated(hidden_states, top_k_weights)))
+                and (self._plan_in_one_launch or not self._differentiated(hidden_states, top_k_weights)))
 
     def _forward_fused(self, hidden_states, top_k_index, top_k_weights):
         """Plan, gate|up (storing act(gate) * up), down, weighted sum per token: four launches (a token's rows too many
