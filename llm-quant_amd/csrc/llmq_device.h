@@ -235,6 +235,33 @@ __device__ __forceinline__ void merge_partials8(const float* rec, int n_splits, 
   for (int e = 0; e < 8; ++e) f[e] *= inv;
 }
 
+// ---- memory straight into LDS -------------------------------------------------------------------
+// A scalar base for buffer loads: an address is base + 32-bit lane offset + 32-bit scalar offset, no vector arithmetic.
+// Transfers into LDS take this form and not the FLAT one (global_load_lds): while a FLAT transfer is in flight the compiler
+// waits for all outstanding LDS reads wherever it needs one of them, so that operands read ahead are not ahead any more.
+#if defined(__HIP_DEVICE_COMPILE__)
+using BufferBase = __amdgpu_buffer_rsrc_t;
+#else
+struct BufferBase {};
+#endif
+__device__ __forceinline__ BufferBase buffer_base(const void* base) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, -1, 0x00020000);   // raw bytes, 4 GiB
+#else
+  return {};
+#endif
+}
+// BYTES (4 or 16) per lane: lane i's go to lds + i * BYTES (lds: uniform over the wave)
+template <int BYTES>
+__device__ __forceinline__ void buffer_to_lds(const BufferBase& base, void* lds, uint32_t lane_offset, uint32_t offset) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(BYTES == 4 || BYTES == 16, "the sizes that are used");
+  auto* to = (__attribute__((address_space(3))) void*)lds;
+  if constexpr (BYTES == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(base, to, 16, lane_offset, offset, 0, 0);
+  else __builtin_amdgcn_raw_ptr_buffer_load_lds(base, to, 4, lane_offset, offset, 0, 0);
+#endif
+}
+
 // ---- codes as 16-bit matrix-core operands without a conversion instruction -------------------------------
 // A 4-bit code is stored with a bias of 8 (n = code + 8, 0..15); placed in the mantissa of 16.0 it IS the value
 // 16 + n in bf16 (0x4180 | n << 3) and in fp16 (0x4c00 | n << 6), two codes per AND-OR. An 8-bit code with its

@@ -14,11 +14,15 @@
 // 32 of the 256 columns and all 128 rows: 4 x 1 MFMA tiles of 32 x 32 (v_mfma_f32_32x32x16_bf16), eight
 // k-steps of 16 per group. A lane converts the codes of one column only, and each converted operand feeds four
 // MFMAs (with 64 x 64 per wave two waves converted the same codes: measured 3-4 % slower on the large shapes).
-// Everything reaches LDS straight from global memory (global_load_lds_dwordx4, 1 KB per wave instruction,
+// Everything reaches LDS straight from global memory (buffer loads into LDS, 1 KB per wave instruction,
 // XOR-swizzled by row so that the operand reads are conflict-free), three stages deep for int4, two for int8:
 // the activation tile, the raw codes of the 256 weight rows, the activation-sum records and the group's scales.
-// The workgroup meets once per group, before the last k-step, and the next group's operands are read from LDS
+// The workgroup meets once per group, when its last operands are in registers, and the next group's are read from LDS
 // behind that barrier.
+// What bounds it: power, then issue. 192 workgroups, 16 to 64 groups: 1.74 us a group with the loop a k-step at a time
+// and FLAT transfers (the same on all-zero operands: 1.64), 1.55 with the loop below (zeros: 1.39); with the transfers
+// taken out 1.24, with the operand reads taken out 1.41, the multiplications alone 1.07. 512 x 14336 x 4096 int4, fp16:
+// 66.9 -> 61.8 us, bf16 with its preparation 75.6 -> 69.9; 2048 x 14336 x 4096 273 -> 255.
 //
 // Codes become bf16 without a conversion instruction: a nibble n = code + 8 placed in the mantissa of
 // 16.0 (bits 0x4180 | n << 3) IS the bf16 value 16 + n, two nibbles per AND-OR (int8: code + 128 through
@@ -90,6 +94,7 @@ template <int BM, int COLS, int KH, int WGS = 1> struct Shape {
   template <int BITS>
   static constexpr int kStages = (160 * 1024 / WGS / kStageBytes<BITS>) >= 4 ? 4 : (160 * 1024 / WGS / kStageBytes<BITS>);
   template <int BITS> static constexpr int kLdsBytes = kStages<BITS> * kStageBytes<BITS>;
+  static constexpr bool kRowBlocks = kMT * KH == 4;   // the loop of wide and narrow tiles (the kernel's main loop has two forms)
 };
 using Wide = Shape<128, 8, 1>;
 using Narrow = Shape<64, 4, 2>;
@@ -365,49 +370,41 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   const int rec_wave = (wv + kWaves - kLeftCodes) % kWaves % (kRecWaves ? kRecWaves : 1);
   const int scale_wave = (wv + kWaves - kLeftCodes - kRecWaves) % kWaves % kScaleWaves;
   const uint32_t r_off = source_row(rec_wave * 64 + lane) * a.G * 16;
-  const float* sw_lane;
+  uint32_t s_off;
   {
     const int n = weight_row(scale_wave * 64 + lane);
-    sw_lane = sw + static_cast<int64_t>(a.out_group > 0 ? n / a.out_group : n) * a.G;
+    s_off = static_cast<uint32_t>(a.out_group > 0 ? n / a.out_group : n) * a.G * 4;
   }
 
-  // (a lane's 32-bit offset goes through an empty asm where it is used: the compiler then adds it to the scalar
-  // base inside the instruction, scalar base + 32-bit lane offset, instead of keeping a 64-bit address per lane
-  // and transfer across the loop and adding the group's step to each with the vector ALU)
-  auto here = [](uint32_t offset) {
-    asm volatile("" : "+v"(offset));
-    return offset;
-  };
-  auto request = [&](int g, int buf) {
+  // Transfer instruction i of a wave for group g into stage `buf`: the activation's, the codes', and the one beyond
+  // the even share.
+  const BufferBase x_base = buffer_base(a.xp), w_base = buffer_base(qw), r_base = buffer_base(a.rec), s_base = buffer_base(sw);
+  auto transfer = [&](int i, int g, int buf) {
     uint8_t* stage = smem + buf * kStageB;
-    const uint8_t* xg = a.xp + static_cast<uint32_t>(g) * kRowBytes;
-#pragma unroll
-    for (int i = 0; i < kXInstr; ++i) {
-      __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(xg + here(x_off[i])),
-                                       reinterpret_cast<u32x4*>(stage + (wv * (kBM / kWaves) + i * 4) * kRowBytes), 16,
-                                       0, 0);
-    }
-    const uint8_t* wg = qw + static_cast<uint32_t>(g) * kCodeRowBytes<BITS>;
-#pragma unroll
-    for (int i = 0; i < kCodeInstr; ++i) {
-      __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(wg + here(w_off[i])),
-                                       reinterpret_cast<u32x4*>(stage + kTileBytes + (wv * kCodeInstr + i) * 1024), 16,
-                                       0, 0);
-    }
-    if (wv < kLeftCodes) {
-      __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(wg + here(w_off[kCodeInstr])),
-                                       reinterpret_cast<u32x4*>(stage + kTileBytes + (kWaves * kCodeInstr + wv) * 1024),
-                                       16, 0, 0);
+    uint8_t* codes = stage + kTileBytes;
+    if (i < kXInstr) {
+      buffer_to_lds<16>(x_base, stage + (wv * (kBM / kWaves) + i * 4) * kRowBytes, x_off[i], g * kRowBytes);
+    } else if (i < kXInstr + kCodeInstr) {
+      const int c = i - kXInstr;
+      buffer_to_lds<16>(w_base, codes + (wv * kCodeInstr + c) * 1024, w_off[c], g * kCodeRowBytes<BITS>);
+    } else if (wv < kLeftCodes) {
+      buffer_to_lds<16>(w_base, codes + (kWaves * kCodeInstr + wv) * 1024, w_off[kCodeInstr], g * kCodeRowBytes<BITS>);
     } else if (wv < kLeftCodes + kRecWaves) {
-      __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(a.rec + static_cast<uint32_t>(g) * 16 + here(r_off)),
-                                       reinterpret_cast<u32x4*>(stage + kTileBytes + kCodeTileB + rec_wave * 1024),
-                                       16, 0, 0);
+      buffer_to_lds<16>(r_base, codes + kCodeTileB + rec_wave * 1024, r_off, g * 16);
     } else if (wv < kExtraWaves) {
-      // the scales of 64 columns, one float per lane
-      __builtin_amdgcn_global_load_lds(
-          sw_lane + g, reinterpret_cast<float*>(stage + kTileBytes + kCodeTileB + kRecTileBytes + scale_wave * 256),
-          4, 0, 0);
+      buffer_to_lds<4>(s_base, codes + kCodeTileB + kRecTileBytes + scale_wave * 256, s_off, g * 4);   // 64 columns' scales
     }
+  };
+  constexpr int kTransfers = kXInstr + kCodeInstr + 1;
+  auto request = [&](int g, int buf) {
+#pragma unroll
+    for (int i = 0; i < kTransfers; ++i) transfer(i, g, buf);
+  };
+  // (part p of `parts` of them)
+  auto request_part = [&](int g, int buf, int p, int parts) {
+#pragma unroll
+    for (int i = 0; i < kTransfers; ++i)
+      if (i * parts / kTransfers == p) transfer(i, g, buf);
   };
   // transfer instructions per wave and group (a compile-time count per branch: the waits below name how many
   // of the youngest may still be in flight)
@@ -446,19 +443,155 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   const u32x4 bias_operand = {nb2, nb2, 0u, 0u};
 
   // ---- prologue: the first groups on their way, the first one's operands in registers ---------------------
+  // (a stage fewer where the loop can ask for it in the first group's blocks: the first group comes sooner)
+  constexpr int kFirstRequests = S::kRowBlocks && kStagesN >= 3 ? kStagesN - 1 : kStagesN;
 #pragma unroll
-  for (int st = 0; st < kStagesN; ++st) {
+  for (int st = 0; st < kFirstRequests; ++st) {
     if (g_begin + st < g_end) request(g_begin + st, st);
   }
-  // (the first group's transfers only, where all kStages batches exist: the loop waits for each later one in turn)
-  if (g_end - g_begin >= kStagesN) {
-    if (wv < kExtraWaves) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStagesN - 1) * kDmaPerWave) : "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStagesN - 1) * (kDmaPerWave - 1)) : "memory");
+  // (the first group's transfers only, where all these batches exist: the loop waits for each later one in turn)
+  if (g_end - g_begin >= kFirstRequests) {
+    if (wv < kExtraWaves) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kFirstRequests - 1) * kDmaPerWave) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kFirstRequests - 1) * (kDmaPerWave - 1)) : "memory");
   } else {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   __builtin_amdgcn_s_barrier();
 
+  if constexpr (S::kRowBlocks) {
+    // Blocks of one 32-row tile x half a group (narrow: x the wave's k-steps): what a lane holds is the activation
+    // operands of the block being multiplied and of the next, the group's converted codes, and the sums of every tile.
+    // Everything that is no multiplication is dealt out over the multiplications, a piece behind each, in this order
+    // (sched_barrier: left alone the compiler gathers it): the next block's operand reads, the conversion of codes half a
+    // group ahead, the finished sums of the tile before into its total (with all of a group's sums folded at its end both
+    // waves of a SIMD do so at once and the matrix core idles), and the transfers of the group kStages ahead.
+    constexpr int kHalves = kSteps == 8 ? 2 : 1, kHS = kSteps / kHalves;   // k-steps of a block
+    constexpr int kBlocks = kHalves * kMT, kLast = kBlocks - 1;
+    constexpr int kLead = 2;                // steps between the request of the next group's codes and their first conversion
+    constexpr int kEarly = kHS - kLead;     // operands of the next group that are converted in the last block
+    constexpr int kParts = kBlocks == 2 || kStagesN < 3 ? 2 : 4;   // a group's transfers in so many pieces, one a block
+    u32x4 fa[2][kHS], fb[kSteps], rec_op = {0u, 0u, 0u, 0u};
+    uint32_t raw[kRawWords];
+    float scale_now, scale_before = 0.0f;
+    v16f acc[kMT];
+#pragma unroll
+    for (int mi = 0; mi < kMT; ++mi)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[mi][r] = 0.0f;
+    auto read_codes = [&](const uint8_t* stage) {
+      if constexpr (kRawBytes == 8) {
+        const u32x2 v = *reinterpret_cast<const u32x2*>(stage + c_base[0]);
+        raw[0] = v.x, raw[1] = v.y;
+      } else {
+#pragma unroll
+        for (int q = 0; q < kRawLoads; ++q) {
+          const u32x4 v = read16(stage, c_base[0] ^ (q << 4));
+          raw[4 * q] = v.x, raw[4 * q + 1] = v.y, raw[4 * q + 2] = v.z, raw[4 * q + 3] = v.w;
+        }
+      }
+    };
+    auto read_scale = [&](const uint8_t* stage) {
+      return *reinterpret_cast<const float*>(stage + kTileBytes + kCodeTileB + kRecTileBytes + (wn * kWaveN + lm) * 4);
+    };
+    auto read_rec = [&](const uint8_t* stage, int mi) {
+      if constexpr (kBiased<T>) rec_op = read16(stage, kTileBytes + kCodeTileB + (mi * 32 + lm) * 16);
+    };
+    auto read_act = [&](const uint8_t* stage, int mi, int j) { return read16(stage, mi * 32 * kRowBytes + (a_base ^ (j << 4))); };
+    auto convert = [&](int j) { fb[j] = operand_words<T, BITS>(raw, j, sixteen); };
+
+    if (kFirstRequests < kStagesN && g_begin + kFirstRequests < g_end)
+      request_part(g_begin + kFirstRequests, kFirstRequests, 0, kParts);
+    read_codes(smem);
+    read_rec(smem, 0);
+    scale_now = read_scale(smem);
+#pragma unroll
+    for (int j = 0; j < kHS; ++j) fa[0][j] = read_act(smem, 0, j);
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) {
+      if (j < kEarly) convert(j);
+      else fb[j] = u32x4{0u, 0u, 0u, 0u};
+    }
+
+    int st = 0, st_fill = kFirstRequests % kStagesN;  // the stage of group g; the one that transfers go to
+    for (int g = g_begin; g < g_end; ++g) {
+      const uint8_t* stage = smem + st * kStageB;
+      const int st_next = st + 1 == kStagesN ? 0 : st + 1;
+      const uint8_t* stage_next = smem + st_next * kStageB;
+      float scale_next = 0.0f;
+#pragma unroll
+      for (int b = 0; b < kBlocks; ++b) {
+        const int h = b / kMT, mi = b % kMT;
+        if (b == kLast) {
+          // The workgroup meets in front of the group's last block, whose operands are in registers: behind the barrier
+          // this stage is free, and the next one is complete (each wave has waited for its own transfers of the next
+          // group; those of later groups may stay in flight).
+          if (kStagesN >= 3 && g + kStagesN - 1 < g_end) {  // (the batches of groups g + 2 .. exist and are younger)
+            if (wv < kExtraWaves) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStagesN - 2) * kDmaPerWave) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStagesN - 2) * (kDmaPerWave - 1)) : "memory");
+          } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          }
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+          st_fill = st;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        {
+          // transfers into the freed stage
+          const int part = b == kLast ? 0 : b + 1, g_fill = b == kLast ? g + kStagesN : g + kStagesN - 1;
+          if (part < kParts && g_fill < g_end && (b == kLast || kFirstRequests < kStagesN || g > g_begin))
+            request_part(g_fill, st_fill, part, kParts);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (h == 0) {
+          // The tile's sums start at -B * xsum[m] (one k-step: the three bf16 pieces of the activation sum against the
+          // constant -B; the upper half of the wave, k' 8..15, multiplies zeros).
+          const v16f zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+          acc[mi] = kBiased<T> && kh == 0 ? mfma<T>(rec_op, bias_operand, zero) : zero;
+        }
+#pragma unroll
+        for (int j = 0; j < kHS; ++j) {
+          acc[mi] = mfma<T>(fa[b & 1][j], fb[h * kHS + j], acc[mi]);
+          if (b == kLast && j == 0) {
+            read_codes(stage_next);   // (past the last group: whatever the stage holds, and unused)
+            scale_next = read_scale(stage_next);
+          }
+          const int next_h = (b + 1) / kMT, next_mi = (b + 1) % kMT;
+          fa[(b + 1) & 1][j] = b == kLast ? read_act(stage_next, 0, j) : read_act(stage, next_mi, next_h * kHS + j);
+          if (j == 0 && b == kLast) read_rec(stage_next, 0);
+          if (j == 0 && b != kLast && next_h == 0) read_rec(stage, next_mi);
+          // codes: the next group's first operands in the last block, the rest of the half in the first; the second half's
+          // while the first is multiplied
+          if (b == kLast && j >= kLead) convert(j - kLead);
+          if (b == 0 && j < kLead) convert(kEarly + j);
+          if (kHalves == 2 && h == 0 && j == kHS - 1) convert(kHS + mi);
+          // finished sums into the totals (two halves: tiles 0 and 1 in blocks 1 and 2 of the second half, tiles 2 and 3 in
+          // those of the next group's first half, away from the conversions; narrow: a tile in the block after its own)
+          const bool early = kHalves == 2 ? h == 1 : mi > 0;
+          const int tile = kHalves == 2 ? (mi == 1 || mi == 2 ? (h == 1 ? mi - 1 : mi + 1) : -1) : (mi + kMT - 1) % kMT;
+          constexpr int kFirstFold = kHS == 4 && kHalves == 2 ? 2 : 1;
+          if (tile >= 0 && j >= kFirstFold) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              if (r * (kHS - kFirstFold) / 16 == j - kFirstFold) {
+                total[tile][0][r] = fmaf(early ? scale_now : scale_before, acc[tile][r], total[tile][0][r]);
+                asm volatile("" : "+v"(total[tile][0][r]));   // (here, and not where the totals are next read)
+              }
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      scale_before = scale_now;
+      scale_now = scale_next;
+      st = st_next;
+    }
+#pragma unroll
+    for (int mi = kHalves == 2 ? kMT / 2 : kMT - 1; mi < kMT; ++mi)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) total[mi][0][r] = fmaf(scale_before, acc[mi][r], total[mi][0][r]);
+  } else {
   // What a lane holds of the group it is about to multiply: the records (operand of the correction
   // step), its raw codes, its columns' scales and the activation operands of k-step 0.
   u32x4 rec[kMT], fa[2][kMT];
@@ -493,6 +626,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   };
   fetch_group_operands(0);
 
+  // (the low tiles of the grouped GEMM, two workgroups a CU: 128 registers a lane do not hold the blocks above)
   // Two waves share a SIMD: while one converts codes or adds its group sums into the totals, the other
   // keeps the matrix core busy. Within a wave the next k-step's activation operands are requested before
   // the current step's multiplications. The workgroup meets once per group, before the last k-step: by
@@ -554,6 +688,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
         for (int r = 0; r < 16; ++r) total[mi][ni][r] = fmaf(scale_now[ni], acc[mi][ni][r], total[mi][ni][r]);
     st = st_next;
   }
+  }
 
   // ---- store: register r of a 32 x 32 tile is row 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32
   if constexpr (EPI == kEpiGateUpSilu) {
@@ -587,22 +722,44 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
     }
     return;
   }
-  // one 32 x 32 tile of totals, whose first row is m_first and whose column (this lane's) is n
-  auto store_tile = [&](const float (&v)[16], int m_first, int n) {
-    if (a.splits == 1) {
+  // Rows that are whole 16-byte packets go out through LDS, a packet a lane and whole rows of the tile at a time
+  // (two bytes a lane as they lie in the registers: 0.7 us more a tile; without any store a launch takes 4.5 us less).
+  const bool whole = GROUPED || a.splits == 1;   // (not a slice of the reduction axis)
+  static_assert(kBM * (kBN * 2 + 16) + (kKH > 1 ? kWaves * (kKH - 1) * 4096 : 0) <= S::template kLdsBytes<BITS>,
+                "a tile of the result in the stages");
+  const bool packets = whole && a.N % 8 == 0;
+  constexpr int kPitch = kBN * 2 + 16;   // 16 bytes of padding: a wave's two halves in different banks
+  uint8_t* const block = smem + (kKH > 1 ? kWaves * (kKH - 1) * 4096 : 0);
+  // one 32 x 32 tile of totals, whose first row and column are rows / columns `row0` / `col0` of the workgroup's tile
+  auto store_tile = [&](const float (&v)[16], int row0, int col0) {
+    const int n = n0 + col0 + lm;
+    if (packets) {
+      uint8_t* to = block + (row0 + 4 * lh) * kPitch + (col0 + lm) * 2;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) *reinterpret_cast<uint16_t*>(to + (8 * (r >> 2) + (r & 3)) * kPitch) = bits16<T>(v[r]);
+    } else if (whole) {
       T* __restrict__ out = static_cast<T*>(a.out);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int m = m_first + 8 * (r >> 2) + 4 * lh + (r & 3);
+        const int m = m0 + row0 + 8 * (r >> 2) + 4 * lh + (r & 3);
         if (m < m_end && n < a.N) out[static_cast<int64_t>(m) * a.N + n] = from_float<T>(v[r]);
       }
     } else {
       float* __restrict__ part = a.partial + static_cast<int64_t>(sp) * a.M * a.N;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int m = m_first + 8 * (r >> 2) + 4 * lh + (r & 3);
+        const int m = m0 + row0 + 8 * (r >> 2) + 4 * lh + (r & 3);
         if (m < m_end && n < a.N) part[static_cast<int64_t>(m) * a.N + n] = v[r];
       }
+    }
+  };
+  auto store_block = [&]() {
+    constexpr int kRowPackets = kBN / 8;
+    T* __restrict__ out = static_cast<T*>(a.out);
+#pragma unroll
+    for (int i = 0; i < kBM * kRowPackets / kThreads; ++i) {
+      const int q = i * kThreads + tid, row = q / kRowPackets, c = q % kRowPackets, m = m0 + row, n = n0 + c * 8;
+      if (m < m_end && n < a.N) store16(out + static_cast<int64_t>(m) * a.N + n, read16(block, row * kPitch + c * 16));
     }
   };
   if constexpr (kKH > 1) {
@@ -633,13 +790,18 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
         sum[r] = from == 0 ? part : sum[r] + part;
       }
     }
-    store_tile(sum, m0 + kh * 32, n0 + wn * kWaveN + lm);
+    store_tile(sum, kh * 32, wn * kWaveN);
   } else {
+    if (packets) __builtin_amdgcn_s_barrier();   // (no wave reads a stage any more)
 #pragma unroll
     for (int ni = 0; ni < kNT; ++ni)
 #pragma unroll
       for (int mi = 0; mi < kMT; ++mi)
-        store_tile(total[mi][ni], m0 + wm * kWaveM + mi * 32, n0 + wn * kWaveN + ni * 32 + lm);
+        store_tile(total[mi][ni], wm * kWaveM + mi * 32, wn * kWaveN + ni * 32);
+  }
+  if (packets) {
+    __syncthreads();
+    store_block();
   }
 }
 
