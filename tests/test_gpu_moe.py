@@ -364,6 +364,15 @@ def test_grouped_gemms_against_real_mode(ext, bits, dtype, tokens, hidden, inter
     assert rel_l2(to_np(got), to_np(want)) <= (1e-2 if dtype == torch.bfloat16 else 1.5e-3)
 
 
+@pytest.mark.parametrize("tokens,hidden,inter,experts,top_k,skew", [
+    (641, 128, 128, 16, 8, False),   # 5128 rows: eight more than the plan's threads keep in registers
+    (512, 128, 128, 80, 10, True),   # 5120, all kept; two experts a lane of the scan; ten rows a token: eight and two
+    (20, 256, 128, 24, 16, False),   # two whole runs of eight rows a token
+])
+def test_a_prompt_past_what_the_plan_and_the_combination_hold_at_once(ext, tokens, hidden, inter, experts, top_k, skew):
+    test_grouped_gemms_against_real_mode(ext, "int4", torch.bfloat16, tokens, hidden, inter, experts, top_k, skew)
+
+
 @pytest.mark.parametrize("tokens", [2, 12])
 def test_an_activation_that_starts_inside_a_packet(ext, tokens):
     """A contiguous view at an odd storage offset, through the two-launch form and the grouped GEMMs: the bits of the
