@@ -52,7 +52,16 @@ struct A16Args {
   void* out;
   int M, N, G, out_group;
   int64_t row_bytes;
+  int scales_at;   // (HELD) where the workgroup's scales lie in LDS
 };
+
+// HELD: the scales come first, all of a workgroup's in one sweep (its weight rows' are one run of memory, whole lines to a
+// load), and wait in LDS. Read group by group, they are a cache line a weight row for four bytes each: of 14336 x 4096 int4,
+// M = 16, 14.4 us, the loads taken out 11.3. Four row tiles, weights rotated through 600 MB, group by group / held, us: int4
+// M = 3 13.0 / 11.5, 16 14.5 / 12.8, 32 17.1 / 16.0, int8 16 18.3 / 18.0. Of one or two row tiles the workgroups are short and
+// the sweep in front costs more than it saves (8192 x 2048 int4, M = 16: 6.4 / 6.8, 4096 x 4096 6.6 / 7.5), and with three
+// activation tiles it takes registers that are not there (48 rows: 19.9 / 21.9).
+__host__ __device__ constexpr int scale_pitch(int G) { return G | 1; }   // (odd: sixteen rows in sixteen banks)
 
 template <typename T> struct Mfma16;
 template <> struct Mfma16<bf16_t> {
@@ -89,7 +98,7 @@ __device__ __forceinline__ typename Mfma16<T>::Vec codes_to_operand(const uint32
   return v;
 }
 
-template <typename T, int BITS, int MT, int NT, bool BIASED>
+template <typename T, int BITS, int MT, int NT, bool BIASED, bool HELD>
 __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A16Args a) {
   using Vec = typename Mfma16<T>::Vec;
   constexpr int kRaw = BITS == 4 ? 4 : 8;  // dwords of codes per lane per group and row tile
@@ -119,6 +128,8 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
     if constexpr (NT == 4) return static_cast<const uint8_t*>(base) + step + at;
     else return at + step;
   };
+  float* const held = reinterpret_cast<float*>(smem + (HELD ? a.scales_at : 0));
+  const int pitch = scale_pitch(G);
   Place wrow[NT], srow[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
@@ -155,7 +166,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
 
   struct Weights {
     uint32_t raw[NT][kRaw];
-    float scale[NT];
+    float scale[HELD ? 1 : NT];
   };
   struct Rows {
     u32x4 xa[MT][4];
@@ -169,7 +180,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
         const u32x4 r = load16(p + 16 * q);
         W.raw[nt][4 * q] = r.x; W.raw[nt][4 * q + 1] = r.y; W.raw[nt][4 * q + 2] = r.z; W.raw[nt][4 * q + 3] = r.w;
       }
-      W.scale[nt] = *reinterpret_cast<const float*>(address(a.ws, srow[nt], static_cast<int64_t>(g) * 4));
+      if constexpr (!HELD) W.scale[nt] = *reinterpret_cast<const float*>(address(a.ws, srow[nt], static_cast<int64_t>(g) * 4));
     }
   };
   auto read_rows = [&](Rows& X) {
@@ -194,14 +205,14 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   // sums x (code + bias); bias * sum_k x comes out per group through four more MFMAs per activation tile against a vector
   // of ones, and the activation's halves are interleaved, both shared by the workgroup's row tiles. It pays where they
   // are: four row tiles, or two with up to two activation tiles. Measured, signed / biased us: 14336 x 4096 int4, four
-  // tiles, M = 16: 14.1 / 12.4, 32: 15.9 / 14.7, 48: 18.1 / 17.8; two, 16: 13.8 / 13.0, 48: 21.2 / 22.1; one,
+  // tiles, M = 16: 14.1 / 12.4, 32: 15.9 / 14.7, 48: 18.1 / 17.8 (before the scales were held); two, 16: 13.8 / 13.0, 48: 21.2 / 22.1; one,
   // 4096 x 14336, 16: 12.4 / 12.8. int8 codes gain nothing: a v_cvt either way.
   using Codes = BiasedCodes<T, BITS>;
   uint32_t magic = Codes::kMagic;
   asm volatile("" : "+v"(magic));   // (in a vector register: see and_or)
   const uint32_t one = __builtin_bit_cast(uint16_t, from_float<T>(1.0f));
   const u32x4 ones = {one | (one << 16), one | (one << 16), one | (one << 16), one | (one << 16)};
-  auto multiply = [&](const Weights& W, const Rows& X) {
+  auto multiply = [&](int g, const Weights& W, const Rows& X) {
     v4f xsum[MT];   // sum_k x of the group: rows 4 blk + r of tile mt, the same in every column
     if constexpr (kBiased) {
 #pragma unroll
@@ -221,7 +232,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
         if constexpr (kBiased) b[s] = __builtin_bit_cast(Vec, Codes::operand(W.raw[nt], s, magic));
         else b[s] = codes_to_operand<T, BITS>(W.raw[nt], s);
       }
-      const float scale = W.scale[nt];
+      const float scale = HELD ? held[(nt * kTileN + j) * pitch + g] : W.scale[HELD ? 0 : nt];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         v4f d = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -239,10 +250,37 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   // The wave's groups wv, wv + wk, ...: this group's rows and codes have arrived (nothing else of the wave is in
   // flight), the rows go from the tile to registers, and with the tile free again the next group's transfer
   // and codes are requested, to arrive under this group's multiplications.
+  // (the scales are asked for in front of everything else, kAhead of a thread's values at once: thread by thread they
+  // are the rows' scales laid end to end)
+  constexpr int kAhead = 8;
+  const int n_scales = kRows * G;
+  float ahead[kAhead] = {};
+  auto scale_of = [&](int e) {
+    const int row = e / G, n = min(n0 + row, a.N - 1);
+    return a.ws + static_cast<int64_t>(a.out_group > 0 ? n / a.out_group : n) * G + (e - row * G);
+  };
+  if constexpr (HELD) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int e = i * blockDim.x + tid;
+      if (e < n_scales) ahead[i] = *scale_of(e);
+    }
+  }
   Weights W0, W1;
   if (wv < G) {
     request_rows(wv);
     load_weights(wv, W0);
+  }
+  if constexpr (HELD) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int e = i * blockDim.x + tid;
+      if (e < n_scales) held[e + (pitch - G) * (e / G)] = ahead[i];
+    }
+    for (int e = kAhead * blockDim.x + tid; e < n_scales; e += blockDim.x) held[e + (pitch - G) * (e / G)] = *scale_of(e);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the scales only: the first group stays in flight)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
   }
   auto step = [&](int g, const Weights& now, Weights& next) {
     Rows X;
@@ -253,7 +291,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
       request_rows(g + wk);
       load_weights(g + wk, next);
     }
-    multiply(now, X);
+    multiply(g, now, X);
   };
   for (int g = wv; g < G; g += 2 * wk) {   // (two groups a round: the register sets swap by name)
     step(g, W0, W1);
@@ -281,14 +319,21 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   }
 }
 
-template <typename T, int BITS, int MT, int NT, bool BIASED>
-int launch_tile(const A16Args& a, int wk, hipStream_t stream) {
+constexpr int kMostScales = 64 * 1024;   // (a workgroup of four row tiles has the CU to itself: 255 groups a row)
+
+template <typename T, int BITS, int MT, int NT, bool BIASED, bool HELD = false>
+int launch_tile(A16Args a, int wk, hipStream_t stream) {
   const int grid = (a.N + NT * kTileN - 1) / (NT * kTileN);
   // the waves' activation tiles, then (the same memory) their partial sums
   const int part = wk * MT * kTileM * NT * kTileN * static_cast<int>(sizeof(float));
   const int tiles = wk * MT * kTileM * kGroup * 2;
-  const int lds = part > tiles ? part : tiles;
-  auto kernel = wq_gemm_a16_kernel<T, BITS, MT, NT, BIASED>;
+  int lds = part > tiles ? part : tiles;
+  if constexpr (HELD) {
+    const int64_t scales = int64_t{NT * kTileN} * scale_pitch(a.G) * static_cast<int>(sizeof(float));
+    if (scales > kMostScales) return launch_tile<T, BITS, MT, NT, BIASED, false>(a, wk, stream);
+    a.scales_at = lds, lds += static_cast<int>(scales);
+  }
+  auto kernel = wq_gemm_a16_kernel<T, BITS, MT, NT, BIASED, HELD>;
   if (lds > 64 * 1024) {
     static bool raised = false;  // per instantiation; worst case two threads both set it
     if (!raised) {
@@ -325,9 +370,10 @@ int launch_typed(const void* x, const void* qw, const float* ws, void* out, int 
   //  32.9 / 27.7, 39.1 / 30.8, int8 39.5 / 35.1; 528, where the third is nearly empty, int4 M = 32 8 % faster, int8 4 %.
   //  Below 192: 8192 x 2048 M = 32 6.7 / 9.1.
   //  Up to 16 rows there is less to share: one round only (288: M = 3 16.7 / 22.1, 16 20.3 / 24.7; 448: 21.9 / 23.2, 26.3 /
-  //  25.9), rows of 32 groups (256 workgroups, M = 3 / 16: K = 2048 7.9 / 8.5, 9.3 / 9.2; K = 4096 14.1 / 13.9, 15.5 / 14.2;
-  //  K = 8192 25.1 / 24.7, 28.1 / 25.7), and for int8 codes nine rows (256: M = 4 17.4 / 18.1, 8 17.8 / 18.1, 12 18.7 / 18.7,
-  //  16 19.7 / 18.9).
+  //  25.9), rows of 32 groups (with the scales held: 256 workgroups, K = 2048, M = 3 / 16: 8.1 / 8.5, 9.3 / 8.9; K = 4096
+  //  14.1 / 12.3 and 15.5 / 13.3; K = 8192, 16: 26.0 / 22.9), and for int8 codes up to eight rows not a whole round of them
+  //  unless rows are long (192: M = 3 / 8 16.5 / 15.1, 16.9 / 15.3; 224: 17.3 / 16.8, 17.3 / 16.6; 256: 17.8 / 18.7, 17.8 /
+  //  19.1; 256 of 64 groups 34.5 / 32.2, 36.2 / 32.2).
   // Four tiles against 64 rows, and int8 codes against 48, are more registers than a wave has (spills: 41 us against 26).
   const bool wide = N >= 2 * kTileN * 256;
   const int quads = (N + 4 * kTileN - 1) / (4 * kTileN);
@@ -344,17 +390,17 @@ int launch_typed(const void* x, const void* qw, const float* ws, void* out, int 
     a.N = N; a.G = G; a.out_group = out_group;
     a.row_bytes = K * BITS / 8;
     const int mt = (a.M + kTileM - 1) / kTileM;
-    const bool few_rows = mt == 1 && quads <= 256 && G >= 32 && (BITS == 4 || a.M > 8);
+    const bool few_rows = mt == 1 && quads <= 256 && G >= 32 && (BITS == 4 || a.M > 8 || quads < 256 || G >= 64);
     const bool more_rows = (mt == 2 || (mt == 3 && BITS == 4)) && (quads <= 256 || quads > 384);
     int rc;
     if (quads >= 192 && offsets32 && (few_rows || more_rows)) {
       constexpr bool kBi = BITS == 4;
       if (mt == 1) {
-        rc = launch_tile<T, BITS, 1, 4, kBi>(a, wk, stream);
+        rc = launch_tile<T, BITS, 1, 4, kBi, true>(a, wk, stream);
       } else if constexpr (BITS == 4) {
-        rc = mt == 2 ? launch_tile<T, BITS, 2, 4, kBi>(a, wk, stream) : launch_tile<T, BITS, 3, 4, kBi>(a, wk, stream);
+        rc = mt == 2 ? launch_tile<T, BITS, 2, 4, kBi, true>(a, wk, stream) : launch_tile<T, BITS, 3, 4, kBi>(a, wk, stream);
       } else {
-        rc = launch_tile<T, BITS, 2, 4, kBi>(a, wk, stream);
+        rc = launch_tile<T, BITS, 2, 4, kBi, true>(a, wk, stream);
       }
     } else if (wide) {
       switch (mt) {

@@ -119,6 +119,35 @@ def test_wide_outputs_take_more_row_tiles_a_workgroup(ext, bits, dtype, m, n, k,
     assert rel_l2(got[:, cols], oracle.gemv_float64(to_np(x), canonical[cols], rows)) <= 2e-3
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,groups,bits,out_group", [
+    (17, 12225, 1, 4, 0),     # one group a row: a scale a row; the last workgroup holds one weight row
+    (32, 12289, 2, 8, 0),
+    (3, 12288, 32, 4, 64),    # one scale row for a workgroup's 64 weight rows
+    (20, 12240, 129, 4, 48),  # more scales than the sweep has ahead of it: 16 for each of 512 threads and some
+    (18, 12300, 255, 4, 0),   # the most that are held
+    (18, 12300, 256, 4, 0),   # one more: read group by group
+])
+def test_scales_of_four_row_tiles(ext, dtype, m, n, groups, bits, out_group):
+    """The scales that a workgroup fetches in front of its loop, at the ends of that sweep, against float64 within the
+    rounding of the output (half a unit: 2^-9 relative in bf16, rel-L2 below 2e-3 as above, 2^-12 in fp16)."""
+    gen = torch.Generator(device="cuda").manual_seed(n + groups)
+    k = groups * GROUP
+    low = torch.randint(-8, 8, (n, groups, GROUP), device="cuda", generator=gen, dtype=torch.int8) if bits == 4 else \
+        torch.randint(-127, 128, (n, groups, GROUP), device="cuda", generator=gen, dtype=torch.int8)
+    q = ((low[..., 0::2] + 8) | ((low[..., 1::2] + 8) << 4)).to(torch.uint8) if bits == 4 else low
+    rows = -(-n // out_group) if out_group else n
+    s = torch.rand(rows, groups, device="cuda", generator=gen) * 0.01 + 1e-3
+    x = torch.randn(m, k, device="cuda", generator=gen).to(dtype)
+    got = ext.wq_gemm_a16(x, q, s, out_group, False).double()
+    want = torch.zeros(m, n, device="cuda", dtype=torch.float64)
+    scale = s.double().repeat_interleave(out_group, 0)[:n] if out_group else s.double()
+    for g in range(groups):
+        part = x[:, g * GROUP:(g + 1) * GROUP].double() @ low[:, g].double().T.contiguous()
+        want += part * scale[:, g]
+    assert float((got - want).norm() / want.norm()) <= (2e-3 if dtype == torch.bfloat16 else 2.5e-4)
+
+
 def test_argument_checks(ext):
     x, q, s, _, _ = make_case(8, 64, 256, 4, torch.bfloat16)
     with pytest.raises(RuntimeError, match="float16 or bfloat16"):
