@@ -70,7 +70,9 @@ template <int BITS> constexpr int kCodeRowBytes = BITS == 4 ? kGroup / 2 : kGrou
 // (still two waves per SIMD, so that one converts codes while the other multiplies), the halves' totals are added
 // through LDS once, at the end, and the smaller stages leave LDS for four of them in flight. WGS: workgroups that
 // share a CU (their stages share its LDS).
-template <int BM, int COLS, int KH, int WGS = 1> struct Shape {
+// CHUNK (the grouped tiles): four groups' scales at a time, see below.
+template <int BM, int COLS, int KH, int WGS = 1, bool CHUNK = false> struct Shape {
+  static constexpr bool kChunk = CHUNK;
   static constexpr int kBM = BM;                 // activation rows per workgroup
   static constexpr int kWaveM = BM;              // ... and per wave
   static constexpr int kWaveN = 32;              // weight rows (output columns) per wave
@@ -83,8 +85,9 @@ template <int BM, int COLS, int KH, int WGS = 1> struct Shape {
   static constexpr int kMT = BM / 32, kNT = kWaveN / 32;
   static constexpr int kRecWaves = BM < 64 ? 1 : BM / 64;   // waves that fetch the activation-sum records (64 rows each)
   static constexpr int kRecTileBytes = kRecWaves * 64 * 16;
-  static constexpr int kScaleTileBytes = kBN * 4;
-  static constexpr int kScaleWaves = kBN / 64;   // ... and, after them, the scales (64 columns each)
+  static constexpr int kScaleTileBytes = CHUNK ? 0 : kBN * 4;         // (of a stage)
+  static constexpr int kChunkBytes = CHUNK ? kBN * 16 : 0;            // (beside the stages)
+  static constexpr int kScaleWaves = CHUNK ? 0 : kBN / 64;   // ... and, after them, the scales (64 columns each)
   template <int BITS> static constexpr int kCodeTileBytes = kBN * kCodeRowBytes<BITS>;
   template <int BITS>
   static constexpr int kStageBytes = kTileBytes + kCodeTileBytes<BITS> + kRecTileBytes + kScaleTileBytes;
@@ -92,8 +95,9 @@ template <int BM, int COLS, int KH, int WGS = 1> struct Shape {
   // before it is multiplied (wide: three for int4, 153 KB, two for int8; narrow: four)
   static constexpr int kWavesPerSimd = (kWaves * WGS + 3) / 4;
   template <int BITS>
-  static constexpr int kStages = (160 * 1024 / WGS / kStageBytes<BITS>) >= 4 ? 4 : (160 * 1024 / WGS / kStageBytes<BITS>);
-  template <int BITS> static constexpr int kLdsBytes = kStages<BITS> * kStageBytes<BITS>;
+  static constexpr int kFitting = (160 * 1024 / WGS - kChunkBytes) / kStageBytes<BITS>;
+  template <int BITS> static constexpr int kStages = kFitting<BITS> >= 4 ? 4 : kFitting<BITS>;
+  template <int BITS> static constexpr int kLdsBytes = kStages<BITS> * kStageBytes<BITS> + kChunkBytes;
   static constexpr bool kRowBlocks = kMT * KH == 4;   // the loop of wide and narrow tiles (the kernel's main loop has two forms)
 };
 using Wide = Shape<128, 8, 1>;
@@ -368,7 +372,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   constexpr int kExtraWaves = kLeftCodes + kRecWaves + kScaleWaves;
   static_assert(kExtraWaves <= kWaves, "at most one transfer instruction per wave beyond the even share");
   const int rec_wave = (wv + kWaves - kLeftCodes) % kWaves % (kRecWaves ? kRecWaves : 1);
-  const int scale_wave = (wv + kWaves - kLeftCodes - kRecWaves) % kWaves % kScaleWaves;
+  const int scale_wave = (wv + kWaves - kLeftCodes - kRecWaves) % kWaves % (kScaleWaves ? kScaleWaves : 1);
   const uint32_t r_off = source_row(rec_wave * 64 + lane) * a.G * 16;
   uint32_t s_off;
   {
@@ -395,6 +399,21 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
       buffer_to_lds<4>(s_base, codes + kCodeTileB + kRecTileBytes + scale_wave * 256, s_off, g * 4);   // 64 columns' scales
     }
   };
+  // CHUNK: a group's scales are a cache line a column for four bytes each, as many lines looked up as the codes' and the
+  // activation's together; four groups' lie side by side. An instruction brings 16 columns' (lane = column, group), two a
+  // wave a chunk, asked for at the first two meetings of a chunk, when every wave has the chunk before in registers, and due
+  // at its last. The waits do not count them: they let that many fewer of the others stay in flight. Group by group /
+  // four at a time, us a call, weights rotated: 64 experts of 2048 x 1024 int4, 300 tokens 106.8 / 102.6, 40 66.1 / 63.4; eight of
+  // 2048 x 4096, 40 tokens 58.3 / 53.9.
+  uint8_t* const chunk_at = smem + kStagesN * kStageB;
+  auto request_scales = [&](int first_group, int part) {
+    const int block = part * kWaves + wv;
+    const int n = weight_row(block * 16 + (lane >> 2)), g = min(first_group + (lane & 3), g_end - 1);
+    const uint32_t at = (static_cast<uint32_t>(a.out_group > 0 ? n / a.out_group : n) * a.G + g) * 4;
+    buffer_to_lds<4>(s_base, chunk_at + block * 256, at, 0);
+  };
+  static_assert(!S::kChunk || kBN == 32 * kWaves, "two instructions a wave bring a chunk");
+  static_assert(!S::kChunk || kStagesN <= 3, "a chunk's last meeting waits for what was asked for two meetings before");
   constexpr int kTransfers = kXInstr + kCodeInstr + 1;
   auto request = [&](int g, int buf) {
 #pragma unroll
@@ -445,6 +464,10 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   // ---- prologue: the first groups on their way, the first one's operands in registers ---------------------
   // (a stage fewer where the loop can ask for it in the first group's blocks: the first group comes sooner)
   constexpr int kFirstRequests = S::kRowBlocks && kStagesN >= 3 ? kStagesN - 1 : kStagesN;
+  if constexpr (S::kChunk) {
+    request_scales(g_begin, 0);
+    request_scales(g_begin, 1);
+  }
 #pragma unroll
   for (int st = 0; st < kFirstRequests; ++st) {
     if (g_begin + st < g_end) request(g_begin + st, st);
@@ -597,7 +620,9 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   u32x4 rec[kMT], fa[2][kMT];
   uint32_t raw[kNT][kRawWords];
   float scale[kNT];
-  auto fetch_group_operands = [&](int st) {
+  static_assert(S::kChunk && kNT == 1, "this loop is the grouped tiles'");
+  u32x4 scales = {0u, 0u, 0u, 0u};   // of this lane's column: the groups still to come of the chunk
+  auto fetch_group_operands = [&](int st, int g) {
     const uint8_t* stage = smem + st * kStageB;
     if constexpr (kBiased<T>) {
 #pragma unroll
@@ -617,14 +642,13 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
         }
       }
     }
-#pragma unroll
-    for (int ni = 0; ni < kNT; ++ni)
-      scale[ni] = *reinterpret_cast<const float*>(stage + kTileBytes + kCodeTileB + kRecTileBytes +
-                                                  (wn * kWaveN + ni * 32 + lm) * 4);
+    if ((g & 3) == 0) scales = read16(chunk_at, (wn * kWaveN + lm) * 16);
+    scale[0] = __builtin_bit_cast(float, scales.x);
+    scales = u32x4{scales.y, scales.z, scales.w, 0u};
 #pragma unroll
     for (int mi = 0; mi < kMT; ++mi) fa[0][mi] = read16(stage, mi * 32 * kRowBytes + a_base);
   };
-  fetch_group_operands(0);
+  fetch_group_operands(0, g_begin);
 
   // (the low tiles of the grouped GEMM, two workgroups a CU: 128 registers a lane do not hold the blocks above)
   // Two waves share a SIMD: while one converts codes or adds its group sums into the totals, the other
@@ -673,7 +697,8 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         if (g + kStagesN < g_end) request(g + kStagesN, st);
-        if (g + 1 < g_end) fetch_group_operands(st_next);  // (fa[0]: the last step multiplies out of fa[1])
+        if ((g & 3) < 2 && (g | 3) + 1 < g_end) request_scales((g | 3) + 1, g & 3);
+        if (g + 1 < g_end) fetch_group_operands(st_next, g + 1);  // (fa[0]: the last step multiplies out of fa[1])
       }
 #pragma unroll
       for (int mi = 0; mi < kMT; ++mi)

@@ -17,7 +17,7 @@
 //
 // Bound: the experts' codes (64 x 2048 x 1024 int4: 201 MB) for up to about 40 rows an expert, the tiled GEMM's rate
 // beyond. Measured, 64 experts, 8 a token, 2048 x 1024, bf16, us a pass, per-expert loop -> here: 300 tokens int4
-// 6970 -> 102; by kernel trace (with the profiler's overhead) at 12 / 60 / 300 / 600 tokens int4 the gate|up GEMM takes
+// 6970 -> 100; by kernel trace (with the profiler's overhead) at 12 / 60 / 300 / 600 tokens int4 the gate|up GEMM takes
 // 33.5 / 39 / 67 / 90 us (4.0 TB/s of codes at 12 tokens), down 18 / 21 / 36 / 48, the plan 4-5, the combination 4.5-5.5.
 #include "wq_gemm_a16_tile.h"
 
@@ -30,10 +30,10 @@ constexpr int kMaxTopK = 256;
 // The shapes: 256 columns (128 gate + 128 up rows of the weight make a whole group of the next reduction axis), rows by
 // what an expert gets. Two workgroups a CU where their stages fit (int4), so that one's first transfers and store run
 // under the other's multiplications: a tile is only 8 to 16 groups long here.
-using Rows32 = Shape<32, 8, 1, 2>;
-using Rows64 = Shape<64, 8, 1, 2>;
-using Rows32Whole = Shape<32, 8, 1, 1>;
-using Rows64Whole = Shape<64, 8, 1, 1>;
+using Rows32 = Shape<32, 8, 1, 2, true>;
+using Rows64 = Shape<64, 8, 1, 2, true>;
+using Rows32Whole = Shape<32, 8, 1, 1, true>;
+using Rows64Whole = Shape<64, 8, 1, 1, true>;
 
 struct PlanArgs {
   const int64_t* expert_of_row;   // [n_rows] (token-major: row i is of token i / top_k)

@@ -373,6 +373,15 @@ def test_a_prompt_past_what_the_plan_and_the_combination_hold_at_once(ext, token
     test_grouped_gemms_against_real_mode(ext, "int4", torch.bfloat16, tokens, hidden, inter, experts, top_k, skew)
 
 
+@pytest.mark.parametrize("bits,dtype", [("int4", torch.bfloat16), ("int8", torch.bfloat16), ("int4", torch.float16)])
+@pytest.mark.parametrize("tokens,hidden,inter,experts,top_k,skew", [
+    (20, 640, 768, 4, 2, False),     # five and six groups: the second run of four groups' scales holds one and two
+    (90, 896, 1152, 2, 2, False),    # seven and nine, 64-row tiles
+])
+def test_scales_of_a_last_run_of_groups(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew):
+    test_grouped_gemms_against_real_mode(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew)
+
+
 @pytest.mark.parametrize("tokens", [2, 12])
 def test_an_activation_that_starts_inside_a_packet(ext, tokens):
     """A contiguous view at an odd storage offset, through the two-launch form and the grouped GEMMs: the bits of the
