@@ -271,13 +271,12 @@ __device__ __forceinline__ void buffer_to_lds(const BufferBase& base, void* lds,
 // group (the products are exact in fp32 either way). Operand element order: the eight codes of a 32-bit word of
 // int4 (two of int8) as (0, 4, 1, 5, 2, 6, 3, 7): the other operand's 16-byte chunks must be in the same
 // order (interleave_halves), which a sum over k does not mind.
-__device__ __forceinline__ uint32_t and_or(uint32_t value, uint32_t mask_scalar, uint32_t bits) {
-  // (value & mask) | bits in one instruction; the compiler leaves it as two. One operand of a VOP3 may come
-  // from a scalar register on this chip, so the mask is scalar and the bits sit in a vector register.
-  uint32_t d;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(d) : "v"(value), "s"(mask_scalar), "v"(bits));
-  return d;
-}
+// (value & mask) | bits. One v_and_or_b32 where the bits sit in a vector register (the callers pin them there: of a VOP3's
+// operands one may come from a scalar register on this chip, and that is the mask). An expression, never inline asm: between a
+// vector instruction's write and a multiplication that reads it two wait states have to pass, the compiler keeps them for the
+// writes it sees, and the result goes straight into a multiplication (as asm one wait state was left at 143 places, and the
+// instructions are the same).
+__device__ __forceinline__ uint32_t and_or(uint32_t value, uint32_t mask, uint32_t bits) { return (value & mask) | bits; }
 // (x0 x1)(x2 x3)(x4 x5)(x6 x7) -> (x0 x4)(x1 x5)(x2 x6)(x3 x7), 16-bit elements
 __device__ __forceinline__ u32x4 interleave_halves(const u32x4 v) {
   u32x4 o;
