@@ -86,7 +86,8 @@ template <int BM, int COLS, int KH, int WGS = 1, bool CHUNK = false> struct Shap
   static constexpr int kRecWaves = BM < 64 ? 1 : BM / 64;   // waves that fetch the activation-sum records (64 rows each)
   static constexpr int kRecTileBytes = kRecWaves * 64 * 16;
   static constexpr int kScaleTileBytes = CHUNK ? 0 : kBN * 4;         // (of a stage)
-  static constexpr int kChunkBytes = CHUNK ? kBN * 16 : 0;            // (beside the stages)
+  static constexpr int kChunks = CHUNK ? (BM >= 64 ? 2 : 1) : 0;      // (beside the stages)
+  static constexpr int kChunkBytes = kChunks * kBN * 16;
   static constexpr int kScaleWaves = CHUNK ? 0 : kBN / 64;   // ... and, after them, the scales (64 columns each)
   template <int BITS> static constexpr int kCodeTileBytes = kBN * kCodeRowBytes<BITS>;
   template <int BITS>
@@ -401,16 +402,28 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   };
   // CHUNK: a group's scales are a cache line a column for four bytes each, as many lines looked up as the codes' and the
   // activation's together; four groups' lie side by side. An instruction brings 16 columns' (lane = column, group), two a
-  // wave a chunk, asked for at the first two meetings of a chunk, when every wave has the chunk before in registers, and due
-  // at its last. The waits do not count them: they let that many fewer of the others stay in flight. Group by group /
-  // four at a time, us a call, weights rotated: 64 experts of 2048 x 1024 int4, 300 tokens 106.8 / 102.6, 40 66.1 / 63.4; eight of
-  // 2048 x 4096, 40 tokens 58.3 / 53.9.
-  uint8_t* const chunk_at = smem + kStagesN * kStageB;
+  // wave a chunk, asked for at the first two meetings of a chunk and due at its last. The waits do not count them: they let
+  // that many fewer of the others stay in flight. The 32-row tiles have LDS for one chunk and hold a column's four scales in
+  // registers, in every wave's by the time the next chunk is asked for; the 64-row tiles have no registers for them (held,
+  // bfloat16 x int4 spilled seven to eight, and each reload in its group loop waited for transfers just asked for) and read a
+  // group's from one of two chunks. Group by group / four at a time, us a call, weights rotated: 64 experts of 2048 x 1024
+  // int4, 300 tokens 107 / 101, 40 71 / 67; eight of 2048 x 4096, 40 tokens 61.5 / 57.0; 64 rows a tile (and held): 64 experts,
+  // 600 tokens 144 / 139 (154), eight, 200 tokens 81.2 / 76.1 (90.1). (An expert's weight row has a scale row of its own:
+  // out_group is not looked at.)
+  uint8_t* const chunks = smem + kStagesN * kStageB;
+  auto chunk_of = [&](int g) { return chunks + (S::kChunks == 2 ? (g >> 2 & 1) * (kBN * 16) : 0); };
+  // (the first instruction's columns lie 16 a wave in the tile's first half, the second's one half on: a scalar distance, so
+  // that one lane offset serves both. Columns of the second half past the weight's end, of which nothing is stored, take the
+  // first half's.)
+  uint32_t c_off = 0, c_half = 0;
+  if constexpr (S::kChunk) {
+    const uint32_t s_row_bytes = static_cast<uint32_t>(a.G) * 4;
+    c_off = static_cast<uint32_t>(n0 + wv * 16 + (lane >> 2)) * s_row_bytes;
+    c_half = static_cast<uint32_t>(EPI == kEpiGateUpSilu ? a.N / 2 : (n0 + kBN / 2 < a.N ? kBN / 2 : 0)) * s_row_bytes;
+  }
   auto request_scales = [&](int first_group, int part) {
-    const int block = part * kWaves + wv;
-    const int n = weight_row(block * 16 + (lane >> 2)), g = min(first_group + (lane & 3), g_end - 1);
-    const uint32_t at = (static_cast<uint32_t>(a.out_group > 0 ? n / a.out_group : n) * a.G + g) * 4;
-    buffer_to_lds<4>(s_base, chunk_at + block * 256, at, 0);
+    const int g = min(lane & 3, g_end - 1 - first_group);
+    buffer_to_lds<4>(s_base, chunk_of(first_group) + (part * kWaves + wv) * 256, c_off + g * 4, first_group * 4 + part * c_half);
   };
   static_assert(!S::kChunk || kBN == 32 * kWaves, "two instructions a wave bring a chunk");
   static_assert(!S::kChunk || kStagesN <= 3, "a chunk's last meeting waits for what was asked for two meetings before");
@@ -619,7 +632,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   // step), its raw codes, its columns' scales and the activation operands of k-step 0.
   u32x4 rec[kMT], fa[2][kMT];
   uint32_t raw[kNT][kRawWords];
-  float scale[kNT];
+  float scale = 0.0f;
   static_assert(S::kChunk && kNT == 1, "this loop is the grouped tiles'");
   u32x4 scales = {0u, 0u, 0u, 0u};   // of this lane's column: the groups still to come of the chunk
   auto fetch_group_operands = [&](int st, int g) {
@@ -642,9 +655,11 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
         }
       }
     }
-    if ((g & 3) == 0) scales = read16(chunk_at, (wn * kWaveN + lm) * 16);
-    scale[0] = __builtin_bit_cast(float, scales.x);
-    scales = u32x4{scales.y, scales.z, scales.w, 0u};
+    if constexpr (S::kChunks == 1) {
+      if ((g & 3) == 0) scales = read16(chunks, (wn * kWaveN + lm) * 16);
+      scale = __builtin_bit_cast(float, scales.x);
+      scales = u32x4{scales.y, scales.z, scales.w, 0u};
+    }
 #pragma unroll
     for (int mi = 0; mi < kMT; ++mi) fa[0][mi] = read16(stage, mi * 32 * kRowBytes + a_base);
   };
@@ -663,9 +678,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   for (int g = g_begin; g < g_end; ++g) {
     const uint8_t* stage = smem + st * kStageB;
     const int st_next = st + 1 == kStagesN ? 0 : st + 1;
-    float scale_now[kNT];
-#pragma unroll
-    for (int ni = 0; ni < kNT; ++ni) scale_now[ni] = scale[ni];
+    float scale_now = scale;
 
     // The group's sums start at -B * xsum[m] (one k-step: the three bf16 pieces of the activation sum
     // against the constant -B; the upper half of the wave, k' 8..15, multiplies zeros), then take the
@@ -686,6 +699,8 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
       if (j < kSteps - 1) {
 #pragma unroll
         for (int mi = 0; mi < kMT; ++mi) fa[(j + 1) & 1][mi] = read16(stage, mi * 32 * kRowBytes + (a_base ^ ((j + 1) << 4)));
+        if (S::kChunks == 2 && j == kSteps - 2)
+          scale_now = *reinterpret_cast<const float*>(chunk_of(g) + (wn * kWaveN + lm) * 16 + (g & 3) * 4);
       } else {
         // own transfers of the next group have landed (the youngest kStages - 2 batches may stay in flight)
         if (kStagesN >= 3 && g + kStagesN - 1 < g_end) {  // (the batches of groups g + 2 .. exist and are younger)
@@ -710,7 +725,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
 #pragma unroll
       for (int ni = 0; ni < kNT; ++ni)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) total[mi][ni][r] = fmaf(scale_now[ni], acc[mi][ni][r], total[mi][ni][r]);
+        for (int r = 0; r < 16; ++r) total[mi][ni][r] = fmaf(scale_now, acc[mi][ni][r], total[mi][ni][r]);
     st = st_next;
   }
   }

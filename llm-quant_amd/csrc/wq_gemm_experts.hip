@@ -243,11 +243,12 @@ int run(const void* x, const int64_t* index, const void* weights, const void* q1
         const float* s2, void* out, uint8_t* ws, int n_tokens, int top_k, int E, int H, int I, hipStream_t stream) {
   const Layout l = layout_for(n_tokens, top_k, E, H, I);
   const int rows = n_tokens * top_k;
-  // 64-row tiles from 40 rows an expert on. Measured, us a pass, 32-row tiles / 64-row: 64 experts of 2048 x 1024 int4 at
-  // 10 rows an expert 58.9 / 68.5, 25: 74.4 / 90.2, 37.5: 89.8 / 92.6, 45: 93.0 / 96.8, 52: 108.5 / 98.5, 75: 128.8 / 122.3;
-  // int8 25: 120.0 / 142.6, 37.5: 147.1 / 146.4, 41: 150.1 / 144.5, 52: 174.1 / 151.2. Eight experts of 2048 x 4096 int4 at
-  // 30: 61.4 / 74.7, 50: 74.6 / 77.8, 75: 77.3 / 79.7, 125: 120.0 / 98.9 (between 40 and 48 rows int4 would keep the lower
-  // tile, int8 would not).
+  // 64-row tiles from 40 rows an expert on: with scales read group by group the two heights met there. Measured since the
+  // scales come in chunks, us a call, 32-row tiles / 64-row, bf16: 64 experts of 2048 x 1024 int4 at 10 rows an expert 76 / 91,
+  // 25: 86 / 85, 37.5: 104 / 86, 45: 106 / 88, 52: 118 / 111, 75: 147 / 144; int8 10: 100 / 117, 25: 119 / 115, 37.5: 146 / 119,
+  // 52: 153 / 127. Eight experts of 2048 x 4096 int4 at 30: 68 / 74, 40: 71 / 75, 50: 71 / 76, 75: 86 / 89, 125: 121 / 110; int8
+  // 30: 91 / 85, 50: 97 / 89, 125: 190 / 145. (Many narrow experts would take the higher tile from 25 rows on, few wide int4 ones
+  // from some 100 on.)
   const int tile_rows = rows > 40 * E ? 64 : 32;
   const PlanArgs p{index, rows, E, top_k, tile_rows, reinterpret_cast<int4*>(ws + l.tiles),
                    reinterpret_cast<int*>(ws + l.n_tiles), reinterpret_cast<int*>(ws + l.row_source),

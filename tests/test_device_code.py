@@ -73,3 +73,12 @@ def test_operands_are_written_two_wait_states_ahead(source):
     text = assembly(source)
     assert text.count("v_mfma") > 100
     assert operands_too_soon(text) == []
+
+
+@needs_hipcc
+@pytest.mark.parametrize("source", ["wq_gemm_experts.hip", "wq_gemm_a16_tile.hip"])
+def test_the_tiles_do_not_spill(source):
+    """A spilled register's reload waits for every transfer into LDS that was asked for before it."""
+    kernels = re.findall(r"\.name:\s+(_Z\S+).*?\.vgpr_spill_count:\s+(\d+)", assembly(source), re.S)
+    assert len(kernels) > 10
+    assert [name for name, spilled in kernels if int(spilled)] == []

@@ -377,6 +377,7 @@ def test_a_prompt_past_what_the_plan_and_the_combination_hold_at_once(ext, token
 @pytest.mark.parametrize("tokens,hidden,inter,experts,top_k,skew", [
     (20, 640, 768, 4, 2, False),     # five and six groups: the second run of four groups' scales holds one and two
     (90, 896, 1152, 2, 2, False),    # seven and nine, 64-row tiles
+    (90, 1536, 1920, 2, 2, False),   # twelve and fifteen: these tiles' two buffers, each used twice
 ])
 def test_scales_of_a_last_run_of_groups(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew):
     test_grouped_gemms_against_real_mode(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew)
