@@ -14,7 +14,7 @@
 // branch rounds code*scale to the activation dtype first; its own test holds the two branches
 // together only within a tolerance, tests/test_kernel_linear.py:62-78.)
 //
-// A workgroup owns 16 or 32 weight rows; its waves split the groups of the reduction axis between them
+// A workgroup owns 16, 32 or 64 weight rows; its waves split the groups of the reduction axis between them
 // (wave w takes groups w, w + waves, ...) and meet in LDS at the end. Per group a wave reads
 //   weights   16 rows x 64 B (4-bit) or 128 B (8-bit), 16 or 32 bytes per lane, straight from HBM
 //             in operand layout: lane = (row j = lane % 16, block = lane / 16) holds k = 32 block ..
@@ -58,8 +58,8 @@ struct A16Args {
 // HELD: the scales come first, all of a workgroup's in one sweep (its weight rows' are one run of memory, whole lines to a
 // load), and wait in LDS. Read group by group, they are a cache line a weight row for four bytes each: of 14336 x 4096 int4,
 // M = 16, 14.4 us, the loads taken out 11.3. Four row tiles, weights rotated through 600 MB, group by group / held, us: int4
-// M = 3 13.0 / 11.5, 16 14.5 / 12.8, 32 17.1 / 16.0, int8 16 18.3 / 18.0. Of one or two row tiles the workgroups are short and
-// the sweep in front costs more than it saves (8192 x 2048 int4, M = 16: 6.4 / 6.8, 4096 x 4096 6.6 / 7.5), and with three
+// M = 3 13.0 / 11.5, 16 14.5 / 12.8, 32 17.1 / 16.0, int8 16 18.3 / 18.0. Short rows do not give the sweep in front back: form_of.
+// Of one or two row tiles the workgroups are short (8192 x 2048 int4, M = 16: 6.4 / 6.8, 4096 x 4096 6.6 / 7.5), and with three
 // activation tiles it takes registers that are not there (48 rows: 19.9 / 21.9).
 __host__ __device__ constexpr int scale_pitch(int G) { return G | 1; }   // (odd: sixteen rows in sixteen banks)
 
@@ -320,6 +320,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
 }
 
 constexpr int kMostScales = 64 * 1024;   // (a workgroup of four row tiles has the CU to itself: 255 groups a row)
+constexpr int64_t held_bytes(int row_tiles, int G) { return int64_t{row_tiles * kTileN} * scale_pitch(G) * 4; }
 
 template <typename T, int BITS, int MT, int NT, bool BIASED, bool HELD = false>
 int launch_tile(A16Args a, int wk, hipStream_t stream) {
@@ -328,11 +329,7 @@ int launch_tile(A16Args a, int wk, hipStream_t stream) {
   const int part = wk * MT * kTileM * NT * kTileN * static_cast<int>(sizeof(float));
   const int tiles = wk * MT * kTileM * kGroup * 2;
   int lds = part > tiles ? part : tiles;
-  if constexpr (HELD) {
-    const int64_t scales = int64_t{NT * kTileN} * scale_pitch(a.G) * static_cast<int>(sizeof(float));
-    if (scales > kMostScales) return launch_tile<T, BITS, MT, NT, BIASED, false>(a, wk, stream);
-    a.scales_at = lds, lds += static_cast<int>(scales);
-  }
+  if constexpr (HELD) a.scales_at = lds, lds += static_cast<int>(held_bytes(NT, a.G));   // (form_of: they fit)
   auto kernel = wq_gemm_a16_kernel<T, BITS, MT, NT, BIASED, HELD>;
   if (lds > 64 * 1024) {
     static bool raised = false;  // per instantiation; worst case two threads both set it
@@ -350,6 +347,53 @@ int launch_tile(A16Args a, int wk, hipStream_t stream) {
   return llmq_host::check_launch("wq_gemm_a16_kernel");
 }
 
+// Which form a slab of activation rows takes: row tiles of a workgroup, and whether its scales are held.
+struct Form {
+  int row_tiles;
+  bool held;
+};
+// Row tiles of a workgroup share the activation rows a wave loads: those come from L2 once per workgroup, and 16
+// weight rows a workgroup make that traffic four times the codes' at M = 16. Two tiles as long as a workgroup per CU
+// and more is left (14336 x 4096 int4 bf16, one / two tiles, us: M = 16 14.6 / 13.0, 32 19.6 / 17.8, 48 29.4 / 21.2; 4096
+// x 4096, M = 64: 10.2 / 13.7).
+// Four tiles (one workgroup a CU) by how full their last round of 256 workgroups is. Measured, two / four tiles, us,
+// weights rotated through 600 MB, bf16; fp16 is within 3 % of it, also where its 33 to 48 rows against int4 spill two
+// registers (14336 x 4096, M = 48: 24.7 / 19.9):
+//  17 rows and more, K = 4096: 192 workgroups int4 M = 17 / 32 / 48: 17.3 / 14.8, 20.7 / 16.4, 24.3 / 19.1, int8 32: 24.3 /
+//  19.8; 256: 18.0 / 15.2, 21.3 / 17.0, 25.2 / 19.8, int8 26.4 / 21.2; but 260 to 384, a second round at most half full:
+//  288 24.9 / 26.8, 29.8 / 30.0, 34.9 / 35.1, int8 17 29.8 / 33.3; 384 26.9 / 27.9, 30.8 / 30.5, int8 17 33.9 / 34.4; 416
+//  32.9 / 27.7, 39.1 / 30.8, int8 39.5 / 35.1; 528, where the third is nearly empty, int4 M = 32 8 % faster, int8 4 %.
+//  Below 192: 8192 x 2048 M = 32 6.7 / 9.1.
+//  Up to 16 rows there is less to share: one round only (288: M = 3 16.7 / 22.1, 16 20.3 / 24.7; 448: 21.9 / 23.2, 26.3 /
+//  25.9), rows of 32 groups (with the scales held: 256 workgroups, K = 2048, M = 3 / 16: 8.1 / 8.5, 9.3 / 8.9; K = 4096
+//  14.1 / 12.3 and 15.5 / 13.3; K = 8192, 16: 26.0 / 22.9), and for int8 codes up to eight rows, the fuller the round the longer
+//  the rows that it takes (in graphs; 192: 32 groups M = 3 / 8 15.0 / 14.2, 15.8 / 14.5; 224: 16.1 / 16.1, 16.7 / 16.1; 240: 32
+//  groups 16.2 / 17.1, 17.0 / 17.2, 48 groups 23.6 / 22.2, 25.4 / 22.3; 256: 64 groups M = 3 / 5 30.3 / 32.0, 30.8 / 32.0, 96
+//  groups 45.3 / 46.3, 46.9 / 45.7, 255 groups M = 3 147.7 / 139.8).
+// Four tiles against 64 rows, and int8 codes against 48, are more registers than a wave has (spills: 41 us against 26).
+constexpr Form form_of(int bits, int rows, int N, int G) {
+  const int quads = (N + 4 * kTileN - 1) / (4 * kTileN), mt = (rows + kTileM - 1) / kTileM;
+  const bool int4 = bits == 4;
+  const int64_t K = static_cast<int64_t>(G) * kGroup, limit = int64_t{1} << 32;   // the four-tile form's offsets from its scalar bases
+  const bool offsets32 = N * (K * bits / 8) < limit && static_cast<int64_t>(N) * G * 4 < limit && kSlabRows * K * 2 < limit;
+  const bool few_codes = int4 || rows > 8 || quads <= 224 || G >= (quads < 256 ? 40 : rows > 4 ? 96 : 192);
+  const bool few_rows = mt == 1 && quads <= 256 && G >= 32 && few_codes;
+  const bool more_rows = (mt == 2 || (mt == 3 && int4)) && (quads <= 256 || quads > 384);
+  if (quads >= 192 && offsets32 && (few_rows || more_rows)) {
+    // The scales of rows that are long enough to pay for the sweep are held, and of somewhat shorter ones where several rounds of
+    // workgroups overlap it and the waves have equal shares. Group by group / held, us, in graphs, M = 17 / 32: int4, 256
+    // workgroups, K = 512 7.8 / 8.4, 8.2 / 8.7; 2048 9.9 / 10.3, 11.3 / 11.5; 2560 11.2 / 11.3, 12.3 / 12.4; 3584 1 and 3 % the
+    // faster held, 4096 4 and 7 %; 2004 workgroups, K = 2048 68.1 / 67.1, 71.9 / 71.1; int8, 256 workgroups, K = 512 7.5 / 8.5, 7.8
+    // / 8.8; 2048 even; 2560 14.9 / 15.6, 15.8 / 16.4 (fp16 13.6 / 15.5, 14.7 / 16.3); 4096 19.2 / 20.1 (21.5 / 21.0 by where the
+    // weights lie), 21.2 / 21.3, M = 9 and 16 1 to 3 % the slower held; 192 and 448 of them 3 to 4 % the faster; 2004, K = 2048
+    // 79.3 / 76.4, 85.4 / 81.1.
+    const bool long_rows = int4 ? mt == 1 || G >= 20 : G >= (quads > 240 && quads <= 256 ? 40 : 32);
+    const bool pays = long_rows || (G >= 16 && G % kMaxWaves == 0 && quads >= (int4 ? 385 : 1024));
+    return {4, mt <= 2 && pays && held_bytes(4, G) <= kMostScales};
+  }
+  return {N >= 2 * kTileN * 256 ? 2 : 1, false};
+}
+
 template <typename T, int BITS>
 int launch_typed(const void* x, const void* qw, const float* ws, void* out, int M, int N, int G, int out_group,
                  hipStream_t stream) {
@@ -357,28 +401,6 @@ int launch_typed(const void* x, const void* qw, const float* ws, void* out, int 
   int wk = G < kMaxWaves ? G : kMaxWaves;
   // rows of few groups: two groups per wave at least
   if (G >= 4 && wk * 2 > G) wk = G / 2;
-  // Row tiles of a workgroup share the activation rows a wave loads: those come from L2 once per workgroup, and 16
-  // weight rows a workgroup make that traffic four times the codes' at M = 16. Two tiles as long as a workgroup per CU
-  // and more is left (14336 x 4096 int4 bf16, one / two tiles, us: M = 16 14.6 / 13.0, 32 19.6 / 17.8, 48 29.4 / 21.2; 4096
-  // x 4096, M = 64: 10.2 / 13.7).
-  // Four tiles (one workgroup a CU) by how full their last round of 256 workgroups is. Measured, two / four tiles, us,
-  // weights rotated through 600 MB, bf16; fp16 is within 3 % of it, also where its 33 to 48 rows against int4 spill two
-  // registers (14336 x 4096, M = 48: 24.7 / 19.9):
-  //  17 rows and more, K = 4096: 192 workgroups int4 M = 17 / 32 / 48: 17.3 / 14.8, 20.7 / 16.4, 24.3 / 19.1, int8 32: 24.3 /
-  //  19.8; 256: 18.0 / 15.2, 21.3 / 17.0, 25.2 / 19.8, int8 26.4 / 21.2; but 260 to 384, a second round at most half full:
-  //  288 24.9 / 26.8, 29.8 / 30.0, 34.9 / 35.1, int8 17 29.8 / 33.3; 384 26.9 / 27.9, 30.8 / 30.5, int8 17 33.9 / 34.4; 416
-  //  32.9 / 27.7, 39.1 / 30.8, int8 39.5 / 35.1; 528, where the third is nearly empty, int4 M = 32 8 % faster, int8 4 %.
-  //  Below 192: 8192 x 2048 M = 32 6.7 / 9.1.
-  //  Up to 16 rows there is less to share: one round only (288: M = 3 16.7 / 22.1, 16 20.3 / 24.7; 448: 21.9 / 23.2, 26.3 /
-  //  25.9), rows of 32 groups (with the scales held: 256 workgroups, K = 2048, M = 3 / 16: 8.1 / 8.5, 9.3 / 8.9; K = 4096
-  //  14.1 / 12.3 and 15.5 / 13.3; K = 8192, 16: 26.0 / 22.9), and for int8 codes up to eight rows not a whole round of them
-  //  unless rows are long (192: M = 3 / 8 16.5 / 15.1, 16.9 / 15.3; 224: 17.3 / 16.8, 17.3 / 16.6; 256: 17.8 / 18.7, 17.8 /
-  //  19.1; 256 of 64 groups 34.5 / 32.2, 36.2 / 32.2).
-  // Four tiles against 64 rows, and int8 codes against 48, are more registers than a wave has (spills: 41 us against 26).
-  const bool wide = N >= 2 * kTileN * 256;
-  const int quads = (N + 4 * kTileN - 1) / (4 * kTileN);
-  const int64_t limit = int64_t{1} << 32;   // the four-tile form's offsets from its scalar bases
-  const bool offsets32 = N * (K * BITS / 8) < limit && static_cast<int64_t>(N) * G * 4 < limit && kSlabRows * K * 2 < limit;
   // (Sixteen waves for few row tiles of long rows, down_proj, measured no faster than eight.)
   for (int m0 = 0; m0 < M; m0 += kSlabRows) {
     A16Args a{};
@@ -390,19 +412,18 @@ int launch_typed(const void* x, const void* qw, const float* ws, void* out, int 
     a.N = N; a.G = G; a.out_group = out_group;
     a.row_bytes = K * BITS / 8;
     const int mt = (a.M + kTileM - 1) / kTileM;
-    const bool few_rows = mt == 1 && quads <= 256 && G >= 32 && (BITS == 4 || a.M > 8 || quads < 256 || G >= 64);
-    const bool more_rows = (mt == 2 || (mt == 3 && BITS == 4)) && (quads <= 256 || quads > 384);
-    int rc;
-    if (quads >= 192 && offsets32 && (few_rows || more_rows)) {
+    const Form form = form_of(BITS, a.M, N, G);
+    int rc = 0;
+    if (form.row_tiles == 4) {
       constexpr bool kBi = BITS == 4;
       if (mt == 1) {
-        rc = launch_tile<T, BITS, 1, 4, kBi, true>(a, wk, stream);
+        rc = form.held ? launch_tile<T, BITS, 1, 4, kBi, true>(a, wk, stream) : launch_tile<T, BITS, 1, 4, kBi>(a, wk, stream);
+      } else if (mt == 2) {
+        rc = form.held ? launch_tile<T, BITS, 2, 4, kBi, true>(a, wk, stream) : launch_tile<T, BITS, 2, 4, kBi>(a, wk, stream);
       } else if constexpr (BITS == 4) {
-        rc = mt == 2 ? launch_tile<T, BITS, 2, 4, kBi, true>(a, wk, stream) : launch_tile<T, BITS, 3, 4, kBi>(a, wk, stream);
-      } else {
-        rc = launch_tile<T, BITS, 2, 4, kBi, true>(a, wk, stream);
+        rc = launch_tile<T, BITS, 3, 4, kBi>(a, wk, stream);
       }
-    } else if (wide) {
+    } else if (form.row_tiles == 2) {
       switch (mt) {
         case 1: rc = launch_tile<T, BITS, 1, 2, BITS == 4>(a, wk, stream); break;
         case 2: rc = launch_tile<T, BITS, 2, 2, BITS == 4>(a, wk, stream); break;

@@ -16,11 +16,15 @@ needs_hipcc = pytest.mark.skipif(not pathlib.Path(HIPCC).exists(), reason="needs
 
 
 @functools.lru_cache(maxsize=None)
+def flags() -> list[str]:
+    return subprocess.run(["make", "-s", "-C", str(PACKAGE), "--no-print-directory", "--eval=flags: ; @echo $(HIPFLAGS)", "flags"],
+                          check=True, capture_output=True, text=True).stdout.split()
+
+
+@functools.lru_cache(maxsize=None)
 def assembly(source: str) -> str:
     """gfx950 assembly of a source, with the Makefile's flags."""
-    flags = subprocess.run(["make", "-s", "-C", str(PACKAGE), "--no-print-directory", "--eval=flags: ; @echo $(HIPFLAGS)", "flags"],
-                           check=True, capture_output=True, text=True).stdout.split()
-    return subprocess.run([HIPCC, *flags, "--cuda-device-only", "-S", str(CSRC / source), "-o", "-"],
+    return subprocess.run([HIPCC, *flags(), "--cuda-device-only", "-S", str(CSRC / source), "-o", "-"],
                           check=True, capture_output=True, text=True).stdout
 
 
@@ -82,3 +86,25 @@ def test_the_tiles_do_not_spill(source):
     kernels = re.findall(r"\.name:\s+(_Z\S+).*?\.vgpr_spill_count:\s+(\d+)", assembly(source), re.S)
     assert len(kernels) > 10
     assert [name for name, spilled in kernels if int(spilled)] == []
+
+
+@needs_hipcc
+def test_forms_of_the_gemm_for_a_few_dozen_rows(tmp_path):
+    """Where one side of a line was measured slower, the other side's form runs: the kernel's own rule, at compile time."""
+    lines = [  # bits, rows, outputs, groups, row tiles, scales held
+        (4, 17, 16384, 1, 4, False), (4, 32, 128256, 8, 4, False), (4, 32, 16384, 16, 4, False), (4, 17, 24577, 16, 4, True),
+        (4, 32, 32000, 18, 4, False), (4, 17, 16384, 19, 4, False), (4, 17, 16384, 20, 4, True), (4, 33, 16384, 64, 4, False),
+        (8, 32, 28672, 4, 4, False), (8, 32, 28672, 16, 4, False), (8, 17, 128256, 16, 4, True), (8, 17, 128256, 20, 4, False),
+        (8, 17, 12288, 31, 4, False), (8, 17, 15360, 32, 4, True), (8, 17, 16384, 39, 4, False), (8, 17, 16384, 40, 4, True),
+        (8, 3, 14336, 32, 4, True), (8, 3, 14337, 32, 2, False), (8, 8, 15360, 39, 2, False), (8, 8, 15360, 40, 4, True),
+        (8, 4, 16384, 191, 2, False), (8, 4, 16384, 192, 4, True), (8, 5, 16384, 64, 2, False), (8, 5, 16384, 96, 4, True),
+        (8, 9, 16384, 32, 4, False), (8, 9, 14336, 32, 4, True), (8, 9, 16384, 31, 2, False), (4, 3, 16384, 32, 4, True), (4, 3, 16448, 32, 2, False),
+        (8, 3, 12288, 255, 4, True), (8, 3, 12288, 256, 4, False), (4, 32, 12288, 256, 4, False),   # what the LDS holds
+        (8, 33, 16384, 32, 2, False), (4, 64, 16384, 32, 2, False), (4, 16, 12224, 32, 2, False), (4, 16, 8176, 32, 1, False),
+    ]
+    checks = [f"static_assert(form_of({b}, {m}, {n}, {g}).row_tiles == {t} && form_of({b}, {m}, {n}, {g}).held == {str(h).lower()});"
+              for b, m, n, g, t, h in lines]
+    source = tmp_path / "forms.hip"
+    source.write_text(f'#include "{CSRC}/wq_gemm_a16.hip"\n' + "\n".join(checks) + "\n")
+    ran = subprocess.run([HIPCC, *flags(), "--cuda-host-only", "-fsyntax-only", str(source)], capture_output=True, text=True)
+    assert ran.returncode == 0, "\n".join(line for line in ran.stderr.splitlines() if "error" in line or "static_assert" in line)

@@ -109,7 +109,7 @@ def test_llama_shapes_on_sampled_entries(ext, n, k, m, split):
     (5, 12225, 4096, 0),                                              # four row tiles, one activation tile; ragged in rows
     (17, 12289, 640, 0), (32, 12352, 512, 64), (33, 12289, 384, 0), (48, 12300, 256, 0),   # two and three activation tiles
     (64, 12289, 256, 0), (16, 16448, 256, 0), (33, 8201, 384, 0),     # two row tiles: past 48 rows, short rows, fewer rows
-    (9, 12225, 4096, 0), (17, 16385, 256, 0), (48, 24577, 256, 0),    # int8's first row count; a full round + 1, 1.5 + 1
+    (9, 12225, 4096, 0), (17, 16385, 256, 0), (48, 24577, 256, 0),    # four row tiles for int8 too; a full round + 1, 1.5 + 1
 ])
 def test_wide_outputs_take_more_row_tiles_a_workgroup(ext, bits, dtype, m, n, k, out_group):
     x, q, s, canonical, scales = make_case(m, n, k, bits, dtype, out_group=out_group, seed=5)
@@ -121,12 +121,16 @@ def test_wide_outputs_take_more_row_tiles_a_workgroup(ext, bits, dtype, m, n, k,
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,groups,bits,out_group", [
-    (17, 12225, 1, 4, 0),     # one group a row: a scale a row; the last workgroup holds one weight row
+    (17, 12225, 1, 4, 0),     # one group a row, read group by group; the last workgroup holds one weight row
     (32, 12289, 2, 8, 0),
-    (3, 12288, 32, 4, 64),    # one scale row for a workgroup's 64 weight rows
+    (3, 12288, 32, 4, 64),    # held: one scale row for a workgroup's 64 weight rows
     (20, 12240, 129, 4, 48),  # more scales than the sweep has ahead of it: 16 for each of 512 threads and some
     (18, 12300, 255, 4, 0),   # the most that are held
     (18, 12300, 256, 4, 0),   # one more: read group by group
+    (17, 24577, 16, 4, 0), (17, 65473, 16, 8, 0),                           # the fewest that are held, over 16 rows: many rounds,
+    (17, 12289, 20, 4, 64), (17, 12225, 32, 8, 0),                          # one round
+    (32, 12225, 19, 4, 0), (17, 12225, 31, 8, 0), (17, 65409, 16, 8, 0),    # one group or workgroup fewer: group by group
+    (5, 16384, 96, 8, 0), (3, 15361, 40, 8, 0),                             # int8 codes, up to eight rows, a (nearly) full round
 ])
 def test_scales_of_four_row_tiles(ext, dtype, m, n, groups, bits, out_group):
     """The scales that a workgroup fetches in front of its loop, at the ends of that sweep, against float64 within the
