@@ -25,7 +25,7 @@
 //             instruction and the address unit, not memory, set the pace), 16-byte slots XOR-swizzled by row,
 //             and come out as operands: the 32 k of row (lane % 16) that the lane's codes belong to
 // and issues 4 MFMAs per activation tile. The next group's transfer and codes are requested once this group's
-// operands are in registers. Rows past M or N are clamped for the loads and dropped at the store, so the load
+// operands are in registers (how far they run under its multiplications: at the loop). Rows past M or N are clamped for the loads and dropped at the store, so the load
 // sequence is the same for every lane.
 #include <type_traits>
 
@@ -249,7 +249,10 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
 
   // The wave's groups wv, wv + wk, ...: this group's rows and codes have arrived (nothing else of the wave is in
   // flight), the rows go from the tile to registers, and with the tile free again the next group's transfer
-  // and codes are requested, to arrive under this group's multiplications.
+  // and codes are requested. The compiler does not count a wait written as assembly: it takes the codes to be on their way
+  // still and waits for everything outstanding once more, somewhere behind a request. Of 14336 x 4096 int4, four row tiles,
+  // scales held, a round's first step waits between the transfer and the codes it requests (the transfer is waited for, the
+  // codes run under the multiplications), its second three multiplications behind both.
   // (the scales are asked for in front of everything else, kAhead of a thread's values at once: thread by thread they
   // are the rows' scales laid end to end)
   constexpr int kAhead = 8;
@@ -278,7 +281,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
       if (e < n_scales) held[e + (pitch - G) * (e / G)] = ahead[i];
     }
     for (int e = kAhead * blockDim.x + tid; e < n_scales; e += blockDim.x) held[e + (pitch - G) * (e / G)] = *scale_of(e);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the scales only: the first group stays in flight)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the first group has arrived too: the sweep's branches end in vmcnt(0))
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   }

@@ -22,7 +22,9 @@
 // What bounds it: power, then issue. 192 workgroups, 16 to 64 groups: 1.74 us a group with the loop a k-step at a time
 // and FLAT transfers (the same on all-zero operands: 1.64), 1.55 with the loop below (zeros: 1.39); with the transfers
 // taken out 1.24, with the operand reads taken out 1.41, the multiplications alone 1.07. 512 x 14336 x 4096 int4, fp16:
-// 66.9 -> 61.8 us, bf16 with its preparation 75.6 -> 69.9; 2048 x 14336 x 4096 273 -> 255.
+// 66.9 -> 61.8 us, bf16 with its preparation 75.6 -> 69.9; 2048 x 14336 x 4096, which callers of a Linear send to the
+// library's product, 273 -> 255. Launches of few narrow tiles on short rows pay 0.1 to 0.2 us for the result's way through
+// LDS (512 x 2048 int4, 72 to 512 rows: 12.0 -> 12.1, 15.3 -> 15.4).
 //
 // Codes become bf16 without a conversion instruction: a nibble n = code + 8 placed in the mantissa of
 // 16.0 (bits 0x4180 | n << 3) IS the bf16 value 16 + n, two nibbles per AND-OR (int8: code + 128 through
@@ -732,9 +734,9 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
 
   // ---- store: register r of a 32 x 32 tile is row 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32
   if constexpr (EPI == kEpiGateUpSilu) {
-    // Waves 0..3 hold the block's gate columns, 4..7 its up columns: both go to LDS as bf16 (no wave reads a
-    // stage any more: the loop's last barrier came after every wave's last operand read), then a lane takes a
-    // 16-byte chunk of a row at a time, 16 lanes a row, as act_prep_kernel does with a tensor in memory.
+    // Waves 0..3 hold the block's gate columns, 4..7 its up columns: both go to LDS as bf16 (the loop's last barrier came
+    // after every wave's last operand read of a group that is multiplied; what the loop of row blocks reads behind it, of the
+    // group past the last, is not used), then a lane takes a 16-byte chunk of a row at a time, 16 lanes a row, as act_prep_kernel does with a tensor in memory.
     __builtin_amdgcn_s_barrier();
     uint8_t* block = smem + (wn >> 2) * (kBM * kEpiRowBytes);
     const int col = (wn & 3) * 32 + lm;
@@ -804,9 +806,10 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
   };
   if constexpr (kKH > 1) {
     // The kKH waves of a column block hold the totals of their parts of every group. Wave kh keeps row tile kh and
-    // hands the others over through LDS (4 KB a tile, [register][lane]; the stages are free: the loop's last
-    // barrier came after every wave's last operand read and its last transfer), then adds the parts of its tile in
-    // the order of the waves, its own in its place.
+    // hands the others over through LDS (4 KB a tile, [register][lane]; the stages are free: the loop's last barrier came
+    // after every wave's last transfer and its last operand read of a group that is multiplied. A slower wave may still read
+    // behind it, of the group past the last, while this one writes: those values are not used), then adds the parts of its
+    // tile in the order of the waves, its own in its place.
     float* exchange = reinterpret_cast<float*>(smem);
     auto slot = [&](int from, int tile) { return ((from * S::kColWaves + wn) * (kKH - 1) + (tile - (tile > from))) * 1024; };
     float own[16];
@@ -832,7 +835,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
     }
     store_tile(sum, kh * 32, wn * kWaveN);
   } else {
-    if (packets) __builtin_amdgcn_s_barrier();   // (no wave reads a stage any more)
+    if (packets) __builtin_amdgcn_s_barrier();   // (no wave reads operands of a group that is multiplied any more)
 #pragma unroll
     for (int ni = 0; ni < kNT; ++ni)
 #pragma unroll

@@ -17,8 +17,9 @@
 //
 // Bound: the experts' codes (64 x 2048 x 1024 int4: 201 MB) for up to about 40 rows an expert, the tiled GEMM's rate
 // beyond. Measured, 64 experts, 8 a token, 2048 x 1024, bf16, us a pass, per-expert loop -> here: 300 tokens int4
-// 6970 -> 100; by kernel trace (with the profiler's overhead) at 12 / 60 / 300 / 600 tokens int4 the gate|up GEMM takes
-// 33.5 / 39 / 67 / 90 us (4.0 TB/s of codes at 12 tokens), down 18 / 21 / 36 / 48, the plan 4-5, the combination 4.5-5.5.
+// 6970 -> 100; by kernel trace (with the profiler's overhead, medians of 24) at 12 / 60 / 300 / 600 tokens int4 the gate|up
+// GEMM takes 33 / 36 / 59 / 97 us (at 12 tokens 51 experts have rows: 3.2 TB/s of their codes; at 600 79 to 108: the clock),
+// down 18.6 / 20 / 33 / 51, the plan 4.8 / 4.9 / 5.2 / 9.2, the combination 4.7 / 4.7 / 5.6 / 8.9.
 #include "wq_gemm_a16_tile.h"
 
 namespace {

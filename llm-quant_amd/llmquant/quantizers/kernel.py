@@ -59,8 +59,11 @@ def _tile_plan_cost(rows: int, out_features: int, groups: int, narrow: bool, int
 
 
 def tiled_gemm_cost(rows: int, out_features: int, groups: int, bits: int = 8, prepared: bool = False) -> float:
-    """Estimated microseconds of llmq_wq_gemm_a16_tile (within a tenth of the measured launches, 128-2048 rows on
-    weights of 2048-28672 rows): rounds of 256 workgroups, each a fixed part plus a time per group, the partial sums'
+    """Estimated microseconds of llmq_wq_gemm_a16_tile, from the figures that the kernel's own plan has (fitted to an earlier
+    main loop: 0.85 to 1.41 times the measured launch over 442 problems, 1.10 in the middle; of the 364 of them up to 1024
+    rows the branch that is then chosen is more than 5 % behind the fastest in 38, more than 10 % in 17, most of all 1024 x 512
+    x 2048, 19.0 us against 14.5 for dequantize + matmul, and 72 x 8192 x 2048 int4, 18.8 against 14.4 for the fused GEMM for a
+    few dozen rows): rounds of 256 workgroups, each a fixed part plus a time per group, the partial sums'
     way through memory where the reduction axis is cut, and 3.5 us for the activation's preparation unless the rows
     arrive prepared (llmq_add_rmsnorm_prepared, the gate|up epilogue). (float16 rows are read as they lie; the estimate
     does not tell the types apart, which leaves them that much in hand.)"""
