@@ -26,7 +26,8 @@
 // (d, half) four keys of its column per read. Among the 16 lanes of a group, that instruction gives lane l, as
 // its element j, element l % 4 of what lane 4 j + l / 4 points at: with lane 4 j + i pointing at key j,
 // columns 4 i .. 4 i + 3, lane l gets column l of keys 0..3. The next block's K and V are requested as soon as
-// this block's K has been consumed, into the tile's other buffer.
+// this block's K has been consumed, into the tile's other buffer. (They run under the softmax and no further: the compiler
+// does not tell the two buffers apart and waits for all of them in front of this block's reads of V.)
 #include "llmq_device.h"
 
 namespace {
