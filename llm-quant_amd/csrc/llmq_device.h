@@ -292,9 +292,11 @@ template <> struct BiasedCodes<bf16_t, 4> {
   static constexpr uint32_t kMagic = 0x41804180u;   // keep it in a vector register: asm volatile("" : "+v"(magic))
   // raw: the lane's codes of a group; step: which eight of them
   static __device__ __forceinline__ u32x4 operand(const uint32_t* raw, int step, uint32_t magic) {
+    return u32x4{word(raw, step, 0, magic), word(raw, step, 1, magic), word(raw, step, 2, magic), word(raw, step, 3, magic)};
+  }
+  static __device__ __forceinline__ uint32_t word(const uint32_t* raw, int step, int i, uint32_t magic) {
     const uint32_t w = raw[step];
-    return u32x4{and_or(w << 3, 0x00780078u, magic), and_or(w >> 1, 0x00780078u, magic),
-                 and_or(w >> 5, 0x00780078u, magic), and_or(w >> 9, 0x00780078u, magic)};
+    return and_or(i == 0 ? w << 3 : w >> (4 * i - 3), 0x00780078u, magic);
   }
 };
 template <> struct BiasedCodes<f16_t, 4> {
@@ -309,16 +311,16 @@ template <> struct BiasedCodes<f16_t, 4> {
 template <> struct BiasedCodes<bf16_t, 8> {
   static constexpr float kBias = 128.0f;
   static constexpr uint32_t kMagic = 0u;
-  static __device__ __forceinline__ u32x4 operand(const uint32_t* raw, int step, uint32_t) {
-    const uint32_t w0 = raw[2 * step] ^ 0x80808080u, w1 = raw[2 * step + 1] ^ 0x80808080u;   // codes 0..3, 4..7
-    uint32_t out[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float lo = static_cast<float>((w0 >> (8 * i)) & 0xffu), hi = static_cast<float>((w1 >> (8 * i)) & 0xffu);
-      // integers below 256: the upper half of the float is the bf16 value, exactly
-      out[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
-    }
-    return u32x4{out[0], out[1], out[2], out[3]};
+  static __device__ __forceinline__ u32x4 operand(const uint32_t* raw, int step, uint32_t magic) {
+    const uint32_t flipped[2] = {raw[2 * step] ^ 0x80808080u, raw[2 * step + 1] ^ 0x80808080u};   // codes 0..3, 4..7
+    return u32x4{word(flipped, 0, 0, magic), word(flipped, 0, 1, magic), word(flipped, 0, 2, magic), word(flipped, 0, 3, magic)};
+  }
+  // (of codes whose sign bits are flipped already)
+  static __device__ __forceinline__ uint32_t word(const uint32_t* flipped, int step, int i, uint32_t) {
+    const uint32_t w0 = flipped[2 * step], w1 = flipped[2 * step + 1];
+    const float lo = static_cast<float>((w0 >> (8 * i)) & 0xffu), hi = static_cast<float>((w1 >> (8 * i)) & 0xffu);
+    // integers below 256: the upper half of the float is the bf16 value, exactly
+    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
   }
 };
 template <> struct BiasedCodes<f16_t, 8> {

@@ -19,12 +19,16 @@
 // the activation tile, the raw codes of the 256 weight rows, the activation-sum records and the group's scales.
 // The workgroup meets once per group, when its last operands are in registers, and the next group's are read from LDS
 // behind that barrier.
-// What bounds it: power, then issue. 192 workgroups, 16 to 64 groups: 1.74 us a group with the loop a k-step at a time
-// and FLAT transfers (the same on all-zero operands: 1.64), 1.55 with the loop below (zeros: 1.39); with the transfers
-// taken out 1.24, with the operand reads taken out 1.41, the multiplications alone 1.07. 512 x 14336 x 4096 int4, fp16:
-// 66.9 -> 61.8 us, bf16 with its preparation 75.6 -> 69.9; 2048 x 14336 x 4096, which callers of a Linear send to the
-// library's product, 273 -> 255. Launches of few narrow tiles on short rows pay 0.1 to 0.2 us for the result's way through
-// LDS (512 x 2048 int4, 72 to 512 rows: 12.0 -> 12.1, 15.3 -> 15.4).
+// What bounds it: issue, and power. Per group a wave issues 36 multiplications of 32 cycles (float16 32), 128 to 160 vector
+// instructions of conversion and folding, 39 LDS reads, and the two waves of a SIMD share one matrix core: 2300 cycles if it never
+// waited, 3100 measured (float16 3020), 224 workgroups. What counts is how evenly the rest lies between the multiplications: a
+// step that carries more than about five vector instructions is longer than its multiplication, whichever wave it is (a
+// multiplication holds the issue slot for 12 cycles, a vector instruction 4). Folds and conversions eight to sixteen a step and
+// none elsewhere: 3316 (3190). Without folds 2460, without conversions 3100 (float16 2730), without transfers 2990 at a clock
+// 10 to 17 % higher: on random codes the chip holds 1.6 to 1.9 GHz under this loop, on zeros 2.2, so that a cycle saved is half
+// a cycle's time. Launches of 512 x 14336 x 4096 int4 us, the lumped loop / this: bf16 with its preparation 77.7 / 75.4, fp16
+// 68.8 / 66.6; 333 x 4096 x 14336 fp16 63.6 / 61.0; 36 problems of both widths 2 % in the middle, 0 to 6. Launches of few narrow
+// tiles on short rows pay 0.1 to 0.2 us for the result's way through LDS.
 //
 // Codes become bf16 without a conversion instruction: a nibble n = code + 8 placed in the mantissa of
 // 16.0 (bits 0x4180 | n << 3) IS the bf16 value 16 + n, two nibbles per AND-OR (int8: code + 128 through
@@ -256,29 +260,75 @@ template <int BITS> __device__ __forceinline__ int code_slot(int row, int c) {
 // one sixteen times as high (1024 + 16 n), and the multiply-add that takes the bias out brings it down, all exact.
 template <typename T, int BITS>
 constexpr uint32_t kOperandMagic = std::is_same<T, f16_t>::value && BITS == 4 ? 0x64006400u : BiasedCodes<T, BITS>::kMagic;
+// word `i` of step `step` (int8: of codes whose sign bits are flipped already)
+template <typename T, int BITS>
+__device__ __forceinline__ uint32_t operand_word(const uint32_t* raw, int step, int i, uint32_t magic) {
+  if constexpr (kBiased<T>) return BiasedCodes<T, BITS>::word(raw, step, i, magic);
+  if constexpr (BITS == 4) {
+    const uint32_t both = __builtin_amdgcn_perm(0u, raw[step], 0x0c000c00u | (i << 16) | i);
+    const h2 v = __builtin_bit_cast(h2, and_or(both, 0x00f0000fu, magic));
+    const h2 down = {static_cast<_Float16>(1.0f), static_cast<_Float16>(0.0625f)};
+    const h2 bias = {static_cast<_Float16>(-1032.0f), static_cast<_Float16>(-72.0f)};
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, down, bias));
+  } else {
+    // bytes 2 i and 2 i + 1 into the two halves, in the mantissa of 256.0
+    const uint32_t w = raw[2 * step + i / 2];
+    const uint32_t pick = i % 2 ? 0x0c030c02u : 0x0c010c00u;
+    const h2 v = __builtin_bit_cast(h2, (__builtin_amdgcn_perm(0u, w, pick) << 2) | magic);
+    const h2 bias = {static_cast<_Float16>(-384.0f), static_cast<_Float16>(-384.0f)};
+    return __builtin_bit_cast(uint32_t, v + bias);
+  }
+}
 template <typename T, int BITS>
 __device__ __forceinline__ u32x4 operand_words(const uint32_t* raw, int step, uint32_t magic) {
   if constexpr (kBiased<T>) return BiasedCodes<T, BITS>::operand(raw, step, magic);
-  uint32_t out[4];
+  uint32_t own[BITS / 4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if constexpr (BITS == 4) {
-      const uint32_t both = __builtin_amdgcn_perm(0u, raw[step], 0x0c000c00u | (i << 16) | i);
-      const h2 v = __builtin_bit_cast(h2, and_or(both, 0x00f0000fu, magic));
-      const h2 down = {static_cast<_Float16>(1.0f), static_cast<_Float16>(0.0625f)};
-      const h2 bias = {static_cast<_Float16>(-1032.0f), static_cast<_Float16>(-72.0f)};
-      out[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, down, bias));
-    } else {
-      // bytes 2 i and 2 i + 1 into the two halves, in the mantissa of 256.0
-      const uint32_t w = raw[2 * step + i / 2] ^ 0x80808080u;
-      const uint32_t pick = i % 2 ? 0x0c030c02u : 0x0c010c00u;
-      const h2 v = __builtin_bit_cast(h2, (__builtin_amdgcn_perm(0u, w, pick) << 2) | magic);
-      const h2 bias = {static_cast<_Float16>(-384.0f), static_cast<_Float16>(-384.0f)};
-      out[i] = __builtin_bit_cast(uint32_t, v + bias);
-    }
-  }
-  return u32x4{out[0], out[1], out[2], out[3]};
+  for (int i = 0; i < BITS / 4; ++i) own[i] = raw[step * (BITS / 4) + i] ^ (BITS == 8 ? 0x80808080u : 0u);
+  return u32x4{operand_word<T, BITS>(own, 0, 0, magic), operand_word<T, BITS>(own, 0, 1, magic),
+               operand_word<T, BITS>(own, 0, 2, magic), operand_word<T, BITS>(own, 0, 3, magic)};
 }
+
+// What the loop of row blocks puts behind which of a group's multiplications (steps): conversions of codes, word by
+// word (four a k-step), and folds of finished sums, register by register (register r of row tile t: 16 t + r). As even
+// as the deadlines allow: the next group's codes are there from the last block's third step on and its first operand is due two
+// steps later; a row tile's sums are finished after its second block and start anew with the next group's first.
+struct Run {
+  int first, count;
+};
+template <int HALVES> struct Dealt;
+// Wide: steps 4 b + j of blocks b = 0..3 (row tiles against the first four k-steps) and 4..7 (against the second four).
+// Row tile t is finished after step 19 + 4 t and starts anew at step 4 t.
+template <> struct Dealt<2> {
+  static constexpr int kEarlyWords = 6;   // of the next group, in the last two steps
+  static constexpr int kMostWords = 4, kMostFolds = 4;
+  static constexpr Run words(int s) {
+    if (s >= 30) return {3 * (s - 30), 3};
+    if (s < 3) return {6 + 3 * s, s < 2 ? 3 : 4};
+    return s >= 10 && s < 18 ? Run{16 + 2 * (s - 10), 2} : Run{0, 0};
+  }
+  static constexpr Run folds(int s) {
+    if (s >= 21 && s < 30) return {4 * (s - 21), 4};
+    return s >= 3 && s < 10 ? Run{36 + 4 * (s - 3), 4} : Run{0, 0};
+  }
+  static constexpr int kLateFolds = 36;   // from this one on: in the next group's steps
+};
+// Narrow: steps 4 b + j of two row tiles, finished after steps 3 and 7. (A k-step's codes at a time: spread over five steps as
+// above, 100 x 14336 x 4096 int4 is 1 to 2 % slower.)
+template <> struct Dealt<1> {
+  static constexpr int kEarlyWords = 8;
+  static constexpr int kMostWords = 4, kMostFolds = 6;
+  static constexpr Run words(int s) {
+    if (s >= 6) return {4 * (s - 6), 4};
+    return s < 2 ? Run{8 + 4 * s, 4} : Run{0, 0};
+  }
+  static constexpr Run folds(int s) {
+    const int k = s % 4;
+    if (s == 0 || k == 0) return {0, 0};
+    return {(s > 4 ? 0 : 16) + (k == 1 ? 0 : 1 + 5 * (k - 1)), k == 1 ? 6 : 5};
+  }
+  static constexpr int kLateFolds = 16;
+};
 
 template <typename T> __device__ __forceinline__ v16f mfma(const u32x4& a, const u32x4& b, const v16f& c) {
   if constexpr (std::is_same<T, bf16_t>::value)
@@ -500,15 +550,14 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
     // Blocks of one 32-row tile x half a group (narrow: x the wave's k-steps): what a lane holds is the activation
     // operands of the block being multiplied and of the next, the group's converted codes, and the sums of every tile.
     // Everything that is no multiplication is dealt out over the multiplications, a piece behind each, in this order
-    // (sched_barrier: left alone the compiler gathers it): the next block's operand reads, the conversion of codes half a
-    // group ahead, the finished sums of the tile before into its total (with all of a group's sums folded at its end both
-    // waves of a SIMD do so at once and the matrix core idles), and the transfers of the group kStages ahead.
+    // (sched_barrier: left alone the compiler gathers it): the next block's operand reads, words of codes converted ahead of
+    // their use, finished sums folded into the totals (Dealt), and the transfers of the group kStages ahead.
     constexpr int kHalves = kSteps == 8 ? 2 : 1, kHS = kSteps / kHalves;   // k-steps of a block
     constexpr int kBlocks = kHalves * kMT, kLast = kBlocks - 1;
-    constexpr int kLead = 2;                // steps between the request of the next group's codes and their first conversion
-    constexpr int kEarly = kHS - kLead;     // operands of the next group that are converted in the last block
+    using Deal = Dealt<kHalves>;
     constexpr int kParts = kBlocks == 2 || kStagesN < 3 ? 2 : 4;   // a group's transfers in so many pieces, one a block
-    u32x4 fa[2][kHS], fb[kSteps], rec_op = {0u, 0u, 0u, 0u};
+    u32x4 fa[2][kHS], rec_op = {0u, 0u, 0u, 0u};
+    uint32_t fb[kSteps * 4];   // (words of the converted codes, four a step)
     uint32_t raw[kRawWords];
     float scale_now, scale_before = 0.0f;
     v16f acc[kMT];
@@ -535,7 +584,11 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
       if constexpr (kBiased<T>) rec_op = read16(stage, kTileBytes + kCodeTileB + (mi * 32 + lm) * 16);
     };
     auto read_act = [&](const uint8_t* stage, int mi, int j) { return read16(stage, mi * 32 * kRowBytes + (a_base ^ (j << 4))); };
-    auto convert = [&](int j) { fb[j] = operand_words<T, BITS>(raw, j, sixteen); };
+    auto convert = [&](int w) {   // (the words of a k-step in order)
+      if (BITS == 8 && w % 4 == 0) raw[w / 2] ^= 0x80808080u, raw[w / 2 + 1] ^= 0x80808080u;
+      fb[w] = operand_word<T, BITS>(raw, w / 4, w % 4, sixteen);
+    };
+    auto operand = [&](int step) { return u32x4{fb[4 * step], fb[4 * step + 1], fb[4 * step + 2], fb[4 * step + 3]}; };
 
     if (kFirstRequests < kStagesN && g_begin + kFirstRequests < g_end)
       request_part(g_begin + kFirstRequests, kFirstRequests, 0, kParts);
@@ -545,9 +598,9 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
 #pragma unroll
     for (int j = 0; j < kHS; ++j) fa[0][j] = read_act(smem, 0, j);
 #pragma unroll
-    for (int j = 0; j < kSteps; ++j) {
-      if (j < kEarly) convert(j);
-      else fb[j] = u32x4{0u, 0u, 0u, 0u};
+    for (int w = 0; w < 4 * kSteps; ++w) {
+      if (w < Deal::kEarlyWords) convert(w);
+      else fb[w] = 0u;
     }
 
     int st = 0, st_fill = kFirstRequests % kStagesN;  // the stage of group g; the one that transfers go to
@@ -590,7 +643,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
         }
 #pragma unroll
         for (int j = 0; j < kHS; ++j) {
-          acc[mi] = mfma<T>(fa[b & 1][j], fb[h * kHS + j], acc[mi]);
+          acc[mi] = mfma<T>(fa[b & 1][j], operand(h * kHS + j), acc[mi]);
           if (b == kLast && j == 0) {
             read_codes(stage_next);   // (past the last group: whatever the stage holds, and unused)
             scale_next = read_scale(stage_next);
@@ -599,23 +652,18 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
           fa[(b + 1) & 1][j] = b == kLast ? read_act(stage_next, 0, j) : read_act(stage, next_mi, next_h * kHS + j);
           if (j == 0 && b == kLast) read_rec(stage_next, 0);
           if (j == 0 && b != kLast && next_h == 0) read_rec(stage, next_mi);
-          // codes: the next group's first operands in the last block, the rest of the half in the first; the second half's
-          // while the first is multiplied
-          if (b == kLast && j >= kLead) convert(j - kLead);
-          if (b == 0 && j < kLead) convert(kEarly + j);
-          if (kHalves == 2 && h == 0 && j == kHS - 1) convert(kHS + mi);
-          // finished sums into the totals (two halves: tiles 0 and 1 in blocks 1 and 2 of the second half, tiles 2 and 3 in
-          // those of the next group's first half, away from the conversions; narrow: a tile in the block after its own)
-          const bool early = kHalves == 2 ? h == 1 : mi > 0;
-          const int tile = kHalves == 2 ? (mi == 1 || mi == 2 ? (h == 1 ? mi - 1 : mi + 1) : -1) : (mi + kMT - 1) % kMT;
-          constexpr int kFirstFold = kHS == 4 && kHalves == 2 ? 2 : 1;
-          if (tile >= 0 && j >= kFirstFold) {
+          const Run words = Deal::words(b * kHS + j), folds = Deal::folds(b * kHS + j);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              if (r * (kHS - kFirstFold) / 16 == j - kFirstFold) {
-                total[tile][0][r] = fmaf(early ? scale_now : scale_before, acc[tile][r], total[tile][0][r]);
-                asm volatile("" : "+v"(total[tile][0][r]));   // (here, and not where the totals are next read)
-              }
+          for (int k = 0; k < Deal::kMostWords; ++k) {
+            const int w = words.first + k;
+            if (k < words.count) convert(w);
+          }
+#pragma unroll
+          for (int k = 0; k < Deal::kMostFolds; ++k) {
+            const int f = folds.first + k, tile = f / 16, r = f % 16;
+            if (k < folds.count) {
+              total[tile][0][r] = fmaf(f >= Deal::kLateFolds ? scale_before : scale_now, acc[tile][r], total[tile][0][r]);
+              asm volatile("" : "+v"(total[tile][0][r]));   // (here, and not where the totals are next read)
             }
           }
           __builtin_amdgcn_sched_barrier(0);
@@ -626,9 +674,8 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
       st = st_next;
     }
 #pragma unroll
-    for (int mi = kHalves == 2 ? kMT / 2 : kMT - 1; mi < kMT; ++mi)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) total[mi][0][r] = fmaf(scale_before, acc[mi][r], total[mi][0][r]);
+    for (int f = Deal::kLateFolds; f < 16 * kMT; ++f)
+      total[f / 16][0][f % 16] = fmaf(scale_before, acc[f / 16][f % 16], total[f / 16][0][f % 16]);
   } else {
   // What a lane holds of the group it is about to multiply: the records (operand of the correction
   // step), its raw codes, its columns' scales and the activation operands of k-step 0.
