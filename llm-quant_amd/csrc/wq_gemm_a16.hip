@@ -20,7 +20,7 @@
 //             in operand layout: lane = (row j = lane % 16, block = lane / 16) holds k = 32 block ..
 //             32 block + 31, eight of them per MFMA step
 //   x         the group's 128 values of every activation row, through the wave's own LDS tile: whole rows
-//             go there straight from L2 (global_load_lds_dwordx4: four rows of 256 bytes per instruction, eight
+//             go there straight from L2 (buffer_load_dwordx4 ... lds: four rows of 256 bytes per instruction, eight
 //             cache lines; as operand loads, 64 bytes per lane at a row each, the same bytes were 64 lines per
 //             instruction and the address unit, not memory, set the pace), 16-byte slots XOR-swizzled by row,
 //             and come out as operands: the 32 k of row (lane % 16) that the lane's codes belong to
@@ -53,6 +53,7 @@ struct A16Args {
   int M, N, G, out_group;
   int64_t row_bytes;
   int scales_at;   // (HELD) where the workgroup's scales lie in LDS
+  uint32_t per_row;   // (HELD, G > 1) ceil(2^32 / G): e / G is the upper half of e * per_row, e a scale's place among the workgroup's
 };
 
 // HELD: the scales come first, all of a workgroup's in one sweep (its weight rows' are one run of memory, whole lines to a
@@ -62,6 +63,9 @@ struct A16Args {
 // Of one or two row tiles the workgroups are short (8192 x 2048 int4, M = 16: 6.4 / 6.8, 4096 x 4096 6.6 / 7.5), and with three
 // activation tiles it takes registers that are not there (48 rows: 19.9 / 21.9).
 __host__ __device__ constexpr int scale_pitch(int G) { return G | 1; }   // (odd: sixteen rows in sixteen banks)
+
+// operands of s_waitcnt: none of the wave's vector loads / LDS reads outstanding, the other counters as they are
+constexpr int kAllLoads = 0x0f70, kAllReads = 0xc07f;
 
 template <typename T> struct Mfma16;
 template <> struct Mfma16<bf16_t> {
@@ -109,7 +113,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
-  const int wv = tid / kWave;
+  const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wk = blockDim.x / kWave;
   const int j = lane & 15;
   const int blk = lane >> 4;
@@ -142,21 +146,19 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   constexpr int kXInstr = MT * 4;
   constexpr int kXTileBytes = MT * kTileM * kGroup * 2;
   unsigned char* xtile = smem + wv * kXTileBytes;
-  Place xsrc[kXInstr];
+  uint32_t xsrc[kXInstr];   // (bytes; launch_typed: a slab's rows span less than 4 GiB)
 #pragma unroll
   for (int i = 0; i < kXInstr; ++i) {
     const int row = 4 * i + (lane >> 4), chunk = (lane & 15) ^ (row & 15);
-    xsrc[i] = place(static_cast<const T*>(a.x), min(row, a.M - 1) * K + chunk * 8);
+    xsrc[i] = static_cast<uint32_t>(min(row, a.M - 1) * K * 2 + chunk * 16);
   }
   auto request_rows = [&](int g) {
+    const BufferBase base = buffer_base(static_cast<const uint8_t*>(a.x) + static_cast<int64_t>(g) * (kGroup * 2));
 #pragma unroll
     for (int i = 0; i < kXInstr; ++i) {
       // (four rows past the activation's end are not fetched: what the tile holds there feeds only result rows
       // that are dropped at the store)
-      if (4 * i < a.M) {
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(address(a.x, xsrc[i], static_cast<int64_t>(g) * (kGroup * 2))),
-                                         reinterpret_cast<u32x4*>(xtile + 1024 * i), 16, 0, 0);
-      }
+      if (4 * i < a.M) buffer_to_lds<16>(base, xtile + 1024 * i, xsrc[i], 0);
     }
   };
   // operand of step s, tile mt: row 16 mt + j, chunk 4 blk + s
@@ -247,58 +249,66 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
     }
   };
 
-  // The wave's groups wv, wv + wk, ...: this group's rows and codes have arrived (nothing else of the wave is in
-  // flight), the rows go from the tile to registers, and with the tile free again the next group's transfer
-  // and codes are requested. The compiler does not count a wait written as assembly: it takes the codes to be on their way
-  // still and waits for everything outstanding once more, somewhere behind a request. Of 14336 x 4096 int4, four row tiles,
-  // scales held, a round's first step waits between the transfer and the codes it requests (the transfer is waited for, the
-  // codes run under the multiplications), its second three multiplications behind both.
   // (the scales are asked for in front of everything else, kAhead of a thread's values at once: thread by thread they
   // are the rows' scales laid end to end)
   constexpr int kAhead = 8;
   const int n_scales = kRows * G;
   float ahead[kAhead] = {};
+  auto row_of = [&](int e) { return static_cast<int>(__umulhi(static_cast<uint32_t>(e), a.per_row)); };   // (e / G)
   auto scale_of = [&](int e) {
-    const int row = e / G, n = min(n0 + row, a.N - 1);
+    const int row = row_of(e), n = min(n0 + row, a.N - 1);
     return a.ws + static_cast<int64_t>(a.out_group > 0 ? n / a.out_group : n) * G + (e - row * G);
   };
+  auto hold = [&](int e, float scale) { held[e + (pitch - G) * row_of(e)] = scale; };
   if constexpr (HELD) {
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
-      const int e = i * blockDim.x + tid;
-      if (e < n_scales) ahead[i] = *scale_of(e);
+      if (i * blockDim.x < n_scales) ahead[i] = *scale_of(min(i * blockDim.x + tid, n_scales - 1));
     }
   }
+
+  // The wave's groups wv, wv + wk, ...: this group's rows and codes have arrived (nothing else of the wave is in
+  // flight), the rows go from the tile to registers, and with the tile free again the next group's transfer
+  // and codes are requested; they run under this group's multiplications. That takes a wait the compiler counts (a builtin:
+  // one written as assembly it does not see, and it waits for everything once more behind the next group's requests) and
+  // transfers that are not FLAT (buffer_to_lds). In graphs, weights rotated, bf16, us, before / now: 14336 x 4096 int4, M =
+  // 5 / 16 / 32 11.9 / 10.5, 12.7 / 11.4, 15.6 / 14.2 (transfers left FLAT: 16 rows 11.9); int8 16.0 / 14.6, 16.8 / 15.7, 19.4 /
+  // 18.2; 128256 x 2048 int4 M = 24 66.4 / 58.7, int8 78.1 / 72.4; 8192 x 2048 int4 3 to 6 % less, 4096 x 4096 and 2048 x 2048 up to
+  // 4 %, 4096 x 14336 up to 3; the other way, 1 to 2 %: 4096 x 4096 int4 and 8192 x 2048 int8 of 12 to 17 rows. What bounds it now:
+  // a wave's chain of groups, and the fixed part of a launch (3.5 us). Two groups on their way (two tiles a wave, exact counts) are
+  // no faster: 14336 x 4096 int4 M = 16 11.3, 4096 x 14336 17.2 against 15.6, 128256 x 2048 int8 M = 16 84.8 against 62.3.
+  const int count = (G - wv + wk - 1) / wk;   // (at least one: wk <= G)
   Weights W0, W1;
-  if (wv < G) {
-    request_rows(wv);
-    load_weights(wv, W0);
-  }
+  auto group = [&](int i) { return wv + i * wk; };
+  request_rows(group(0));
+  load_weights(group(0), W0);
   if constexpr (HELD) {
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
       const int e = i * blockDim.x + tid;
-      if (e < n_scales) held[e + (pitch - G) * (e / G)] = ahead[i];
+      if (e < n_scales) hold(e, ahead[i]);
     }
-    for (int e = kAhead * blockDim.x + tid; e < n_scales; e += blockDim.x) held[e + (pitch - G) * (e / G)] = *scale_of(e);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the first group has arrived too: the sweep's branches end in vmcnt(0))
+    for (int e = kAhead * blockDim.x + tid; e < n_scales; e += blockDim.x) hold(e, *scale_of(e));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   }
-  auto step = [&](int g, const Weights& now, Weights& next) {
+  auto step = [&](int i, const Weights& now, Weights& next) {
     Rows X;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(kAllLoads);
+    __builtin_amdgcn_sched_barrier(0);
     read_rows(X);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (g + wk < G) {
-      request_rows(g + wk);
-      load_weights(g + wk, next);
+    __builtin_amdgcn_s_waitcnt(kAllReads);
+    __builtin_amdgcn_sched_barrier(0);
+    if (i + 1 < count) {
+      request_rows(group(i + 1));
+      load_weights(group(i + 1), next);
     }
-    multiply(g, now, X);
+    multiply(group(i), now, X);
   };
-  for (int g = wv; g < G; g += 2 * wk) {   // (two groups a round: the register sets swap by name)
-    step(g, W0, W1);
-    if (g + wk < G) step(g + wk, W1, W0);
+  for (int i = 0; i < count; i += 2) {   // (two groups a round: the register sets swap by name)
+    step(i, W0, W1);
+    if (i + 1 < count) step(i + 1, W1, W0);
   }
   __syncthreads();   // every wave is done with its tile: the partial sums take the same memory
 
@@ -332,7 +342,10 @@ int launch_tile(A16Args a, int wk, hipStream_t stream) {
   const int part = wk * MT * kTileM * NT * kTileN * static_cast<int>(sizeof(float));
   const int tiles = wk * MT * kTileM * kGroup * 2;
   int lds = part > tiles ? part : tiles;
-  if constexpr (HELD) a.scales_at = lds, lds += static_cast<int>(held_bytes(NT, a.G));   // (form_of: they fit)
+  if constexpr (HELD) {   // (form_of: they fit)
+    a.scales_at = lds, lds += static_cast<int>(held_bytes(NT, a.G));
+    a.per_row = static_cast<uint32_t>(((uint64_t{1} << 32) + a.G - 1) / a.G);
+  }
   auto kernel = wq_gemm_a16_kernel<T, BITS, MT, NT, BIASED, HELD>;
   if (lds > 64 * 1024) {
     static bool raised = false;  // per instantiation; worst case two threads both set it
@@ -405,13 +418,16 @@ int launch_typed(const void* x, const void* qw, const float* ws, void* out, int 
   // rows of few groups: two groups per wave at least
   if (G >= 4 && wk * 2 > G) wk = G / 2;
   // (Sixteen waves for few row tiles of long rows, down_proj, measured no faster than eight.)
-  for (int m0 = 0; m0 < M; m0 += kSlabRows) {
+  // (a slab's offsets have 32 bits)
+  const int64_t fit = (int64_t{1} << 32) / (K * 2);
+  const int slab = fit >= kSlabRows ? kSlabRows : (fit > 0 ? static_cast<int>(fit) : 1);
+  for (int m0 = 0; m0 < M; m0 += slab) {
     A16Args a{};
     a.x = static_cast<const T*>(x) + static_cast<int64_t>(m0) * K;
     a.qw = static_cast<const uint8_t*>(qw);
     a.ws = ws;
     a.out = static_cast<T*>(out) + static_cast<int64_t>(m0) * N;
-    a.M = M - m0 < kSlabRows ? M - m0 : kSlabRows;
+    a.M = M - m0 < slab ? M - m0 : slab;
     a.N = N; a.G = G; a.out_group = out_group;
     a.row_bytes = K * BITS / 8;
     const int mt = (a.M + kTileM - 1) / kTileM;

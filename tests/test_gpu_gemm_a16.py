@@ -103,6 +103,22 @@ def test_llama_shapes_on_sampled_entries(ext, n, k, m, split):
     assert rel_l2(got[:, cols], exact) <= 2e-3
 
 
+def test_rows_whose_offsets_need_more_than_32_bits(ext):
+    """64 activation rows of 4 GiB and a little: they are taken in slabs whose offsets have 32 bits. The bar is that of the
+    closed form above (the output's rounding alone is 1.1e-3)."""
+    m, n, groups = 64, 2, 262145
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(m, groups * GROUP, device="cuda", generator=gen, dtype=torch.bfloat16)
+    q = torch.randint(-128, 128, (n, groups, GROUP), device="cuda", generator=gen, dtype=torch.int8)
+    s = torch.rand(n, groups, device="cuda", generator=gen) * 0.01
+    got = ext.wq_gemm_a16(x, q, s, 0, False)
+    want = torch.zeros(m, n, dtype=torch.float64, device="cuda")
+    for g in range(0, groups, 8192):
+        part = (q[:, g:g + 8192].float() * s[:, g:g + 8192, None]).flatten(1)
+        want += (x[:, g * GROUP:(g + 8192) * GROUP].float() @ part.T.contiguous()).double()
+    assert rel_l2(to_np(got), want.cpu().numpy()) <= 2e-3
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k,out_group", [
