@@ -21,13 +21,16 @@
 // reductions plus one exchange between the two halves; O^T = V^T P^T (A = head_dim x keys, B = keys x queries)
 // takes the probabilities straight out of those registers as its B operand (the k index of the MFMA is just a
 // naming of the keys, the same on both operands) and V^T from the wave's own LDS tile: the block's rows of V go
-// there as they lie in memory (global_load_lds_dwordx4, no register in between, the 16-byte pieces of odd keys
+// there as they lie in memory (buffer_load_dwordx4 ... lds, no register in between, the 16-byte pieces of odd keys
 // XOR-swizzled by four so that the reads below spread over the banks), and ds_read_b64_tr_b16 hands lane
 // (d, half) four keys of its column per read. Among the 16 lanes of a group, that instruction gives lane l, as
 // its element j, element l % 4 of what lane 4 j + l / 4 points at: with lane 4 j + i pointing at key j,
-// columns 4 i .. 4 i + 3, lane l gets column l of keys 0..3. The next block's K and V are requested as soon as
-// this block's K has been consumed, into the tile's other buffer. (They run under the softmax and no further: the compiler
-// does not tell the two buffers apart and waits for all of them in front of this block's reads of V.)
+// columns 4 i .. 4 i + 3, lane l gets column l of keys 0..3. The reads of V stand behind the first product's
+// multiplications; with both operands of the block in registers the next block's K and V are requested, into the
+// same tile, and run under the softmax and the second product. us in graphs, 32 query / 8 kv heads, bf16, with the
+// reads of V behind the softmax, where the compiler waits for all transfers, the next block's too / now: head_dim 64, 256 tokens 5.0 /
+// 4.9, 500 9.1 / 8.6, 800 14.9 / 14.3, 1100 22.1 / 20.1, 2048 67.8 / 67.0; head_dim 128, 500 15.6 / 15.2, 1100 44.8 / 43.1, 2048
+// 140 / 135, 4096 425 / 410; up to 128 tokens within 2 %.
 #include "llmq_device.h"
 
 namespace {
@@ -40,6 +43,7 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 
+constexpr int kAllLoads = 0x0f70;   // operand of s_waitcnt: no vector load outstanding, the other counters as they are
 constexpr int kQueriesPerGroup = 32, kWavesPerGroup = 4, kKeysPerBlock = 32;
 
 template <typename T> __device__ __forceinline__ v16f mfma16(u32x4 a, u32x4 b, v16f c);
@@ -52,7 +56,7 @@ template <> __device__ __forceinline__ v16f mfma16<f16_t>(u32x4 a, u32x4 b, v16f
 
 template <typename T> __device__ __forceinline__ uint32_t pack2(float lo, float hi);
 template <> __device__ __forceinline__ uint32_t pack2<bf16_t>(float lo, float hi) {
-  return static_cast<uint32_t>(bf16_bits_rne(lo)) | (static_cast<uint32_t>(bf16_bits_rne(hi)) << 16);
+  return bf16_pair_rne(lo, hi);
 }
 template <> __device__ __forceinline__ uint32_t pack2<f16_t>(float lo, float hi) {
   const _Float16 a = static_cast<_Float16>(lo), b = static_cast<_Float16>(hi);
@@ -63,8 +67,33 @@ template <> __device__ __forceinline__ uint32_t pack2<f16_t>(float lo, float hi)
 // 8 (r / 4) + 4 lh + r % 4).
 __device__ __forceinline__ int key_of(int lh, int r) { return 8 * (r >> 2) + 4 * lh + (r & 3); }
 
+__device__ __forceinline__ uint32_t lds_offset(const void* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
+#else
+  return 0;
+#endif
+}
+
+// The transposing reads of two row tiles, eight keys apart four times. (Assembly, with their wait: in front of the builtin the
+// compiler waits for every transfer into LDS, the next block's as well.)
+template <int ROW>
+__device__ __forceinline__ void read_transposed(uint32_t at0, uint32_t at1, u32x2* a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %8 offset:%10\n\t"
+      "ds_read_b64_tr_b16 %4, %9\n\tds_read_b64_tr_b16 %5, %9 offset:%10\n\t"
+      "ds_read_b64_tr_b16 %2, %8 offset:%11\n\tds_read_b64_tr_b16 %3, %8 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %6, %9 offset:%11\n\tds_read_b64_tr_b16 %7, %9 offset:%12\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(a[4]), "=&v"(a[5]), "=&v"(a[6]), "=&v"(a[7])
+      : "v"(at0), "v"(at1), "n"(8 * ROW), "n"(16 * ROW), "n"(24 * ROW)
+      : "memory");
+#endif
+}
+
 template <int D> struct Lds {
-  static constexpr int kTile = 2 * kKeysPerBlock * D * 2;          // bytes of one wave's V tile, two buffers
+  static constexpr int kTile = kKeysPerBlock * D * 2;              // bytes of one wave's V tile
   static constexpr int kRow = D + 4;                               // floats of a row of a partial result
   static constexpr int kPartial = kQueriesPerGroup * kRow * 4;     // bytes of one wave's partial result
   static constexpr int kBody = kWavesPerGroup * (kPartial > kTile ? kPartial : kTile);
@@ -112,17 +141,15 @@ __global__ __launch_bounds__(kWavesPerGroup * kWave, 2) void prefill_attention_k
     v_off[i] = static_cast<uint32_t>((slot ^ ((key & 1) << 2)) * 16);
   }
   u32x4 kreg[kDSteps];
-  auto request = [&](int b, int buf) {
+  auto request = [&](int b) {
     const int j0 = b * kKeysPerBlock;
     const T* row = kh + static_cast<int64_t>(min(j0 + lm, tokens - 1)) * D + 8 * lh;
+    const BufferBase block = buffer_base(vh + static_cast<int64_t>(j0) * D);
 #pragma unroll
     for (int t = 0; t < kDSteps; ++t) kreg[t] = load16(row + 16 * t);
 #pragma unroll
     for (int i = 0; i < kVInstr; ++i) {
-      const unsigned char* src = reinterpret_cast<const unsigned char*>(vh) +
-                                 static_cast<int64_t>(min(j0 + v_key[i], tokens - 1)) * kRowBytes + v_off[i];
-      __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(src),
-                                       reinterpret_cast<u32x4*>(tile + buf * kTileBytes + 1024 * i), 16, 0, 0);
+      buffer_to_lds<16>(block, tile + 1024 * i, min(v_key[i], tokens - 1 - j0) * kRowBytes + v_off[i], 0);
     }
   };
   // where this lane points for the transposing reads: key 4 lh + j of a group of eight, columns
@@ -144,19 +171,23 @@ __global__ __launch_bounds__(kWavesPerGroup * kWave, 2) void prefill_attention_k
     for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;   // of this lane's query, in units of log2
 
-  if (wv < n_blocks) request(wv, 0);
-  int buf = 0;
-  for (int b = wv; b < n_blocks; b += kWavesPerGroup, buf ^= 1) {
+  const uint32_t vt = lds_offset(tile);
+  if (wv < n_blocks) request(wv);
+  for (int b = wv; b < n_blocks; b += kWavesPerGroup) {
     const int j0 = b * kKeysPerBlock;
     // this block's K and V have arrived (nothing else of this wave is in flight)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(kAllLoads);
+    __builtin_amdgcn_sched_barrier(0);
     v16f s;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = 0.0f;
 #pragma unroll
     for (int t = 0; t < kDSteps; ++t) s = mfma16<T>(kreg[t], qreg[t], s);
-    // (the other buffer: its last readers were the previous block's MFMAs, whose operands have long arrived)
-    if (b + kWavesPerGroup < n_blocks) request(b + kWavesPerGroup, buf ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x2 vreg[kDTiles][4];   // V^T operands of row tile t: keys 4 lh + 0..3 of each eight of the block
+#pragma unroll
+    for (int t = 0; t < kDTiles; t += 2) read_transposed<kRowBytes>(vt + tr_at[t], vt + tr_at[t + 1], vreg[t]);
+    if (b + kWavesPerGroup < n_blocks) request(b + kWavesPerGroup);   // (K and V of this block are in registers)
 
     // keys beyond the query or the prompt out (only the blocks on the diagonal and at the prompt's end have any)
     if (j0 + kKeysPerBlock - 1 > min(q0, tokens - 1)) {
@@ -199,18 +230,13 @@ __global__ __launch_bounds__(kWavesPerGroup * kWave, 2) void prefill_attention_k
 
     // O^T += V^T P^T: k-step st covers the keys that registers 8 st .. 8 st + 7 hold (key_of): two transposing
     // reads, keys 16 st + 4 lh + 0..3 and 16 st + 8 + 4 lh + 0..3
-    const unsigned char* vt = tile + buf * kTileBytes;
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       const u32x4 pb = {p[4 * st], p[4 * st + 1], p[4 * st + 2], p[4 * st + 3]};
 #pragma unroll
       for (int t = 0; t < kDTiles; ++t) {
-        const unsigned char* at = vt + tr_at[t] + 16 * st * kRowBytes;
-        const uint2 a_lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) v4s*)(at)));
-        const uint2 a_hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) v4s*)(at + 8 * kRowBytes)));
-        o[t] = mfma16<T>(u32x4{a_lo.x, a_lo.y, a_hi.x, a_hi.y}, pb, o[t]);
+        const u32x2 lo = vreg[t][2 * st], hi = vreg[t][2 * st + 1];
+        o[t] = mfma16<T>(u32x4{lo.x, lo.y, hi.x, hi.y}, pb, o[t]);
       }
     }
   }
