@@ -195,6 +195,35 @@ def test_rope_and_append_in_one_launch_equal_the_two_launches(ext, dtype, bits, 
     assert torch.equal(bare.k_codes, two.k_codes) and torch.equal(bare.v_scale, two.v_scale)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("tokens", [767, 768, 1031])
+def test_rope_and_append_of_rows_that_start_anywhere(ext, dtype, bits, head_dim, tokens):
+    """Rows that are no whole packets (an odd row stride, a tensor that starts one element in) against the same values in
+    packets (taken from 6144 head vectors on): the same bits, and tokens past the cache's end are left out on both ways."""
+    from llmquant.runtime.kv_cache import KernelQuantCache
+
+    q_heads, kv_heads, max_len = 4, 2, 760
+    torch.manual_seed(head_dim + bits)
+    width = (q_heads + 2 * kv_heads) * head_dim
+    loose = (torch.randn(tokens, width + 3, device="cuda") * 2.0).to(dtype)
+    loose[5, 1:] = 0.0
+    q_width, kv_width = q_heads * head_dim, kv_heads * head_dim
+    emb = torch.rand(tokens, head_dim, device="cuda") * 6.28
+    cos, sin = emb.cos().to(dtype), emb.sin().to(dtype)
+    results = []
+    for qkv in (loose[:, 1:width + 1], loose[:, 1:width + 1].contiguous()):
+        q, k, v = qkv[:, :q_width], qkv[:, q_width:q_width + kv_width], qkv[:, q_width + kv_width:]
+        cache = KernelQuantCache(1, kv_heads, head_dim, max_len, bits, q_heads=q_heads)
+        out = ext.rope_kv_append(q, k, v, cos, sin, cache.k_codes[0], cache.v_codes[0], cache.k_scale[0], cache.v_scale[0],
+                                 cache.position, q_heads, True)
+        results.append([out[0], out[1][:, :max_len], out[2][:, :max_len], cache.k_codes, cache.v_codes, cache.k_scale,
+                        cache.v_scale])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
 def test_rope_and_append_argument_checks(ext):
     from llmquant.runtime.kv_cache import KernelQuantCache
 
