@@ -160,75 +160,6 @@ __global__ __launch_bounds__(256) void rope_kv_append_kernel(
   }
 }
 
-// The same for rows and tensors that are whole 16-byte packets: D / V lanes a head, each with its own packet of the vector and
-// the one its elements are rotated with (same rounding points, same bits). Bound: a chain of memory trips (rows, then stores) of one
-// short launch; a wave a head, an element or two a lane, is eight times the waves (line between the two: llmq_rope_kv_append).
-template <typename T, int BITS, int D>
-__global__ __launch_bounds__(256) void rope_kv_append_packets_kernel(
-    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, const int64_t q_stride,
-    const int64_t k_stride, const int64_t v_stride, const T* __restrict__ cos_rows,
-    const T* __restrict__ sin_rows, T* __restrict__ q_out, uint8_t* __restrict__ k_codes,
-    uint8_t* __restrict__ v_codes, float* __restrict__ k_scale, float* __restrict__ v_scale,
-    T* __restrict__ dq_k, T* __restrict__ dq_v, const int32_t* __restrict__ pos_dev, const int tokens,
-    const int q_heads, const int kv_heads, const int t_max) {
-  constexpr int V = Pack<T>::N, kLanes = D / V;
-  static_assert(kLanes == 8 || kLanes == 16 || kLanes == 32, "a head's lanes are a group of group_max");
-  const uint32_t item = blockIdx.x * blockDim.x + threadIdx.x;   // (below 2^31: the host's rule)
-  const uint32_t heads = q_heads + 2 * kv_heads, vector = item / kLanes;
-  if (vector >= tokens * heads) return;   // a head's lanes leave together
-  const int p = static_cast<int>(item % kLanes);
-  const int tok = static_cast<int>(vector / heads), h = static_cast<int>(vector % heads);
-  const bool is_q = h < q_heads;
-  const bool is_v = h >= q_heads + kv_heads;
-  const int head = is_q ? h : (is_v ? h - q_heads - kv_heads : h - q_heads);
-  const int pos = is_q ? 0 : pos_dev[0] + tok;
-  const T* src = is_q   ? q + tok * q_stride + static_cast<int64_t>(head) * D
-                 : is_v ? v + tok * v_stride + static_cast<int64_t>(head) * D
-                        : k + tok * k_stride + static_cast<int64_t>(head) * D;
-  float f[V];
-  Pack<T>::unpack(load16(src + p * V), f);
-  if (!is_v) {
-    float other[V], c[V], s[V];
-    Pack<T>::unpack(load16(src + (p ^ (kLanes / 2)) * V), other);
-    Pack<T>::unpack(load16(cos_rows + static_cast<int64_t>(tok) * D + p * V), c);
-    Pack<T>::unpack(load16(sin_rows + static_cast<int64_t>(tok) * D + p * V), s);
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-      const float rot = p < kLanes / 2 ? -other[e] : other[e];
-      f[e] = round_through<T>(round_through<T>(f[e] * c[e]) + round_through<T>(rot * s[e]));
-    }
-  }
-  if (is_q) {
-    store16(q_out + (static_cast<int64_t>(tok) * q_heads + head) * D + p * V, Pack<T>::pack(f));
-    return;
-  }
-  if (pos < 0 || pos >= t_max) return;
-  const float qmax = static_cast<float>((1 << (BITS - 1)) - 1);
-  const float qmin = -qmax - 1.0f;
-  float amax = 0.0f;
-#pragma unroll
-  for (int e = 0; e < V; ++e) amax = fmaxf(amax, fabsf(f[e]));
-  amax = group_max<kLanes>(amax);
-  const float scale = scale_from_amax(amax, qmax);
-  const int64_t slot = static_cast<int64_t>(head) * t_max + pos;
-  if (p == 0) (is_v ? v_scale : k_scale)[slot] = scale;
-  T* dq = is_v ? dq_v : dq_k;
-  uint32_t words[2] = {0u, 0u};   // V codes: V x BITS bits
-#pragma unroll
-  for (int e = 0; e < V; ++e) {
-    const float qv = quant_code(f[e], scale, qmin, qmax);
-    f[e] = qv * scale;
-    const int code = static_cast<int>(qv);
-    if constexpr (BITS == 8) words[e / 4] |= (static_cast<uint32_t>(code) & 0xffu) << (8 * (e % 4));
-    else words[0] |= (static_cast<uint32_t>(code + 8) & 0xfu) << (4 * e);
-  }
-  if (dq != nullptr) store16(dq + (static_cast<int64_t>(head) * tokens + tok) * D + p * V, Pack<T>::pack(f));
-  uint8_t* codes = (is_v ? v_codes : k_codes) + (slot * D + p * V) * BITS / 8;
-  if constexpr (V * BITS == 64) *reinterpret_cast<u32x2*>(codes) = u32x2{words[0], words[1]};
-  else if constexpr (V * BITS == 32) *reinterpret_cast<uint32_t*>(codes) = words[0];
-  else *reinterpret_cast<uint16_t*>(codes) = static_cast<uint16_t>(words[0]);
-}
-
 // ---- dequantize a range of the cache (what update() hands back outside of decode) ---------------
 template <typename T, int BITS>
 __global__ __launch_bounds__(256) void kv_dequant_kernel(
@@ -1607,20 +1538,20 @@ extern "C" int llmq_rope_kv_append(const void* q, const void* k, const void* v, 
   const uintptr_t codes_at = reinterpret_cast<uintptr_t>(k_codes) | reinterpret_cast<uintptr_t>(v_codes);
   const bool packets = waves >= 6144 && at % 16 == 0 && codes_at % 8 == 0 && (q_row_stride | k_row_stride | v_row_stride) % packet == 0 &&
                        lanes < (int64_t{1} << 31) - 256;
-  const dim3 grid(static_cast<unsigned>(packets ? (lanes + 255) / 256 : (waves + 3) / 4)), block(256);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define LLMQ_ROPE_APPEND_AS(KERNEL, T, B, D)                                                                 \
-  hipLaunchKernelGGL((KERNEL<T, B, D>), grid, block, 0, s, static_cast<const T*>(q),                         \
+  if (packets) {
+    return llmq_host::rope_kv_append_packets(q, k, v, q_row_stride, k_row_stride, v_row_stride, cos_rows, sin_rows, q_out,
+                                             k_codes, v_codes, k_scale, v_scale, dq_k_or_null, dq_v_or_null, pos_dev, tokens,
+                                             q_heads, kv_heads, head_dim, t_max, bits, dtype, s);
+  }
+  const dim3 grid(static_cast<unsigned>((waves + 3) / 4)), block(256);
+#define LLMQ_ROPE_APPEND(T, B, D)                                                                          \
+  hipLaunchKernelGGL((rope_kv_append_kernel<T, B, D>), grid, block, 0, s, static_cast<const T*>(q),         \
                      static_cast<const T*>(k), static_cast<const T*>(v), q_row_stride, k_row_stride,        \
                      v_row_stride, static_cast<const T*>(cos_rows), static_cast<const T*>(sin_rows),        \
                      static_cast<T*>(q_out), static_cast<uint8_t*>(k_codes), static_cast<uint8_t*>(v_codes), \
                      k_scale, v_scale, static_cast<T*>(dq_k_or_null), static_cast<T*>(dq_v_or_null), pos_dev, \
                      tokens, q_heads, kv_heads, t_max)
-#define LLMQ_ROPE_APPEND(T, B, D)                                        \
-  do {                                                                   \
-    if (packets) LLMQ_ROPE_APPEND_AS(rope_kv_append_packets_kernel, T, B, D); \
-    else LLMQ_ROPE_APPEND_AS(rope_kv_append_kernel, T, B, D);            \
-  } while (0)
 #define LLMQ_ROPE_APPEND_T(T)                                             \
   do {                                                                    \
     if (bits == 8 && head_dim == 64) LLMQ_ROPE_APPEND(T, 8, 64);          \
@@ -1635,7 +1566,6 @@ extern "C" int llmq_rope_kv_append(const void* q, const void* k, const void* v, 
   }
 #undef LLMQ_ROPE_APPEND_T
 #undef LLMQ_ROPE_APPEND
-#undef LLMQ_ROPE_APPEND_AS
   return llmq_host::check_launch("rope_kv_append_kernel");
 }
 

@@ -371,6 +371,12 @@ int experts_direct_launch(const void* x, const int64_t* index, const void* weigh
                           const float* gate_up_scale, const void* down, const float* down_scale, void* out, void* act,
                           int tokens, int top_k, int n_experts, int hidden, int intermediate, int wformat, int dtype,
                           hipStream_t stream);
+// The cache append of a prompt whose rows are whole packets (kv_cache.hip checks them, prefill_ops.hip launches).
+int rope_kv_append_packets(const void* q, const void* k, const void* v, int64_t q_row_stride, int64_t k_row_stride,
+                           int64_t v_row_stride, const void* cos_rows, const void* sin_rows, void* q_out, void* k_codes,
+                           void* v_codes, float* k_scale, float* v_scale, void* dq_k_or_null, void* dq_v_or_null,
+                           const int32_t* pos_dev, int tokens, int q_heads, int kv_heads, int head_dim, int t_max, int bits,
+                           int dtype, hipStream_t s);
 int gemv_batched_mfma_launch(const void* x, const void* qw, const float* ws, void* out, const int32_t* block_expert,
                              const int32_t* block_row0, const int32_t* block_rows, int n_blocks, int n_rows,
                              int n_experts, int N, int G, int out_group, int wformat, int dtype,
