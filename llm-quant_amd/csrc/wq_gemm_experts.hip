@@ -239,18 +239,31 @@ int run_shape(const TileArgs& gate_up, const TileArgs& down, int max_row_tiles, 
   return launch_grouped<T, BITS, kEpiStore, S>(down, max_row_tiles, stream);
 }
 
+// Rows of a tile: 32 or 64. The host does not know the experts' counts; an expert's last tile is half full on average, so
+// that there are about rows / height + E / 2 row tiles (no fewer than experts with rows), each with I / 128 column tiles in the
+// gate|up launch, on 512 places at once (int8: 256, one a CU). A launch takes a round at least, and half of one more than the tiles fill on
+// average; a round of 64-row tiles takes 1.4 of 32-row ones. Measured, both heights, 96 problems each of int4 and int8 (bf16, a router
+// that prefers some experts to others; 8 to 128 experts, 4 to 200 rows an expert), us a call, 32 / 64 rows: 64 experts of 2048 x
+// 1024 int4 at 10 rows an expert 65 / 74, 30: 86 / 96, 37.5: 96 / 100, 45: 103 / 103, 75: 143 / 130, 200: 285 / 243; int8 30: 119 /
+// 134, 37.5: 140 / 136, 52: 169 / 145; eight of 2048 x 4096 int4 at 45: 67 / 79, 64: 78 / 85, 90: 90 / 88, 130: 118 / 106, int8 37.5: 90
+// / 104, 45: 94 / 103, 52: 109 / 104, 130: 187 / 136; eight of 4096 x 14336 int4 30: 264 / 286, 37.5: 324 / 298; sixteen of 4096 x 6400
+// int4 30: 247 / 257, 37.5: 282 / 260. A line at 40 rows an expert was up to 19 % behind (eight of 2048 x 4096).
+int tile_rows_for(int rows, int E, int I, bool int4) {
+  const double hit = rows < E ? rows : E, places = int4 ? 512.0 : 256.0;
+  auto cost = [&](int height) {
+    const double row_tiles = static_cast<double>(rows) / height + 0.5 * E;
+    const double rounds = (row_tiles > hit ? row_tiles : hit) * (I / kGroup) / places + 0.5;
+    return rounds > 1.0 ? rounds : 1.0;
+  };
+  return 1.4 * cost(64) < cost(32) ? 64 : 32;
+}
+
 template <typename T, int BITS>
 int run(const void* x, const int64_t* index, const void* weights, const void* q1, const float* s1, const void* q2,
         const float* s2, void* out, uint8_t* ws, int n_tokens, int top_k, int E, int H, int I, hipStream_t stream) {
   const Layout l = layout_for(n_tokens, top_k, E, H, I);
   const int rows = n_tokens * top_k;
-  // 64-row tiles from 40 rows an expert on: with scales read group by group the two heights met there. Measured since the
-  // scales come in chunks, us a call, 32-row tiles / 64-row, bf16: 64 experts of 2048 x 1024 int4 at 10 rows an expert 76 / 91,
-  // 25: 86 / 85, 37.5: 104 / 86, 45: 106 / 88, 52: 118 / 111, 75: 147 / 144; int8 10: 100 / 117, 25: 119 / 115, 37.5: 146 / 119,
-  // 52: 153 / 127. Eight experts of 2048 x 4096 int4 at 30: 68 / 74, 40: 71 / 75, 50: 71 / 76, 75: 86 / 89, 125: 121 / 110; int8
-  // 30: 91 / 85, 50: 97 / 89, 125: 190 / 145. (Many narrow experts would take the higher tile from 25 rows on, few wide int4 ones
-  // from some 100 on.)
-  const int tile_rows = rows > 40 * E ? 64 : 32;
+  const int tile_rows = tile_rows_for(rows, E, I, BITS == 4);
   const PlanArgs p{index, rows, E, top_k, tile_rows, reinterpret_cast<int4*>(ws + l.tiles),
                    reinterpret_cast<int*>(ws + l.n_tiles), reinterpret_cast<int*>(ws + l.row_source),
                    reinterpret_cast<int*>(ws + l.sorted)};
