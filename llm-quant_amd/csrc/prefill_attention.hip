@@ -43,7 +43,8 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 
-constexpr int kAllLoads = 0x0f70;   // operand of s_waitcnt: no vector load outstanding, the other counters as they are
+// operands of s_waitcnt: none of the wave's vector loads / LDS reads outstanding, the other counters as they are
+constexpr int kAllLoads = 0x0f70, kAllReads = 0xc07f;
 constexpr int kQueriesPerGroup = 32, kWavesPerGroup = 4, kKeysPerBlock = 32;
 
 template <typename T> __device__ __forceinline__ v16f mfma16(u32x4 a, u32x4 b, v16f c);
@@ -66,31 +67,6 @@ template <> __device__ __forceinline__ uint32_t pack2<f16_t>(float lo, float hi)
 // Key of a 32-key block that register r of an S^T tile holds in lane half lh (the MFMA's result layout: row
 // 8 (r / 4) + 4 lh + r % 4).
 __device__ __forceinline__ int key_of(int lh, int r) { return 8 * (r >> 2) + 4 * lh + (r & 3); }
-
-__device__ __forceinline__ uint32_t lds_offset(const void* p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
-#else
-  return 0;
-#endif
-}
-
-// The transposing reads of two row tiles, eight keys apart four times. (Assembly, with their wait: in front of the builtin the
-// compiler waits for every transfer into LDS, the next block's as well.)
-template <int ROW>
-__device__ __forceinline__ void read_transposed(uint32_t at0, uint32_t at1, u32x2* a) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile(
-      "ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %8 offset:%10\n\t"
-      "ds_read_b64_tr_b16 %4, %9\n\tds_read_b64_tr_b16 %5, %9 offset:%10\n\t"
-      "ds_read_b64_tr_b16 %2, %8 offset:%11\n\tds_read_b64_tr_b16 %3, %8 offset:%12\n\t"
-      "ds_read_b64_tr_b16 %6, %9 offset:%11\n\tds_read_b64_tr_b16 %7, %9 offset:%12\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(a[4]), "=&v"(a[5]), "=&v"(a[6]), "=&v"(a[7])
-      : "v"(at0), "v"(at1), "n"(8 * ROW), "n"(16 * ROW), "n"(24 * ROW)
-      : "memory");
-#endif
-}
 
 template <int D> struct Lds {
   static constexpr int kTile = kKeysPerBlock * D * 2;              // bytes of one wave's V tile
@@ -171,12 +147,12 @@ __global__ __launch_bounds__(kWavesPerGroup * kWave, 2) void prefill_attention_k
     for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;   // of this lane's query, in units of log2
 
-  const uint32_t vt = lds_offset(tile);
   if (wv < n_blocks) request(wv);
   for (int b = wv; b < n_blocks; b += kWavesPerGroup) {
     const int j0 = b * kKeysPerBlock;
     // this block's K and V have arrived (nothing else of this wave is in flight)
     __builtin_amdgcn_s_waitcnt(kAllLoads);
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     v16f s;
 #pragma unroll
@@ -186,7 +162,14 @@ __global__ __launch_bounds__(kWavesPerGroup * kWave, 2) void prefill_attention_k
     __builtin_amdgcn_sched_barrier(0);
     u32x2 vreg[kDTiles][4];   // V^T operands of row tile t: keys 4 lh + 0..3 of each eight of the block
 #pragma unroll
-    for (int t = 0; t < kDTiles; t += 2) read_transposed<kRowBytes>(vt + tr_at[t], vt + tr_at[t + 1], vreg[t]);
+    for (int t = 0; t < kDTiles; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        vreg[t][e] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) v4s*)(tile + tr_at[t] + 8 * e * kRowBytes)));
+    __builtin_amdgcn_s_waitcnt(kAllReads);   // (the next block's transfers take the tile)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
     if (b + kWavesPerGroup < n_blocks) request(b + kWavesPerGroup);   // (K and V of this block are in registers)
 
     // keys beyond the query or the prompt out (only the blocks on the diagonal and at the prompt's end have any)

@@ -296,9 +296,11 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   auto step = [&](int i, const Weights& now, Weights& next) {
     Rows X;
     __builtin_amdgcn_s_waitcnt(kAllLoads);
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     read_rows(X);
     __builtin_amdgcn_s_waitcnt(kAllReads);
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     if (i + 1 < count) {
       request_rows(group(i + 1));
