@@ -383,6 +383,18 @@ def test_scales_of_a_last_run_of_groups(ext, bits, dtype, tokens, hidden, inter,
     test_grouped_gemms_against_real_mode(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew)
 
 
+@pytest.mark.parametrize("bits,dtype", [("int4", torch.bfloat16), ("int8", torch.bfloat16), ("int4", torch.float16)])
+@pytest.mark.parametrize("tokens,hidden,inter,experts,top_k,skew", [
+    (601, 896, 2176, 2, 2, False),   # nine 64-row tiles an expert and one of 25; seven and seventeen groups
+    (400, 1536, 4736, 2, 2, True),   # six and one of 16; twelve and thirty-seven
+    (333, 640, 4096, 3, 2, True),    # the first expert takes every token, the others what is left
+])
+def test_prompts_whose_rounds_take_the_higher_tiles(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew):
+    """Shapes that fill the chip with 64-row tiles (where 1.4 rounds of them are fewer than those of 32-row ones), ragged in
+    rows and in groups."""
+    test_grouped_gemms_against_real_mode(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew)
+
+
 @pytest.mark.parametrize("tokens", [2, 12])
 def test_an_activation_that_starts_inside_a_packet(ext, tokens):
     """A contiguous view at an odd storage offset, through the two-launch form and the grouped GEMMs: the bits of the
