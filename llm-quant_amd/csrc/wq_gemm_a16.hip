@@ -52,6 +52,7 @@ struct A16Args {
   void* out;
   int M, N, G, out_group;
   int64_t row_bytes;
+  int wk, each, more;   // waves of a workgroup; groups of a wave, and waves that have one more
   int scales_at;   // (HELD) where the workgroup's scales lie in LDS
   uint32_t per_row;   // (HELD, G > 1) ceil(2^32 / G): e / G is the upper half of e * per_row, e a scale's place among the workgroup's
 };
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int wk = blockDim.x / kWave;
+  const int wk = a.wk;
   const int j = lane & 15;
   const int blk = lane >> 4;
   const int G = a.G;
@@ -271,17 +272,18 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
   // flight), the rows go from the tile to registers, and with the tile free again the next group's transfer
   // and codes are requested; they run under this group's multiplications. That takes a wait the compiler counts (a builtin:
   // one written as assembly it does not see, and it waits for everything once more behind the next group's requests) and
-  // transfers that are not FLAT (buffer_to_lds). In graphs, weights rotated, bf16, us, before / now: 14336 x 4096 int4, M =
-  // 5 / 16 / 32 11.9 / 10.5, 12.7 / 11.4, 15.6 / 14.2 (transfers left FLAT: 16 rows 11.9); int8 16.0 / 14.6, 16.8 / 15.7, 19.4 /
-  // 18.2; 128256 x 2048 int4 M = 24 66.4 / 58.7, int8 78.1 / 72.4; 8192 x 2048 int4 3 to 6 % less, 4096 x 4096 and 2048 x 2048 up to
-  // 4 %, 4096 x 14336 up to 3; the other way, 1 to 2 %: 4096 x 4096 int4 and 8192 x 2048 int8 of 12 to 17 rows. What bounds it now:
-  // a wave's chain of groups, and the fixed part of a launch (3.5 us). Two groups on their way (two tiles a wave, exact counts) are
-  // no faster: 14336 x 4096 int4 M = 16 11.3, 4096 x 14336 17.2 against 15.6, 128256 x 2048 int8 M = 16 84.8 against 62.3.
-  const int count = (G - wv + wk - 1) / wk;   // (at least one: wk <= G)
+  // transfers that are not FLAT (buffer_to_lds). And nothing slow lies in front of the first request: the host sends the waves'
+  // shares along (a division here, and the workgroup's size out of the dispatch packet, are 0.1 to 0.4 us). In graphs, weights
+  // rotated, bf16, us, with the waits and FLAT transfers / with a division in front / now: 14336 x 4096 int4, M = 4 / 16 / 32 11.8 /
+  // 10.2 / 9.7, 12.7 / 11.4 / 11.0, 15.6 / 14.3 / 13.7; int8 16.0 / 14.7 / 14.4, 16.9 / 15.8 / 15.4, 19.3 / 18.1 / 17.8; 128256 x
+  // 2048 int4 M = 24 64.8 / 57.6 / 55.8, int8 78.4 / 73.1 / 71.9; 8192 x 2048 int4 M = 16 6.2 / 6.1 / 6.0, int8 7.1 / 7.3 / 7.0; 4096 x
+  // 4096 int4 M = 12 6.2 / 6.2 / 6.2, 32 8.7 / 8.5 / 8.5; the other way: 4096 x 4096 of 16 rows, int4 6.5 / 6.6 / 6.6, int8 7.4 / 7.5
+  // / 7.5. What bounds it now: a wave's chain of groups, and the fixed part of a launch (3.5 us). Two groups on their way (two
+  // tiles a wave, exact counts) are no faster: 14336 x 4096 int4 M = 16 11.3, 4096 x 14336 17.2 against 15.6, 128256 x 2048 int8 M =
+  // 16 84.8 against 62.3.
   Weights W0, W1;
-  auto group = [&](int i) { return wv + i * wk; };
-  request_rows(group(0));
-  load_weights(group(0), W0);
+  request_rows(wv);   // (wv < wk <= G)
+  load_weights(wv, W0);
   if constexpr (HELD) {
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
@@ -293,7 +295,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   }
-  auto step = [&](int i, const Weights& now, Weights& next) {
+  auto step = [&](int g, bool last, const Weights& now, Weights& next) {
     Rows X;
     __builtin_amdgcn_s_waitcnt(kAllLoads);
     asm volatile("" ::: "memory");
@@ -302,15 +304,27 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void wq_gemm_a16_kernel(const A1
     __builtin_amdgcn_s_waitcnt(kAllReads);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    if (i + 1 < count) {
-      request_rows(group(i + 1));
-      load_weights(group(i + 1), next);
+    if (!last) {
+      request_rows(g + wk);
+      load_weights(g + wk, next);
     }
-    multiply(group(i), now, X);
+    multiply(g, now, X);
   };
-  for (int i = 0; i < count; i += 2) {   // (two groups a round: the register sets swap by name)
-    step(i, W0, W1);
-    if (i + 1 < count) step(i + 1, W1, W0);
+  // (Two groups a round: the register sets swap by name. By counts, the loop of four row tiles is 0 to 3 % slower, 14336 x 4096 int4
+  // M = 17 12.8 us; by groups, short launches of one tile are: 512 x 2048 int8 M = 4 3 %, 1024 x 4096 int4 2.)
+  if constexpr (NT == 4) {
+    int g = wv;
+    do {
+      step(g, g + wk >= G, W0, W1);
+      if (g + wk < G) step(g + wk, g + 2 * wk >= G, W1, W0);
+      g += 2 * wk;
+    } while (g < G);
+  } else {
+    const int count = a.each + (wv < a.more);
+    for (int i = 0; i < count; i += 2) {
+      step(wv + i * wk, i + 1 >= count, W0, W1);
+      if (i + 1 < count) step(wv + (i + 1) * wk, i + 2 >= count, W1, W0);
+    }
   }
   __syncthreads();   // every wave is done with its tile: the partial sums take the same memory
 
@@ -339,6 +353,7 @@ constexpr int64_t held_bytes(int row_tiles, int G) { return int64_t{row_tiles * 
 
 template <typename T, int BITS, int MT, int NT, bool BIASED, bool HELD = false>
 int launch_tile(A16Args a, int wk, hipStream_t stream) {
+  a.wk = wk, a.each = a.G / wk, a.more = a.G % wk;
   const int grid = (a.N + NT * kTileN - 1) / (NT * kTileN);
   // the waves' activation tiles, then (the same memory) their partial sums
   const int part = wk * MT * kTileM * NT * kTileN * static_cast<int>(sizeof(float));
