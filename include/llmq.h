@@ -152,6 +152,8 @@ int llmq_wq_experts_direct(const void* x, const int64_t* top_k_index, const void
  * experts, 256 experts a token, activations and one expert's weight below 4 GiB. */
 int llmq_wq_experts_supported(int n_tokens, int top_k, int n_experts, int hidden, int intermediate);
 size_t llmq_wq_experts_workspace_bytes(int n_tokens, int top_k, int n_experts, int hidden, int intermediate);
+/* Rows of a tile that the call takes (0: not supported): for timing and tests; the result does not depend on it. */
+int llmq_wq_experts_tile_rows(int n_tokens, int top_k, int n_experts, int hidden, int intermediate, int wformat);
 int llmq_wq_experts(const void* x, const int64_t* top_k_index, const void* top_k_weights, const void* gate_up,
                     const float* gate_up_scale, const void* down, const float* down_scale, void* out,
                     void* workspace, size_t workspace_bytes, int n_tokens, int top_k, int n_experts, int hidden,

@@ -239,23 +239,31 @@ int run_shape(const TileArgs& gate_up, const TileArgs& down, int max_row_tiles, 
   return launch_grouped<T, BITS, kEpiStore, S>(down, max_row_tiles, stream);
 }
 
-// Rows of a tile: 32 or 64. The host does not know the experts' counts; an expert's last tile is half full on average, so
-// that there are about rows / height + E / 2 row tiles (no fewer than experts with rows), each with I / 128 column tiles in the
-// gate|up launch, on 512 places at once (int8: 256, one a CU). A launch takes a round at least, and half of one more than the tiles fill on
-// average; a round of 64-row tiles takes 1.4 of 32-row ones. Measured, both heights, 96 problems each of int4 and int8 (bf16, a router
-// that prefers some experts to others; 8 to 128 experts, 4 to 200 rows an expert), us a call, 32 / 64 rows: 64 experts of 2048 x
-// 1024 int4 at 10 rows an expert 65 / 74, 30: 86 / 96, 37.5: 96 / 100, 45: 103 / 103, 75: 143 / 130, 200: 285 / 243; int8 30: 119 /
-// 134, 37.5: 140 / 136, 52: 169 / 145; eight of 2048 x 4096 int4 at 45: 67 / 79, 64: 78 / 85, 90: 90 / 88, 130: 118 / 106, int8 37.5: 90
-// / 104, 45: 94 / 103, 52: 109 / 104, 130: 187 / 136; eight of 4096 x 14336 int4 30: 264 / 286, 37.5: 324 / 298; sixteen of 4096 x 6400
-// int4 30: 247 / 257, 37.5: 282 / 260. A line at 40 rows an expert was up to 19 % behind (eight of 2048 x 4096).
-int tile_rows_for(int rows, int E, int I, bool int4) {
-  const double hit = rows < E ? rows : E, places = int4 ? 512.0 : 256.0;
-  auto cost = [&](int height) {
-    const double row_tiles = static_cast<double>(rows) / height + 0.5 * E;
-    const double rounds = (row_tiles > hit ? row_tiles : hit) * (I / kGroup) / places + 0.5;
-    return rounds > 1.0 ? rounds : 1.0;
+// Rows of a tile: 32 or 64. The host does not know the experts' counts; an expert's last tile is about half full, so that
+// there are some rows / height + 0.45 E row tiles (no fewer than experts with rows), each with I / 128 column tiles of H / 128
+// groups in the gate|up launch and H / 256 of I / 128 in the down launch. A launch's time goes by rounds of one workgroup a CU: one
+// that does not fill the chip takes part of a round, one that is just begun a quarter; a round of 64-row tiles takes 1.5 (int8
+// 1.46) of 32-row ones. Measured, both heights, 968 problems in graphs (bf16, routers without and with favourites; 4 to 128 experts, H
+// from 0.3 I to 32 I, 4 to 200 rows an expert), us a call, 32 / 64 rows: 64 experts of 2048 x 1024 int4 at 10 rows an expert
+// 65 / 74, 30: 86 / 96, 37.5: 96 / 100, 75: 143 / 130, 200: 285 / 243; int8 30: 119 / 134, 37.5: 140 / 136, 52: 169 / 145; eight of
+// 2048 x 4096 int4 at 45: 67 / 79, 64: 78 / 85, 130: 118 / 106, int8 45: 94 / 103, 52: 109 / 104, 130: 187 / 136; eight of 4096 x
+// 14336 int8 37.5: 489 / 395; forty of 1024 x 512 int8 30: 32 / 36, 45: 47 / 37, 75: 50 / 59; 64 of 7168 x 256 int8 45: 158 / 164,
+// 64: 228 / 179. Of the 448 that the figures were fitted to, the height taken is 0.3 % (int8 0.6) behind the better one on average,
+// 16 % (13) at worst (sixteen of 6144 x 1024 int4, 52: 92 / 106; 32 of 2048 x 2048 int8, 16: 117 / 104); of the 520 others 0.7
+// (1.1) and 16 % (35, a round begun by a few tiles more than were reckoned with). By the gate|up launch's rounds alone 0.9 (1.4) and 15 %
+// (30), 1.3 (2.4) and 16 % (40); by a line at 40 rows an expert 2.9 (2.3) and 22 % (30), 2.6 (3.6) and 40 % (47).
+int tile_rows_for(int rows, int E, int H, int I, bool int4) {
+  const double hit = rows < E ? rows : E, least = int4 ? 0.5 : 0.25;
+  auto rounds = [&](double tiles) {
+    const double all = tiles / 256.0, whole = static_cast<int64_t>(all);
+    if (all <= 1.0) return least + (1.0 - least) * all;
+    return all > whole ? whole + 0.25 + 0.75 * (all - whole) : whole;
   };
-  return 1.4 * cost(64) < cost(32) ? 64 : 32;
+  auto cost = [&](int height) {
+    const double by_rows = static_cast<double>(rows) / height + 0.45 * E, row_tiles = by_rows > hit ? by_rows : hit;
+    return rounds(row_tiles * (I / kGroup)) * (H / kGroup) + rounds(row_tiles * ((H + 255) / 256)) * (I / kGroup);
+  };
+  return (int4 ? 1.5 : 1.46) * cost(64) < cost(32) ? 64 : 32;
 }
 
 template <typename T, int BITS>
@@ -263,7 +271,7 @@ int run(const void* x, const int64_t* index, const void* weights, const void* q1
         const float* s2, void* out, uint8_t* ws, int n_tokens, int top_k, int E, int H, int I, hipStream_t stream) {
   const Layout l = layout_for(n_tokens, top_k, E, H, I);
   const int rows = n_tokens * top_k;
-  const int tile_rows = tile_rows_for(rows, E, I, BITS == 4);
+  const int tile_rows = tile_rows_for(rows, E, H, I, BITS == 4);
   const PlanArgs p{index, rows, E, top_k, tile_rows, reinterpret_cast<int4*>(ws + l.tiles),
                    reinterpret_cast<int*>(ws + l.n_tiles), reinterpret_cast<int*>(ws + l.row_source),
                    reinterpret_cast<int*>(ws + l.sorted)};
@@ -317,6 +325,11 @@ extern "C" int llmq_wq_experts_supported(int n_tokens, int top_k, int n_experts,
 extern "C" size_t llmq_wq_experts_workspace_bytes(int n_tokens, int top_k, int n_experts, int hidden, int intermediate) {
   if (!llmq_wq_experts_supported(n_tokens, top_k, n_experts, hidden, intermediate)) return 0;
   return layout_for(n_tokens, top_k, n_experts, hidden, intermediate).total;
+}
+
+extern "C" int llmq_wq_experts_tile_rows(int n_tokens, int top_k, int n_experts, int hidden, int intermediate, int wformat) {
+  if (!llmq_wq_experts_supported(n_tokens, top_k, n_experts, hidden, intermediate)) return 0;
+  return tile_rows_for(n_tokens * top_k, n_experts, hidden, intermediate, wformat == LLMQ_W_INT4_PACKED);
 }
 
 extern "C" int llmq_wq_experts(const void* x, const int64_t* top_k_index, const void* top_k_weights,

@@ -99,6 +99,8 @@ def load_capi() -> ctypes.CDLL:
     lib.llmq_wq_experts_direct.restype = c_int
     lib.llmq_wq_experts_supported.argtypes = [c_int] * 5
     lib.llmq_wq_experts_supported.restype = c_int
+    lib.llmq_wq_experts_tile_rows.argtypes = [c_int] * 6
+    lib.llmq_wq_experts_tile_rows.restype = c_int
     lib.llmq_wq_experts_workspace_bytes.argtypes = [c_int] * 5
     lib.llmq_wq_experts_workspace_bytes.restype = ctypes.c_size_t
     lib.llmq_wq_experts.argtypes = [c_p] * 9 + [ctypes.c_size_t] + [c_int] * 7 + [c_p]

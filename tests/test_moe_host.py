@@ -159,3 +159,29 @@ def test_which_prompts_the_grouped_gemms_take(experts, hidden, inter, packed, ro
 
     module = SimpleNamespace(num_experts=experts, hidden_dim=hidden, intermediate_dim=inter, _packed=packed)
     assert KernelQuantExperts._grouped_pays(module, rows) is grouped
+
+
+@pytest.mark.parametrize("experts,top_k,hidden,inter,bits,tokens,height", [
+    (40, 8, 1024, 512, 8, 225, 64),    # 47 us a call with 32-row tiles, 37 with 64 (two rounds of either launch against one)
+    (64, 8, 7168, 256, 8, 416, 64),    # 218, 170: the down launch has fourteen times the column tiles of gate|up
+    (16, 4, 6144, 1024, 8, 256, 64),   # 174, 139
+    (8, 2, 4096, 1024, 4, 800, 64),    # 91, 79
+    (64, 8, 2048, 1024, 4, 300, 32),   # 96, 100
+    (64, 8, 2048, 1024, 4, 600, 64),   # 142, 130
+    (8, 2, 2048, 4096, 4, 180, 32),    # 67, 79
+    (8, 2, 2048, 4096, 8, 180, 32),    # 94, 103
+    (8, 2, 4096, 14336, 8, 150, 64),   # 489, 395
+    (2, 1, 128, 128, 4, 9, 32),
+])
+def test_the_faster_height_of_the_row_tiles(experts, top_k, hidden, inter, bits, tokens, height):
+    """Where one height was measured to be the faster by 4 % and more, on either side of the line."""
+    from llmquant.hip.build import load_capi
+
+    assert load_capi().llmq_wq_experts_tile_rows(tokens, top_k, experts, hidden, inter, bits) == height
+
+
+def test_the_row_tiles_of_calls_that_are_not_taken():
+    from llmquant.hip.build import load_capi
+
+    assert load_capi().llmq_wq_experts_tile_rows(8, 2, 4, 100, 128, 4) == 0
+    assert load_capi().llmq_wq_experts_tile_rows(0, 2, 4, 128, 128, 8) == 0
