@@ -328,13 +328,19 @@ def test_direct_launches_equal_the_planned_ones(ext, bits, dtype, tokens, hidden
             assert torch.equal(quant(x, ids, weights), quant._forward_fused(x, ids, weights))
 
 
+def tile_rows(bits, tokens, hidden, inter, experts, top_k):
+    from llmquant.hip.build import load_capi
+
+    return load_capi().llmq_wq_experts_tile_rows(tokens, top_k, experts, hidden, inter, 4 if bits == "int4" else 8)
+
+
 @pytest.mark.parametrize("bits,dtype", [("int4", torch.bfloat16), ("int8", torch.bfloat16), ("int4", torch.float16),
                                         ("int8", torch.float16)])
 @pytest.mark.parametrize("tokens,hidden,inter,experts,top_k,skew", [
     (9, 128, 128, 4, 2, False),      # one group a row, one column tile, runs of a few rows
     (33, 384, 256, 3, 1, True),      # a run of 33 rows: one more than a row tile; columns that fill half a tile
-    (64, 512, 384, 8, 8, False),     # every expert takes every token: two full 32-row tiles each
-    (150, 512, 512, 2, 2, True),     # 150 rows an expert: 64-row tiles, the last of 22
+    (64, 512, 384, 8, 8, False),     # every expert takes every token: two full tiles each
+    (150, 512, 512, 2, 2, True),     # 150 rows an expert: five tiles, the last of 22
     (40, 2048, 1024, 64, 8, False),  # experts that nobody picked among many
 ])
 def test_grouped_gemms_against_real_mode(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew):
@@ -376,22 +382,26 @@ def test_a_prompt_past_what_the_plan_and_the_combination_hold_at_once(ext, token
 @pytest.mark.parametrize("bits,dtype", [("int4", torch.bfloat16), ("int8", torch.bfloat16), ("int4", torch.float16)])
 @pytest.mark.parametrize("tokens,hidden,inter,experts,top_k,skew", [
     (20, 640, 768, 4, 2, False),     # five and six groups: the second run of four groups' scales holds one and two
-    (90, 896, 1152, 2, 2, False),    # seven and nine, 64-row tiles
-    (90, 1536, 1920, 2, 2, False),   # twelve and fifteen: these tiles' two buffers, each used twice
+    (90, 896, 1152, 2, 2, False),    # seven and nine
+    (90, 1536, 1920, 2, 2, False),   # twelve and fifteen: three and almost four whole runs
 ])
 def test_scales_of_a_last_run_of_groups(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew):
+    assert tile_rows(bits, tokens, hidden, inter, experts, top_k) == 32
     test_grouped_gemms_against_real_mode(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew)
 
 
-@pytest.mark.parametrize("bits,dtype", [("int4", torch.bfloat16), ("int8", torch.bfloat16), ("int4", torch.float16)])
-@pytest.mark.parametrize("tokens,hidden,inter,experts,top_k,skew", [
-    (601, 896, 2176, 2, 2, False),   # nine 64-row tiles an expert and one of 25; seven and seventeen groups
-    (400, 1536, 4736, 2, 2, True),   # six and one of 16; twelve and thirty-seven
-    (333, 640, 4096, 3, 2, True),    # the first expert takes every token, the others what is left
+@pytest.mark.parametrize("bits,dtype", [("int4", torch.bfloat16), ("int8", torch.bfloat16), ("int4", torch.float16),
+                                        ("int8", torch.float16)])
+@pytest.mark.parametrize("tokens,hidden,inter,experts,top_k,skew,heights", [
+    (601, 896, 2176, 2, 2, False, (64, 64)),   # nine 64-row tiles an expert and one of 25; seven and seventeen groups
+    (400, 1536, 4736, 2, 2, True, (64, 64)),   # six and one of 16; twelve and thirty-seven
+    (333, 640, 4096, 3, 2, True, (32, 64)),    # the first expert takes every token, the others what is left
+    (190, 1024, 512, 40, 8, False, (64, 64)),  # 38 rows an expert: one or two tiles each, most of them not full
+    (150, 768, 1664, 3, 2, False, (32, 32)),   # about a hundred rows each: four 32-row tiles; six and thirteen groups
 ])
-def test_prompts_whose_rounds_take_the_higher_tiles(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew):
-    """Shapes that fill the chip with 64-row tiles (where 1.4 rounds of them are fewer than those of 32-row ones), ragged in
-    rows and in groups."""
+def test_prompts_by_the_height_of_their_row_tiles(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew, heights):
+    """Shapes on both sides of the line between the heights, ragged in rows and in groups (heights: int4, int8)."""
+    assert tile_rows(bits, tokens, hidden, inter, experts, top_k) == heights[bits == "int8"]
     test_grouped_gemms_against_real_mode(ext, bits, dtype, tokens, hidden, inter, experts, top_k, skew)
 
 
