@@ -201,7 +201,8 @@ def test_rope_and_append_in_one_launch_equal_the_two_launches(ext, dtype, bits, 
 @pytest.mark.parametrize("tokens", [767, 768, 1031])
 def test_rope_and_append_of_rows_that_start_anywhere(ext, dtype, bits, head_dim, tokens):
     """Rows that are no whole packets (an odd row stride, a tensor that starts one element in) against the same values in
-    packets (taken from 6144 head vectors on): the same bits, and tokens past the cache's end are left out on both ways."""
+    packets (taken from 6144 head vectors on): the same bits, the sign of zeros among them, NaN in the same places, and
+    tokens past the cache's end are left out on both ways."""
     from llmquant.runtime.kv_cache import KernelQuantCache
 
     q_heads, kv_heads, max_len = 4, 2, 760
@@ -209,6 +210,10 @@ def test_rope_and_append_of_rows_that_start_anywhere(ext, dtype, bits, head_dim,
     width = (q_heads + 2 * kv_heads) * head_dim
     loose = (torch.randn(tokens, width + 3, device="cuda") * 2.0).to(dtype)
     loose[5, 1:] = 0.0
+    loose[6, 1:] = -0.0
+    loose[7, 1::7] = -0.0
+    loose[8, 1::9], loose[9, 2::11] = float("inf"), float("-inf")
+    loose[10, 1::13] = loose[11, 1:] = float("nan")
     q_width, kv_width = q_heads * head_dim, kv_heads * head_dim
     emb = torch.rand(tokens, head_dim, device="cuda") * 6.28
     cos, sin = emb.cos().to(dtype), emb.sin().to(dtype)
@@ -220,8 +225,13 @@ def test_rope_and_append_of_rows_that_start_anywhere(ext, dtype, bits, head_dim,
                                  cache.position, q_heads, True)
         results.append([out[0], out[1][:, :max_len], out[2][:, :max_len], cache.k_codes, cache.v_codes, cache.k_scale,
                         cache.v_scale])
+    as_bits = {1: torch.uint8, 2: torch.int16, 4: torch.int32}
     for a, b in zip(*results):
-        assert torch.equal(a, b)
+        both = [t.contiguous() for t in (a, b)]
+        if a.is_floating_point():
+            assert torch.equal(both[0].isnan(), both[1].isnan())
+            both = [torch.nan_to_num(t, nan=0.0, posinf=float("inf"), neginf=float("-inf")) for t in both]
+        assert torch.equal(*[t.view(as_bits[t.element_size()]) for t in both])
 
 
 def test_rope_and_append_argument_checks(ext):
