@@ -330,6 +330,42 @@ template <> struct Dealt<1> {
   static constexpr int kLateFolds = 16;
 };
 
+// Whether the tables above deal out a group of HALVES x MT blocks of HS steps: every word and fold once, in order within a
+// k-step, no more of them a step than the loop has room for; a word behind the last multiplication that reads the group's before
+// and ahead of its own first, with its codes there (asked for behind the last block's first step, two steps before they
+// are used) and not yet overwritten; a fold behind its tile's last multiplication and ahead of the tile's first of the next group.
+template <int HALVES, int MT, int HS> constexpr bool dealt_in_time() {
+  using D = Dealt<HALVES>;
+  constexpr int kAll = HALVES * MT * HS, kWords = 4 * HALVES * HS, kFolds = 16 * MT, kCodes = (HALVES * MT - 1) * HS;
+  int word_at[kWords] = {}, fold_at[kFolds] = {};   // (step + 1; 0: none yet)
+  for (int s = 0; s < kAll; ++s) {
+    const Run words = D::words(s), folds = D::folds(s);
+    if (words.count > D::kMostWords || folds.count > D::kMostFolds) return false;
+    for (int w = words.first; w < words.first + words.count; ++w) {
+      if (w >= kWords || word_at[w] != 0) return false;
+      word_at[w] = s + 1;
+    }
+    for (int f = folds.first; f < folds.first + folds.count; ++f) {
+      if (f >= kFolds || fold_at[f] != 0) return false;
+      fold_at[f] = s + 1;
+    }
+  }
+  int before = -kAll;
+  for (int w = 0; w < kWords; ++w) {
+    const int s = word_at[w] - 1, block = w / 4 / HS * MT, j = w / 4 % HS;
+    const bool early = w < D::kEarlyWords;   // (in the steps of the group before)
+    if (s < 0 || (early ? s < kCodes + 2 : s >= kCodes)) return false;
+    const int when = early ? s - kAll : s, first = block * HS + j, last = (block + MT - 1) * HS + j;
+    if (when >= first || when < last - kAll || (w % 4 != 0 && when < before)) return false;
+    before = when;
+  }
+  for (int f = 0; f < kFolds; ++f) {
+    const int s = fold_at[f] - 1, tile = f / 16, done = ((HALVES - 1) * MT + tile) * HS + HS - 1;
+    if (s < 0 || (f >= D::kLateFolds ? s >= tile * HS : s <= done)) return false;
+  }
+  return true;
+}
+
 template <typename T> __device__ __forceinline__ v16f mfma(const u32x4& a, const u32x4& b, const v16f& c) {
   if constexpr (std::is_same<T, bf16_t>::value)
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
@@ -555,6 +591,7 @@ __global__ __launch_bounds__(S::kThreads, GROUPED ? S::kWavesPerSimd : 1) void w
     constexpr int kHalves = kSteps == 8 ? 2 : 1, kHS = kSteps / kHalves;   // k-steps of a block
     constexpr int kBlocks = kHalves * kMT, kLast = kBlocks - 1;
     using Deal = Dealt<kHalves>;
+    static_assert(dealt_in_time<kHalves, kMT, kHS>(), "the conversions and folds of this shape");
     constexpr int kParts = kBlocks == 2 || kStagesN < 3 ? 2 : 4;   // a group's transfers in so many pieces, one a block
     u32x4 fa[2][kHS], rec_op = {0u, 0u, 0u, 0u};
     uint32_t fb[kSteps * 4];   // (words of the converted codes, four a step)
