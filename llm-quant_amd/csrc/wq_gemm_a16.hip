@@ -58,11 +58,11 @@ struct A16Args {
 };
 
 // HELD: the scales come first, all of a workgroup's in one sweep (its weight rows' are one run of memory, whole lines to a
-// load), and wait in LDS. Read group by group, they are a cache line a weight row for four bytes each: of 14336 x 4096 int4,
-// M = 16, 14.4 us, the loads taken out 11.3. Four row tiles, weights rotated through 600 MB, group by group / held, us: int4
-// M = 3 13.0 / 11.5, 16 14.5 / 12.8, 32 17.1 / 16.0, int8 16 18.3 / 18.0. Short rows do not give the sweep in front back: form_of.
-// Of one or two row tiles the workgroups are short (8192 x 2048 int4, M = 16: 6.4 / 6.8, 4096 x 4096 6.6 / 7.5), and with three
-// activation tiles it takes registers that are not there (48 rows: 19.9 / 21.9).
+// load), and wait in LDS. Read group by group, they are a cache line a weight row for four bytes each. Four row tiles, weights
+// rotated through 600 MB, in graphs, group by group / held, us: 14336 x 4096 int4 M = 3 12.1 / 9.7, 16 13.6 / 11.1, 32 16.2 / 13.6,
+// int8 16 17.6 / 15.7. Short rows do not give the sweep in front back: form_of. Of two row tiles 14336 x 4096 int4, M = 16 14.2 /
+// 12.1, but 8192 x 2048 6.0 / 6.1; of one 4096 x 4096 6.7 / 6.8: neither is built. Nor is it for three activation tiles: with an
+// earlier loop they had no registers left for it (48 rows: 19.9 / 21.9); with this one they have (18.5 / 16.4).
 __host__ __device__ constexpr int scale_pitch(int G) { return G | 1; }   // (odd: sixteen rows in sixteen banks)
 
 // operands of s_waitcnt: none of the wave's vector loads / LDS reads outstanding, the other counters as they are
@@ -387,23 +387,24 @@ struct Form {
 };
 // Row tiles of a workgroup share the activation rows a wave loads: those come from L2 once per workgroup, and 16
 // weight rows a workgroup make that traffic four times the codes' at M = 16. Two tiles as long as a workgroup per CU
-// and more is left (14336 x 4096 int4 bf16, one / two tiles, us: M = 16 14.6 / 13.0, 32 19.6 / 17.8, 48 29.4 / 21.2; 4096
-// x 4096, M = 64: 10.2 / 13.7).
-// Four tiles (one workgroup a CU) by how full their last round of 256 workgroups is. Measured, two / four tiles, us,
-// weights rotated through 600 MB, bf16; fp16 is within 3 % of it, also where its 33 to 48 rows against int4 spill two
-// registers (14336 x 4096, M = 48: 24.7 / 19.9):
-//  17 rows and more, K = 4096: 192 workgroups int4 M = 17 / 32 / 48: 17.3 / 14.8, 20.7 / 16.4, 24.3 / 19.1, int8 32: 24.3 /
-//  19.8; 256: 18.0 / 15.2, 21.3 / 17.0, 25.2 / 19.8, int8 26.4 / 21.2; but 260 to 384, a second round at most half full:
-//  288 24.9 / 26.8, 29.8 / 30.0, 34.9 / 35.1, int8 17 29.8 / 33.3; 384 26.9 / 27.9, 30.8 / 30.5, int8 17 33.9 / 34.4; 416
-//  32.9 / 27.7, 39.1 / 30.8, int8 39.5 / 35.1; 528, where the third is nearly empty, int4 M = 32 8 % faster, int8 4 %.
-//  Below 192: 8192 x 2048 M = 32 6.7 / 9.1.
-//  Up to 16 rows there is less to share: one round only (288: M = 3 16.7 / 22.1, 16 20.3 / 24.7; 448: 21.9 / 23.2, 26.3 /
-//  25.9), rows of 32 groups (with the scales held: 256 workgroups, K = 2048, M = 3 / 16: 8.1 / 8.5, 9.3 / 8.9; K = 4096
-//  14.1 / 12.3 and 15.5 / 13.3; K = 8192, 16: 26.0 / 22.9), and for int8 codes up to eight rows, the fuller the round the longer
-//  the rows that it takes (in graphs; 192: 32 groups M = 3 / 8 15.0 / 14.2, 15.8 / 14.5; 224: 16.1 / 16.1, 16.7 / 16.1; 240: 32
-//  groups 16.2 / 17.1, 17.0 / 17.2, 48 groups 23.6 / 22.2, 25.4 / 22.3; 256: 64 groups M = 3 / 5 30.3 / 32.0, 30.8 / 32.0, 96
-//  groups 45.3 / 46.3, 46.9 / 45.7, 255 groups M = 3 147.7 / 139.8).
-// Four tiles against 64 rows, and int8 codes against 48, are more registers than a wave has (spills: 41 us against 26).
+// and more is left (in graphs, weights rotated through 600 MB, bf16, us, one / two tiles: 14336 x 4096 int4 M = 16 17.8 / 14.2, 32
+// 24.2 / 18.2, 48 33.9 / 23.5; 4096 x 4096, M = 64: 12.1 / 14.4).
+// Four tiles (one workgroup a CU) by how full their last round of 256 workgroups is. The lines are those of an earlier loop;
+// measured with the present one, as above, two tiles / four / four with the scales held (fp16 within 3 %):
+//  17 rows and more, K = 4096: 192 workgroups int4 M = 17 / 32 / 48: 15.1 / 14.5 / 12.1, 17.9 / 15.9 / 13.4, 23.0 / 18.1 / 16.1, int8
+//  32: 23.8 / 19.9 / 17.5; 256: 15.0 / 14.6 / 12.3, 17.8 / 16.1 / 13.6, 23.2 / 18.4 / 16.3, int8 25.9 / 20.9 / 19.4; two for 260 to
+//  384, a second round at most half full: 288 20.2 / 26.0 / 21.3, 24.7 / 28.9 / 23.9, 32.9 / 33.0 / 28.9, int8 17 28.8 / 33.3 / 29.5;
+//  384 21.5 / 26.6 / 21.9, 25.6 / 29.5 / 24.6, int8 17 32.2 / 34.3 / 31.4; 416 25.6 / 26.9 / 22.2, 31.8 / 29.8 / 24.9, int8 32 45.2 /
+//  38.1 / 34.0; 528 int4 32 38.6 / 42.2 / 34.9, int8 56.0 / 54.8 / 47.6. Below 192: 8192 x 2048 M = 32 7.4 / 9.5 (four).
+//  Up to 16 rows there is less to share: one round only (288, M = 3 / 16: 15.2 / 19.9 / 14.4, 19.2 / 23.0 / 17.6; 448: 20.2 / 20.5 /
+//  15.1, 24.9 / 23.7 / 18.6), rows of 32 groups (256 workgroups, K = 2048: 7.5 / 8.1 / 7.3, 8.6 / 8.5 / 7.8; K = 4096 11.3 / 12.0 /
+//  9.7, 14.0 / 13.4 / 11.0; K = 8192, 16: 26.8 / 25.2 / 19.6), and for int8 codes up to eight rows, the fuller the round the longer
+//  the rows that it takes (two / held; 192: 32 groups M = 3 / 8 15.9 / 13.3, 16.5 / 13.7; 224: 17.0 / 14.6, 17.0 / 14.5; 240: 32
+//  groups 17.1 / 15.4, 17.1 / 15.4, 48 groups 22.2 / 19.2, 24.5 / 19.7; 256: 32 groups M = 3 17.0 / 16.8, 64 groups M = 3 / 5 30.1 /
+//  29.9, 30.6 / 30.0, 96 groups 44.9 / 43.7, 46.3 / 43.6, 255 groups M = 3 143 / 134).
+//  With the scales held four tiles are ahead of where the lines lie, by most at 288 and 448 workgroups of up to 16 rows and at
+//  33 to 48 rows; two are at 2004 workgroups of K = 2048 int4, M = 17 (50.7 / 52.4).
+// Four tiles against 64 rows, and int8 codes against 48, are more registers than a wave has (spills: 39, int8 50 and 3).
 constexpr Form form_of(int bits, int rows, int N, int G) {
   const int quads = (N + 4 * kTileN - 1) / (4 * kTileN), mt = (rows + kTileM - 1) / kTileM;
   const bool int4 = bits == 4;
@@ -414,12 +415,11 @@ constexpr Form form_of(int bits, int rows, int N, int G) {
   const bool more_rows = (mt == 2 || (mt == 3 && int4)) && (quads <= 256 || quads > 384);
   if (quads >= 192 && offsets32 && (few_rows || more_rows)) {
     // The scales of rows that are long enough to pay for the sweep are held, and of somewhat shorter ones where several rounds of
-    // workgroups overlap it and the waves have equal shares. Group by group / held, us, in graphs, M = 17 / 32: int4, 256
-    // workgroups, K = 512 7.8 / 8.4, 8.2 / 8.7; 2048 9.9 / 10.3, 11.3 / 11.5; 2560 11.2 / 11.3, 12.3 / 12.4; 3584 1 and 3 % the
-    // faster held, 4096 4 and 7 %; 2004 workgroups, K = 2048 68.1 / 67.1, 71.9 / 71.1; int8, 256 workgroups, K = 512 7.5 / 8.5, 7.8
-    // / 8.8; 2048 even; 2560 14.9 / 15.6, 15.8 / 16.4 (fp16 13.6 / 15.5, 14.7 / 16.3); 4096 19.2 / 20.1 (21.5 / 21.0 by where the
-    // weights lie), 21.2 / 21.3, M = 9 and 16 1 to 3 % the slower held; 192 and 448 of them 3 to 4 % the faster; 2004, K = 2048
-    // 79.3 / 76.4, 85.4 / 81.1.
+    // workgroups overlap it and the waves have equal shares: with an earlier loop the sweep cost shorter ones up to 16 %. With the
+    // present one, group by group / held, us, in graphs, M = 17 / 32, int4, 256 workgroups: K = 512 7.1 / 7.0, 7.4 / 7.4; 2048 9.3 /
+    // 8.5, 10.2 / 9.4; 2560 10.9 / 9.5, 11.5 / 11.0; 3584 13.5 / 11.6, 14.5 / 13.1; 4096 14.6 / 12.3, 16.1 / 13.6; 2004 workgroups, K =
+    // 2048 59.8 / 52.4, 65.5 / 58.7; int8, 256 workgroups, K = 512 7.9 / 7.8, 8.2 / 8.2; 2048 11.7 / 10.5, 11.9 / 11.4; 2560 13.4 / 12.9,
+    // 14.4 / 14.0 (fp16 15.2 / 13.4, 14.7 / 14.6); 4096 19.3 / 18.5, 20.9 / 19.4; 2004, K = 2048 76.5 / 68.8, 82.2 / 75.2.
     const bool long_rows = int4 ? mt == 1 || G >= 20 : G >= (quads > 240 && quads <= 256 ? 40 : 32);
     const bool pays = long_rows || (G >= 16 && G % kMaxWaves == 0 && quads >= (int4 ? 385 : 1024));
     return {4, mt <= 2 && pays && held_bytes(4, G) <= kMostScales};
@@ -434,7 +434,7 @@ int launch_typed(const void* x, const void* qw, const float* ws, void* out, int 
   int wk = G < kMaxWaves ? G : kMaxWaves;
   // rows of few groups: two groups per wave at least
   if (G >= 4 && wk * 2 > G) wk = G / 2;
-  // (Sixteen waves for few row tiles of long rows, down_proj, measured no faster than eight.)
+  // (Sixteen waves for few row tiles of long rows, down_proj, measured no faster than eight, with an earlier loop.)
   // (a slab's offsets have 32 bits)
   const int64_t fit = (int64_t{1} << 32) / (K * 2);
   const int slab = fit >= kSlabRows ? kSlabRows : (fit > 0 ? static_cast<int>(fit) : 1);

@@ -22,12 +22,13 @@
 // What bounds it: issue, and power. Per group a wave issues 36 multiplications of 32 cycles (float16 32), 128 to 160 vector
 // instructions of conversion and folding, 39 LDS reads, and the two waves of a SIMD share one matrix core: 2300 cycles if it never
 // waited, 3100 measured (float16 3020), 224 workgroups. What counts is how evenly the rest lies between the multiplications: a
-// step that carries more than about five vector instructions is longer than its multiplication, whichever wave it is (a
-// multiplication holds the issue slot for 12 cycles, a vector instruction 4). Folds and conversions eight to sixteen a step and
-// none elsewhere: 3316 (3190). Without folds 2460, without conversions 3100 (float16 2730), without transfers 2990 at a clock
-// 10 to 17 % higher: on random codes the chip holds 1.6 to 1.9 GHz under this loop, on zeros 2.2, so that a cycle saved is half
-// a cycle's time. Launches of 512 x 14336 x 4096 int4 us, the lumped loop / this: bf16 with its preparation 77.7 / 75.4, fp16
-// 68.8 / 66.6; 333 x 4096 x 14336 fp16 63.6 / 61.0; 36 problems of both widths 2 % in the middle, 0 to 6. Launches of few narrow
+// step that carries more than six vector instructions is longer than its multiplication (independent multiplications on two
+// waves a SIMD, cycles each with 0 / 4 / 6 / 8 / 12 / 16 vector instructions behind it: 33 / 35 / 35 / 44 / 56 / 67). Folds and
+// conversions eight to sixteen a step and none elsewhere: 3316 (3190). Without folds 2460, without conversions 3100 (float16 2730),
+// without transfers 2990 at a clock 10 to 17 % higher: on random codes the chip holds 1.6 to 1.9 GHz under this loop, on zeros 2.2,
+// so that a cycle saved is half a cycle's time. Launches of 512 x 14336 x 4096 int4 us, the lumped loop / this, in turn on one
+// card: bf16 with its preparation 77.7 / 75.4 (another card 72.5), fp16 68.8 / 66.6; 333 x 4096 x 14336 fp16 63.6 / 61.0 (another
+// 56.2); 36 problems of both widths 2 % in the middle, 0 to 6. Launches of few narrow
 // tiles on short rows pay 0.1 to 0.2 us for the result's way through LDS.
 //
 // Codes become bf16 without a conversion instruction: a nibble n = code + 8 placed in the mantissa of

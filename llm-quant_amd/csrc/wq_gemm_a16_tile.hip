@@ -99,10 +99,10 @@ Plan plan_for(int M, int N, int G, bool narrow = false) {
 // part (first transfers from memory, the store) plus a time per group of the reduction axis (wide 8 + 1.93 / 2.1 a
 // group for int4 / int8, narrow 6 + 0.75 / 1.0), and where the axis is cut the partial tiles' way through memory
 // and the second launch (3 us + 8 bytes per partial value at 9 TB/s: most of it overlaps the tiles). The figures are of
-// the kernel whose loop went a k-step at a time; the present one is faster and they were not fitted again: over 442
-// problems (72 to 2048 rows, weights of 512 to 28672 rows of 16 to 112 groups) the cheaper plan's estimate with the
-// preparation is 0.85 to 1.41 times the measured launch, 1.10 in the middle, half of them within a tenth, 92 of 100 within a
-// fifth.
+// the kernel whose loop went a k-step at a time; the present one is faster and they were not fitted again: over 420
+// problems (72 to 1024 rows, weights of 512 to 28672 rows of 16 to 112 groups) the cheaper plan's estimate with the
+// preparation is 0.84 to 1.39 times the measured launch, 1.05 in the middle, half of them 1.00 to 1.11; the other width would
+// be faster by 0.3 % on average.
 double plan_cost(const Plan& p, int M, int N, bool narrow, bool int4) {
   const double fixed = narrow ? 6.0 : 8.0;
   const double per_group = narrow ? (int4 ? 0.75 : 1.0) : (int4 ? 1.93 : 2.1);

@@ -31,7 +31,7 @@ FUSED_GEMM_MAX_ROWS = 64
 FUSED_GEMM_WHOLE_ROWS = FUSED_GEMM_MAX_ROWS
 #: ... and from this many rows on it is also faster than the GEMV kernel, which multiplies its rows
 #: as int8 digit planes and slows down with each row (14336 x 4096 int4, graph replay: GEMV 9.6 /
-#: 13.0 / 14.8 / 21.0 us for 1-4 rows, the fused GEMM 13.4-14.3 us for any of them)
+#: 13.1 / 14.9 / 21.0 us for 1-4 rows, the fused GEMM 9.2-9.4 us for any of them; two rows stay with the GEMV)
 FUSED_GEMM_MIN_ROWS = 3
 FUSED_GEMM_SPLIT_GROUPS = 1 << 30   # (no row is long enough for the split form to win)
 
@@ -60,10 +60,10 @@ def _tile_plan_cost(rows: int, out_features: int, groups: int, narrow: bool, int
 
 def tiled_gemm_cost(rows: int, out_features: int, groups: int, bits: int = 8, prepared: bool = False) -> float:
     """Estimated microseconds of llmq_wq_gemm_a16_tile, from the figures that the kernel's own plan has (fitted to an earlier
-    main loop: 0.85 to 1.41 times the measured launch over 442 problems, 1.10 in the middle; of the 364 of them up to 1024
-    rows the branch that is then chosen is more than 5 % behind the fastest in 38, more than 10 % in 17, most of all 1024 x 512
-    x 2048, 19.0 us against 14.5 for dequantize + matmul, and 72 x 8192 x 2048 int4, 18.8 against 14.4 for the fused GEMM for a
-    few dozen rows): rounds of 256 workgroups, each a fixed part plus a time per group, the partial sums'
+    main loop: 0.84 to 1.39 times the measured launch over 420 problems of 72 to 1024 rows, 1.05 in the middle; the branch that
+    is then chosen is 2.5 % behind the fastest on average, more than 5 % in 70 of them, more than 10 % in 35, most of all 1024
+    x 512 x 2048, 19.6 us against 13.5 for dequantize + matmul, and 72 x 8192 x 2048 int4, 18.0 against 13.9 for the fused GEMM
+    for a few dozen rows): rounds of 256 workgroups, each a fixed part plus a time per group, the partial sums'
     way through memory where the reduction axis is cut, and 3.5 us for the activation's preparation unless the rows
     arrive prepared (llmq_add_rmsnorm_prepared, the gate|up epilogue). (float16 rows are read as they lie; the estimate
     does not tell the types apart, which leaves them that much in hand.)"""
@@ -85,23 +85,25 @@ def tiled_gemm_pays(rows: int, out_features: int, groups: int, bits: int = 8, pr
     """Whether the tiled fused GEMM is the branch for this many activation rows. Up to 128 rows: wide or long
     weights, and mid-sized ones (the fused GEMM for a few dozen rows keeps the narrow short ones). Beyond: where its
     estimated time is within 5 % of dequantize + matmul's (a tie goes to the branch that builds no dense weight).
-    Measured, M x N x K int4, tiled / dense us: 512 x 16384 x 2048 46 / 54, 640 x 16384 x 2048 77 / 59 (320 tiles:
-    a second round), 512 x 28672 x 4096 143 / 164, 640 x 4096 x 14336 102 / 120, 1024 x 14336 x 4096 149 / 122;
-    int8: 512 x 3072 x 2048 24.2 / 24.9, 192 x 3072 x 2048 17.1 / 24.4, 1024 x 3072 x 2048 33.0 / 28.7,
-    136 x 512 x 2048 12.6 / 13.8."""
+    Measured, M x N x K int4, tiled / dense us: 512 x 16384 x 2048 44 / 52, 640 x 16384 x 2048 69 / 59 (320 tiles:
+    a second round), 512 x 28672 x 4096 136 / 158, 640 x 4096 x 14336 93 / 126, 1024 x 14336 x 4096 135 / 119;
+    int8: 512 x 3072 x 2048 22.3 / 23.9, 192 x 3072 x 2048 17.3 / 25.5, 1024 x 3072 x 2048 31.6 / 29.4; behind the line,
+    160 x 512 x 2048 12.5 / 11.5."""
     if not FUSED_GEMM_MAX_ROWS < rows <= TILED_GEMM_MAX_ROWS:
         return False
     if rows <= FUSED_GEMM_SLAB_MAX_ROWS:
-        # one tile of rows on a mid-sized weight (Llama-3-8B's q|k|v, 6144 x 4096 int8, M = 65-128: 24.8-27.1 us
-        # against 32.7-36.0 for dequantize + matmul); smaller weights take the fused GEMM for a few dozen rows twice
+        # one tile of rows on a mid-sized weight (Llama-3-8B's q|k|v, 6144 x 4096 int8, 72 / 128 rows: 24.6 / 26.3 us
+        # against 33.0 / 35.8 for dequantize + matmul); smaller weights take the fused GEMM for a few dozen rows twice.
+        # (8192 x 2048 is on the wrong side since that kernel's loop got faster: int4 72 / 128 rows 18.0 / 20.2, 13.9 / 18.2 there)
         return out_features >= 8192 or groups >= 64 or out_features * groups > FUSED_GEMM_SLAB_MAX_GROUP_ROWS
     return (tiled_gemm_cost(rows, out_features, groups, bits, prepared)
             <= 1.05 * dense_branch_cost(rows, out_features, groups, bits))
 
 
 #: Narrow, short weights (N * groups up to 4096 x 32: q|k|v and o_proj of the 1B and 8B models) keep the fused GEMM up
-#: to this many rows, 64 at a time: two launches of it beat both dequantize + matmul and the tiled GEMM there
-#: (3072 x 2048 int8, M = 128: 14.1 us against 21.7 and 21.2; 4096 x 4096: 24.4 against 32.0 and 27.4).
+#: to this many rows, 64 at a time: two launches of it beat dequantize + matmul, and the tiled GEMM or are level with it (3072 x
+#: 2048 int8, M = 128: 13.6 us against 21.7 and 16.2; 4096 x 4096 int4 20.1 / 31.7 / 20.3, int8 24.3 / 31.6 / 22.6; 1024 x 4096
+#: int4 17.9 / 19.1 / 15.3).
 FUSED_GEMM_SLAB_MAX_ROWS = 128
 FUSED_GEMM_SLAB_MAX_GROUP_ROWS = 4096 * 32
 

@@ -90,7 +90,8 @@ def test_the_tiles_do_not_spill(source):
 
 @needs_hipcc
 def test_forms_of_the_gemm_for_a_few_dozen_rows(tmp_path):
-    """Where one side of a line was measured slower, the other side's form runs: the kernel's own rule, at compile time."""
+    """The lines between the forms, on both sides: the kernel's own rule, at compile time. (They were drawn with an earlier loop;
+    what either side takes with the present one stands at the rule.)"""
     lines = [  # bits, rows, outputs, groups, row tiles, scales held
         (4, 17, 16384, 1, 4, False), (4, 32, 128256, 8, 4, False), (4, 32, 16384, 16, 4, False), (4, 17, 24577, 16, 4, True),
         (4, 32, 32000, 18, 4, False), (4, 17, 16384, 19, 4, False), (4, 17, 16384, 20, 4, True), (4, 33, 16384, 64, 4, False),
